@@ -1,0 +1,105 @@
+"""fp32 products on the fp16 MFMA units (operands as two fp16 parts) against float64.
+
+The parts hold 22 bits of a value scaled by its row's (or output channel's) power of
+two, and the sums are fp32.  Error model of an output element: each of the two operands
+is off by at most 2^-23 of itself plus 2^-39 of its row's largest entry, lo * lo (at most
+2^-22 of the product) is left out, and the fp32 accumulators round 3 K / 8 times (K = 4 d_in
+real terms, in blocks of eight) by 2^-24 of partial sums of random terms.  In the 2-norm that
+stays below (2^-22 + 2^-24 sqrt(3 K / 16)) of the result: 6.6e-7 for d_in = 128, 1.1e-6 for
+512; the bound used is 2e-6.
+"""
+
+import numpy as np
+import pytest
+import torch
+
+from _gpu_helpers import say
+from oracle import dense
+
+pytestmark = pytest.mark.gpu
+
+TOL = 2e-6
+
+
+def _rel(got, ref):
+    got, ref = np.asarray(got, np.float64), np.asarray(ref, np.float64)
+    return float(np.linalg.norm(got - ref) / np.linalg.norm(ref))
+
+
+def _gm(a, b):
+    from yggdrasil_amd import ops
+
+    return ops.geom_matmul(torch.from_numpy(a).cuda(), torch.from_numpy(b).cuda()).cpu().numpy()
+
+
+def _truth(a, b):
+    return np.transpose(dense.linear(np.transpose(b, (1, 0, 2)), a), (1, 0, 2))
+
+
+@pytest.mark.parametrize("M,K,N", [(64, 128, 6400), (65, 129, 6333), (130, 136, 3300), (513, 143, 800), (66, 255, 6300)])
+def test_geom_matmul_sizes(M, K, N):
+    """Sizes from which the split product runs, on and off its tiles (64 x 64, blocks of 8 inputs)."""
+    g = np.random.default_rng(M + K + N)
+    a = (g.standard_normal((M, K, 8)) / np.sqrt(8 * K)).astype(np.float32)
+    b = g.standard_normal((K, N, 8)).astype(np.float32)
+    say(f"split geom_matmul M={M} K={K} N={N}")
+    assert _rel(_gm(a, b), _truth(a, b)) < TOL
+
+
+def test_geom_matmul_scales_and_non_finite():
+    """Rows and channels over 200 binades, zero rows, entries 2^-20 below their row's largest, and rows
+    with an infinity or NaN: those give non-finite rows, and every other row is as without them."""
+    g = np.random.default_rng(4)
+    M, K, N = 70, 130, 6000
+    a = (g.standard_normal((M, K, 8)) / np.sqrt(8 * K)).astype(np.float32)
+    b = g.standard_normal((K, N, 8)).astype(np.float32)
+    a *= np.ldexp(1.0, g.integers(-60, 40, (M, 1, 1))).astype(np.float32)
+    b *= np.ldexp(1.0, g.integers(-60, 40, (1, N, 1))).astype(np.float32)
+    b[:40] *= np.float32(2.0 ** -20)
+    b[:, 17] = 0.0
+    bad = b.copy()
+    bad[3, 100, 2] = np.inf
+    bad[5, 2000, 0] = np.nan
+    say("split geom_matmul scales, non-finite")
+    ref = _truth(a, b)
+    out, out_bad = _gm(a, b), _gm(a, bad)
+    # sqrt(8 K) random terms of the largest size in the row and the channel
+    scale = np.abs(a).max(axis=(1, 2))[:, None] * np.abs(b).max(axis=(0, 2))[None, :] * np.sqrt(8 * K)
+    err = np.linalg.norm(out - ref, axis=2)
+    assert np.isfinite(out).all() and not out[:, 17].any()
+    assert (err <= 1e-6 * scale).all()
+    assert not np.isfinite(out_bad[:, [100, 2000]]).any()
+    keep = np.ones(N, bool)
+    keep[[100, 2000]] = False
+    assert np.array_equal(out_bad[:, keep], out[:, keep])
+
+
+@pytest.mark.parametrize("N,d,F,E,k,act,empty", [(1700, 128, 256, 5, 2, "gelu", False), (3300, 133, 141, 3, 1, "sigmoid", True),
+                                                 (1300, 150, 128, 8, 4, "relu", False)])
+def test_layer(N, d, F, E, k, act, empty):
+    """The fp32 layer with both products split: widths off the blocks of 8, an expert without rows, odd row
+    counts, tokens over many binades, biases and a residual."""
+    import yggdrasil_amd
+
+    g = np.random.default_rng(N + d)
+    x = g.standard_normal((N, d, 8)).astype(np.float32) * np.ldexp(1.0, g.integers(-12, 4, (N, 1, 1))).astype(np.float32)
+    lg = g.standard_normal((N, E)).astype(np.float32)
+    if empty:
+        lg[:, 1] = -30.0
+    wu = (g.standard_normal((E, F, d, 8)) / np.sqrt(8 * d)).astype(np.float32)
+    wd = (g.standard_normal((E, d, F, 8)) / np.sqrt(8 * F)).astype(np.float32)
+    bu, bd = ((0.1 * g.standard_normal(s)).astype(np.float32) for s in ((E, F, 8), (E, d, 8)))
+    res = g.standard_normal((N, d, 8)).astype(np.float32)
+    cfg = yggdrasil_amd.MoEHLMConfig(d_model=d, d_ff=F, n_experts=E, top_k=k, activation=act, router="logits")
+    layer = yggdrasil_amd.CliffordMoELayer(cfg, device="cuda")
+    layer.load_reference_weights(w_up=wu, b_up=bu, w_down=wd, b_down=bd)
+    say(f"split layer N={N} d={d} F={F} E={E} k={k} {act}")
+    with torch.no_grad():
+        out = layer.moe_forward(torch.from_numpy(x).cuda()[None], logits=torch.from_numpy(lg).cuda(),
+                                residual=torch.from_numpy(res).cuda()[None])[0].cpu().numpy()
+    idx = layer.last_routing["topk_idx"].cpu().numpy()
+    w = layer.last_routing["topk_w"].cpu().numpy()
+    ref = dense.moe_layer(x, idx, w, wu, bu, wd, bd, act, residual=res)
+    # two products in turn (their errors add), the activation's fast exponential (2^-21)
+    assert _rel(out, ref) < 2 * TOL
+    assert _rel(out - res, ref - res) < 4 * TOL  # (and the residual's rounding, 2^-24 of a larger sum)

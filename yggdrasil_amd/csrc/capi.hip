@@ -10,6 +10,7 @@
 #include <stdarg.h>
 #include <stdio.h>
 
+#include <algorithm>
 #include <mutex>
 
 #include "ygg_common.h"
@@ -80,18 +81,45 @@ static size_t ys_bytes(size_t P, int E, int d, int F, int dtype, int w_format) {
   return P * d * 8 * es;
 }
 
-YGG_API size_t ygg_moe_workspace_bytes(int N, int d, int F, int E, int k, int dtype, int w_format) {
+// Whether a layer's two fp32 Pauli products run as split products (fp32 operands as two
+// fp16 parts), and the regions of its workspace that this enlarges or adds.
+static bool f32_split(int N, int d, int F, int E, int k, int w_format) {
+  const long long P = (long long)N * k;
+  return w_format == kWPauliF32 && N > 0 && P <= 0x7fffffffLL && ygg::pauli_split_pays(P, E, d, F) &&
+         ygg::pauli_split_pays(P, E, F, d) && ygg::pauli_split_fits(E, (int)P, N, true, d, F, false) &&
+         ygg::pauli_split_fits(E, (int)P, (int)P, false, F, d, false);
+}
+struct SplitSizes {
+  size_t x, h, w, col_exp, norms;
+};
+static SplitSizes split_sizes(size_t N, size_t P, int d, int F, int E) {
+  SplitSizes z;
+  z.x = N * pauli_split_row_bytes(d);
+  z.h = P * pauli_split_row_bytes(F);
+  z.w = std::max((size_t)F * pauli_split_row_bytes(d), (size_t)d * pauli_split_row_bytes(F)) * E;  // both products, in turn
+  z.col_exp = (size_t)E * std::max(d, F) * 4;
+  z.norms = (size_t)E * 2 * pauli_split_norm_blocks(F) * 4;
+  return z;
+}
+
+static size_t moe_workspace(int N, int d, int F, int E, int k, int dtype, int w_format, bool allow_split) {
   const size_t P = (size_t)N * k;
   const size_t es = (dtype == kF32) ? 4 : 2;
   size_t b = 0;
+  const bool split = allow_split && f32_split(N, d, F, E, k, w_format);
+  const SplitSizes z = split_sizes(N, P, d, F, E);
   b += align256((size_t)N * E * 4);       // logits
   b += align256(P * 4) * 2;               // perm, slot_pos
   b += align256(ygg_route_workspace_bytes(N, E, k));
-  b += align256(P * d * 8 * es);          // x_sorted (Pauli half-rows of x for format 3)
-  b += align256(P * F * 8 * es);          // h
+  b += align256(std::max(P * d * 8 * es, split ? z.x : 0));  // x_sorted (Pauli half-rows of x for format 3, split rows)
+  b += align256(std::max(P * F * 8 * es, split ? z.h : 0));  // h
   b += align256(ys_bytes(P, E, d, F, dtype, w_format));  // y_sorted
   if (w_format == kWPauliF32) b += align256(P * 4);       // row_slot: each row's slot, for the partial planes
+  if (split) b += align256(z.w) + align256(z.col_exp) + align256(z.norms) + 2 * align256(P * 4);  // row and h exponents
   return b;
+}
+YGG_API size_t ygg_moe_workspace_bytes(int N, int d, int F, int E, int k, int dtype, int w_format) {
+  return moe_workspace(N, d, F, E, k, dtype, w_format, true);
 }
 
 // Sizes the layer's kernels cannot address, refused before the first launch: more
@@ -119,7 +147,7 @@ static int moe_forward_impl(const void* x, int dtype, int N, int d, int F, int E
                             const float* b_down, int w_format, const void* residual, void* out, int32_t* topk_idx,
                             float* topk_w, int32_t* counts, int32_t* offsets, void* workspace,
                             size_t workspace_bytes, hipStream_t stream,
-                            float* h_pre_out) {
+                            float* h_pre_out, bool allow_split = true) {
   // every path checks the sizes here, also those that route inside a product
   YGG_CHECK_ARG(N >= 0 && d >= 1 && F >= 1, "ygg_moe_forward: bad sizes N=%d d=%d F=%d", N, d, F);
   YGG_CHECK_ARG(E >= 1 && E <= kMaxExperts, "ygg_moe_forward: E=%d out of range [1, %d]", E, kMaxExperts);
@@ -142,9 +170,9 @@ static int moe_forward_impl(const void* x, int dtype, int N, int d, int F, int E
   YGG_CHECK_ARG(w_format != kWPauli || (d % 2 == 0 && F % 2 == 0),
                 "ygg_moe_forward: the Pauli weight format needs even d and F (d=%d F=%d)", d, F);
   if (layer_size_check("ygg_moe_forward", N, d, F, E, k, w_format)) return -1;
-  YGG_CHECK_ARG(workspace_bytes >= ygg_moe_workspace_bytes(N, d, F, E, k, dtype, w_format),
-                "ygg_moe_forward: workspace of %zu bytes, need %zu", workspace_bytes,
-                ygg_moe_workspace_bytes(N, d, F, E, k, dtype, w_format));
+  const size_t ws_need = moe_workspace(N, d, F, E, k, dtype, w_format, allow_split);
+  YGG_CHECK_ARG(workspace_bytes >= ws_need, "ygg_moe_forward: workspace of %zu bytes, need %zu", workspace_bytes,
+                ws_need);
   YGG_CHECK_ARG(N == 0 || logits || (router_w && router_b), "ygg_moe_forward: need logits or router parameters");
   if (N == 0)  // no tokens: every expert's count and offset is zero, as ygg_route writes them
     return (counts && offsets) ? ygg_route(nullptr, 0, E, k, nullptr, nullptr, counts, offsets, nullptr, nullptr,
@@ -162,10 +190,12 @@ static int moe_forward_impl(const void* x, int dtype, int N, int d, int F, int E
   void* rws = p;
   const size_t rws_bytes = align256(ygg_route_workspace_bytes(N, E, k));
   p += rws_bytes;
+  const bool split = allow_split && f32_split(N, d, F, E, k, w_format);
+  const SplitSizes z = split_sizes(N, P, d, F, E);
   void* xs = p;
-  p += align256(P * d * 8 * es);
+  p += align256(std::max(P * d * 8 * es, split ? z.x : 0));
   void* h = p;
-  p += align256(P * F * 8 * es);
+  p += align256(std::max(P * F * 8 * es, split ? z.h : 0));
   void* ys = p;
 
   if (w_format == kWPauliI8) {
@@ -205,7 +235,7 @@ static int moe_forward_impl(const void* x, int dtype, int N, int d, int F, int E
   // the Pauli formats' conversion of x to Pauli rows (into the x_sorted region: N <= P
   // rows) runs as extra workgroups of the routing's first launch
   ygg::RowConvert cv;
-  if ((w_format == kWPauli || w_format == kWPauliF32) && !f32_routed_up) {
+  if ((w_format == kWPauli || w_format == kWPauliF32) && !f32_routed_up && !split) {
     cv.x = x;
     cv.out = xs;
     cv.n = (long long)N * d;
@@ -216,7 +246,7 @@ static int moe_forward_impl(const void* x, int dtype, int N, int d, int F, int E
   // partial planes at slot rows t k + s (the combine's plane loads then need no
   // routing array)
   int32_t* row_slot = nullptr;
-  if (w_format == kWPauliF32) {
+  if (w_format == kWPauliF32 && !split) {
     row_slot = reinterpret_cast<int32_t*>(static_cast<char*>(ys) + align256(ys_bytes(P, E, d, F, dtype, w_format)));
     cv.row_slot = row_slot;
   }
@@ -229,6 +259,37 @@ static int moe_forward_impl(const void* x, int dtype, int N, int d, int F, int E
   } else if (ygg::route_convert(logits, N, E, k, topk_idx, topk_w, counts, offsets, perm, slot_pos, rws, rws_bytes,
                                 cv, stream)) {
     return -1;
+  }
+  if (split) {
+    // fp32 Pauli, enough rows: both operands of each product as two fp16 parts.  The up
+    // product gathers x's split rows and writes h as split rows, whose exponents come
+    // from a bound taken with x's; the weights are split into one region in turn.
+    char* q = static_cast<char*>(ys) + align256(ys_bytes(P, E, d, F, dtype, w_format)) + align256(P * 4);
+    auto take = [&](size_t bytes) {
+      char* r = q;
+      q += align256(bytes);
+      return r;
+    };
+    void* ws = take(z.w);
+    int32_t* col_exp = reinterpret_cast<int32_t*>(take(z.col_exp));
+    float* norms = reinterpret_cast<float*>(take(z.norms));
+    int32_t* row_exp = reinterpret_cast<int32_t*>(take(P * 4));
+    ygg::SplitHidden hid;
+    hid.k = k;
+    hid.d_ff = F;
+    hid.act = act;
+    hid.slot_pos = slot_pos;
+    hid.topk_idx = topk_idx;
+    hid.norms = norms;
+    hid.h_exp = reinterpret_cast<int32_t*>(take(P * 4));
+    if (pauli_split_weights(static_cast<const float*>(w_up), E, F, d, b_up, ws, col_exp, norms, stream) ||
+        pauli_split_rows(static_cast<const float*>(x), N, d, xs, row_exp, hid, stream) ||
+        pauli_split_up(xs, N, row_exp, perm, (int)P, ws, col_exp, b_up, offsets, E, d, F, act, h, hid.h_exp, h_pre_out,
+                       stream) ||
+        pauli_split_weights(static_cast<const float*>(w_down), E, d, F, nullptr, ws, col_exp, nullptr, stream) ||
+        pauli_split_linear(h, hid.h_exp, (int)P, ws, col_exp, b_down, offsets, E, F, d, static_cast<float*>(ys), stream))
+      return -1;
+    return ygg_combine(ys, kF32, /*y_mask=*/0, N, k, d, topk_idx, topk_w, slot_pos, residual, out, dtype, stream);
   }
   if (w_format == kWPauliF32) {
     // fp32 Pauli: x's Pauli rows (converted with the routing) are gathered through perm
@@ -366,7 +427,8 @@ YGG_API int ygg_moe_forward_noalloc(const void* x, int dtype, int N, int d, int 
                                     hipStream_t stream) {
   YGG_CHECK_ARG(N >= 0 && d >= 1 && F >= 1 && k >= 1, "ygg_moe_forward_noalloc: bad sizes N=%d d=%d F=%d k=%d", N, d,
                 F, k);
-  const size_t need = ygg_moe_workspace_bytes(N, d, F, E, k, dtype, w_format);
+  // (without the split products' regions, so that the calls which fit do not depend on them)
+  const size_t need = moe_workspace(N, d, F, E, k, dtype, w_format, false);
   YGG_CHECK_ARG(need <= kNoAllocScratchBytes,
                 "ygg_moe_forward_noalloc: this layer call needs %zu bytes of scratch, more than the %zu the library "
                 "holds per device; use ygg_moe_forward with a workspace",
@@ -375,7 +437,7 @@ YGG_API int ygg_moe_forward_noalloc(const void* x, int dtype, int N, int d, int 
   if (N > 0 && device_scratch(stream, &ws)) return -1;
   return moe_forward_impl(x, dtype, N, d, F, E, k, act, logits, router_w, router_b, w_up, s_up, b_up, w_down, s_down,
                           b_down, w_format, residual, out, topk_idx, topk_w, counts, offsets, ws,
-                          kNoAllocScratchBytes, stream, nullptr);
+                          kNoAllocScratchBytes, stream, nullptr, /*allow_split=*/false);
 }
 
 // The forward of a training step (fp32 Pauli weights): ygg_moe_forward, and the

@@ -15,8 +15,10 @@
 namespace ygg {
 
 typedef __bf16 pbf16x8_t __attribute__((ext_vector_type(8)));
+typedef _Float16 pf16x8_t __attribute__((ext_vector_type(8)));
 typedef __bf16 pbf16x2_t __attribute__((ext_vector_type(2)));
 typedef float pf32x2_t __attribute__((ext_vector_type(2)));
+typedef float pf32x4_t __attribute__((ext_vector_type(4)));
 typedef float pf32x16_t __attribute__((ext_vector_type(16)));
 
 // ---------------------------------------------------------------------------
@@ -112,6 +114,27 @@ __device__ inline void store_pauli_f32(float* dst, const float* x) {
   float4* q = reinterpret_cast<float4*>(dst);
   q[0] = make_float4(c0[0], c0[2], c0[1], c0[3]);
   q[1] = make_float4(c1[0], c1[2], c1[1], c1[3]);
+}
+
+// ---- fp32 values as two fp16 parts (the split products of pauli_gemm.hip) ----------
+typedef _Float16 pf16x4_t __attribute__((ext_vector_type(4)));
+// the scale exponent of values whose largest magnitude is m: it brings them below 2^15
+// (m zero or not finite: unscaled)
+__device__ __forceinline__ int split_exp(float m) {
+  if (!(m > 0.f) || !(m < INFINITY)) return 0;
+  return 15 - __builtin_amdgcn_frexp_expf(m);
+}
+// four values scaled by 2^s -> their hi and lo parts, 8 bytes each, rounded to nearest
+__device__ __forceinline__ void split4_f16(const float* v, int s, uint2& hi, uint2& lo) {
+  pf16x4_t h, l;
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    const float x = __builtin_ldexpf(v[q], s);
+    h[q] = (_Float16)x;
+    l[q] = (_Float16)(x - (float)h[q]);
+  }
+  hi = __builtin_bit_cast(uint2, h);
+  lo = __builtin_bit_cast(uint2, l);
 }
 
 // two floats -> packed bf16 pair (v_cvt_pk_bf16_f32, round to nearest even)

@@ -714,6 +714,28 @@ YGG_API size_t ygg_geom_matmul_f32_workspace_bytes(int M, int K, int N) {
   return gm_w_bytes(M, K) + gm_x_bytes(K, N) + kGmAlign;
 }
 
+namespace {
+// The split product's operands in the workspace: split weights at 0, then these offsets.
+struct GmSplit {
+  size_t x, col_exp, row_exp, partial, offsets, end;
+};
+GmSplit gm_split_layout(int M, int K, int N) {
+  GmSplit g;
+  g.x = gm_align((size_t)M * pauli_split_row_bytes(K));
+  g.col_exp = g.x + gm_align((size_t)N * pauli_split_row_bytes(K));
+  g.row_exp = g.col_exp + gm_align((size_t)M * 4);
+  g.partial = g.row_exp + gm_align((size_t)N * 4);
+  g.offsets = g.partial + gm_align(pauli_split_gm_partials(K, N) * 4);
+  g.end = g.offsets + kGmAlign;
+  return g;
+}
+// geom_matmul through the split product, within the workspace of the fp32 MFMA one.
+bool gm_split(int M, int K, int N) {
+  return pauli_split_pays((long long)N, 1, K, M) && pauli_split_fits(1, N, N, false, K, M, true) &&
+         gm_split_layout(M, K, N).end <= ygg_geom_matmul_f32_workspace_bytes(M, K, N);
+}
+}  // namespace
+
 YGG_API int ygg_geom_matmul_f32_ws(const float* a, const float* b, float* out, int M, int K, int N, void* workspace,
                                    size_t workspace_bytes, hipStream_t stream) {
   YGG_CHECK_ARG(M >= 0 && K >= 0 && N >= 0, "ygg_geom_matmul_f32: bad sizes M=%d K=%d N=%d", M, K, N);
@@ -731,6 +753,16 @@ YGG_API int ygg_geom_matmul_f32_ws(const float* a, const float* b, float* out, i
   YGG_CHECK_ARG(workspace != nullptr && workspace_bytes >= need,
                 "ygg_geom_matmul_f32: workspace of %zu bytes, %zu needed", workspace_bytes, need);
   char* ws = static_cast<char*>(workspace);
+  if (gm_split(M, K, N)) {
+    const GmSplit g = gm_split_layout(M, K, N);
+    int32_t* off = reinterpret_cast<int32_t*>(ws + g.offsets);
+    int32_t* ce = reinterpret_cast<int32_t*>(ws + g.col_exp);
+    int32_t* re = reinterpret_cast<int32_t*>(ws + g.row_exp);
+    if (pauli_split_gm_operands(a, b, M, K, N, ws, ce, ws + g.x, re, reinterpret_cast<float*>(ws + g.partial), off,
+                                stream))
+      return -1;
+    return pauli_split_linear_t(ws + g.x, re, N, ws, ce, off, K, M, out, stream);
+  }
   float* wp = reinterpret_cast<float*>(ws);
   float* xp = reinterpret_cast<float*>(ws + gm_w_bytes(M, K));
   int32_t* off = reinterpret_cast<int32_t*>(ws + gm_w_bytes(M, K) + gm_x_bytes(K, N));

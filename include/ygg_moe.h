@@ -211,6 +211,13 @@ int ygg_pauli_grouped_linear_f32(const float* x, const int32_t* gather, int P_ma
                                  const float* bias_prepared, const int32_t* offsets, int E, int d_in, int d_out,
                                  int act, float* y, int y_layout, ygg_stream_t stream);
 
+/* CliffordLinear.forward (clifford_linear.py:101-123) of one weight: x (rows, d_in, 8) ->
+ * y (rows, d_out, 8), both blade order, dtype 0 (w prepared in format 4) or 1 (format 1);
+ * bias (d_out, 8) prepared (mask order) or NULL. */
+size_t ygg_clifford_linear_workspace_bytes(int dtype, int rows, int d_in, int d_out);
+int ygg_clifford_linear(const void* x, int dtype, int rows, const void* w, const float* bias, int d_in, int d_out,
+                        void* y, void* workspace, size_t workspace_bytes, ygg_stream_t stream);
+
 /* Blade-order fp32 rows (rows, d, 8) -> fp32 Pauli rows (rows, d, 2, 2, 2): element
  * [m][i][b][k][c] is the real (k = 0) or imaginary (k = 1) part of entry (c, b) of
  * multivector x[m][i] as a 2x2 complex matrix. */

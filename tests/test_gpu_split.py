@@ -103,3 +103,37 @@ def test_layer(N, d, F, E, k, act, empty):
     # two products in turn (their errors add), the activation's fast exponential (2^-21)
     assert _rel(out, ref) < 2 * TOL
     assert _rel(out - res, ref - res) < 4 * TOL  # (and the residual's rounding, 2^-24 of a larger sum)
+
+
+@pytest.mark.parametrize("rows,d_in,d_out,bias,dtype", [
+    (6400, 128, 64, True, "f32"), (1637, 131, 257, False, "f32"),   # split product
+    (6399, 127, 65, True, "f32"), (1, 1, 1, True, "f32"), (33, 300, 5, False, "f32"),  # fp32 MFMA product
+    (200, 9, 40, True, "bf16"), (17, 128, 33, False, "bf16"), (0, 16, 8, True, "f32")])
+def test_clifford_linear_module(rows, d_in, d_out, bias, dtype):
+    """The module on each of its paths, from a strided and from a misaligned input."""
+    import yggdrasil_amd
+
+    g = np.random.default_rng(rows + d_in)
+    dt = torch.float32 if dtype == "f32" else torch.bfloat16
+    x = torch.from_numpy(g.standard_normal((rows, d_in, 8)).astype(np.float32)).to(dt)
+    w = (g.standard_normal((d_out, d_in, 8)) / np.sqrt(8 * d_in)).astype(np.float32)
+    b = g.standard_normal((d_out, 8)).astype(np.float32)
+    lin = yggdrasil_amd.CliffordLinear(d_in, d_out, bias=bias, dtype=dt, device="cuda")
+    with torch.no_grad():
+        lin.weight.copy_(torch.from_numpy(w))
+        if bias:
+            lin.bias.copy_(torch.from_numpy(b))
+    say(f"CliffordLinear {rows} x {d_in} -> {d_out} {dtype}")
+    shifted = torch.empty(rows * d_in * 8 + 1, dtype=dt, device="cuda")[1:].view(rows, d_in, 8)
+    strided = torch.empty((rows, 2 * d_in, 8), dtype=dt, device="cuda")[:, ::2]
+    shifted.copy_(x)
+    strided.copy_(x)
+    y = lin(x.cuda())
+    assert y.shape == (rows, d_out, 8) and y.dtype == dt
+    assert torch.equal(lin(shifted), y) and torch.equal(lin(strided), y)
+    assert torch.equal(lin(x.cuda()[None])[0], y)
+    if rows:
+        w_held = torch.from_numpy(w).to(dt).double().numpy()
+        ref = dense.linear(x.double().numpy(), w_held, b if bias else None)
+        # bf16: the output's rounding, 2^-9 of each element at most
+        assert _rel(y.double().cpu().numpy(), ref) < (TOL if dtype == "f32" else 2.0 ** -9)

@@ -786,3 +786,93 @@ YGG_API int ygg_geom_matmul_f32(const float* a, const float* b, float* out, int 
   YGG_CHECK_ARG(fe == hipSuccess, "ygg_geom_matmul_f32: freeing the workspace: %s", hipGetErrorString(fe));
   return 0;
 }
+
+// ---------------------------------------------------------------------------
+// CliffordLinear on its own: the rows as a single expert's
+// ---------------------------------------------------------------------------
+
+namespace {
+// x (rows, d, 8) blade order -> the product's input rows, and the one-expert offsets
+// {0, rows}, in one launch.  fp32: Pauli rows; bf16: mask order.  One thread per
+// multivector.
+template <int DT>
+__global__ __launch_bounds__(256) void linear_rows_kernel(const void* __restrict__ x, int rows, size_t n_mv,
+                                                          void* __restrict__ out, int32_t* __restrict__ offsets) {
+  const size_t n = (size_t)blockIdx.x * 256 + threadIdx.x;
+  if (n < 2) offsets[n] = n == 0 ? 0 : rows;
+  if (n >= n_mv) return;
+  if constexpr (DT == kF32) {
+    pauli_rows_f32_one(static_cast<const float*>(x), n, static_cast<float*>(out));
+  } else {
+    uint4 q = static_cast<const uint4*>(x)[n];  // components 3 and 4 exchanged
+    const uint32_t c3 = q.y >> 16, c4 = q.z & 0xffffu;
+    q.y = (q.y & 0xffffu) | (c4 << 16);
+    q.z = (q.z & 0xffff0000u) | c3;
+    static_cast<uint4*>(out)[n] = q;
+  }
+}
+
+struct LinearLayout {
+  bool split;
+  size_t x, w, col_exp, row_exp, offsets, end;
+};
+LinearLayout linear_layout(int dtype, int rows, int d_in, int d_out) {
+  LinearLayout l;
+  l.split = dtype == kF32 && pauli_split_pays(rows, 1, d_in, d_out) &&
+            pauli_split_fits(1, rows, rows, false, d_in, d_out, false);
+  l.x = 0;
+  l.w = gm_align(l.split ? (size_t)rows * pauli_split_row_bytes(d_in) : (size_t)rows * d_in * (dtype == kF32 ? 32 : 16));
+  l.col_exp = l.w + gm_align(l.split ? (size_t)d_out * pauli_split_row_bytes(d_in) : 0);
+  l.row_exp = l.col_exp + gm_align(l.split ? (size_t)d_out * 4 : 0);
+  l.offsets = l.row_exp + gm_align(l.split ? (size_t)rows * 4 : 0);
+  l.end = l.offsets + kGmAlign;
+  return l;
+}
+}  // namespace
+
+extern "C" int ygg_grouped_clifford_linear(const void*, int, const void*, int, const float*, const float*,
+                                           const int32_t*, int, int, int, int, void*, int, int, hipStream_t);
+
+YGG_API size_t ygg_clifford_linear_workspace_bytes(int dtype, int rows, int d_in, int d_out) {
+  if (rows <= 0 || d_in <= 0 || d_out <= 0) return 0;
+  return linear_layout(dtype, rows, d_in, d_out).end;
+}
+
+// fp32: the split product from the sizes where it pays (4096 x 128 -> 512: 71 us a call;
+// the L(w) blocks on the vector units, 64 multiply-adds a pair, took 363 of the 398 us of a
+// call that also copied its row range from the host and waited for it), the fp32
+// MFMA product below; bf16: the L(w) blocks.
+YGG_API int ygg_clifford_linear(const void* x, int dtype, int rows, const void* w, const float* bias, int d_in,
+                                int d_out, void* y, void* workspace, size_t workspace_bytes, hipStream_t stream) {
+  YGG_CHECK_ARG(dtype == kF32 || dtype == kBF16, "ygg_clifford_linear: dtype %d", dtype);
+  YGG_CHECK_ARG(rows >= 0 && d_in >= 1 && d_out >= 1, "ygg_clifford_linear: bad sizes rows=%d d_in=%d d_out=%d", rows,
+                d_in, d_out);
+  if (rows == 0) return 0;
+  YGG_CHECK_ARG(x && w && y && workspace, "ygg_clifford_linear: null pointer");
+  const LinearLayout l = linear_layout(dtype, rows, d_in, d_out);
+  YGG_CHECK_ARG(workspace_bytes >= l.end, "ygg_clifford_linear: workspace of %zu bytes, need %zu", workspace_bytes, l.end);
+  char* ws = static_cast<char*>(workspace);
+  int32_t* off = reinterpret_cast<int32_t*>(ws + l.offsets);
+  if (l.split) {
+    int32_t* ce = reinterpret_cast<int32_t*>(ws + l.col_exp);
+    int32_t* re = reinterpret_cast<int32_t*>(ws + l.row_exp);
+    SplitHidden none;
+    none.one_offsets = off;
+    if (pauli_split_weights(static_cast<const float*>(w), 1, d_out, d_in, nullptr, ws + l.w, ce, nullptr, stream) ||
+        pauli_split_rows(static_cast<const float*>(x), rows, d_in, ws + l.x, re, none, stream))
+      return -1;
+    return pauli_split_linear(ws + l.x, re, rows, ws + l.w, ce, bias, off, 1, d_in, d_out, static_cast<float*>(y),
+                              stream);
+  }
+  const size_t n = (size_t)rows * d_in;
+  const unsigned grid = (unsigned)((n + 255) / 256);
+  if (dtype == kF32) linear_rows_kernel<kF32><<<grid, 256, 0, stream>>>(x, rows, n, ws, off);
+  else linear_rows_kernel<kBF16><<<grid, 256, 0, stream>>>(x, rows, n, ws, off);
+  if (check_launch("linear_rows")) return -1;
+  if (dtype == kF32)
+    return launch_f32_act<kF32OutBlade>(kActNone, 1, stream, reinterpret_cast<const float*>(ws), nullptr,
+                                        static_cast<const float*>(w), bias, off, 1, d_in, d_out, rows,
+                                        static_cast<float*>(y));
+  return ygg_grouped_clifford_linear(ws, rows, w, kWBF16, nullptr, bias, off, 1, d_in, d_out, kActNone, y, kBF16, 1,
+                                     stream);
+}

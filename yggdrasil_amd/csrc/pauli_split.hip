@@ -214,6 +214,7 @@ __global__ __launch_bounds__(256) void split_rows_kernel(const float* __restrict
   }
   if (hid.k == 0) {
     if (lane == 0) row_exp[t] = s;
+    if (hid.one_offsets != nullptr && t == 0 && lane < 2) hid.one_offsets[lane] = lane * N;
     return;
   }
 #pragma unroll

@@ -219,6 +219,7 @@ struct SplitHidden {
   const int32_t* topk_idx = nullptr;
   const float* norms = nullptr;  // of pauli_split_weights
   int32_t* h_exp = nullptr;
+  int32_t* one_offsets = nullptr;  // k = 0: when set, takes the one-expert offsets {0, N}
 };
 int pauli_split_rows(const float* x, int N, int d, void* out, int32_t* row_exp, const SplitHidden& hid,
                      hipStream_t stream);

@@ -317,17 +317,15 @@ class CliffordLinear(nn.Module):
     def _prepared(self):
         key = (self.weight._version, None if self.bias is None else self.bias._version, self.weight.device)
         if self._prep is None or self._prep[0] != key:
-            fmt = "f32" if self.dtype == torch.float32 else "bf16"
+            fmt = "pauli_f32" if self.dtype == torch.float32 else "bf16"
             self._prep = (key, ops.prepare_weights(self.weight.detach().unsqueeze(0), fmt),
                           ops.prepare_bias(self.bias.detach().unsqueeze(0)) if self.bias is not None else None)
         return self._prep
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         batch = x.shape[:-2]
-        flat = ops.to_mask_order(x.reshape(-1, self.d_in, 8).to(self.dtype))
         _, pw, pb = self._prepared()
-        offsets = torch.tensor([0, flat.shape[0]], device=x.device, dtype=torch.int32)
-        y = ops.grouped_clifford_linear(flat, pw, offsets, pb, "none", out_dtype=self.dtype)
+        y = ops.clifford_linear(x.reshape(-1, self.d_in, 8).to(self.dtype).contiguous(), pw, pb)
         return y.reshape(*batch, self.d_out, 8)
 
 

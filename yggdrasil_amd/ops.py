@@ -423,6 +423,27 @@ def pauli_grouped_linear_f32(x: torch.Tensor, pw: PreparedWeights, offsets: torc
     return y
 
 
+def clifford_linear(x: torch.Tensor, pw: PreparedWeights, bias_prepared: torch.Tensor | None = None) -> torch.Tensor:
+    """CliffordLinear (``clifford_linear.py:101-123``) of one weight: x (rows, d_in, 8) blade order -> (rows, d_out, 8).
+
+    fp32 rows take weights prepared as 'pauli_f32', bf16 rows as 'bf16' (E = 1)."""
+    dev = _dev(x, bias_prepared)
+    if x.dim() != 3 or tuple(x.shape[1:]) != (pw.d_in, 8):
+        raise ValueError(f"x must be (rows, {pw.d_in}, 8), got {tuple(x.shape)}")
+    want = "pauli_f32" if _dtype_code(x) == 0 else "bf16"
+    if pw.fmt != want or pw.E != 1:
+        raise ValueError(f"{x.dtype} rows take one weight prepared as {want!r}")
+    if x.data_ptr() % 16:  # the kernels load 16 bytes at a time
+        x = x.clone()
+    rows, code = x.shape[0], _dtype_code(x)
+    y = torch.empty((rows, pw.d_out, 8), device=dev, dtype=x.dtype)
+    nbytes = lib().ygg_clifford_linear_workspace_bytes(code, rows, pw.d_in, pw.d_out)
+    ws = torch.empty((max(nbytes, 1),), device=dev, dtype=torch.uint8)
+    check(lib().ygg_clifford_linear(ptr(x), code, rows, ptr(pw.data), ptr(bias_prepared), pw.d_in, pw.d_out, ptr(y),
+                                    ptr(ws), nbytes, stream_handle(dev)), "clifford_linear")
+    return y
+
+
 def pauli_rows_from_blade_f32(x: torch.Tensor) -> torch.Tensor:
     """(rows, d, 8) fp32 blade order -> (rows, d, 2, 2, 2) fp32 Pauli rows.
 

@@ -137,3 +137,42 @@ def test_clifford_linear_module(rows, d_in, d_out, bias, dtype):
         ref = dense.linear(x.double().numpy(), w_held, b if bias else None)
         # bf16: the output's rounding, 2^-9 of each element at most
         assert _rel(y.double().cpu().numpy(), ref) < (TOL if dtype == "f32" else 2.0 ** -9)
+
+
+@pytest.mark.parametrize("N,d,F,E,k,act,router", [(3300, 133, 150, 3, 1, "gelu", "logits"),
+                                                  (1700, 128, 260, 5, 2, "sigmoid", "energy"),
+                                                  (1301, 150, 128, 8, 4, "relu", "logits")])
+def test_layer_backward(N, d, F, E, k, act, router):
+    """Gradients through the split products and weight gradients: widths off every block, an expert without
+    rows, chunks with odd tails, tokens over many binades (rows of one weight-gradient sum have different
+    scales), one token of zeros."""
+    import yggdrasil_amd
+
+    g = np.random.default_rng(N + d)
+    x = g.standard_normal((N, d, 8)).astype(np.float32) * np.ldexp(1.0, g.integers(-9, 4, (N, 1, 1))).astype(np.float32)
+    x[7] = 0.0
+    lg = g.standard_normal((N, E)).astype(np.float32)
+    if E == 3:
+        lg[:, 1] = -30.0
+    wu = (g.standard_normal((E, F, d, 8)) / np.sqrt(8 * d)).astype(np.float32)
+    wd = (g.standard_normal((E, d, F, 8)) / np.sqrt(8 * F)).astype(np.float32)
+    bu, bd = ((0.1 * g.standard_normal(s)).astype(np.float32) for s in ((E, F, 8), (E, d, 8)))
+    dout = g.standard_normal((N, d, 8)).astype(np.float32) * np.ldexp(1.0, g.integers(-9, 4, (N, 1, 1))).astype(np.float32)
+    cfg = yggdrasil_amd.MoEHLMConfig(d_model=d, d_ff=F, n_experts=E, top_k=k, activation=act, router=router)
+    layer = yggdrasil_amd.CliffordMoELayer(cfg, device="cuda")
+    layer.load_reference_weights(w_up=wu, b_up=bu, w_down=wd, b_down=bd)
+    say(f"split backward N={N} d={d} F={F} E={E} k={k} {act}")
+    xt = torch.from_numpy(x).cuda()[None].requires_grad_(True)
+    out = layer.moe_forward(xt, logits=torch.from_numpy(lg).cuda() if router == "logits" else None)
+    grads = torch.autograd.grad(out, (xt, layer.w_up, layer.b_up, layer.w_down, layer.b_down),
+                                torch.from_numpy(dout).cuda()[None])
+    idx = layer.last_routing["topk_idx"].cpu().numpy()
+    w = layer.last_routing["topk_w"].cpu().numpy()
+    assert _rel(out[0].detach().cpu().numpy(), dense.moe_layer(x, idx, w, wu, bu, wd, bd, act)) < 2 * TOL
+    ref = dense.moe_layer_backward(x, idx, w, wu, bu, wd, bd, dout, act)
+    for name, got, want in zip(("dx", "dw_up", "db_up", "dw_down", "db_down"), grads, ref):
+        got = got.cpu().numpy().reshape(want.shape)
+        # the sums' error of two products and the activation's derivative in fp32
+        assert np.isfinite(got).all() and _rel(got, want) < 4 * TOL, (name, _rel(got, want))
+        if E == 3 and name != "dx":
+            assert not got[1].any()

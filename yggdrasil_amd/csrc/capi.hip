@@ -497,20 +497,29 @@ static int bw_regions(int N, int d, int F, int E, int k, size_t* r) {
   r[n++] = P * 4;              // slot_pos
   r[n++] = (size_t)N * E * 4;  // logits scratch
   r[n++] = ygg_route_workspace_bytes(N, E, k);
-  r[n++] = (size_t)N * d * 32;  // x in Pauli rows
-  for (int q = 0; q < 4; ++q) r[n++] = P * F * 32;  // h_pre, h, Pauli rows of h / dh_pre, dh / dh_pre
-  for (int q = 0; q < 3; ++q) r[n++] = P * d * 32;  // y / dx rows, dy, Pauli rows of dy
+  const bool split = f32_split(N, d, F, E, k, kWPauliF32);  // (split rows are padded to blocks of 8 multivectors)
+  const size_t row_d = split ? pauli_split_row_bytes(d) : (size_t)d * 32;
+  const size_t row_f = split ? pauli_split_row_bytes(F) : (size_t)F * 32;
+  r[n++] = N * row_d;  // x in Pauli rows
+  for (int q = 0; q < 4; ++q) r[n++] = P * row_f;  // h_pre, h, Pauli rows of h / dh_pre, dh / dh_pre
+  for (int q = 0; q < 3; ++q) r[n++] = P * row_d;  // y / dx rows, dy, Pauli rows of dy
   // weight-gradient partial sums, reused by both products: the up product's
   // (d_in = d, d_out = F) and the down product's (d_in = F, d_out = d, whose
   // bias planes are d-wide), so the larger of the two
   const size_t wg_up = weight_grad_pauli_workspace_bytes((int)P, E, d, F);
   const size_t wg_down = weight_grad_pauli_workspace_bytes((int)P, E, F, d);
   r[n++] = wg_up > wg_down ? wg_up : wg_down;
+  if (split) {
+    const SplitSizes z = split_sizes(N, P, d, F, E);
+    r[n++] = z.w;        // split weights of one product at a time
+    r[n++] = z.col_exp;
+    for (int q = 0; q < 4; ++q) r[n++] = P * 4;  // exponents of the rows of x (N), h, dy, dh_pre
+  }
   return n;
 }
 
 YGG_API size_t ygg_moe_backward_workspace_bytes(int N, int d, int F, int E, int k) {
-  size_t r[24], b = 0;
+  size_t r[32], b = 0;
   const int n = bw_regions(N, d, F, E, k, r);
   for (int q = 0; q < n; ++q) b += align256(r[q]);
   return b;
@@ -538,7 +547,7 @@ YGG_API int ygg_moe_backward(const float* x, int N, int d, int F, int E, int k, 
   }
   YGG_CHECK_ARG(x && dout && dx, "ygg_moe_backward: null x, dout or dx");
   const size_t P = (size_t)N * k;
-  size_t sz[24];
+  size_t sz[32];
   bw_regions(N, d, F, E, k, sz);
   char* base = static_cast<char*>(workspace);
   int next = 0;
@@ -571,9 +580,12 @@ YGG_API int ygg_moe_backward(const float* x, int N, int d, int F, int E, int k, 
   // the MFMA weight gradient pays off with enough rows per expert; below that the
   // vector-ALU kernel, which spreads a tile's pairs over more waves, is faster
   const bool wg_mfma = P >= (size_t)kWgradMfmaRowsPerExpert * E;
+  // split products and weight gradients, where the forward's products were split
+  const bool split = hp_in && f32_split(N, d, F, E, k, kWPauliF32) && weight_grad_split_fits(N, true, d, F) &&
+                     weight_grad_split_fits((int)P, false, F, d);
   // x's Pauli rows, when needed, are converted by extra workgroups of the routing launch
   ygg::RowConvert cv;
-  if (!hp_in || wg_mfma) {
+  if ((!hp_in || wg_mfma) && !split) {
     cv.x = x;
     cv.out = xp;
     cv.n = (long long)N * d;
@@ -586,6 +598,32 @@ YGG_API int ygg_moe_backward(const float* x, int N, int d, int F, int E, int k, 
   } else if (ygg::route_energy_convert(x, kF32, N, d, router_w, router_b, E, k, idx, tw, counts, offsets, perm,
                                        slot_pos, lg, rws, rws_bytes, cv, stream)) {
     return -1;
+  }
+  if (split) {
+    void* ws = take();
+    int32_t* col_exp = static_cast<int32_t*>(take());
+    int32_t* x_exp = static_cast<int32_t*>(take());
+    int32_t* h_exp = static_cast<int32_t*>(take());
+    int32_t* dy_exp = static_cast<int32_t*>(take());
+    int32_t* dh_exp = static_cast<int32_t*>(take());
+    // split rows of x, h (from h before the activation) and, by the combine's backward, dy
+    if (pauli_split_rows(x, N, d, xp, x_exp, ygg::SplitHidden{}, stream) ||
+        activation_split_rows(hp_in, nullptr, P, F, act, h, h_exp, stream))
+      return -1;
+    if (dtopk_w && (pauli_split_weights(w_down, E, d, F, nullptr, ws, col_exp, nullptr, stream) ||
+                    pauli_split_linear(h, h_exp, (int)P, ws, col_exp, b_down, offsets, E, F, d, y, stream)))
+      return -1;
+    if (combine_backward(dout, dtopk_w ? y : nullptr, N, k, d, tw, slot_pos, nullptr, nullptr, dtopk_w, stream, dp,
+                         dy_exp) ||
+        pauli_split_weights(w_down_adj, E, F, d, nullptr, ws, col_exp, nullptr, stream) ||
+        pauli_split_linear(dp, dy_exp, (int)P, ws, col_exp, nullptr, offsets, E, d, F, dh, stream) ||
+        weight_grad_split(dp, dy_exp, h, (int)P, h_exp, nullptr, offsets, (int)P, E, F, d, dw_down, db_down, wg, stream) ||
+        activation_split_rows(hp_in, dh, P, F, act, fp, dh_exp, stream) ||
+        pauli_split_weights(w_up_adj, E, d, F, nullptr, ws, col_exp, nullptr, stream) ||
+        pauli_split_linear(fp, dh_exp, (int)P, ws, col_exp, nullptr, offsets, E, F, d, y, stream) ||
+        weight_grad_split(fp, dh_exp, xp, N, x_exp, perm, offsets, (int)P, E, d, F, dw_up, db_up, wg, stream))
+      return -1;
+    return dispatch_backward(y, N, k, d, slot_pos, residual ? dout : nullptr, dx, stream);
   }
   if (!hp_in) {
     if (ygg_pauli_grouped_linear_f32(xp, perm, (int)P, w_up, b_up, offsets, E, d, F, kActNone, h_pre, 1, stream))

@@ -117,12 +117,32 @@ __device__ inline void store_pauli_f32(float* dst, const float* x) {
 }
 
 // ---- fp32 values as two fp16 parts (the split products of pauli_gemm.hip) ----------
+typedef _Float16 pf16x2_t __attribute__((ext_vector_type(2)));
 typedef _Float16 pf16x4_t __attribute__((ext_vector_type(4)));
 // the scale exponent of values whose largest magnitude is m: it brings them below 2^15
-// (m zero or not finite: unscaled)
+// (m not finite: unscaled; m zero: as if they were small, so that a row of zeros does
+// not set the common scale of the rows summed with it)
+constexpr int kSplitExpZero = 100;
 __device__ __forceinline__ int split_exp(float m) {
-  if (!(m > 0.f) || !(m < INFINITY)) return 0;
+  if (m == 0.f) return kSplitExpZero;
+  if (!(m < INFINITY)) return 0;
   return 15 - __builtin_amdgcn_frexp_expf(m);
+}
+// magnitudes compared as integers, which orders a NaN above every number
+__device__ __forceinline__ uint32_t mag_bits(float v) { return __builtin_bit_cast(uint32_t, v) & 0x7fffffffu; }
+__device__ __forceinline__ uint32_t wave_max_u32(uint32_t v) {
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) v = max(v, (uint32_t)__shfl_xor((int)v, o));
+  return v;
+}
+// the largest magnitude of a multivector's Pauli entries (as bits)
+__device__ __forceinline__ uint32_t pauli_mag(const float* x) {
+  float c0[4], c1[4];
+  uint32_t m = 0;
+  blade_to_pauli(x, c0, c1);
+#pragma unroll
+  for (int c = 0; c < 4; ++c) m = max(m, max(mag_bits(c0[c]), mag_bits(c1[c])));
+  return m;
 }
 // four values scaled by 2^s -> their hi and lo parts, 8 bytes each, rounded to nearest
 __device__ __forceinline__ void split4_f16(const float* v, int s, uint2& hi, uint2& lo) {
@@ -135,6 +155,20 @@ __device__ __forceinline__ void split4_f16(const float* v, int s, uint2& hi, uin
   }
   hi = __builtin_bit_cast(uint2, h);
   lo = __builtin_bit_cast(uint2, l);
+}
+
+// multivector i of a split row (`row` its start, d_pad multivectors per half-row)
+__device__ __forceinline__ void store_split_mv(unsigned char* row, int d_pad, int i, const float* x, int s) {
+  float c0[4], c1[4];
+  blade_to_pauli(x, c0, c1);
+  uint2 h0, l0, h1, l1;
+  split4_f16(c0, s, h0, l0);
+  split4_f16(c1, s, h1, l1);
+  unsigned char* p = row + (size_t)(i >> 3) * 128 + (i & 7) * 8;
+  *reinterpret_cast<uint2*>(p) = h0;
+  *reinterpret_cast<uint2*>(p + 64) = l0;
+  *reinterpret_cast<uint2*>(p + (size_t)d_pad * 16) = h1;
+  *reinterpret_cast<uint2*>(p + (size_t)d_pad * 16 + 64) = l1;
 }
 
 // two floats -> packed bf16 pair (v_cvt_pk_bf16_f32, round to nearest even)

@@ -17,15 +17,6 @@
 namespace ygg {
 namespace {
 
-// magnitudes compared as integers, which orders a NaN above every number
-__device__ __forceinline__ uint32_t mag_bits(float v) { return __builtin_bit_cast(uint32_t, v) & 0x7fffffffu; }
-
-__device__ __forceinline__ uint32_t wave_max_u32(uint32_t v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v = max(v, (uint32_t)__shfl_xor((int)v, o));
-  return v;
-}
-
 // entries of a weight multivector as the product's B operand: per a, (c0 u, c0 -v,
 // c1 u, c1 -v) of W / 2 (the 1/2 makes the inverse map a plain sum)
 __device__ __forceinline__ void w_entries(const float* w8, float (&e0)[4], float (&e1)[4]) {
@@ -184,11 +175,9 @@ __global__ __launch_bounds__(256) void split_rows_kernel(const float* __restrict
   const float* row = x + (size_t)t * d * 8;
   uint32_t m = 0;
   for (int i = lane; i < d; i += 64) {
-    float v[8], c0[4], c1[4];
+    float v[8];
     load8(row + (size_t)i * 8, v);
-    blade_to_pauli(v, c0, c1);
-#pragma unroll
-    for (int c = 0; c < 4; ++c) m = max(m, max(mag_bits(c0[c]), mag_bits(c1[c])));
+    m = max(m, pauli_mag(v));
   }
   const int s = split_exp(__builtin_bit_cast(float, wave_max_u32(m)));
   const int d_pad = (d + 7) & ~7;
@@ -203,14 +192,7 @@ __global__ __launch_bounds__(256) void split_rows_kernel(const float* __restrict
       const float a = __builtin_ldexpf(c0[c], s), b = __builtin_ldexpf(c1[c], s);
       n2 += a * a + b * b;
     }
-    uint2 h0, l0, h1, l1;
-    split4_f16(c0, s, h0, l0);
-    split4_f16(c1, s, h1, l1);
-    unsigned char* p = o + (size_t)(i >> 3) * 128 + (i & 7) * 8;
-    *reinterpret_cast<uint2*>(p) = h0;
-    *reinterpret_cast<uint2*>(p + 64) = l0;
-    *reinterpret_cast<uint2*>(p + (size_t)d_pad * 16) = h1;
-    *reinterpret_cast<uint2*>(p + (size_t)d_pad * 16 + 64) = l1;
+    store_split_mv(o, d_pad, i, v, s);
   }
   if (hid.k == 0) {
     if (lane == 0) row_exp[t] = s;
@@ -273,11 +255,9 @@ __global__ __launch_bounds__(256) void split_gm_first_kernel(const float* __rest
     for (int u = 0; u < kGmKBlock / 8; ++u) {
       const int k = kb * kGmKBlock + u * 8 + (t >> 5);
       if (k < K) {
-        float v[8], c0[4], c1[4];
+        float v[8];
         load8(b + ((size_t)k * N + n) * 8, v);
-        blade_to_pauli(v, c0, c1);
-#pragma unroll
-        for (int c = 0; c < 4; ++c) m = max(m, max(mag_bits(c0[c]), mag_bits(c1[c])));
+        m = max(m, pauli_mag(v));
       }
     }
   }

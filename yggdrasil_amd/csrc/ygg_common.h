@@ -299,13 +299,25 @@ size_t weight_grad_pauli_workspace_bytes(int P_max, int E, int d_in, int d_out);
 int weight_grad_pauli(const float* dy_pauli, const float* a_pauli, const int32_t* gather, const int32_t* offsets,
                       int P_max, int E, int d_in, int d_out, float* dW, float* db, void* workspace,
                       hipStream_t stream);
+// The same on the fp16 MFMA units from split rows (pauli_split.hip) of dy and a with
+// their exponents (a's per source row); same workspace.
+bool weight_grad_split_fits(int a_rows, bool gathered, int d_in, int d_out);
+int weight_grad_split(const void* dy, const int32_t* dy_exp, const void* a, int a_rows, const int32_t* a_exp,
+                      const int32_t* gather, const int32_t* offsets, int P_max, int E, int d_in, int d_out, float* dW,
+                      float* db, void* workspace, hipStream_t stream);
+// The activation's forward (g NULL) or backward (of g at h) over P blade rows of d
+// multivectors, as split rows.
+int activation_split_rows(const float* h, const float* g, size_t P, int d, int act, void* out, int32_t* row_exp,
+                          hipStream_t stream);
 // (out may alias g; out and out_pauli -- fp32 Pauli rows -- are each optional)
 int activation_backward(const float* h, const float* g, size_t n_mv, int act, float* out, float* out_pauli,
                         hipStream_t stream);
 int activation_forward(const float* h, size_t n_mv, int act, float* out, float* out_pauli, hipStream_t stream);
 int fill_zero_f32(float* p, size_t n, hipStream_t stream);  // n floats at p set to zero
+// dy goes out as blade rows, fp32 Pauli rows and / or split rows with their exponents
 int combine_backward(const float* dout, const float* y_sorted, int N, int k, int d, const float* topk_w,
-                     const int32_t* slot_pos, float* dy_sorted, float* dy_pauli, float* dtopk_w, hipStream_t stream);
+                     const int32_t* slot_pos, float* dy_sorted, float* dy_pauli, float* dtopk_w, hipStream_t stream,
+                     void* dy_split = nullptr, int32_t* dy_exp = nullptr);
 int dispatch_backward(const float* dxs, int N, int k, int d, const int32_t* slot_pos, const float* residual_grad,
                       float* dx, hipStream_t stream);
 

@@ -1,0 +1,71 @@
+"""bf16 Pauli layers of few rows (products that stream the weights, K ranges of the down product) and the
+routing's paths by batch size."""
+
+import numpy as np
+import pytest
+import torch
+
+from _gpu_helpers import TOL_BF16, bf16_round, normwise_err, say
+from oracle import dense, moe
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("N,d,F,E,k,act", [
+    (1, 2, 2, 1, 1, "gelu"),        # one input pair, one column
+    (3, 30, 34, 3, 2, "relu"),      # chunks of 8 inputs with tails, columns off 32
+    (17, 66, 530, 7, 3, "gelu"),    # two and more row tiles, K ranges with a short last one
+    (40, 520, 72, 2, 1, "sigmoid"),  # up contraction past the activations' register range
+    (640, 36, 1030, 64, 2, "gelu"),  # the largest row count, empty and many experts
+    (320, 64, 300, 5, 4, "none"),
+])
+def test_layer(N, d, F, E, k, act):
+    import yggdrasil_amd
+
+    if act == "none":
+        act = "relu"
+    g = np.random.default_rng(N + F)
+    x = bf16_round(g.standard_normal((N, d, 8)).astype(np.float32))
+    lg = g.standard_normal((N, E)).astype(np.float32)
+    lg[:, 0] -= 20.0 * (E > k)  # an expert without rows
+    wu = bf16_round((g.standard_normal((E, F, d, 8)) / np.sqrt(8 * d)).astype(np.float32))
+    wd = bf16_round((g.standard_normal((E, d, F, 8)) / np.sqrt(8 * F)).astype(np.float32))
+    bu, bd = ((0.1 * g.standard_normal(s)).astype(np.float32) for s in ((E, F, 8), (E, d, 8)))
+    res = bf16_round(g.standard_normal((N, d, 8)).astype(np.float32))
+    cfg = yggdrasil_amd.MoEHLMConfig(d_model=d, d_ff=F, n_experts=E, top_k=k, activation=act, dtype=torch.bfloat16,
+                                     weight_format="pauli", router="logits")
+    layer = yggdrasil_amd.CliffordMoELayer(cfg, device="cuda")
+    layer.load_reference_weights(w_up=wu, b_up=bu, w_down=wd, b_down=bd)
+    say(f"few rows N={N} d={d} F={F} E={E} k={k} {act}")
+    out = layer.moe_forward(torch.from_numpy(x).cuda().bfloat16()[None], logits=torch.from_numpy(lg).cuda(),
+                            residual=torch.from_numpy(res).cuda().bfloat16()[None])[0]
+    idx = layer.last_routing["topk_idx"].cpu().numpy()
+    w = layer.last_routing["topk_w"].cpu().numpy()
+    ref = dense.moe_layer(x, idx, w, wu, bu, wd, bd, act, residual=res)
+    assert normwise_err(out.float().cpu().numpy(), ref) < TOL_BF16
+
+
+@pytest.mark.parametrize("E,k", [(1, 1), (7, 2), (33, 4), (64, 3)])
+@pytest.mark.parametrize("N", [1, 9, 90, 91, 300, 301, 1024])
+def test_route_paths_agree(N, E, k):
+    """The same routing on the one- and the two-launch path, from logits and from x (whose logits the one-
+    workgroup kernel and the separate launch sum in one order), against the oracle's selection."""
+    from yggdrasil_amd import ops
+
+    g = np.random.default_rng(N * E)
+    lg = g.standard_normal((N, E)).astype(np.float32)
+    say(f"route N={N} E={E} k={k}")
+    r = ops.route(torch.from_numpy(lg).cuda(), k)
+    idx, w = moe.route_topk(moe.softmax(lg), k)
+    counts, offsets, perm, slot_pos = moe.dispatch_plan(idx, E)
+    for got, want in ((r.topk_idx, idx), (r.counts, counts), (r.offsets, offsets), (r.perm, perm), (r.slot_pos, slot_pos)):
+        assert np.array_equal(got.cpu().numpy().reshape(want.shape), want)
+    for dt in (torch.float32, torch.bfloat16):
+        for d in (13, 70):
+            x = torch.from_numpy(g.standard_normal((N, d, 8)).astype(np.float32)).cuda().to(dt)
+            rw, rb = torch.randn(E, 4).cuda(), torch.randn(E).cuda()
+            a = ops.route_energy(x, rw, rb, k)
+            one = ops.route_energy(x[:1].contiguous(), rw, rb, k)  # one token: always the one-workgroup kernel
+            assert torch.equal(a.topk_idx[0], one.topk_idx[0]) and torch.equal(a.topk_w[0], one.topk_w[0])
+            sep = ops.route(ops.router_energy_logits(x, rw, rb), k)
+            assert (a.topk_idx != sep.topk_idx).float().mean().item() < 0.02  # another order of the sums: ties only

@@ -371,6 +371,32 @@ __global__ __launch_bounds__(256) void router_energy_logits_kernel(const void* _
 using namespace ygg;
 
 namespace {
+// Whether a batch routes in one workgroup: its time grows with the tokens (16 at a time)
+// and the logits a lane holds, the two launches' does not (one / two, us: E = 8: 256 tokens
+// 6.9 / 8.0, 512 10.8 / 8.4, 1024 19.0 / 8.4; E = 32: 128 8.4 / 9.5, 256 13.0 / 9.6; E = 64:
+// 64 7.4 / 7.6, 128 9.2 / 8.1, 1024 43.3 / 8.7).
+bool route_in_one(int N, int E) { return N <= kSmallMaxN && N * ((E + 7) / 8 + 2) <= 900; }
+
+// ... and the logits with it, while the workgroup's reading of x is short beside a launch of
+// its own (one / three launches, us: E = 8, d = 64: 128 tokens 6.0 / 6.5, 256 8.8 / 8.0; d = 256: 32
+// tokens 5.9 / 7.0, 64 7.5 / 7.1, 256 19.1 / 9.3).
+bool energy_in_one(int N, int E, int d) { return route_in_one(N, E) && (long long)N * d <= 13000; }
+
+// The grade-energy logits of energy_logits (the sums of the one-workgroup kernel, in its
+// order) for batches that do not route in one workgroup: eight lanes per token.
+template <int Q>
+__global__ __launch_bounds__(64) void router_energy_logits8_kernel(const void* __restrict__ x, int x_dtype, int N,
+                                                                   int d, const float* __restrict__ rw,
+                                                                   const float* __restrict__ rb, int E,
+                                                                   float* __restrict__ logits) {
+  const int j = threadIdx.x & (kSelLanes - 1), t = blockIdx.x * (64 / kSelLanes) + threadIdx.x / kSelLanes;
+  float p[Q];
+  energy_logits<Q>(x, x_dtype, d, rw, rb, E, t, t < N, j, p);
+#pragma unroll
+  for (int q = 0; q < Q; ++q)
+    if (t < N && j + kSelLanes * q < E) logits[(size_t)t * E + j + kSelLanes * q] = p[q];
+}
+
 template <bool FROM_X>
 int launch_route_small(const float* logits, const void* x, int x_dtype, int d, const float* rw, const float* rb, int N,
                        int E, int k, int32_t* topk_idx, float* topk_w, int32_t* counts, int32_t* offsets,
@@ -436,7 +462,7 @@ int ygg::route_convert(const float* logits, int N, int E, int k, int32_t* topk_i
   YGG_CHECK_ARG(N == 0 || (logits && topk_idx && topk_w && perm && slot_pos && workspace),
                 "ygg_route: null pointer argument");
   YGG_CHECK_ARG(counts && offsets, "ygg_route: null counts/offsets");
-  if (N > 0 && N <= kSmallMaxN)
+  if (N > 0 && route_in_one(N, E))
     return launch_route_small<false>(logits, nullptr, 0, 0, nullptr, nullptr, N, E, k, topk_idx, topk_w, counts,
                                      offsets, perm, slot_pos, cv, stream);
   const int nb = (N + kSelTokens - 1) / kSelTokens;
@@ -592,6 +618,20 @@ int ygg::route_energy_convert(const void* x, int x_dtype, int N, int d, const fl
   if (N > 0 && N <= kSmallMaxN) {
     YGG_CHECK_ARG(x && router_w && router_b && topk_idx && topk_w && perm && slot_pos,
                   "ygg_route_energy: null pointer argument");
+    if (logits_scratch != nullptr && !energy_in_one(N, E, d)) {
+      const unsigned grid = (unsigned)((N + 64 / kSelLanes - 1) / (64 / kSelLanes));
+      switch ((E + 7) / 8) {
+#define YGG_EL(Q)                                                                                                     \
+  case Q:                                                                                                             \
+    router_energy_logits8_kernel<Q><<<grid, 64, 0, stream>>>(x, x_dtype, N, d, router_w, router_b, E, logits_scratch); \
+    break;
+        YGG_EL(1) YGG_EL(2) YGG_EL(3) YGG_EL(4) YGG_EL(5) YGG_EL(6) YGG_EL(7) YGG_EL(8)
+#undef YGG_EL
+      }
+      if (check_launch("router_energy_logits8")) return -1;
+      return ygg::route_convert(logits_scratch, N, E, k, topk_idx, topk_w, counts, offsets, perm, slot_pos, workspace,
+                                workspace_bytes, cv, stream);
+    }
     return launch_route_small<true>(nullptr, x, x_dtype, d, router_w, router_b, N, E, k, topk_idx, topk_w, counts,
                                     offsets, perm, slot_pos, cv, stream);
   }

@@ -417,25 +417,47 @@ __global__ __launch_bounds__(256) void weight_grad_kernel(const float* __restric
 // operand it is Im(D conj(A)).  A wave owns 32 j x 32 i, eight 32 x 32
 // accumulators ((a, c) x (re, im)), 16 MFMAs per row.
 //
-// The rows of one expert are cut into chunks of kWgmChunk rows; every
-// (chunk, 64 x 64 tile) is one workgroup, which writes its Pauli sums to a
-// partial plane of its chunk.  The reduction adds an expert's chunks in chunk
-// order, so the result does not depend on scheduling.  The workgroups of the
-// first i tile also sum the D rows of their chunk for the bias gradient.
-constexpr int kWgmChunk = 384;  // rows per chunk (measured best of 128-2048 at the C3 shape)
+// The rows of one expert are cut into chunks; every (chunk, 64 x 64 tile) is one
+// workgroup, which writes its Pauli sums to a partial plane of its chunk -- or, when the
+// expert has no other chunk, the gradient itself.  The reduction adds the other
+// experts' chunks in chunk order, so the result does not depend on scheduling.  The
+// workgroups of the first i tile also sum the D rows of their chunk for the bias gradient.
+constexpr int kWgmChunk = 384;  // rows per chunk (measured best of 128-2048 at 32768 rows, 512 x 128)
 constexpr int kWgmTile = 64;     // j and i per workgroup (2 x 2 waves of 32)
 constexpr int kWgmU = 2;         // rows per register-buffered block
 
-__device__ inline bool wgm_find_chunk(const int32_t* __restrict__ offsets, int E, int chunk, int& e, int& r0,
-                                      int& r1) {
+// The chunk-th chunk over the experts' ranges: its expert, rows [r0, r1) and whether it is
+// the expert's only one.  Up to 64 experts: a lane each, a scan finds the chunk's.
+__device__ inline bool wgm_find_chunk(const int32_t* __restrict__ offsets, int E, int chunk, int lane, int& e, int& r0,
+                                      int& r1, bool& only) {
+  constexpr int rows = kWgmChunk;
+  if (E <= 64) {
+    const int beg = lane < E ? offsets[lane] : 0, end = lane < E ? offsets[lane + 1] : 0;
+    const int nt = (end - beg + rows - 1) / rows;
+    int incl = nt;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const int v = __shfl_up(incl, o);
+      if (lane >= o) incl += v;
+    }
+    const uint64_t after = __ballot(incl > chunk);
+    if (after == 0) return false;
+    e = (int)__builtin_ctzll(after);
+    const int n = __builtin_amdgcn_readlane(nt, e), first = __builtin_amdgcn_readlane(incl, e) - n;
+    r0 = __builtin_amdgcn_readlane(beg, e) + (chunk - first) * rows;
+    r1 = min(__builtin_amdgcn_readlane(end, e), r0 + rows);
+    only = n == 1;
+    return true;
+  }
   int acc = 0, beg = offsets[0];
   for (int x = 0; x < E; ++x) {
     const int end = offsets[x + 1];
-    const int n = (end - beg + kWgmChunk - 1) / kWgmChunk;
+    const int n = (end - beg + rows - 1) / rows;
     if (chunk < acc + n) {
       e = x;
-      r0 = beg + (chunk - acc) * kWgmChunk;
-      r1 = min(end, r0 + kWgmChunk);
+      r0 = beg + (chunk - acc) * rows;
+      r1 = min(end, r0 + rows);
+      only = n == 1;
       return true;
     }
     acc += n;
@@ -444,28 +466,55 @@ __device__ inline bool wgm_find_chunk(const int32_t* __restrict__ offsets, int E
   return false;
 }
 
-// grid (chunks bound, ceil(d_out / 64), ceil(d_in / 64)), 256 threads.
+// One weight's and one output channel's gradient from the Pauli sums s ([a][c][re, im] of
+// D conj(A), [b][re, im][a] of D): half the blade form.
+__device__ __forceinline__ void store_dw(float* __restrict__ dst, const float* s) {
+  float o[8];
+  pauli_to_blade(s[0], s[1], s[2], s[3], s[4], s[5], s[6], s[7], o);
+  float4* q = reinterpret_cast<float4*>(dst);
+  q[0] = make_float4(0.5f * o[0], 0.5f * o[1], 0.5f * o[2], 0.5f * o[3]);
+  q[1] = make_float4(0.5f * o[4], 0.5f * o[5], 0.5f * o[6], 0.5f * o[7]);
+}
+__device__ __forceinline__ void store_db(float* __restrict__ dst, const float* t) {
+  const float s[8] = {t[0], t[2], t[4], t[6], t[1], t[3], t[5], t[7]};  // entry (a, b): re at b * 4 + a, im at + 2
+  store_dw(dst, s);
+}
+
+// grid (chunks bound, ceil(d_out / T), ceil(d_in / T)), 256 threads: RS = 1, T = 64, a wave per
+// 32 x 32 quadrant; RS = 4, T = 32, the four waves take every fourth block of rows of one
+// 32 x 32 tile and add their sums in wave order through LDS.  RS = 4 serves the grids that
+// would leave CUs idle: a row is a chain of 16 MFMAs of 64 cycles, 0.5 us, so an expert's 64
+// rows took 31 us in one wave (512 rows over 8 experts, skewed, 64 x 256: 42 us each with
+// the longest expert's chain, where the vector-ALU kernel on 32 x 32 tiles took 112).
 // part: (chunks, d_out, d_in, 8) Pauli sums [a][c][re, im]; dbpart: (chunks, d_out, 8)
 // Pauli-row sums [b][re, im][a] of D, or NULL.
-__global__ __launch_bounds__(256) void weight_grad_mfma_kernel(const float* __restrict__ Dp,
+template <int RS>
+__global__ __launch_bounds__(256, 2) void weight_grad_mfma_kernel(const float* __restrict__ Dp,
                                                                const float* __restrict__ Ap,
                                                                const int32_t* __restrict__ gather,
                                                                const int32_t* __restrict__ offsets, int E, int d_in,
                                                                int d_out, float* __restrict__ part,
-                                                               float* __restrict__ dbpart) {
-  int e, r0, r1;
-  if (!wgm_find_chunk(offsets, E, blockIdx.x, e, r0, r1)) return;
-  (void)e;
+                                                               float* __restrict__ dbpart, float* __restrict__ dW,
+                                                               float* __restrict__ db) {
   const int lane = threadIdx.x & 63;
+  int e, r0, r1;
+  bool only;
+  if (!wgm_find_chunk(offsets, E, blockIdx.x, lane, e, r0, r1, only)) return;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   r0 = __builtin_amdgcn_readfirstlane(r0);
   r1 = __builtin_amdgcn_readfirstlane(r1);
   const int l32 = lane & 31, kk = lane >> 5;
-  const int j0 = blockIdx.y * kWgmTile + (wave & 1) * 32, i0 = blockIdx.z * kWgmTile + (wave >> 1) * 32;
+  const int j0 = RS == 1 ? blockIdx.y * kWgmTile + (wave & 1) * 32 : blockIdx.y * 32;
+  const int i0 = RS == 1 ? blockIdx.z * kWgmTile + (wave >> 1) * 32 : blockIdx.z * 32;
+  if constexpr (RS > 1) {  // this wave's share of the rows
+    const int per = (r1 - r0 + RS - 1) / RS;
+    r0 = min(r0 + wave * per, r1);
+    r1 = min(r0 + per, r1);
+  }
   const int jc = min(j0 + l32, d_out - 1), ic = min(i0 + l32, d_in - 1);  // clamped loads, not stored
   const float* dcol = Dp + (size_t)jc * 8 + kk * 2;  // + row * d_out * 8; b = 0 at +0, b = 1 at +4
   const float* acol = Ap + (size_t)ic * 8;           // + src * d_in * 8
-  const bool bias_wave = dbpart != nullptr && blockIdx.z == 0 && (wave >> 1) == 0;
+  const bool bias_wave = dbpart != nullptr && blockIdx.z == 0 && (RS > 1 || (wave >> 1) == 0);
 
   pf32x16_t acc[2][2][2];
 #pragma unroll
@@ -545,23 +594,75 @@ __global__ __launch_bounds__(256) void weight_grad_mfma_kernel(const float* __re
     mma_row(o);
   }
 
+  if constexpr (RS > 1) {  // the waves' sums into wave 0's, (0 + 2) + (1 + 3)
+    __shared__ float4 red[2][8][4][64];
+    __shared__ float4 red_b[3][64];
+    auto put = [&](int slot) __attribute__((always_inline)) {
+#pragma unroll
+      for (int a = 0; a < 8; ++a)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+          const pf32x16_t& x = acc[a >> 2][(a >> 1) & 1][a & 1];
+          red[slot][a][v][lane] = make_float4(x[4 * v], x[4 * v + 1], x[4 * v + 2], x[4 * v + 3]);
+        }
+    };
+    auto add = [&](int slot) __attribute__((always_inline)) {
+#pragma unroll
+      for (int a = 0; a < 8; ++a)
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+          const float4 o = red[slot][a][v][lane];
+          pf32x16_t& x = acc[a >> 2][(a >> 1) & 1][a & 1];
+          x[4 * v] += o.x; x[4 * v + 1] += o.y; x[4 * v + 2] += o.z; x[4 * v + 3] += o.w;
+        }
+    };
+    if (wave >= 2) put(wave - 2);
+    if (wave >= 1) red_b[wave - 1][lane] = make_float4(bs[0], bs[1], bs[2], bs[3]);
+    __syncthreads();
+    if (wave < 2) add(wave);
+    __syncthreads();
+    if (wave == 1) put(0);
+    __syncthreads();
+    if (wave > 0) return;
+    add(0);
+#pragma unroll
+    for (int w = 0; w < RS - 1; ++w) {
+      const float4 o = red_b[w][lane];
+      bs[0] += o.x; bs[1] += o.y; bs[2] += o.z; bs[3] += o.w;
+    }
+  }
   // lane holds column i0 + l32, rows j0 + 8 (v / 4) + 4 kk + v % 4
   const int i = i0 + l32;
-  float* pc = part + (size_t)blockIdx.x * d_out * d_in * 8;
+  float* pc = only ? dW + (size_t)e * d_out * d_in * 8 : part + (size_t)blockIdx.x * d_out * d_in * 8;
   if (i < d_in) {
 #pragma unroll
     for (int v = 0; v < 16; ++v) {
       const int j = j0 + 8 * (v >> 2) + 4 * kk + (v & 3);
       if (j >= d_out) continue;
-      float4* q = reinterpret_cast<float4*>(pc + ((size_t)j * d_in + i) * 8);
-      q[0] = make_float4(acc[0][0][0][v], acc[0][0][1][v], acc[0][1][0][v], acc[0][1][1][v]);
-      q[1] = make_float4(acc[1][0][0][v], acc[1][0][1][v], acc[1][1][0][v], acc[1][1][1][v]);
+      const float o[8] = {acc[0][0][0][v], acc[0][0][1][v], acc[0][1][0][v], acc[0][1][1][v],
+                          acc[1][0][0][v], acc[1][0][1][v], acc[1][1][0][v], acc[1][1][1][v]};
+      float* dst = pc + ((size_t)j * d_in + i) * 8;
+      if (only) {
+        store_dw(dst, o);
+      } else {
+        reinterpret_cast<float4*>(dst)[0] = make_float4(o[0], o[1], o[2], o[3]);
+        reinterpret_cast<float4*>(dst)[1] = make_float4(o[4], o[5], o[6], o[7]);
+      }
     }
   }
-  if (bias_wave && j0 + l32 < d_out) {
-    float* q = dbpart + ((size_t)blockIdx.x * d_out + j0 + l32) * 8 + kk * 2;  // [b][k][a]
-    *reinterpret_cast<float2*>(q) = make_float2(bs[0], bs[1]);
-    *reinterpret_cast<float2*>(q + 4) = make_float2(bs[2], bs[3]);
+  if (bias_wave) {  // this lane's (re or im) entries of the row sums, its partner's the others
+    const float x0 = __shfl_xor(bs[0], 32), x1 = __shfl_xor(bs[1], 32), x2 = __shfl_xor(bs[2], 32),
+                x3 = __shfl_xor(bs[3], 32);
+    const float t[8] = {bs[0], bs[1], x0, x1, bs[2], bs[3], x2, x3};  // [b][k][a]
+    if (kk == 0 && j0 + l32 < d_out) {
+      if (only) {
+        store_db(db + ((size_t)e * d_out + j0 + l32) * 8, t);
+      } else {
+        float4* q = reinterpret_cast<float4*>(dbpart + ((size_t)blockIdx.x * d_out + j0 + l32) * 8);
+        q[0] = make_float4(t[0], t[1], t[2], t[3]);
+        q[1] = make_float4(t[4], t[5], t[6], t[7]);
+      }
+    }
   }
 }
 
@@ -579,8 +680,8 @@ __global__ __launch_bounds__(256) void weight_grad_mfma_kernel(const float* __re
 __global__ __launch_bounds__(256, 2) void weight_grad_split_kernel(
     const unsigned char* __restrict__ Ds, const int32_t* __restrict__ d_exp, const unsigned char* __restrict__ As,
     uint32_t a_bytes, const int32_t* __restrict__ a_exp, const int32_t* __restrict__ gather,
-    const int32_t* __restrict__ offsets, int E, int d_in, int d_out, int n_chunks, int n_xcd, float* __restrict__ part,
-    float* __restrict__ dbpart) {
+    const int32_t* __restrict__ offsets, int E, int d_in, int d_out, int n_chunks, int n_xcd,
+    float* __restrict__ part, float* __restrict__ dbpart, float* __restrict__ dW, float* __restrict__ db) {
   typedef unsigned int u32x2_t __attribute__((ext_vector_type(2)));
   __shared__ alignas(8) uint32_t s_delta[kWgmChunk];  // the row's ratio, twice, as fp16
   __shared__ alignas(8) uint32_t s_src[kWgmChunk];    // byte offset of the row of A
@@ -589,10 +690,10 @@ __global__ __launch_bounds__(256, 2) void weight_grad_split_kernel(
   const int nj = (d_out + kWgmTile - 1) / kWgmTile, ni = (d_in + kWgmTile - 1) / kWgmTile, nt = nj * ni;
   const int xcd = blockIdx.x % n_xcd, bq = blockIdx.x / n_xcd;
   const int chunk = bq / nt * n_xcd + xcd, tile = bq % nt;
-  int e, r0, r1;
-  if (chunk >= n_chunks || !wgm_find_chunk(offsets, E, chunk, e, r0, r1)) return;
-  (void)e;
   const int tid = threadIdx.x, lane = tid & 63;
+  int e, r0, r1;
+  bool only;
+  if (chunk >= n_chunks || !wgm_find_chunk(offsets, E, chunk, lane, e, r0, r1, only)) return;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   r0 = __builtin_amdgcn_readfirstlane(r0);
   r1 = __builtin_amdgcn_readfirstlane(r1);
@@ -723,7 +824,7 @@ __global__ __launch_bounds__(256, 2) void weight_grad_split_kernel(
 
   // lane holds column i0 + l32, rows j0 + 8 (v / 4) + 4 g + v % 4
   const int i = i0 + l32;
-  float* pc = part + (size_t)chunk * d_out * d_in * 8;
+  float* pc = only ? dW + (size_t)e * d_out * d_in * 8 : part + (size_t)chunk * d_out * d_in * 8;
   if (i < d_in) {
 #pragma unroll
     for (int v = 0; v < 16; ++v) {
@@ -736,67 +837,69 @@ __global__ __launch_bounds__(256, 2) void weight_grad_split_kernel(
         for (int c = 0; c < 2; ++c)
 #pragma unroll
           for (int q = 0; q < 2; ++q) o[a * 4 + c * 2 + q] = __builtin_ldexpf(acc[a][c][q][v], -Q);
-      float4* q = reinterpret_cast<float4*>(pc + ((size_t)j * d_in + i) * 8);
-      q[0] = make_float4(o[0], o[1], o[2], o[3]);
-      q[1] = make_float4(o[4], o[5], o[6], o[7]);
+      float* dst = pc + ((size_t)j * d_in + i) * 8;
+      if (only) {
+        store_dw(dst, o);
+      } else {
+        reinterpret_cast<float4*>(dst)[0] = make_float4(o[0], o[1], o[2], o[3]);
+        reinterpret_cast<float4*>(dst)[1] = make_float4(o[4], o[5], o[6], o[7]);
+      }
     }
   }
   if (bias_wave) {
-    float* o = &bs[0][0][0];
+    float t[8];  // [b][k][a]
 #pragma unroll
-    for (int q = 0; q < 8; ++q) o[q] += __shfl_xor(o[q], 32);
+    for (int q = 0; q < 8; ++q) {
+      t[q] = bs[q >> 2][(q >> 1) & 1][q & 1];
+      t[q] += __shfl_xor(t[q], 32);
+    }
     if (g == 0 && j0 + l32 < d_out) {
-      float4* q = reinterpret_cast<float4*>(dbpart + ((size_t)chunk * d_out + j0 + l32) * 8);  // [b][k][a]
-      q[0] = make_float4(bs[0][0][0], bs[0][0][1], bs[0][1][0], bs[0][1][1]);
-      q[1] = make_float4(bs[1][0][0], bs[1][0][1], bs[1][1][0], bs[1][1][1]);
+      if (only) {
+        store_db(db + ((size_t)e * d_out + j0 + l32) * 8, t);
+      } else {
+        float4* q = reinterpret_cast<float4*>(dbpart + ((size_t)chunk * d_out + j0 + l32) * 8);
+        q[0] = make_float4(t[0], t[1], t[2], t[3]);
+        q[1] = make_float4(t[4], t[5], t[6], t[7]);
+      }
     }
   }
 }
 
 // dW[e, j, i] = (1/2) blade(sum over the expert's chunks, in order, of the Pauli sums);
-// db[e, j] likewise from the D-row sums.  One thread per (e, j, i) multivector.
+// db[e, j] likewise from the D-row sums; zero for an expert without rows.  (An expert of
+// one chunk has its gradient already.)  One thread per multivector, blockIdx.y the expert.
 __global__ __launch_bounds__(256) void weight_grad_reduce_kernel(const float* __restrict__ part,
                                                                  const float* __restrict__ dbpart,
                                                                  const int32_t* __restrict__ offsets, int E, int d_in,
                                                                  int d_out, float* __restrict__ dW,
                                                                  float* __restrict__ db) {
-  const size_t n = (size_t)blockIdx.x * 256 + threadIdx.x;
-  if (n >= (size_t)E * d_out * d_in) return;
-  const size_t ji = n % ((size_t)d_out * d_in);
-  const int e = (int)(n / ((size_t)d_out * d_in));
-  int cb = 0, beg = offsets[0];
-  for (int x = 0; x < e; ++x) {
-    const int end = offsets[x + 1];
-    cb += (end - beg + kWgmChunk - 1) / kWgmChunk;
-    beg = end;
-  }
-  const int ce = cb + (offsets[e + 1] - beg + kWgmChunk - 1) / kWgmChunk;
-  float s[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-  for (int c = cb; c < ce; ++c) {
-    const float4* q = reinterpret_cast<const float4*>(part + ((size_t)c * d_out * d_in + ji) * 8);
-    const float4 u = q[0], w = q[1];
-    s[0] += u.x; s[1] += u.y; s[2] += u.z; s[3] += u.w;
-    s[4] += w.x; s[5] += w.y; s[6] += w.z; s[7] += w.w;
-  }
-  float o[8];
-  pauli_to_blade(s[0], s[1], s[2], s[3], s[4], s[5], s[6], s[7], o);
-  float4* dst = reinterpret_cast<float4*>(dW + n * 8);
-  dst[0] = make_float4(0.5f * o[0], 0.5f * o[1], 0.5f * o[2], 0.5f * o[3]);
-  dst[1] = make_float4(0.5f * o[4], 0.5f * o[5], 0.5f * o[6], 0.5f * o[7]);
-  if (db != nullptr && ji % d_in == 0) {
-    const int j = (int)(ji / d_in);
-    float t[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};  // [b][k][a]
-    for (int c = cb; c < ce; ++c) {
-      const float4* q = reinterpret_cast<const float4*>(dbpart + ((size_t)c * d_out + j) * 8);
+  constexpr int rows = kWgmChunk;
+  const int e = blockIdx.y, lane = threadIdx.x & 63;
+  const int ce = (offsets[e + 1] - offsets[e] + rows - 1) / rows;
+  if (ce == 1) return;
+  int cb = 0;  // the chunks before the expert's
+  for (int x = lane; x < e; x += 64) cb += (offsets[x + 1] - offsets[x] + rows - 1) / rows;
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) cb += __shfl_xor(cb, o);
+  const size_t ji = (size_t)blockIdx.x * 256 + threadIdx.x, n = (size_t)d_out * d_in;
+  if (ji >= n) return;
+  auto sum = [&](const float* p, size_t stride, float* s) __attribute__((always_inline)) {
+#pragma unroll
+    for (int c = 0; c < 8; ++c) s[c] = 0.f;
+#pragma unroll 4
+    for (int c = 0; c < ce; ++c) {
+      const float4* q = reinterpret_cast<const float4*>(p + (size_t)c * stride);
       const float4 u = q[0], w = q[1];
-      t[0] += u.x; t[1] += u.y; t[2] += u.z; t[3] += u.w;
-      t[4] += w.x; t[5] += w.y; t[6] += w.z; t[7] += w.w;
+      s[0] += u.x; s[1] += u.y; s[2] += u.z; s[3] += u.w;
+      s[4] += w.x; s[5] += w.y; s[6] += w.z; s[7] += w.w;
     }
-    // entry (a, b): re at b * 4 + a, im at b * 4 + 2 + a
-    pauli_to_blade(t[0], t[2], t[4], t[6], t[1], t[3], t[5], t[7], o);
-    float4* q = reinterpret_cast<float4*>(db + ((size_t)e * d_out + j) * 8);
-    q[0] = make_float4(0.5f * o[0], 0.5f * o[1], 0.5f * o[2], 0.5f * o[3]);
-    q[1] = make_float4(0.5f * o[4], 0.5f * o[5], 0.5f * o[6], 0.5f * o[7]);
+  };
+  float s[8];
+  sum(part + ((size_t)cb * n + ji) * 8, n * 8, s);
+  store_dw(dW + ((size_t)e * n + ji) * 8, s);
+  if (db != nullptr && ji < (size_t)d_out) {
+    sum(dbpart + ((size_t)cb * d_out + ji) * 8, (size_t)d_out * 8, s);
+    store_db(db + ((size_t)e * d_out + ji) * 8, s);
   }
 }
 
@@ -823,14 +926,17 @@ int weight_grad_pauli(const float* dy_pauli, const float* a_pauli, const int32_t
   float* part = static_cast<float*>(workspace);
   float* dbpart = db ? part + chunks * d_out * d_in * 8 : nullptr;
   if (P_max > 0) {
-    hipLaunchKernelGGL(weight_grad_mfma_kernel,
-                       dim3((unsigned)chunks, (d_out + kWgmTile - 1) / kWgmTile, (d_in + kWgmTile - 1) / kWgmTile),
-                       dim3(256), 0, stream, dy_pauli, a_pauli, gather, offsets, E, d_in, d_out, part, dbpart);
+    const dim3 g64((unsigned)chunks, (d_out + kWgmTile - 1) / kWgmTile, (d_in + kWgmTile - 1) / kWgmTile);
+    if ((size_t)g64.x * g64.y * g64.z >= 512)  // two workgroups per CU
+      hipLaunchKernelGGL(weight_grad_mfma_kernel<1>, g64, dim3(256), 0, stream, dy_pauli, a_pauli, gather, offsets, E,
+                         d_in, d_out, part, dbpart, dW, db);
+    else
+      hipLaunchKernelGGL(weight_grad_mfma_kernel<4>, dim3((unsigned)chunks, (d_out + 31) / 32, (d_in + 31) / 32),
+                         dim3(256), 0, stream, dy_pauli, a_pauli, gather, offsets, E, d_in, d_out, part, dbpart, dW, db);
     if (check_launch("weight gradient (MFMA)")) return -1;
   }
-  const size_t n = (size_t)E * d_out * d_in;
-  hipLaunchKernelGGL(weight_grad_reduce_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, stream, part, dbpart,
-                     offsets, E, d_in, d_out, dW, db);
+  hipLaunchKernelGGL(weight_grad_reduce_kernel, dim3((unsigned)(((size_t)d_out * d_in + 255) / 256), E), dim3(256), 0,
+                     stream, part, dbpart, offsets, E, d_in, d_out, dW, db);
   return check_launch("weight gradient (reduction)");
 }
 
@@ -854,12 +960,11 @@ int weight_grad_split(const void* dy, const int32_t* dy_exp, const void* a, int 
                        dim3(256), 0, stream, static_cast<const unsigned char*>(dy), dy_exp,
                        static_cast<const unsigned char*>(a),
                        gather ? (uint32_t)((size_t)a_rows * pauli_split_row_bytes(d_in)) : 0u, a_exp, gather, offsets, E,
-                       d_in, d_out, (int)chunks, n_xcd, part, dbpart);
+                       d_in, d_out, (int)chunks, n_xcd, part, dbpart, dW, db);
     if (check_launch("weight gradient (split)")) return -1;
   }
-  const size_t n = (size_t)E * d_out * d_in;
-  hipLaunchKernelGGL(weight_grad_reduce_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, stream, part, dbpart,
-                     offsets, E, d_in, d_out, dW, db);
+  hipLaunchKernelGGL(weight_grad_reduce_kernel, dim3((unsigned)(((size_t)d_out * d_in + 255) / 256), E), dim3(256), 0,
+                     stream, part, dbpart, offsets, E, d_in, d_out, dW, db);
   return check_launch("weight gradient (reduction)");
 }
 

@@ -503,8 +503,6 @@ YGG_API int ygg_moe_block_ffn(const void* x, int dtype, int N, int d, int F, int
 // same inputs), so perm, slot_pos and offsets match the forward's; so are the
 // activations the backward needs (h before and after the activation, y).
 // The regions of its workspace, in order (each 256-byte aligned).
-constexpr int kWgradMfmaRowsPerExpert = 256;  // mean rows per expert from which the MFMA weight gradient runs
-
 static int bw_regions(int N, int d, int F, int E, int k, size_t* r) {
   const size_t P = (size_t)N * k;
   int n = 0;
@@ -590,21 +588,18 @@ YGG_API int ygg_moe_backward(const float* x, int N, int d, int F, int E, int k, 
   float* fp = static_cast<float*>(take());  // Pauli rows of h, then of dh_pre
   float* dh = static_cast<float*>(take());  // dh, then dh_pre in place
   float* y = static_cast<float*>(take());   // y, then dx rows
-  float* dy = static_cast<float*>(take());
+  take();  // (a region of dy's size: the workspace's layout is kept)
   float* dp = static_cast<float*>(take());  // Pauli rows of dy
   void* wg = take();                        // weight-gradient partial sums
 
   // forward recompute: h_pre (unless the forward kept it), h (Pauli rows), y (blade, for dtopk_w)
   const float* hp_in = h_pre_saved;
-  // the MFMA weight gradient pays off with enough rows per expert; below that the
-  // vector-ALU kernel, which spreads a tile's pairs over more waves, is faster
-  const bool wg_mfma = P >= (size_t)kWgradMfmaRowsPerExpert * E;
   // split products and weight gradients, where the forward's products were split
   const bool split = hp_in && f32_split(N, d, F, E, k, kWPauliF32) && weight_grad_split_fits(N, true, d, F) &&
                      weight_grad_split_fits((int)P, false, F, d);
-  // x's Pauli rows, when needed, are converted by extra workgroups of the routing launch
+  // x's Pauli rows are converted by extra workgroups of the routing launch
   ygg::RowConvert cv;
-  if ((!hp_in || wg_mfma) && !split) {
+  if (!split) {
     cv.x = x;
     cv.out = xp;
     cv.n = (long long)N * d;
@@ -649,27 +644,22 @@ YGG_API int ygg_moe_backward(const float* x, int N, int d, int F, int E, int k, 
       return -1;
     hp_in = h_pre;
   }
-  // h as Pauli rows for the down product (and in blade order for the vector-ALU weight gradient)
-  if (activation_forward(hp_in, P * F, act, wg_mfma ? nullptr : h, fp, stream)) return -1;
+  // h as Pauli rows for the down product and its weight gradient
+  if (activation_forward(hp_in, P * F, act, nullptr, fp, stream)) return -1;
   if (dtopk_w &&
       ygg_pauli_grouped_linear_f32(fp, nullptr, (int)P, w_down, b_down, offsets, E, F, d, kActNone, y, 1, stream))
     return -1;
   // combine backward -> dy; down backward -> dh, dW_down, db_down
-  if (combine_backward(dout, dtopk_w ? y : nullptr, N, k, d, tw, slot_pos, wg_mfma ? nullptr : dy, dp, dtopk_w,
-                       stream))
+  if (combine_backward(dout, dtopk_w ? y : nullptr, N, k, d, tw, slot_pos, nullptr, dp, dtopk_w, stream))
     return -1;
   if (ygg_pauli_grouped_linear_f32(dp, nullptr, (int)P, w_down_adj, nullptr, offsets, E, d, F, kActNone, dh, 1, stream))
     return -1;
-  if (wg_mfma ? weight_grad_pauli(dp, fp, nullptr, offsets, (int)P, E, F, d, dw_down, db_down, wg, stream)
-              : grouped_weight_grad(dy, h, nullptr, offsets, E, F, d, dw_down, db_down, stream))
-    return -1;
+  if (weight_grad_pauli(dp, fp, nullptr, offsets, (int)P, E, F, d, dw_down, db_down, wg, stream)) return -1;
   // activation backward -> Pauli rows of dh before the activation; up backward -> dx rows, dW_up, db_up
-  if (activation_backward(hp_in, dh, P * F, act, wg_mfma ? nullptr : dh, fp, stream)) return -1;
+  if (activation_backward(hp_in, dh, P * F, act, nullptr, fp, stream)) return -1;
   if (ygg_pauli_grouped_linear_f32(fp, nullptr, (int)P, w_up_adj, nullptr, offsets, E, F, d, kActNone, y, 1, stream))
     return -1;
-  if (wg_mfma ? weight_grad_pauli(fp, xp, perm, offsets, (int)P, E, d, F, dw_up, db_up, wg, stream)
-              : grouped_weight_grad(dh, x, perm, offsets, E, d, F, dw_up, db_up, stream))
-    return -1;
+  if (weight_grad_pauli(fp, xp, perm, offsets, (int)P, E, d, F, dw_up, db_up, wg, stream)) return -1;
   // dispatch backward: each token's rows summed, plus dout when the forward added x
   return dispatch_backward(y, N, k, d, slot_pos, residual ? dout : nullptr, dx, stream);
 }

@@ -261,6 +261,14 @@ int ygg_moe_forward_noalloc(const void* x, int dtype, int N, int d, int F, int E
                             int w_format, const void* residual, void* out, int32_t* topk_idx, float* topk_w,
                             int32_t* counts, int32_t* offsets, ygg_stream_t stream);
 
+/* sum_e (f_e - 1/E)^2 with f = counts / (sum of counts + 1e-12), fp32
+ * (CliffordRouter.load_balance_loss, clifford_router.py:108-117): one value at out. */
+int ygg_balance_loss(const int32_t* counts, int E, float* out, ygg_stream_t stream);
+
+/* ygg_adjoint_weights_f32 prepared in format 4 (E experts, d_in outputs, d_out inputs), in
+ * one pass over W (E, d_out, d_in, 8) fp32. */
+int ygg_prepare_adjoint_weights_f32(const float* W, int E, int d_out, int d_in, void* out, ygg_stream_t stream);
+
 /* ---- backward (fp32) ---------------------------------------------------------------
  * The reference has no MoE backward (hlm_block.py:202-206); these follow
  * CliffordLinear.backward (holograph/layers/clifford_linear.py:125-163) and

@@ -69,3 +69,43 @@ def test_route_paths_agree(N, E, k):
             assert torch.equal(a.topk_idx[0], one.topk_idx[0]) and torch.equal(a.topk_w[0], one.topk_w[0])
             sep = ops.route(ops.router_energy_logits(x, rw, rb), k)
             assert (a.topk_idx != sep.topk_idx).float().mean().item() < 0.02  # another order of the sums: ties only
+
+
+@pytest.mark.parametrize("E,d_in,d_out,counts", [
+    (3, 33, 40, (0, 5, 1)),          # a row split over more waves than rows, an empty expert
+    (8, 64, 256, (120, 3, 0, 64, 65, 63, 130, 67)),
+    (2, 20, 30, (400, 1000)),        # several chunks per expert
+    (70, 9, 17, tuple(range(70))),   # more experts than lanes
+])
+def test_weight_gradient_row_split(E, d_in, d_out, counts):
+    """The weight gradient of few rows: each expert against float64 (sums of up to 1000 rows x 4 terms in fp32:
+    2^-24 sqrt(4000) of a random sum; 1e-5)."""
+    from yggdrasil_amd import ops
+
+    g = np.random.default_rng(E + d_in)
+    P = sum(counts)
+    off = np.concatenate([[0], np.cumsum(counts)]).astype(np.int32)
+    a, dy = (g.standard_normal((P, n, 8)).astype(np.float32) for n in (d_in, d_out))
+    say(f"weight gradient E={E} {d_in} x {d_out}")
+    dW, db = ops.grouped_weight_grad_pauli(ops.pauli_rows_from_blade_f32(torch.from_numpy(dy).cuda()),
+                                           ops.pauli_rows_from_blade_f32(torch.from_numpy(a).cuda()),
+                                           torch.from_numpy(off).cuda(), E)
+    for e in range(E):
+        _, want, want_b = dense.linear_backward(a[off[e]:off[e + 1]], np.zeros((d_out, d_in, 8)), dy[off[e]:off[e + 1]])
+        if counts[e] == 0:
+            assert not dW[e].any() and not db[e].any()
+        else:
+            assert normwise_err(dW[e].cpu().numpy(), want) < 1e-5 and normwise_err(db[e].cpu().numpy(), want_b) < 1e-5
+
+
+def test_adjoint_preparation_and_balance_loss():
+    """One-pass adjoint weights equal the two-pass ones bit for bit; the balance loss is the formula's."""
+    from yggdrasil_amd import ops
+
+    w = torch.randn(3, 37, 50, 8, device="cuda")
+    assert torch.equal(ops.prepare_adjoint_weights(w).data, ops.prepare_weights(ops.adjoint_weights(w), "pauli_f32").data)
+    for E in (1, 8, 64, 100):
+        c = torch.randint(0, 3000, (E,), device="cuda", dtype=torch.int32)
+        f = c.double() / (c.double().sum() + 1e-12)
+        assert abs(ops.balance_loss(c).item() - ((f - 1.0 / E) ** 2).sum().item()) <= 1e-6 * max(1.0 / E, 1e-3)
+    assert ops.balance_loss(torch.zeros(8, device="cuda", dtype=torch.int32)).item() == pytest.approx(1.0 / 8)

@@ -55,6 +55,8 @@ SIGNATURES = {
                                  _c_size, _vp]),
     "ygg_moe_forward_noalloc": (_c_int, [_vp, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _vp, _vp, _vp,
                                          _vp, _vp, _vp, _vp, _vp, _vp, _c_int, _vp, _vp, _vp, _vp, _vp, _vp, _vp]),
+    "ygg_balance_loss": (_c_int, [_vp, _c_int, _vp, _vp]),
+    "ygg_prepare_adjoint_weights_f32": (_c_int, [_vp, _c_int, _c_int, _c_int, _vp, _vp]),
     "ygg_adjoint_weights_f32": (_c_int, [_vp, _c_int, _c_int, _c_int, _vp, _vp]),
     "ygg_grouped_weight_grad_f32": (_c_int, [_vp, _vp, _vp, _vp, _c_int, _c_int, _c_int, _vp, _vp, _vp]),
     "ygg_grouped_weight_grad_pauli_f32_workspace_bytes": (_c_size, [_c_int, _c_int, _c_int, _c_int]),
@@ -108,6 +110,9 @@ def check(status: int, what: str = "") -> None:
 
 
 def stream_handle(device=None) -> int:
+    """The current stream of a tensor's device (read on every call, without building a Stream object)."""
+    if device is not None and device.index is not None:
+        return torch._C._cuda_getCurrentRawStream(device.index)
     return torch.cuda.current_stream(device).cuda_stream
 
 

@@ -484,6 +484,32 @@ __global__ __launch_bounds__(256) void pauli_f32_prep_kernel(const float* __rest
     }
 }
 
+// The adjoint weights Wadj[e, i, j] = ~W[e, j, i] in format 4 from W (E, d_out, d_in, 8)
+// blade: reversion is the conjugate transpose of the matrix, so entry (a, c) of Wadj is the
+// conjugate of entry (c, a) of W.  One thread per (e, j, i); the records of one (e, j) are
+// contiguous over i, as W is.
+__global__ __launch_bounds__(256) void pauli_f32_prep_adjoint_kernel(const float* __restrict__ W, int E, int d_out,
+                                                                     int d_in, float* __restrict__ out) {
+  const size_t n = (size_t)blockIdx.x * 256 + threadIdx.x;
+  if (n >= (size_t)E * d_out * d_in) return;
+  const int i = (int)(n % d_in);
+  const size_t ej = n / d_in;
+  const float4 p0 = reinterpret_cast<const float4*>(W + n * 8)[0], p1 = reinterpret_cast<const float4*>(W + n * 8)[1];
+  const float x[8] = {0.5f * p0.x, 0.5f * p0.y, 0.5f * p0.z, 0.5f * p0.w, 0.5f * p1.x, 0.5f * p1.y, 0.5f * p1.z, 0.5f * p1.w};
+  float c0[4], c1[4];
+  blade_to_pauli(x, c0, c1);  // c0 = (M00, M10), c1 = (M01, M11)
+  // [c][a] of Wadj: conj(W[c][a])
+  const float u[2][2] = {{c0[0], c1[0]}, {c0[2], c1[2]}}, v[2][2] = {{-c0[1], -c1[1]}, {-c0[3], -c1[3]}};
+  // Wadj has d_out inputs (j) and d_in outputs (i): record k of input j, output i
+  float4* r0 = reinterpret_cast<float4*>(out + ((ej * 2 + 0) * d_in + i) * 8);
+  float4* r1 = reinterpret_cast<float4*>(out + ((ej * 2 + 1) * d_in + i) * 8);
+#pragma unroll
+  for (int c = 0; c < 2; ++c) {
+    r0[c] = make_float4(u[c][0], v[c][0], u[c][1], v[c][1]);
+    r1[c] = make_float4(-v[c][0], u[c][0], -v[c][1], u[c][1]);
+  }
+}
+
 // blade fp32 rows (rows, d, 8) -> Pauli rows; one thread per multivector
 __global__ __launch_bounds__(256) void blade_to_pauli_f32_rows_kernel(const float* __restrict__ x, int rows, int d,
                                                                       float* __restrict__ out) {
@@ -612,6 +638,17 @@ int ygg::pauli_f32_prepare_weights(const float* W, int E, int d_out, int d_in, v
   pauli_f32_prep_kernel<<<(unsigned)((total + 255) / 256), 256, 0, stream>>>(W, E, d_out, d_in,
                                                                              static_cast<float*>(out));
   return check_launch("pauli_f32_prep");
+}
+
+YGG_API int ygg_prepare_adjoint_weights_f32(const float* W, int E, int d_out, int d_in, void* out,
+                                            hipStream_t stream) {
+  YGG_CHECK_ARG(E >= 0 && d_out >= 0 && d_in >= 0, "ygg_prepare_adjoint_weights_f32: bad sizes");
+  const size_t total = (size_t)E * d_out * d_in;
+  if (total == 0) return 0;
+  YGG_CHECK_ARG(W && out, "ygg_prepare_adjoint_weights_f32: null pointer");
+  pauli_f32_prep_adjoint_kernel<<<(unsigned)((total + 255) / 256), 256, 0, stream>>>(W, E, d_out, d_in,
+                                                                                     static_cast<float*>(out));
+  return check_launch("pauli_f32_prep_adjoint");
 }
 
 // Contraction splits of the partial-plane product: as many as keep every workgroup of

@@ -641,3 +641,30 @@ int ygg::route_energy_convert(const void* x, int x_dtype, int N, int d, const fl
   return ygg::route_convert(logits_scratch, N, E, k, topk_idx, topk_w, counts, offsets, perm, slot_pos, workspace,
                             workspace_bytes, cv, stream);
 }
+
+namespace {
+// one wave: the counts' sum (whole numbers), then the squares of f_e - 1 / E in lane order
+__global__ __launch_bounds__(64) void balance_loss_kernel(const int32_t* __restrict__ counts, int E,
+                                                          float* __restrict__ out) {
+  const int lane = threadIdx.x;
+  long long n = 0;
+  for (int e = lane; e < E; e += 64) n += counts[e];
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) n += __shfl_xor(n, o);
+  const float total = (float)n + 1e-12f, even = 1.0f / (float)E;
+  float s = 0.f;
+  for (int e = lane; e < E; e += 64) {
+    const float f = (float)counts[e] / total - even;
+    s += f * f;
+  }
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o);
+  if (lane == 0) *out = s;
+}
+}  // namespace
+
+YGG_API int ygg_balance_loss(const int32_t* counts, int E, float* out, hipStream_t stream) {
+  YGG_CHECK_ARG(E >= 1 && counts && out, "ygg_balance_loss: bad arguments (E=%d)", E);
+  balance_loss_kernel<<<1, 64, 0, stream>>>(counts, E, out);
+  return check_launch("balance_loss");
+}

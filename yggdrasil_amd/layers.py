@@ -140,8 +140,21 @@ class CliffordMoELayer(nn.Module):
                 p.copy_(deq)
         self._prepared = None
 
+    @property
+    def last_routing(self):
+        """The last call's ``topk_idx``, ``topk_w``, ``counts`` and ``offsets`` (None before the first)."""
+        r = self.__dict__.get("_last_routing")
+        if isinstance(r, ops.LayerRouting):  # the tensors are made when they are asked for
+            r = self.__dict__["_last_routing"] = r.arrays()
+        return r
+
+    @last_routing.setter
+    def last_routing(self, routing):
+        self.__dict__["_last_routing"] = routing
+
     def _param_versions(self):
-        return tuple(p._version for p in self.parameters()) + (self.w_up.device,)
+        p = self._parameters
+        return [v._version for v in p.values() if v is not None] + [p["w_up"].device]
 
     @torch.no_grad()
     def prepare(self):
@@ -178,41 +191,51 @@ class CliffordMoELayer(nn.Module):
             raise ValueError(f"expected (B, T, {cfg.d_model}, 8), got {tuple(x.shape)}")
         if x.dtype != cfg.dtype:
             raise ValueError(f"layer dtype is {cfg.dtype}, input is {x.dtype}")
-        B, T = x.shape[:2]
-        flat = x.reshape(B * T, cfg.d_model, 8).contiguous()
+        B, T, d = x.shape[:3]
+        N, E = B * T, cfg.n_experts
+        if not x.is_contiguous():
+            x = x.contiguous()
         prep = self._get_prepared()
         if cfg.router == "logits":
             if logits is None:
                 raise ValueError("router='logits' needs logits")
         elif cfg.router == "clifford_head" and logits is None:
-            logits = self._head_logits(flat, prep)
-        if logits is not None:
-            logits = logits.reshape(B * T, cfg.n_experts).float().contiguous()
-        res = residual.reshape(B * T, cfg.d_model, 8).contiguous() if residual is not None else None
-        ws_bytes = ops.moe_workspace_bytes(B * T, cfg.d_model, cfg.d_ff, cfg.n_experts, cfg.top_k, cfg.dtype,
-                                           cfg.weight_format)
-        if self._workspace is None or self._workspace.numel() < ws_bytes or self._workspace.device != x.device:
-            self._workspace = torch.empty((max(ws_bytes, 1),), device=x.device, dtype=torch.uint8)
+            logits = self._head_logits(x.reshape(N, d, 8), prep)
+        if logits is not None and not (logits.dtype == torch.float32 and logits.dim() > 0 and logits.shape[-1] == E and
+                                       logits.numel() == N * E and logits.is_contiguous()):
+            logits = logits.reshape(N, E).float().contiguous()
+        if residual is not None:
+            if residual.shape != x.shape or not residual.is_contiguous():
+                residual = residual.reshape(x.shape).contiguous()
+            if residual.dtype != x.dtype:
+                raise ValueError("residual must have x's shape and dtype")
+        ws_bytes = ops.moe_workspace_bytes(N, d, cfg.d_ff, E, cfg.top_k, cfg.dtype, cfg.weight_format)
+        ws = self.__dict__["_workspace"]
+        if ws is None or ws.numel() < ws_bytes or ws.device != x.device:
+            ws = self.__dict__["_workspace"] = torch.empty((max(ws_bytes, 1),), device=x.device, dtype=torch.uint8)
         if self._needs_grad(x, residual):
-            out = _MoEFunction.apply(flat, res, self.w_up, self.b_up, self.w_down, self.b_down, self, logits)
-        else:
-            out = self._forward_flat(flat, logits, res)
-        return out.reshape(B, T, cfg.d_model, 8)
-
-    def _forward_flat(self, flat, logits, res):
-        cfg, prep = self.cfg, self._get_prepared()
-        out, routing = ops.moe_forward(flat, cfg.top_k, prep["w_up"], prep["w_down"], prep["b_up"], prep["b_down"],
-                                       cfg.activation, logits=logits,
-                                       router_weight=self.router_weight.detach() if logits is None else None,
-                                       router_bias=self.router_bias.detach() if logits is None else None,
-                                       residual=res, workspace=self._workspace)
-        self.last_routing = routing
+            flat = x.reshape(N, d, 8)
+            res = residual.reshape(N, d, 8) if residual is not None else None
+            lg = logits.reshape(N, E) if logits is not None else None
+            return _MoEFunction.apply(flat, res, self.w_up, self.b_up, self.w_down, self.b_down, self, lg).reshape(B, T, d, 8)
+        rw = rb = None
+        if logits is None:
+            p = self._parameters
+            rw, rb = p["router_weight"].detach(), p["router_bias"].detach()
+            if rw.dtype != torch.float32 or not rw.is_contiguous():
+                rw = rw.float().contiguous()
+            if rb.dtype != torch.float32 or not rb.is_contiguous():
+                rb = rb.float().contiguous()
+        ops._dev(x, logits, residual, rw, rb, prep["b_up"], prep["b_down"])
+        out, routing = ops.layer_forward(x, N, cfg.top_k, prep["w_up"], prep["w_down"], prep["b_up"], prep["b_down"],
+                                         cfg.activation, logits, rw, rb, residual, ws, ws_bytes)
+        self.__dict__["_last_routing"] = routing
         return out
 
     def _needs_grad(self, x, residual) -> bool:
         """Autograd runs for fp32 layers with 'pauli_f32' weights (the backward's format);
         other formats compute the forward only and their output carries no graph."""
-        if not torch.is_grad_enabled() or self.cfg.weight_format != "pauli_f32":
+        if self.cfg.weight_format != "pauli_f32" or not torch.is_grad_enabled():
             return False
         return x.requires_grad or (residual is not None and residual.requires_grad) or any(
             p.requires_grad for p in (self.w_up, self.b_up, self.w_down, self.b_down))
@@ -222,11 +245,8 @@ class CliffordMoELayer(nn.Module):
         """Adjoint expert weights (reverse, channel axes exchanged) in the 'pauli_f32' layout."""
         key = self._param_versions()
         if getattr(self, "_adjoint", None) is None or self._adjoint["key"] != key:
-            self._adjoint = dict(key=key,
-                                 w_up=ops.prepare_weights(ops.adjoint_weights(self.w_up.detach().contiguous()),
-                                                          "pauli_f32"),
-                                 w_down=ops.prepare_weights(ops.adjoint_weights(self.w_down.detach().contiguous()),
-                                                            "pauli_f32"))
+            self._adjoint = dict(key=key, w_up=ops.prepare_adjoint_weights(self.w_up.detach().contiguous()),
+                                 w_down=ops.prepare_adjoint_weights(self.w_down.detach().contiguous()))
         return self._adjoint
 
     def forward(self, x: torch.Tensor, logits: torch.Tensor | None = None):
@@ -260,9 +280,7 @@ class CliffordMoELayer(nn.Module):
         """
         if self.last_routing is None:
             return torch.zeros((), device=self.w_up.device)
-        c = self.last_routing["counts"].float()
-        f = c / (c.sum() + 1e-12)
-        return ((f - 1.0 / self.cfg.n_experts) ** 2).sum()
+        return ops.balance_loss(self.last_routing["counts"])
 
 
 class _MoEFunction(torch.autograd.Function):

@@ -568,6 +568,57 @@ def moe_forward(x: torch.Tensor, k: int, w_up: PreparedWeights, w_down: Prepared
     return out, dict(topk_idx=topk_idx, topk_w=topk_w, counts=counts, offsets=offsets)
 
 
+class LayerRouting:
+    """The routing of one layer call, in one int32 buffer: ``arrays()`` are its tensors."""
+
+    __slots__ = ("block", "N", "k", "E")
+    ALIGN = 64  # int32 values: each array starts on 256 bytes
+
+    def __init__(self, N: int, k: int, E: int, device):
+        self.N, self.k, self.E = N, k, E
+        a, slots = self.ALIGN, (N * k + self.ALIGN - 1) // self.ALIGN * self.ALIGN
+        self.block = torch.empty(2 * slots + (E + a - 1) // a * a + E + 1, device=device, dtype=torch.int32)
+
+    def pointers(self):
+        a, p = self.ALIGN, self.block.data_ptr()
+        slots = (self.N * self.k + a - 1) // a * a
+        counts = p + 8 * slots
+        return p, p + 4 * slots, counts, counts + 4 * ((self.E + a - 1) // a * a)
+
+    def arrays(self) -> dict:
+        b, a, n = self.block, self.ALIGN, self.N * self.k
+        slots = (n + a - 1) // a * a
+        off = 2 * slots + (self.E + a - 1) // a * a
+        return dict(topk_idx=b[:n].view(self.N, self.k), topk_w=b[slots:slots + n].view(torch.float32).view(self.N, self.k),
+                    counts=b[2 * slots:2 * slots + self.E], offsets=b[off:off + self.E + 1])
+
+
+def layer_forward(x: torch.Tensor, N: int, k: int, w_up: PreparedWeights, w_down: PreparedWeights, b_up: torch.Tensor,
+                  b_down: torch.Tensor, act: str, logits: torch.Tensor | None, router_weight: torch.Tensor | None,
+                  router_bias: torch.Tensor | None, residual: torch.Tensor | None, workspace: torch.Tensor,
+                  ws_bytes: int):
+    """:func:`moe_forward` for ``CliffordMoELayer``, whose prepared weights fit each other: x contiguous of any shape
+    that holds (N, d, 8), logits and router parameters contiguous fp32.  Returns ``(out like x, LayerRouting)``."""
+    dev = x.device
+    out = torch.empty_like(x)
+    r = LayerRouting(N, k, w_up.E, dev)
+    idx, w, counts, offsets = r.pointers()
+    check(lib().ygg_moe_forward(x.data_ptr(), DTYPE_CODE[x.dtype], N, w_up.d_in, w_up.d_out, w_up.E, k, ACT_CODE[act],
+                                ptr(logits), ptr(router_weight), ptr(router_bias), w_up.data.data_ptr(),
+                                ptr(w_up.scales), ptr(b_up), w_down.data.data_ptr(), ptr(w_down.scales), ptr(b_down),
+                                WFORMAT_CODE[w_up.fmt], ptr(residual), out.data_ptr(), idx, w, counts, offsets,
+                                workspace.data_ptr(), ws_bytes, stream_handle(dev)), "moe_forward")
+    return out, r
+
+
+def balance_loss(counts: torch.Tensor) -> torch.Tensor:
+    """``sum_e (f_e - 1/E)^2`` with f = counts / (sum + 1e-12) (``clifford_router.py:108-117``), 0-d fp32; counts int32."""
+    dev = _dev(counts)
+    out = torch.empty((), device=dev, dtype=torch.float32)
+    check(lib().ygg_balance_loss(ptr(counts), counts.numel(), ptr(out), stream_handle(dev)), "balance_loss")
+    return out
+
+
 def clifford_layer_norm(x: torch.Tensor, gamma: torch.Tensor, beta: torch.Tensor, eps: float = 1e-6,
                         out_dtype: torch.dtype | None = None, out: torch.Tensor | None = None) -> torch.Tensor:
     """CliffordLayerNorm.forward (``normalization.py:44-67``). x: (..., d, 8); gamma, beta: (d, 8)."""
@@ -645,6 +696,19 @@ def adjoint_weights(w: torch.Tensor) -> torch.Tensor:
     out = torch.empty((E, d_in, d_out, 8), device=dev, dtype=torch.float32)
     check(lib().ygg_adjoint_weights_f32(ptr(w), E, d_out, d_in, ptr(out), stream_handle(dev)), "adjoint_weights")
     return out
+
+
+def prepare_adjoint_weights(w: torch.Tensor) -> PreparedWeights:
+    """``prepare_weights(adjoint_weights(w), "pauli_f32")`` in one pass. w: (E, d_out, d_in, 8) fp32."""
+    dev = _dev(w)
+    if w.dtype != torch.float32 or w.dim() != 4 or w.shape[-1] != 8:
+        raise ValueError("prepare_adjoint_weights: w must be fp32 (E, d_out, d_in, 8)")
+    E, d_out, d_in = w.shape[:3]
+    data = torch.empty((lib().ygg_prepared_weight_bytes(E, d_in, d_out, WFORMAT_CODE["pauli_f32"]),), device=dev,
+                       dtype=torch.uint8)
+    check(lib().ygg_prepare_adjoint_weights_f32(ptr(w), E, d_out, d_in, ptr(data), stream_handle(dev)),
+          "prepare_adjoint_weights")
+    return PreparedWeights(data, None, "pauli_f32", E, d_in, d_out)
 
 
 def grouped_weight_grad(dy: torch.Tensor, a: torch.Tensor, offsets: torch.Tensor, E: int,

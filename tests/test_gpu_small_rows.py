@@ -109,3 +109,39 @@ def test_adjoint_preparation_and_balance_loss():
         f = c.double() / (c.double().sum() + 1e-12)
         assert abs(ops.balance_loss(c).item() - ((f - 1.0 / E) ** 2).sum().item()) <= 1e-6 * max(1.0 / E, 1e-3)
     assert ops.balance_loss(torch.zeros(8, device="cuda", dtype=torch.int32)).item() == pytest.approx(1.0 / 8)
+
+
+@pytest.mark.parametrize("N,d,F,E,k,act", [
+    (200, 17, 18, 3, 2, "gelu"),     # two chunks of the contraction, the second one input long; odd width
+    (333, 101, 131, 5, 2, "sigmoid"),  # odd widths, columns off 64 and 32
+    (900, 64, 129, 4, 1, "relu"),    # odd hidden width (a padding column between the products)
+    (160, 150, 70, 2, 2, "gelu"),
+])
+def test_int8_layer_of_enough_rows(N, d, F, E, k, act):
+    """int8 weights in whole-number fp16 products: the layer on the dequantized weights (x, weights exact; h rounded
+    to 11 bits, y and the output to bf16), tokens over many binades, an expert without rows, a token of zeros."""
+    import yggdrasil_amd
+
+    g = np.random.default_rng(N + F)
+    x = g.standard_normal((N, d, 8)).astype(np.float32) * np.ldexp(1.0, g.integers(-12, 5, (N, 1, 1))).astype(np.float32)
+    x[5] = 0.0
+    x = bf16_round(x)
+    lg = g.standard_normal((N, E)).astype(np.float32)
+    lg[:, 0] -= 30.0 * (E > k)
+    wu = (g.standard_normal((E, F, d, 8)) / np.sqrt(8 * d)).astype(np.float32)
+    wd = (g.standard_normal((E, d, F, 8)) / np.sqrt(8 * F)).astype(np.float32)
+    bu, bd = ((0.1 * g.standard_normal(s)).astype(np.float32) for s in ((E, F, 8), (E, d, 8)))
+    cfg = yggdrasil_amd.MoEHLMConfig(d_model=d, d_ff=F, n_experts=E, top_k=k, activation=act, dtype=torch.bfloat16,
+                                     weight_format="int8", router="logits")
+    layer = yggdrasil_amd.CliffordMoELayer(cfg, device="cuda")
+    layer.load_reference_weights(w_up=wu, b_up=bu, w_down=wd, b_down=bd)
+    say(f"int8 layer N={N} d={d} F={F} E={E} k={k} {act}")
+    out = layer.moe_forward(torch.from_numpy(x).cuda().bfloat16()[None], logits=torch.from_numpy(lg).cuda())[0]
+    idx = layer.last_routing["topk_idx"].cpu().numpy()
+    w = layer.last_routing["topk_w"].cpu().numpy()
+    ref = dense.moe_layer(x, idx, w, moe.dequantize_int8(*moe.quantize_int8(wu)), bu,
+                          moe.dequantize_int8(*moe.quantize_int8(wd)), bd, act)
+    got = out.float().cpu().numpy()
+    # y and the output are rounded once each, 2^-9 of an element at most, and k rows of y are added
+    assert np.linalg.norm(got - ref) / np.linalg.norm(ref) < 2.0 ** -8
+    assert normwise_err(got, ref) < TOL_BF16

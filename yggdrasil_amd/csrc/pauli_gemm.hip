@@ -1318,6 +1318,16 @@ namespace {
 // 512-thread 64 x 128 workgroup per CU.)
 using Tile = PauliTile</*WR*/ 2, /*WC*/ 1, /*BWT*/ 2, /*BWJ*/ 2, /*KC*/ 16>;
 constexpr int kWgPerCu = 2;
+// Fewer tiles than workgroups: one workgroup per tile -- unless every tile cut in halves
+// still gets a CU of its own (a split product: a workgroup's place): then the whole grid
+// runs and the kernel cuts them, which shortens a workgroup's steps.  Half tiles stage as
+// much as whole ones, so two to a CU are no faster where a staged operand feeds one MFMA
+// instead of three.  (geom_matmul 512 x 128 x 1024, 128 tiles: 57 -> 46 us, 512 x 512 x 1024 138 -> 106;
+// bf16 layer of 1024 tokens, d = 64, F = 128, E = 4, 36 and 72 tiles: 39 -> 34; of 1500 tokens,
+// 144 tiles in the down product: 65 -> 66, left as it was.)
+bool clip_grid(long long tiles, int grid, int halves_per_place) {
+  return tiles < grid && halves_per_place * tiles > grid;
+}
 
 // persistent grid: as many workgroups as fit on the chip at once
 struct DeviceShape {
@@ -1350,7 +1360,7 @@ int launch_pauli(hipStream_t st, const uint16_t* X, uint64_t x_bytes, const int3
       ((long long)(P_max + Tile::T - 1) / Tile::T + E) * ((d_out + Tile::BN - 1) / Tile::BN);
   int grid = ds.cus * kWgPerCu;
   int xcds = ds.xcds;
-  if (max_tiles < grid) {
+  if (clip_grid(max_tiles, grid, 4)) {
     grid = (int)max_tiles;
     xcds = 1;
   }
@@ -1412,7 +1422,7 @@ int launch_split(const void* x, int x_rows, int P_max, const void* w, const floa
   const long long max_tiles = ((long long)(P_max + PauliDmaTile::T - 1) / PauliDmaTile::T + E) *
                               ((d_out + PauliDmaTile::BN - 1) / PauliDmaTile::BN);
   int grid = ds.cus * kWgPerCu, xcds = ds.xcds;
-  if (max_tiles < grid) {
+  if (clip_grid(max_tiles, grid, 2)) {
     grid = (int)max_tiles;
     xcds = 1;
   }
@@ -1474,7 +1484,7 @@ int launch_half(const void* x, int x_rows, const int32_t* row_exp, const int32_t
   const long long max_tiles = ((long long)(P_max + PauliDmaTile::T - 1) / PauliDmaTile::T + E) *
                               ((d_out + PauliDmaTile::BN - 1) / PauliDmaTile::BN);
   int grid = ds.cus * kWgPerCu, xcds = ds.xcds;
-  if (max_tiles < grid) {
+  if (clip_grid(max_tiles, grid, 4)) {
     grid = (int)max_tiles;
     xcds = 1;
   }

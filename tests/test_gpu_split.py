@@ -141,7 +141,8 @@ def test_clifford_linear_module(rows, d_in, d_out, bias, dtype):
 
 @pytest.mark.parametrize("N,d,F,E,k,act,router", [(3300, 133, 150, 3, 1, "gelu", "logits"),
                                                   (1700, 128, 260, 5, 2, "sigmoid", "energy"),
-                                                  (1301, 150, 128, 8, 4, "relu", "logits")])
+                                                  (1301, 150, 128, 8, 4, "relu", "logits"),
+                                                  (1201, 261, 180, 2, 2, "gelu", "logits")])
 def test_layer_backward(N, d, F, E, k, act, router):
     """Gradients through the split products and weight gradients: widths off every block, an expert without
     rows, chunks with odd tails, tokens over many binades (rows of one weight-gradient sum have different

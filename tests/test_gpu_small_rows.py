@@ -145,3 +145,27 @@ def test_int8_layer_of_enough_rows(N, d, F, E, k, act):
     # y and the output are rounded once each, 2^-9 of an element at most, and k rows of y are added
     assert np.linalg.norm(got - ref) / np.linalg.norm(ref) < 2.0 ** -8
     assert normwise_err(got, ref) < TOL_BF16
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_layer_with_pruned_and_parametrized_weights(dtype):
+    """A pruned weight is no parameter of that name any more, a parametrized one lies in a submodule: same outputs, bit
+    for bit, and a change of the tensor behind it is seen."""
+    import copy
+
+    import torch.nn.utils.parametrize as parametrize
+    import torch.nn.utils.prune as prune
+    import yggdrasil_amd
+
+    cfg = yggdrasil_amd.MoEHLMConfig(d_model=32, d_ff=64, n_experts=4, top_k=2, dtype=dtype)
+    layer = yggdrasil_amd.CliffordMoELayer(cfg, device="cuda")
+    other = copy.deepcopy(layer)
+    prune.identity(other, "w_up")
+    prune.identity(other, "router_weight")
+    parametrize.register_parametrization(other, "b_down", torch.nn.Identity())
+    x = torch.randn(1, 40, 32, 8, device="cuda").to(dtype)
+    with torch.no_grad():
+        assert torch.equal(layer.moe_forward(x), other.moe_forward(x))
+        layer.b_down.add_(1.0)
+        other.parametrizations.b_down.original.add_(1.0)
+        assert torch.equal(layer.moe_forward(x), other.moe_forward(x))

@@ -154,6 +154,8 @@ class CliffordMoELayer(nn.Module):
 
     def _param_versions(self):
         p = self._parameters
+        if self._modules or "w_up" not in p:  # parametrized or pruned: other names, or none, hold the weights
+            return [v._version for v in self.parameters()] + [self.w_up.device]
         return [v._version for v in p.values() if v is not None] + [p["w_up"].device]
 
     @torch.no_grad()
@@ -220,8 +222,7 @@ class CliffordMoELayer(nn.Module):
             return _MoEFunction.apply(flat, res, self.w_up, self.b_up, self.w_down, self.b_down, self, lg).reshape(B, T, d, 8)
         rw = rb = None
         if logits is None:
-            p = self._parameters
-            rw, rb = p["router_weight"].detach(), p["router_bias"].detach()
+            rw, rb = self.router_weight.detach(), self.router_bias.detach()
             if rw.dtype != torch.float32 or not rw.is_contiguous():
                 rw = rw.float().contiguous()
             if rb.dtype != torch.float32 or not rb.is_contiguous():

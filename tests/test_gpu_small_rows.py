@@ -46,7 +46,7 @@ def test_layer(N, d, F, E, k, act):
 
 
 @pytest.mark.parametrize("E,k", [(1, 1), (7, 2), (33, 4), (64, 3)])
-@pytest.mark.parametrize("N", [1, 9, 90, 91, 300, 301, 1024])
+@pytest.mark.parametrize("N", [1, 9, 90, 91, 128, 129, 300, 301, 1024])
 def test_route_paths_agree(N, E, k):
     """The same routing on the one- and the two-launch path, from logits and from x (whose logits the one-
     workgroup kernel and the separate launch sum in one order), against the oracle's selection."""
@@ -61,7 +61,7 @@ def test_route_paths_agree(N, E, k):
     for got, want in ((r.topk_idx, idx), (r.counts, counts), (r.offsets, offsets), (r.perm, perm), (r.slot_pos, slot_pos)):
         assert np.array_equal(got.cpu().numpy().reshape(want.shape), want)
     for dt in (torch.float32, torch.bfloat16):
-        for d in (13, 70):
+        for d in (13, 64, 70):
             x = torch.from_numpy(g.standard_normal((N, d, 8)).astype(np.float32)).cuda().to(dt)
             rw, rb = torch.randn(E, 4).cuda(), torch.randn(E).cuda()
             a = ops.route_energy(x, rw, rb, k)

@@ -250,12 +250,13 @@ __global__ __launch_bounds__(kSmallThreads) void route_small(const float* __rest
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int j = tid & (kSelLanes - 1);
   const int ngroups = (N + 7) / 8;
+  // the thread's last slot stays in registers, those before it go through slot_pos
+  int e = -1, rank = 0;
   // a real loop (not unrolled): this kernel runs once per layer call, cold, and
   // its instruction fetch, not its arithmetic, sets its latency
 #pragma unroll 1
   for (int grp = wave; grp < ngroups; grp += kSmallWaves) {
     const int t = grp * 8 + lane / kSelLanes;
-    int e;
     float w;
     if constexpr (FROM_X) {
       float p[Q];
@@ -264,7 +265,7 @@ __global__ __launch_bounds__(kSmallThreads) void route_small(const float* __rest
     } else {
       select_token<Q>(logits, E, k, t, t < N, j, lane, e, w);
     }
-    const int rank = rank_in_wave(e, E, lane, &cnt[0][grp], kSmallGroups);
+    rank = rank_in_wave(e, E, lane, &cnt[0][grp], kSmallGroups);
     if (e >= 0) {  // rank within the group for now; the placement below turns it into the row
       topk_idx[(size_t)t * k + j] = e;
       topk_w[(size_t)t * k + j] = w;
@@ -272,9 +273,21 @@ __global__ __launch_bounds__(kSmallThreads) void route_small(const float* __rest
     }
   }
   __syncthreads();
-  // per expert (one wave each): exclusive scan of its group counts in group
-  // order; lane l holds groups 2l and 2l + 1
-  for (int x = wave; x < E; x += kSmallWaves) {
+  // per expert: exclusive scan of its group counts in group order.  Up to 16 groups (128
+  // tokens) 16 lanes each, every expert at once; else a wave each, lane l with groups 2l and 2l + 1
+  static_assert(kSmallThreads >= 16 * kMaxExperts, "16 lanes per expert");
+  if (ngroups <= 16) {
+    const int x = tid >> 4, g = tid & 15;
+    const int c = x < E && g < ngroups ? cnt[x][g] : 0;
+    int incl = c;
+#pragma unroll
+    for (int o = 1; o < 16; o <<= 1) {
+      const int v = __shfl_up(incl, o, 16);
+      if (g >= o) incl += v;
+    }
+    if (x < E && g < ngroups) cnt[x][g] = incl - c;
+    if (x < E && g == 15) tot[x] = incl;
+  } else for (int x = wave; x < E; x += kSmallWaves) {
     const int g0 = 2 * lane, g1 = g0 + 1;
     const int c0 = g0 < ngroups ? cnt[x][g0] : 0;
     const int c1 = g1 < ngroups ? cnt[x][g1] : 0;
@@ -312,8 +325,12 @@ __global__ __launch_bounds__(kSmallThreads) void route_small(const float* __rest
     const int t = grp * 8 + lane / kSelLanes;
     if (t < N && j < k) {
       const size_t f = (size_t)t * k + j;
-      const int e = topk_idx[f];
-      const int pos = eoff[e] + cnt[e][grp] + slot_pos[f];
+      int ee = e, r = rank;
+      if (grp + kSmallWaves < ngroups) {
+        ee = topk_idx[f];
+        r = slot_pos[f];
+      }
+      const int pos = eoff[ee] + cnt[ee][grp] + r;
       slot_pos[f] = pos;
       perm[pos] = t;
       if (cv.row_slot != nullptr) cv.row_slot[pos] = (int32_t)f;
@@ -378,8 +395,9 @@ namespace {
 bool route_in_one(int N, int E) { return N <= kSmallMaxN && N * ((E + 7) / 8 + 2) <= 900; }
 
 // ... and the logits with it, while the workgroup's reading of x is short beside a launch of
-// its own (one / three launches, us: E = 8, d = 64: 128 tokens 6.0 / 6.5, 256 8.8 / 8.0; d = 256: 32
-// tokens 5.9 / 7.0, 64 7.5 / 7.1, 256 19.1 / 9.3).
+// its own (one / three launches, us, measured while both loaded a row in smaller batches and
+// the map after it: E = 8, d = 64: 128 tokens 6.0 / 6.5, 256 8.8 / 8.0; d = 256: 32 tokens
+// 5.9 / 7.0, 64 7.5 / 7.1, 256 19.1 / 9.3).
 bool energy_in_one(int N, int E, int d) { return route_in_one(N, E) && (long long)N * d <= 13000; }
 
 // The grade-energy logits of energy_logits (the sums of the one-workgroup kernel, in its

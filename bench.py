@@ -588,6 +588,7 @@ def run_gm(torch, ops, name, c, steps, warmup):
         ms = time_fn(torch, lambda: ops.geom_matmul(a, b, workspace=ws, out=out), steps, warmup)
         flops = 128.0 * M * K * N  # the reference's arithmetic: 64 multiply-adds per multivector pair
         res[tag] = dict(M=M, K=K, N=N, ms=ms, tflops=flops / 2 / (ms * 1e-3) / 1e12,
+                        # against the fp32 units' peak: products on the fp16 units can pass 1
                         mfma_frac_f32=flops / 2 / (ms * 1e-3) / PEAK_F32,
                         dense_equiv_tflops=flops / (ms * 1e-3) / 1e12)
         del a, b, ws, out

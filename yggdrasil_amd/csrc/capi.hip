@@ -110,33 +110,20 @@ static size_t small_planes_bytes(int N, int d, int F, int E, int k, int w_format
   return (size_t)ygg::pauli_small_splits((int)P, E, F, d) * P * d * 32;
 }
 
-// Whether a bf16 layer's int8 weights (format 2) run as HALF products, and their regions
-static bool i8_half(int N, int d, int F, int E, int k, int w_format) {
-  const long long P = (long long)N * k;
-  return w_format == kWI8 && N > 0 && P <= 0x7fffffffLL && !decode_shape((int)P, E, w_format) &&
-         ygg::pauli_half_pays(N, P, E, d, F);
-}
-static size_t half_x_bytes(size_t N, int d) { return N * ((d + 1) & ~1) * 16; }
-static size_t half_w_bytes(int E, int d, int F) {
-  return (size_t)E * 16 * std::max((size_t)F * ((d + 1) & ~1), (size_t)d * ((F + 1) & ~1));  // both products, in turn
-}
-
 static size_t moe_workspace(int N, int d, int F, int E, int k, int dtype, int w_format, bool allow_split) {
   const size_t P = (size_t)N * k;
   const size_t es = (dtype == kF32) ? 4 : 2;
   size_t b = 0;
   const bool split = allow_split && f32_split(N, d, F, E, k, w_format);
   const SplitSizes z = split_sizes(N, P, d, F, E);
-  const bool half = allow_split && i8_half(N, d, F, E, k, w_format);
   b += align256((size_t)N * E * 4);       // logits
   b += align256(P * 4) * 2;               // perm, slot_pos
   b += align256(ygg_route_workspace_bytes(N, E, k));
-  b += align256(std::max(P * d * 8 * es, split ? z.x : half ? half_x_bytes(N, d) : 0));  // x_sorted (Pauli half-rows of x for format 3, split rows)
-  b += align256(std::max(P * F * 8 * es, split ? z.h : half ? half_x_bytes(P, F) : 0));  // h
+  b += align256(std::max(P * d * 8 * es, split ? z.x : 0));  // x_sorted (Pauli half-rows of x for format 3, split rows)
+  b += align256(std::max(P * F * 8 * es, split ? z.h : 0));  // h
   b += align256(std::max(ys_bytes(P, E, d, F, dtype, w_format),
                          allow_split ? small_planes_bytes(N, d, F, E, k, w_format) : 0));  // y_sorted
   if (w_format == kWPauliF32) b += align256(P * 4);       // row_slot: each row's slot, for the partial planes
-  if (half) b += align256(half_w_bytes(E, d, F)) + align256((size_t)E * 2 * pauli_half_norm_blocks(F) * 4) + 2 * align256(P * 4);
   if (split) b += align256(z.w) + align256(z.col_exp) + align256(z.norms) + 2 * align256(P * 4);  // row and h exponents
   return b;
 }
@@ -214,11 +201,10 @@ static int moe_forward_impl(const void* x, int dtype, int N, int d, int F, int E
   p += rws_bytes;
   const bool split = allow_split && f32_split(N, d, F, E, k, w_format);
   const SplitSizes z = split_sizes(N, P, d, F, E);
-  const bool half = allow_split && i8_half(N, d, F, E, k, w_format);
   void* xs = p;
-  p += align256(std::max(P * d * 8 * es, split ? z.x : half ? half_x_bytes(N, d) : 0));
+  p += align256(std::max(P * d * 8 * es, split ? z.x : 0));
   void* h = p;
-  p += align256(std::max(P * F * 8 * es, split ? z.h : half ? half_x_bytes(P, F) : 0));
+  p += align256(std::max(P * F * 8 * es, split ? z.h : 0));
   void* ys = p;
 
   if (w_format == kWPauliI8) {
@@ -304,7 +290,6 @@ static int moe_forward_impl(const void* x, int dtype, int N, int d, int F, int E
     hid.slot_pos = slot_pos;
     hid.topk_idx = topk_idx;
     hid.norms = norms;
-    hid.norm_blocks = pauli_split_norm_blocks(F);
     hid.h_exp = reinterpret_cast<int32_t*>(take(P * 4));
     if (pauli_split_weights(static_cast<const float*>(w_up), E, F, d, b_up, ws, col_exp, norms, stream) ||
         pauli_split_rows(static_cast<const float*>(x), N, d, xs, row_exp, hid, stream) ||
@@ -374,34 +359,6 @@ static int moe_forward_impl(const void* x, int dtype, int N, int d, int F, int E
       return -1;
     return combine_planes(static_cast<const float*>(ys), decode_splits(F), (int)P, N, k, d, topk_idx, topk_w,
                           slot_pos, residual, out, dtype, stream);
-  }
-  if (half) {
-    // int8 weights, enough rows: the codes' Pauli entries against fp16 Pauli rows of x and h
-    char* q = static_cast<char*>(ys) + align256(ys_bytes(P, E, d, F, dtype, w_format));
-    auto take = [&](size_t bytes) {
-      char* r = q;
-      q += align256(bytes);
-      return r;
-    };
-    void* ws = take(half_w_bytes(E, d, F));
-    float* norms = reinterpret_cast<float*>(take((size_t)E * 2 * pauli_half_norm_blocks(F) * 4));
-    int32_t* row_exp = reinterpret_cast<int32_t*>(take(P * 4));
-    ygg::SplitHidden hid;
-    hid.k = k;
-    hid.d_ff = F;
-    hid.act = act;
-    hid.slot_pos = slot_pos;
-    hid.topk_idx = topk_idx;
-    hid.norms = norms;
-    hid.norm_blocks = pauli_half_norm_blocks(F);
-    hid.h_exp = reinterpret_cast<int32_t*>(take(P * 4));
-    if (pauli_half_weights(static_cast<const int8_t*>(w_up), s_up, E, F, d, b_up, ws, norms, stream) ||
-        pauli_half_rows(static_cast<const uint16_t*>(x), N, d, xs, row_exp, hid, stream) ||
-        pauli_half_up(xs, N, row_exp, perm, (int)P, ws, s_up, b_up, offsets, E, d, F, act, h, hid.h_exp, stream) ||
-        pauli_half_weights(static_cast<const int8_t*>(w_down), s_down, E, d, F, nullptr, ws, nullptr, stream) ||
-        pauli_half_down(h, hid.h_exp, (int)P, ws, s_down, b_down, offsets, E, F, d, ys, stream))
-      return -1;
-    return ygg_combine(ys, kBF16, /*y_mask=*/0, N, k, d, topk_idx, topk_w, slot_pos, residual, out, dtype, stream);
   }
   if (ygg_dispatch(x, dtype, N, k, d, slot_pos, xs, /*to_mask_order=*/1, stream)) return -1;
   if (ygg_grouped_clifford_linear(xs, (int)P, w_up, w_format, s_up, b_up, offsets, E, d, F, act, h, dtype,

@@ -53,7 +53,6 @@
 // Activation rows are gathered through the expert-grouped row index, which
 // fuses the dispatch copy into the up projection.
 
-#include <algorithm>
 #include <type_traits>
 
 #include "pauli_common.h"
@@ -272,63 +271,6 @@ __device__ __forceinline__ void pauli_split_epilogue(const pf32x4_t (&acc)[4][2]
         }
       }
     }
-  }
-}
-
-// Epilogue of one tile of a HALF product (fp16 rows scaled by 2^row_e, whole-number weights
-// times col_f): bias, activation, bf16 blade rows or the next product's fp16 Pauli half-rows
-// scaled by 2^out_e (their width d_out rounded up to even, the padding column zero).
-template <int ACT, int OUT, int WR, int BWT>
-__device__ __forceinline__ void pauli_half_epilogue(const pf32x16_t (&acc)[WR][1][2][2], const float (&bv)[8],
-                                                    const PauliTileInfo& ti, int wave, int g, int l32, int d_out,
-                                                    const int* row_e, const float* col_f, const int32_t* out_e,
-                                                    __amdgpu_buffer_rsrc_t y_rsrc) {
-  typedef unsigned int pu32x2_t __attribute__((ext_vector_type(2)));
-  typedef unsigned int pu32x4_t __attribute__((ext_vector_type(4)));
-  const int wt = wave % BWT, wj = wave / BWT;
-  const int jl = wj * 32 + l32, j = ti.col0 + jl, d_pad = (d_out + 1) & ~1;
-  if (j >= (OUT == kOutPauliRows ? d_pad : d_out)) return;
-  const float cf = j < d_out ? 0.5f * col_f[jl] : 0.f;
-#pragma unroll
-  for (int rb = 0; rb < WR; ++rb) {
-    if (ti.half >= 0 && rb > 0) break;  // a half tile: the first accumulators hold block `half`
-    const int rbr = ti.half >= 0 ? ti.half : rb;
-#pragma unroll
-    for (int q = 0; q < 4; ++q)
-#pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        const int rl = (ti.compact ? wt * 16 : (wt * WR + rbr) * 16) + 4 * q + h + 2 * g;  // row of the tile
-        if (ti.row0 + rl >= ti.row_end) continue;
-        const int v0 = 4 * q + 2 * h;  // b = 0 at v0, b = 1 at v0 + 1
-        float y[8];
-        pauli_to_blade(acc[rb][0][0][0][v0], acc[rb][0][0][1][v0], acc[rb][0][0][0][v0 + 1], acc[rb][0][0][1][v0 + 1],
-                       acc[rb][0][1][0][v0], acc[rb][0][1][1][v0], acc[rb][0][1][0][v0 + 1], acc[rb][0][1][1][v0 + 1], y);
-        const int ex = -row_e[rl];
-#pragma unroll
-        for (int c = 0; c < 8; ++c) y[c] = __builtin_fmaf(__builtin_ldexpf(y[c], ex), cf, bv[c]);
-        activate_blade<ACT>(y);
-        if constexpr (OUT == kOutPauliRows) {
-          float c0[4], c1[4];
-          if (j >= d_out) {
-#pragma unroll
-            for (int c = 0; c < 8; ++c) y[c] = 0.f;
-          }
-          blade_to_pauli(y, c0, c1);
-          const int oe = out_e[rl];
-          pf16x4_t f0, f1;
-#pragma unroll
-          for (int c = 0; c < 4; ++c) {
-            f0[c] = (_Float16)__builtin_ldexpf(c0[c], oe);
-            f1[c] = (_Float16)__builtin_ldexpf(c1[c], oe);
-          }
-          const uint32_t off = ((uint32_t)rl * 2 * d_pad + j) * 8;
-          __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(pu32x2_t, f0), y_rsrc, off, 0, 0);
-          __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(pu32x2_t, f1), y_rsrc, off + (uint32_t)d_pad * 8, 0, 0);
-        } else {
-          const pu32x4_t o = {pack2_bf16(y[0], y[1]), pack2_bf16(y[2], y[3]), pack2_bf16(y[4], y[5]), pack2_bf16(y[6], y[7])};
-          __builtin_amdgcn_raw_buffer_store_b128(o, y_rsrc, ((uint32_t)rl * d_out + j) * 16, 0, 0);
-        }
-      }
   }
 }
 
@@ -715,29 +657,21 @@ __device__ __forceinline__ void lds_barrier() { asm volatile("s_barrier" ::: "me
 // 2 GiB; rows taken in place, and the output, are addressed from buffer resources
 // whose 64-bit base is the tile's first row, so only one tile's span needs 32-bit
 // offsets and the number of rows is not limited by them.
-// KIND: bf16 operands; SPLIT (above); HALF: one fp16 part, rows of x scaled by 2^row_exp,
-// the weights whole numbers (int8 codes' Pauli entries, at most 254) times a factor per
-// output channel.  Against the int8 L(w) blocks on bf16 this halves the MFMA work (32
-// multiply-adds a pair for 64) and rounds x's entries and h to 11 bits in the place of h's
-// 8 (layer of 2048 tokens, d = 128, F = 512, E = 32, k = 2: 220 -> 131 us with the codes'
-// expansion, error against float64 2.9e-3 -> 2.4e-3).
-enum PauliKind : int { kPauliBf16 = 0, kPauliSplit = 1, kPauliHalf = 2 };
 struct PauliSplitExps {
   const int32_t* row = nullptr;  // per product row
-  const int32_t* col = nullptr;  // per (expert, output channel): an exponent (SPLIT) or an fp32 factor (HALF)
+  const int32_t* col = nullptr;  // per (expert, output channel)
   int n_rows = 0;                // rows of `row` (and of the transposed output)
   const int32_t* out = nullptr;  // split rows out: the exponents to write them with, per product row
   float* pre = nullptr;          // split rows out: when set, takes the blade rows before the activation
 };
-template <int ACT, int OUT, int OUT_DT, int KIND = kPauliBf16>
+template <int ACT, int OUT, int OUT_DT, bool SPLIT = false>
 __global__ __launch_bounds__(PauliDmaTile::NT) __attribute__((amdgpu_waves_per_eu(2))) void pauli_gemm_dma_kernel(
     const uint16_t* __restrict__ X, const int32_t* __restrict__ gather, const uint16_t* __restrict__ Wp,
     const float* __restrict__ bias, const int32_t* __restrict__ offsets, int E, int d_in, int d_out,
     void* __restrict__ Y, int n_xcd, uint64_t x_bytes, uint64_t y_bytes, PauliSplitExps exps = PauliSplitExps{}) {
   using C = PauliDmaTile;
-  constexpr bool SPLIT = KIND == kPauliSplit, HALF = KIND == kPauliHalf;
   constexpr int NT = C::NT, T = C::T, BN = C::BN, KC = C::KC, WR = C::WR, WC = C::WC, BWT = C::BWT;
-  __shared__ __attribute__((aligned(1024))) unsigned char smem[SPLIT || HALF ? C::LDS_SPLIT : C::LDS];
+  __shared__ __attribute__((aligned(1024))) unsigned char smem[SPLIT ? C::LDS_SPLIT : C::LDS];
   __shared__ int s_off[kPauliMaxExperts + 1];   // expert row offsets
   __shared__ int s_tbeg[kPauliMaxExperts + 1];  // first whole row tile of each expert
   __shared__ int s_cbeg[kPauliMaxExperts + 1];  // first compact row tile of each expert
@@ -853,9 +787,9 @@ __global__ __launch_bounds__(PauliDmaTile::NT) __attribute__((amdgpu_waves_per_e
       const_cast<float*>(bias), (short)0, bias ? (uint32_t)E * d_out * 32 : 0u, kBufferFlags);
   __amdgpu_buffer_rsrc_t w_rsrc = x_rsrc;
   const __amdgpu_buffer_rsrc_t re_rsrc = __builtin_amdgcn_make_buffer_rsrc(
-      const_cast<int32_t*>(exps.row), (short)0, SPLIT || HALF ? (uint32_t)exps.n_rows * 4 : 0u, kBufferFlags);
+      const_cast<int32_t*>(exps.row), (short)0, SPLIT ? (uint32_t)exps.n_rows * 4 : 0u, kBufferFlags);
   const __amdgpu_buffer_rsrc_t ce_rsrc = __builtin_amdgcn_make_buffer_rsrc(
-      const_cast<int32_t*>(exps.col), (short)0, SPLIT || HALF ? (uint32_t)E * d_out * 4 : 0u, kBufferFlags);
+      const_cast<int32_t*>(exps.col), (short)0, SPLIT ? (uint32_t)E * d_out * 4 : 0u, kBufferFlags);
 
   // this lane's pieces: A loads 4 w .. 4 w + 3 (half-rows 8 q .. 8 q + 7, one
   // 128-byte line each), W loads 2 w and 2 w + 1 (columns 8 q .. 8 q + 7)
@@ -935,7 +869,7 @@ __global__ __launch_bounds__(PauliDmaTile::NT) __attribute__((amdgpu_waves_per_e
         dma_to_lds<16>(b_rsrc, smem + C::B_OFF + (iwm & 1) * BN * 32 + wave * 1024,
                        j < d_out ? (uint32_t)(t.e * d_out + j) * 32 + (lane & 1) * 16 : kOff);
       }
-      if constexpr (SPLIT || HALF) {  // the tile's scales: rows (wave 2), columns (wave 3)
+      if constexpr (SPLIT) {  // the tile's scale exponents: rows (wave 2), columns (wave 3)
         unsigned char* es = smem + C::S_OFF + (iwm & 1) * (T + BN) * 4;
         if (wave == 2) {
           dma_to_lds<4>(re_rsrc, es, (uint32_t)min(t.row0 + lane, t.row_end - 1) * 4);
@@ -1025,28 +959,16 @@ __global__ __launch_bounds__(PauliDmaTile::NT) __attribute__((amdgpu_waves_per_e
       for (int rb = 0; rb < NR; ++rb) {
         const uint4 x = av[s][rb];
         const uint4 ap = make_uint4(rot_conj(x.x), rot_conj(x.y), rot_conj(x.z), rot_conj(x.w));
-        if constexpr (HALF) {
-          const pf16x8_t A0 = __builtin_bit_cast(pf16x8_t, x), A1 = __builtin_bit_cast(pf16x8_t, ap);
+        const pbf16x8_t A0 = __builtin_bit_cast(pbf16x8_t, x);
+        const pbf16x8_t A1 = __builtin_bit_cast(pbf16x8_t, ap);
 #pragma unroll
-          for (int cb = 0; cb < WC; ++cb)
+        for (int cb = 0; cb < WC; ++cb)
 #pragma unroll
-            for (int a = 0; a < 2; ++a) {
-              const pf16x8_t B = __builtin_bit_cast(pf16x8_t, wv[s][cb][a]);
-              acc[rb][cb][a][0] = __builtin_amdgcn_mfma_f32_32x32x16_f16(A0, B, acc[rb][cb][a][0], 0, 0, 0);
-              acc[rb][cb][a][1] = __builtin_amdgcn_mfma_f32_32x32x16_f16(A1, B, acc[rb][cb][a][1], 0, 0, 0);
-            }
-        } else {
-          const pbf16x8_t A0 = __builtin_bit_cast(pbf16x8_t, x);
-          const pbf16x8_t A1 = __builtin_bit_cast(pbf16x8_t, ap);
-#pragma unroll
-          for (int cb = 0; cb < WC; ++cb)
-#pragma unroll
-            for (int a = 0; a < 2; ++a) {
-              const pbf16x8_t B = __builtin_bit_cast(pbf16x8_t, wv[s][cb][a]);
-              acc[rb][cb][a][0] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(A0, B, acc[rb][cb][a][0], 0, 0, 0);
-              acc[rb][cb][a][1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(A1, B, acc[rb][cb][a][1], 0, 0, 0);
-            }
-        }
+          for (int a = 0; a < 2; ++a) {
+            const pbf16x8_t B = __builtin_bit_cast(pbf16x8_t, wv[s][cb][a]);
+            acc[rb][cb][a][0] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(A0, B, acc[rb][cb][a][0], 0, 0, 0);
+            acc[rb][cb][a][1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(A1, B, acc[rb][cb][a][1], 0, 0, 0);
+          }
       }
     __builtin_amdgcn_s_setprio(0);
   };
@@ -1128,17 +1050,6 @@ __global__ __launch_bounds__(PauliDmaTile::NT) __attribute__((amdgpu_waves_per_e
           for (int a = 0; a < 2; ++a)
 #pragma unroll
             for (int ri = 0; ri < 2; ++ri) sacc[rb][cb][a][ri] = pf32x4_t{0.f, 0.f, 0.f, 0.f};
-    } else if constexpr (HALF) {  // the scales come off before the bias
-#pragma unroll
-      for (int rb = 0; rb < WR; ++rb)
-#pragma unroll
-        for (int cb = 0; cb < WC; ++cb)
-#pragma unroll
-          for (int a = 0; a < 2; ++a)
-#pragma unroll
-            for (int ri = 0; ri < 2; ++ri)
-#pragma unroll
-              for (int v = 0; v < 16; ++v) acc[rb][cb][a][ri][v] = 0.f;
     } else {
       load_bias(m);
       pauli_acc_from_bias<WR, WC>(acc, bvs);
@@ -1159,15 +1070,7 @@ __global__ __launch_bounds__(PauliDmaTile::NT) __attribute__((amdgpu_waves_per_e
           rsrc_from(Y, y_bytes, first), rsrc_from(exps.pre, pre_bytes, (uint64_t)ti.row0 * d_out * 32),
           (uint32_t)exps.n_rows * 32);
     }
-    if constexpr (HALF) {
-      load_bias(m);
-      const int* es = reinterpret_cast<const int*>(smem + C::S_OFF + (m & 1) * (T + BN) * 4);
-      const uint64_t row_bytes = (uint64_t)(OUT == kOutPauliRows ? (d_out + 1) & ~1 : d_out) * 16;
-      pauli_half_epilogue<ACT, OUT, WR, BWT>(acc, bvs[0], ti, wave, g, l32, d_out, es,
-                                             reinterpret_cast<const float*>(es + T),
-                                             OUT == kOutPauliRows ? exps.out + ti.row0 : nullptr,
-                                             rsrc_from(Y, y_bytes, (uint64_t)ti.row0 * row_bytes));
-    } else if constexpr (!SPLIT) {
+    if constexpr (!SPLIT) {
       const __amdgpu_buffer_rsrc_t y_rsrc = rsrc_from(Y, y_bytes, (uint64_t)ti.row0 * d_out * Y_MV_BYTES);
       pauli_tile_epilogue<ACT, OUT, OUT_DT, WR, WC, BWT, true>(acc, bvs, ti, wave, g, l32, d_out, y_rsrc, ti.row0);
     }
@@ -1426,7 +1329,7 @@ int launch_split(const void* x, int x_rows, int P_max, const void* w, const floa
     grid = (int)max_tiles;
     xcds = 1;
   }
-  pauli_gemm_dma_kernel<ACT, OUT, kF32, kPauliSplit><<<grid, PauliDmaTile::NT, 0, st>>>(
+  pauli_gemm_dma_kernel<ACT, OUT, kF32, true><<<grid, PauliDmaTile::NT, 0, st>>>(
       static_cast<const uint16_t*>(x), gather, static_cast<const uint16_t*>(w), bias, offsets, E, dv, d_out, y, xcds,
       (uint64_t)x_rows * dv * 16, (uint64_t)P_max * y_row, ex);
   return check_launch("pauli_split");
@@ -1472,66 +1375,6 @@ int ygg::pauli_split_up(const void* x, int x_rows, const int32_t* row_exp, const
     default: YGG_SU(kActSigmoid);
   }
 #undef YGG_SU
-}
-
-// ---- HALF products (int8 weights, enough rows) --------------------------------------
-namespace {
-template <int ACT, int OUT>
-int launch_half(const void* x, int x_rows, const int32_t* row_exp, const int32_t* gather, int P_max, const void* w,
-                const float* col_f, const float* bias, const int32_t* offsets, int E, int d_in, int d_out, void* y,
-                const int32_t* out_exp, hipStream_t st) {
-  const DeviceShape ds = device_shape();
-  const long long max_tiles = ((long long)(P_max + PauliDmaTile::T - 1) / PauliDmaTile::T + E) *
-                              ((d_out + PauliDmaTile::BN - 1) / PauliDmaTile::BN);
-  int grid = ds.cus * kWgPerCu, xcds = ds.xcds;
-  if (clip_grid(max_tiles, grid, 4)) {
-    grid = (int)max_tiles;
-    xcds = 1;
-  }
-  PauliSplitExps ex;
-  ex.row = row_exp;
-  ex.col = reinterpret_cast<const int32_t*>(col_f);
-  ex.n_rows = P_max;
-  ex.out = out_exp;
-  const int dp = (d_in + 1) & ~1;
-  pauli_gemm_dma_kernel<ACT, OUT, kBF16, kPauliHalf><<<grid, PauliDmaTile::NT, 0, st>>>(
-      static_cast<const uint16_t*>(x), gather, static_cast<const uint16_t*>(w), bias, offsets, E, dp, d_out, y, xcds,
-      (uint64_t)x_rows * dp * 16, (uint64_t)P_max * (OUT == kOutPauliRows ? (d_out + 1) & ~1 : d_out) * 16, ex);
-  return check_launch("pauli_half");
-}
-}  // namespace
-
-// Wherever the sizes fit: from 20 rows per expert on (fewer take the decode kernels) it was
-// 1.2 to 2.1 times as fast as the L(w) blocks over d = 64-128, F = 128-512, E = 4-64 (d = 128,
-// F = 512, E = 32: 20 rows each 181 -> 96 us, 256 each 317 -> 160; d = 64, F = 128, E = 4: 64 each
-// 70 -> 60, 512 each 99 -> 58).
-bool ygg::pauli_half_pays(int N, long long P, int E, int d, int F) {
-  const uint64_t lim = (uint64_t)1 << 31, dp = (d + 1) & ~1, fp = (F + 1) & ~1;
-  return E >= 1 && E <= kPauliMaxExperts && d > 2 * PauliDmaTile::KC && F > 2 * PauliDmaTile::KC && P >= 16LL * E &&
-         (uint64_t)P * 4 < lim && (F + 64) * dp * 16 < lim && (d + 64) * fp * 16 < lim &&
-         (uint64_t)E * std::max(d, F) * 32 < lim && N * dp * 16 < lim && PauliDmaTile::T * std::max(dp, fp) * 32 < lim;
-}
-
-int ygg::pauli_half_up(const void* x, int x_rows, const int32_t* row_exp, const int32_t* gather, int P_max,
-                       const void* w, const float* col_f, const float* bias, const int32_t* offsets, int E, int d_in,
-                       int d_out, int act, void* h, const int32_t* h_exp, hipStream_t stream) {
-#define YGG_HU(A)                                                                                              \
-  return launch_half<A, kOutPauliRows>(x, x_rows, row_exp, gather, P_max, w, col_f, bias, offsets, E, d_in, d_out, \
-                                       h, h_exp, stream)
-  switch (act) {
-    case kActNone: YGG_HU(kActNone);
-    case kActGelu: YGG_HU(kActGelu);
-    case kActRelu: YGG_HU(kActRelu);
-    default: YGG_HU(kActSigmoid);
-  }
-#undef YGG_HU
-}
-
-int ygg::pauli_half_down(const void* h, const int32_t* h_exp, int P_max, const void* w, const float* col_f,
-                         const float* bias, const int32_t* offsets, int E, int d_in, int d_out, void* y,
-                         hipStream_t stream) {
-  return launch_half<kActNone, kOutBlade>(h, P_max, h_exp, nullptr, P_max, w, col_f, bias, offsets, E, d_in, d_out, y,
-                                          nullptr, stream);
 }
 
 // Pauli weight preparation, called by ygg_prepare_weights (format 3).

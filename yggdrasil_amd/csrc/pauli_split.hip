@@ -167,35 +167,6 @@ __global__ __launch_bounds__(256) void split_weights_kernel(const float* __restr
 // component (sigmoid's stay within 1), and an entry of M(h) is at most its norm.  The
 // bound is some 2^4 above the largest entry in practice, which leaves the parts their 22
 // bits down to 2^-12 of it.
-__device__ __forceinline__ void slot_exponents(const SplitHidden& hid, int t, int lane, int s, float n2,
-                                               int32_t* __restrict__ row_exp) {
-#pragma unroll
-  for (int q = 32; q > 0; q >>= 1) n2 += __shfl_xor(n2, q);
-  const float xn = __builtin_ldexpf(__builtin_sqrtf(n2), -s);
-  const int nb = hid.norm_blocks;
-  for (int q = 0; q < hid.k; ++q) {
-    const int e = hid.topk_idx[(size_t)t * hid.k + q];
-    float a = 0.f, b = 0.f;
-    for (int u = lane; u < nb; u += 64) {
-      a = fmaxf(a, hid.norms[(size_t)e * 2 * nb + u]);
-      b = fmaxf(b, hid.norms[(size_t)e * 2 * nb + nb + u]);
-    }
-#pragma unroll
-    for (int u = 32; u > 0; u >>= 1) {
-      a = fmaxf(a, __shfl_xor(a, u));
-      b = fmaxf(b, __shfl_xor(b, u));
-    }
-    if (lane == 0) {
-      // 1.5: |M(b)| = sqrt(2) |b|, and the rounding of the sums behind it
-      float bound = 1.01f * (a * xn) + 1.5f * b;
-      if (hid.act == kActSigmoid) bound = fmaxf(bound, 3.f);
-      const int r = hid.slot_pos[(size_t)t * hid.k + q];
-      row_exp[r] = s;
-      hid.h_exp[r] = bound == INFINITY ? 15 - 128 : split_exp(bound);
-    }
-  }
-}
-
 __global__ __launch_bounds__(256) void split_rows_kernel(const float* __restrict__ x, int N, int d,
                                                          unsigned char* __restrict__ out,
                                                          int32_t* __restrict__ row_exp, SplitHidden hid) {
@@ -228,120 +199,31 @@ __global__ __launch_bounds__(256) void split_rows_kernel(const float* __restrict
     if (hid.one_offsets != nullptr && t == 0 && lane < 2) hid.one_offsets[lane] = lane * N;
     return;
   }
-  slot_exponents(hid, t, lane, s, n2, row_exp);
-}
-
-// ---- int8 codes -> the HALF products' weights -----------------------------------------
-// Codes (format 2): [E][d_out / 32][d_in / 2][32 j][2 i] of 8 bytes, mask order, signs folded.
-// Workgroup: 32 channels of one expert, eight input pairs at a time through LDS (the codes
-// are contiguous over channels, the records over pairs); blockIdx.y splits the pairs when
-// no norms are asked for.  An entry is a sum of two codes, exact in fp16.
-__global__ __launch_bounds__(256) void half_weights_kernel(const int8_t* __restrict__ w,
-                                                           const float* __restrict__ scales, int d_out, int d_in,
-                                                           const float* __restrict__ bias,
-                                                           unsigned char* __restrict__ out, float* __restrict__ norms) {
-  __shared__ uint4 tile[32][8][2];  // [channel][pair][a]
-  __shared__ float sq[8][32];
-  const int JB = (d_out + 31) / 32, IP = (d_in + 1) / 2;
-  const int e = blockIdx.x / JB, jb = blockIdx.x - e * JB;
-  const int t = threadIdx.x, pp = t >> 5, jj = t & 31;
-  const int per = ((IP + 7) / 8 + gridDim.y - 1) / gridDim.y * 8, p_beg = blockIdx.y * per, p_end = min(IP, p_beg + per);
-  const int8_t* src = w + (((size_t)e * JB + jb) * IP * 32 + jj) * 16;
-  float n2 = 0.f;
-  uint4 q = make_uint4(0, 0, 0, 0);
-  if (p_beg + pp < p_end) q = *reinterpret_cast<const uint4*>(src + (size_t)(p_beg + pp) * 512);
-  for (int p0 = p_beg; p0 < p_end; p0 += 8) {
-    const uint32_t u[4] = {q.x, q.y, q.z, q.w};
-    uint2 rec[2][2];  // [a][input of the pair]
 #pragma unroll
-    for (int ih = 0; ih < 2; ++ih) {
-      float x[8];
-#pragma unroll
-      for (int m = 0; m < 8; ++m)
-        x[mask_to_blade(m)] = (float)(kWFold(m) * (int)(int8_t)(u[ih * 2 + (m >> 2)] >> (8 * (m & 3))));
-      float c0[4], c1[4];
-      blade_to_pauli(x, c0, c1);  // c0 = (M00, M10), c1 = (M01, M11)
-#pragma unroll
-      for (int c = 0; c < 4; ++c) n2 += c0[c] * c0[c] + c1[c] * c1[c];
-      const pf16x4_t a0 = {(_Float16)c0[0], (_Float16)-c0[1], (_Float16)c1[0], (_Float16)-c1[1]};
-      const pf16x4_t a1 = {(_Float16)c0[2], (_Float16)-c0[3], (_Float16)c1[2], (_Float16)-c1[3]};
-      rec[0][ih] = __builtin_bit_cast(uint2, a0);
-      rec[1][ih] = __builtin_bit_cast(uint2, a1);
-    }
-    tile[jj][pp][0] = make_uint4(rec[0][0].x, rec[0][0].y, rec[0][1].x, rec[0][1].y);
-    tile[jj][pp][1] = make_uint4(rec[1][0].x, rec[1][0].y, rec[1][1].x, rec[1][1].y);
-    q = make_uint4(0, 0, 0, 0);
-    if (p0 + 8 + pp < p_end) q = *reinterpret_cast<const uint4*>(src + (size_t)(p0 + 8 + pp) * 512);
-    __syncthreads();
-    const int oj = t >> 3, op = t & 7;
-    if (jb * 32 + oj < d_out && p0 + op < p_end) {
-      uint4* dst = reinterpret_cast<uint4*>(out + (((size_t)e * d_out + jb * 32 + oj) * IP + p0 + op) * 32);
-      dst[0] = tile[oj][op][0];
-      dst[1] = tile[oj][op][1];
-    }
-    __syncthreads();
-  }
-  if (norms == nullptr) return;
-  sq[pp][jj] = n2;
-  __syncthreads();
-  if (t < 32) {
+  for (int q = 32; q > 0; q >>= 1) n2 += __shfl_xor(n2, q);
+  const float xn = __builtin_ldexpf(__builtin_sqrtf(n2), -s);
+  const int nb = (hid.d_ff + 7) / 8;
+  for (int q = 0; q < hid.k; ++q) {
+    const int e = hid.topk_idx[(size_t)t * hid.k + q];
     float a = 0.f, b = 0.f;
-    const int j = min(jb * 32 + t, d_out - 1);
-    for (int r = 0; r < 8; ++r) a += sq[r][t];  // (channels past d_out hold zero codes)
-    a = __builtin_sqrtf(a) * scales[(size_t)e * d_out + j];
-    if (bias != nullptr) {
-      for (int c = 0; c < 8; ++c) b = fmaxf(b, fabsf(bias[((size_t)e * d_out + j) * 8 + c]));
-      b *= 2.8284272f;  // at least the norm of the eight
+    for (int u = lane; u < nb; u += 64) {
+      a = fmaxf(a, hid.norms[(size_t)e * 2 * nb + u]);
+      b = fmaxf(b, hid.norms[(size_t)e * 2 * nb + nb + u]);
     }
 #pragma unroll
-    for (int o = 16; o > 0; o >>= 1) {
-      a = fmaxf(a, __shfl_xor(a, o));
-      b = fmaxf(b, __shfl_xor(b, o));
+    for (int u = 32; u > 0; u >>= 1) {
+      a = fmaxf(a, __shfl_xor(a, u));
+      b = fmaxf(b, __shfl_xor(b, u));
     }
-    if (t == 0) {
-      norms[(size_t)e * 2 * JB + jb] = a;
-      norms[(size_t)e * 2 * JB + JB + jb] = b;
+    if (lane == 0) {
+      // 1.5: |M(b)| = sqrt(2) |b|, and the rounding of the sums behind it
+      float bound = 1.01f * (a * xn) + 1.5f * b;
+      if (hid.act == kActSigmoid) bound = fmaxf(bound, 3.f);
+      const int r = hid.slot_pos[(size_t)t * hid.k + q];
+      row_exp[r] = s;
+      hid.h_exp[r] = bound == INFINITY ? 15 - 128 : split_exp(bound);
     }
   }
-}
-
-// bf16 blade rows -> fp16 Pauli half-rows scaled by 2^exponent; one wave per row
-__global__ __launch_bounds__(256) void half_rows_kernel(const uint16_t* __restrict__ x, int N, int d,
-                                                        uint2* __restrict__ out, int32_t* __restrict__ row_exp,
-                                                        SplitHidden hid) {
-  const int lane = threadIdx.x & 63, t = blockIdx.x * 4 + (threadIdx.x >> 6);
-  if (t >= N) return;
-  const uint4* row = reinterpret_cast<const uint4*>(x) + (size_t)t * d;
-  auto load = [&](int i, float* v) __attribute__((always_inline)) {
-    const uint4 q = row[i];
-    v[0] = bf_lo(q.x); v[1] = bf_hi(q.x); v[2] = bf_lo(q.y); v[3] = bf_hi(q.y);
-    v[4] = bf_lo(q.z); v[5] = bf_hi(q.z); v[6] = bf_lo(q.w); v[7] = bf_hi(q.w);
-  };
-  uint32_t m = 0;
-  for (int i = lane; i < d; i += 64) {
-    float v[8];
-    load(i, v);
-    m = max(m, pauli_mag(v));
-  }
-  const int s = split_exp(__builtin_bit_cast(float, wave_max_u32(m)));
-  const int dp = (d + 1) & ~1;
-  float n2 = 0.f;
-  for (int i = lane; i < dp; i += 64) {
-    float v[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f}, c0[4], c1[4];
-    if (i < d) load(i, v);
-    blade_to_pauli(v, c0, c1);
-    pf16x4_t f0, f1;
-#pragma unroll
-    for (int c = 0; c < 4; ++c) {
-      const float a = __builtin_ldexpf(c0[c], s), b = __builtin_ldexpf(c1[c], s);
-      n2 += a * a + b * b;
-      f0[c] = (_Float16)a;
-      f1[c] = (_Float16)b;
-    }
-    out[(size_t)t * 2 * dp + i] = __builtin_bit_cast(uint2, f0);
-    out[((size_t)t * 2 + 1) * dp + i] = __builtin_bit_cast(uint2, f1);
-  }
-  slot_exponents(hid, t, lane, s, n2, row_exp);
 }
 
 constexpr int kGmKBlock = 64;  // inputs whose maxima one workgroup of the first launch takes
@@ -445,20 +327,6 @@ int ygg::pauli_split_rows(const float* x, int N, int d, void* out, int32_t* row_
   split_rows_kernel<<<(unsigned)((N + 3) / 4), 256, 0, stream>>>(x, N, d, static_cast<unsigned char*>(out), row_exp,
                                                                  hid);
   return check_launch("pauli_split_rows");
-}
-
-int ygg::pauli_half_weights(const int8_t* w, const float* scales, int E, int d_out, int d_in, const float* bias,
-                            void* out, float* norms, hipStream_t stream) {
-  const int IP = (d_in + 1) / 2;
-  const dim3 grid((unsigned)(E * ((d_out + 31) / 32)), norms ? 1u : (unsigned)((IP + 63) / 64));
-  half_weights_kernel<<<grid, 256, 0, stream>>>(w, scales, d_out, d_in, bias, static_cast<unsigned char*>(out), norms);
-  return check_launch("pauli_half_weights");
-}
-
-int ygg::pauli_half_rows(const uint16_t* x, int N, int d, void* out, int32_t* row_exp, const SplitHidden& hid,
-                         hipStream_t stream) {
-  half_rows_kernel<<<(unsigned)((N + 3) / 4), 256, 0, stream>>>(x, N, d, static_cast<uint2*>(out), row_exp, hid);
-  return check_launch("pauli_half_rows");
 }
 
 size_t ygg::pauli_split_gm_partials(int K, int N) { return (size_t)((K + kGmKBlock - 1) / kGmKBlock) * N; }

@@ -233,8 +233,7 @@ struct SplitHidden {
   int k = 0, d_ff = 0, act = 0;
   const int32_t* slot_pos = nullptr;
   const int32_t* topk_idx = nullptr;
-  const float* norms = nullptr;  // of pauli_split_weights or pauli_half_weights
-  int norm_blocks = 0;           // per expert, of either kind
+  const float* norms = nullptr;  // of pauli_split_weights
   int32_t* h_exp = nullptr;
   int32_t* one_offsets = nullptr;  // k = 0: when set, takes the one-expert offsets {0, N}
 };
@@ -246,22 +245,6 @@ int pauli_split_rows(const float* x, int N, int d, void* out, int32_t* row_exp, 
 size_t pauli_split_gm_partials(int K, int N);
 int pauli_split_gm_operands(const float* a, const float* b, int M, int K, int N, void* w, int32_t* col_exp, void* x,
                             int32_t* row_exp, float* partial, int32_t* offsets, hipStream_t stream);
-
-// bf16 layers with int8 weights (format 2) and enough rows: the products on one fp16 part
-// (pauli_gemm.hip, HALF).  Rows: Pauli half-rows of an even number of multivectors (the
-// padding one zero), scaled by 2^exponent; weights: format 3's records holding the
-// codes' Pauli entries, expanded from the codes on each call, with the codes' scales as factors.
-bool pauli_half_pays(int N, long long P, int E, int d, int F);
-inline int pauli_half_norm_blocks(int d_out) { return (d_out + 31) / 32; }
-int pauli_half_weights(const int8_t* w, const float* scales, int E, int d_out, int d_in, const float* bias, void* out,
-                       float* norms, hipStream_t stream);
-int pauli_half_rows(const uint16_t* x, int N, int d, void* out, int32_t* row_exp, const SplitHidden& hid,
-                    hipStream_t stream);
-int pauli_half_up(const void* x, int x_rows, const int32_t* row_exp, const int32_t* gather, int P_max, const void* w,
-                  const float* col_f, const float* bias, const int32_t* offsets, int E, int d_in, int d_out, int act,
-                  void* h, const int32_t* h_exp, hipStream_t stream);
-int pauli_half_down(const void* h, const int32_t* h_exp, int P_max, const void* w, const float* col_f,
-                    const float* bias, const int32_t* offsets, int E, int d_in, int d_out, void* y, hipStream_t stream);
 
 // decode-shape int8 products (clifford_gemm.hip): whether (P_max rows, E
 // experts, format) takes the weight-streaming kernel, its number of K splits

@@ -377,3 +377,15 @@ def test_geom_matmul_workspace_checks_before_touching_a_device():
     assert L.ygg_geom_matmul_f32_ws(None, fake, fake, M, K, N, fake, need, None) == -1
     # empty outputs are a no-op that touches nothing
     assert L.ygg_geom_matmul_f32_ws(None, None, None, 0, K, N, None, 0, None) == 0
+
+
+def test_bf16_layer_workspace_grows_with_the_batch():
+    """A workspace sized for N tokens serves every smaller batch of a bf16 Pauli layer."""
+    from yggdrasil_amd import _native
+
+    if not os.path.exists(_native.LIB_PATH):
+        pytest.skip("library not built")
+    L = _native.lib()
+    for d, F, E, k in ((128, 512, 32, 2), (256, 1024, 64, 2), (64, 128, 4, 1), (100, 302, 12, 3)):
+        sizes = [L.ygg_moe_workspace_bytes(N, d, F, E, k, 1, 3) for N in range(1, 2100)]
+        assert all(a <= b for a, b in zip(sizes, sizes[1:])), (d, F, E, k)

@@ -41,3 +41,52 @@ def test_int8_layer_multiplies_the_given_bf16_inputs(N):
                           moe.dequantize_int8(*moe.quantize_int8(wd)), zeros[1], "relu")
     err = out.float().cpu().numpy() - ref
     assert np.linalg.norm(err) < 2.0 ** -7 * np.linalg.norm(ref)
+
+
+def _bf16_layer(d, F, E, k, act="gelu", router="logits"):
+    import yggdrasil_amd
+
+    torch.manual_seed(d + F + E)
+    cfg = yggdrasil_amd.MoEHLMConfig(d_model=d, d_ff=F, n_experts=E, top_k=k, activation=act, dtype=torch.bfloat16,
+                                     weight_format="pauli", router=router)
+    layer = yggdrasil_amd.CliffordMoELayer(cfg, device="cuda")
+    with torch.no_grad():
+        for p in (layer.b_up, layer.b_down):
+            p.normal_(0.0, 0.1)
+    return layer
+
+
+@pytest.mark.parametrize("N,d,F,E,k,act", [
+    (1, 2, 2, 1, 1, "gelu"), (9, 16, 18, 3, 2, "relu"), (40, 18, 16, 4, 3, "sigmoid"), (17, 24, 40, 64, 2, "gelu"),
+    (33, 66, 258, 2, 1, "gelu"), (16, 256, 1024, 64, 2, "gelu"), (64, 128, 512, 8, 2, "relu"), (160, 100, 302, 12, 4, "sigmoid"),
+    (701, 34, 98, 5, 2, "gelu"), (300, 200, 798, 4, 2, "relu"), (1201, 10, 16, 3, 1, "gelu")])
+def test_few_rows_equal_the_tiles(N, d, F, E, k, act):
+    """bf16 Pauli layers: a call of few rows gives, bit for bit, what the separate products give (which take
+    the 64 x 64 tiles at every size), on both sides of d_in = 16, where the tiles change."""
+    from yggdrasil_amd import ops
+
+    layer = _bf16_layer(d, F, E, k, act)
+    x = torch.randn(1, N, d, 8, device="cuda").bfloat16()
+    lg = torch.randn(N, E, device="cuda")
+    lg[:, 0] -= 20.0 * (E > k)  # an expert without rows
+    say(f"few rows against tiles N={N} d={d} F={F} E={E} k={k} {act}")
+    out = layer.moe_forward(x, logits=lg)
+    prep = layer._get_prepared()
+    r = ops.route(lg, k)
+    h = ops.pauli_grouped_linear(ops.pauli_rows_from_blade(x[0]), prep["w_up"], r.offsets, prep["b_up"], act,
+                                 gather=r.perm, x_layout="pauli", y_layout="pauli")
+    y = ops.pauli_grouped_linear(h, prep["w_down"], r.offsets, prep["b_down"], "none", x_layout="pauli",
+                                 y_layout="blade", out_dtype=torch.bfloat16)
+    assert torch.equal(out[0], ops.combine(y, r))
+
+
+@pytest.mark.parametrize("d,F,E,k", [(128, 512, 32, 2), (64, 130, 3, 1), (16, 32, 4, 2)])
+def test_bf16_rows_do_not_depend_on_the_batch(d, F, E, k):
+    """A token's output row is the same bits in a batch of 1, 7, 500, 900 and 3000 tokens."""
+    layer = _bf16_layer(d, F, E, k)
+    x = torch.randn(1, 3000, d, 8, device="cuda").bfloat16()
+    lg = torch.randn(3000, E, device="cuda")
+    say(f"batch invariance d={d} F={F} E={E} k={k}")
+    full = layer.moe_forward(x, logits=lg)
+    for n in (1, 7, 500, 900):
+        assert torch.equal(layer.moe_forward(x[:, :n].contiguous(), logits=lg[:n].contiguous()), full[:, :n])

@@ -102,14 +102,6 @@ static SplitSizes split_sizes(size_t N, size_t P, int d, int F, int E) {
   return z;
 }
 
-// fp32 planes of the down product when a bf16 Pauli layer's products take the few-rows
-// kernels (else 0)
-static size_t small_planes_bytes(int N, int d, int F, int E, int k, int w_format) {
-  const long long P = (long long)N * k;
-  if (w_format != kWPauli || P > ygg::kPauliSmallRows || !ygg::pauli_small_pays(N, (int)P, E, d, F)) return 0;
-  return (size_t)ygg::pauli_small_splits((int)P, E, F, d) * P * d * 32;
-}
-
 static size_t moe_workspace(int N, int d, int F, int E, int k, int dtype, int w_format, bool allow_split) {
   const size_t P = (size_t)N * k;
   const size_t es = (dtype == kF32) ? 4 : 2;
@@ -121,8 +113,7 @@ static size_t moe_workspace(int N, int d, int F, int E, int k, int dtype, int w_
   b += align256(ygg_route_workspace_bytes(N, E, k));
   b += align256(std::max(P * d * 8 * es, split ? z.x : 0));  // x_sorted (Pauli half-rows of x for format 3, split rows)
   b += align256(std::max(P * F * 8 * es, split ? z.h : 0));  // h
-  b += align256(std::max(ys_bytes(P, E, d, F, dtype, w_format),
-                         allow_split ? small_planes_bytes(N, d, F, E, k, w_format) : 0));  // y_sorted
+  b += align256(ys_bytes(P, E, d, F, dtype, w_format));  // y_sorted
   if (w_format == kWPauliF32) b += align256(P * 4);       // row_slot: each row's slot, for the partial planes
   if (split) b += align256(z.w) + align256(z.col_exp) + align256(z.norms) + 2 * align256(P * 4);  // row and h exponents
   return b;
@@ -321,24 +312,20 @@ static int moe_forward_impl(const void* x, int dtype, int N, int d, int F, int E
     return combine_planes(static_cast<const float*>(ys), splits, (int)P, N, k, d, topk_idx, topk_w, slot_pos,
                           residual, out, dtype, stream, /*slot rows*/ true);
   }
-  if (w_format == kWPauli && allow_split && small_planes_bytes(N, d, F, E, k, w_format) > 0) {
-    const int splits = pauli_small_splits((int)P, E, F, d);
-    if (pauli_small_up(xs, N, perm, (int)P, w_up, b_up, offsets, E, d, F, act, h, stream) ||
-        pauli_small_down(h, (int)P, w_down, b_down, offsets, E, F, d, splits, static_cast<float*>(ys), stream))
-      return -1;
-    return combine_planes(static_cast<const float*>(ys), splits, (int)P, N, k, d, topk_idx, topk_w, slot_pos, residual,
-                          out, dtype, stream);
-  }
   if (w_format == kWPauli) {
     // x's Pauli half-rows (converted with the routing); up: gather those rows through
     // perm inside the product -> h in Pauli half-rows; down: h -> y_sorted in blade
     // order.  No expert-grouped copy of x is made.
-    if (ygg_pauli_grouped_linear(xs, /*Pauli rows*/ 1, N, perm, (int)P, w_up, b_up, offsets, E, d, F, act, h,
-                                 /*Pauli rows*/ 0, kBF16, stream))
+    if (pauli_small_pays(N, (long long)P, E, d, F)) {  // few rows: the same outputs
+      if (pauli_small_up(xs, N, perm, (int)P, w_up, b_up, offsets, E, d, F, act, h, stream) ||
+          pauli_small_down(h, (int)P, w_down, b_down, offsets, E, F, d, ys, stream))
+        return -1;
+    } else if (ygg_pauli_grouped_linear(xs, /*Pauli rows*/ 1, N, perm, (int)P, w_up, b_up, offsets, E, d, F, act, h,
+                                        /*Pauli rows*/ 0, kBF16, stream) ||
+               ygg_pauli_grouped_linear(h, /*Pauli rows*/ 1, (int)P, nullptr, (int)P, w_down, b_down, offsets, E, F, d,
+                                        kActNone, ys, /*blade*/ 1, kBF16, stream)) {
       return -1;
-    if (ygg_pauli_grouped_linear(h, /*Pauli rows*/ 1, (int)P, nullptr, (int)P, w_down, b_down, offsets, E, F, d, kActNone, ys,
-                                 /*blade*/ 1, kBF16, stream))
-      return -1;
+    }
     return ygg_combine(ys, kBF16, /*y_mask=*/0, N, k, d, topk_idx, topk_w, slot_pos, residual, out, dtype, stream);
   }
   if (decode) {
@@ -444,8 +431,8 @@ YGG_API int ygg_moe_forward_noalloc(const void* x, int dtype, int N, int d, int 
                                     hipStream_t stream) {
   YGG_CHECK_ARG(N >= 0 && d >= 1 && F >= 1 && k >= 1, "ygg_moe_forward_noalloc: bad sizes N=%d d=%d F=%d k=%d", N, d,
                 F, k);
-  // the paths that need a larger workspace (split fp32 products, K ranges of few-row bf16
-  // products) only where it fits the scratch, so that they refuse no call
+  // the split fp32 products, which need a larger workspace, only where it fits the scratch, so
+  // that they refuse no call
   const bool allow = moe_workspace(N, d, F, E, k, dtype, w_format, true) <= kNoAllocScratchBytes;
   const size_t need = moe_workspace(N, d, F, E, k, dtype, w_format, allow);
   YGG_CHECK_ARG(need <= kNoAllocScratchBytes,

@@ -55,14 +55,9 @@
 
 #include <type_traits>
 
-#include "pauli_common.h"
+#include "pauli_tile.h"
 
 namespace ygg {
-
-enum PauliIn : int { kInBladeGather = 0, kInPauliRows = 1 };
-// split products (fp32 operands as two fp16 parts) write fp32 blade rows, blade columns
-// (d_out, P), or the split rows of the next product
-enum PauliOut : int { kOutPauliRows = 0, kOutBlade = 1, kOutBladeT = 2, kOutSplitRows = 3 };
 
 constexpr int kPauliMaxExperts = 64;
 
@@ -85,86 +80,6 @@ struct PauliTile {
   static_assert(KC % 4 == 0, "KC must be a multiple of the MFMA K step (4 multivectors)");
   static_assert(A_ITEMS_ROWS % NT == 0 && W_ITEMS % NT == 0, "staging split");
 };
-
-struct PauliTileInfo {
-  int e, row0, row_end, col0;
-  int half;  // -1: the whole tile; 0 / 1: only row block `half` of every wave
-  // a compact tile (the last row tile of an expert, at most 32 rows): computed as a
-  // half tile (block 0 of every wave), its rows staged at the token slots that block
-  // covers, 0-15 and 32-47, so wave row group wt holds rows 16 wt .. 16 wt + 15
-  bool compact = false;
-};
-
-// Epilogue of one tile for one wave: the inverse Pauli map, bias, grade-wise
-// activation and the output layout, all in the lane that holds the 8 reals of
-// an output multivector.  acc[rb][cb][a][re/im] is wave row block rb (of WR,
-// each 16 tokens x b = 0, 1), column block cb (of WC, 32 output multivectors);
-// bv[cb] is the bias of this lane's column in blade order, added here unless
-// BIAS_IN_ACC (the accumulators started from it).  The output is written by
-// buffer stores: y_rsrc starts at output row `row_base` and ends at the output's
-// true end, the row-dependent part of each offset is a scalar, the lane's part a
-// fixed per-lane offset.
-template <int ACT, int OUT, int OUT_DT, int WR, int WC, int BWT, bool BIAS_IN_ACC>
-__device__ __forceinline__ void pauli_tile_epilogue(const pf32x16_t (&acc)[WR][WC][2][2], const float (&bvs)[WC][8],
-                                                    const PauliTileInfo& ti, int wave, int g, int l32, int d_out,
-                                                    __amdgpu_buffer_rsrc_t y_rsrc, int row_base) {
-  typedef unsigned int pu32x2_t __attribute__((ext_vector_type(2)));
-  typedef unsigned int pu32x4_t __attribute__((ext_vector_type(4)));
-  const int wt = wave % BWT, wj = wave / BWT;
-  // bytes per output row (Pauli half-row pair, bf16 blade or fp32 blade row)
-  constexpr int MV_BYTES = (OUT == kOutPauliRows || OUT_DT == kBF16) ? 16 : 32;
-#pragma unroll
-  for (int cb = 0; cb < WC; ++cb) {
-    const int j = ti.col0 + (wj * WC + cb) * 32 + l32;
-    if (j >= d_out) continue;
-    const float* bv = bvs[cb];
-    // lane part of the offset: token 2 g of the group of four, column j
-    const uint32_t v_off = OUT == kOutPauliRows ? (uint32_t)((4 * g) * d_out + j) * 8
-                                                : (uint32_t)((2 * g) * d_out + j) * MV_BYTES;
-#pragma unroll
-    for (int rb = 0; rb < WR; ++rb) {
-      if (ti.half >= 0 && rb > 0) break;  // a half tile: the first accumulators hold block `half`
-      const int rbr = ti.half >= 0 ? ti.half : rb;
-#pragma unroll
-      for (int q = 0; q < 4; ++q)
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-          const int rs = ti.row0 + (ti.compact ? wt * 16 : (wt * WR + rbr) * 16) + 4 * q + h;  // row of lanes with g = 0
-          if (rs + 2 * g >= ti.row_end) continue;
-          const uint32_t s_off = (uint32_t)(rs - row_base) * d_out * MV_BYTES;
-          const int v0 = 4 * q + 2 * h;  // b = 0 at v0, b = 1 at v0 + 1
-          float y[8];
-          pauli_to_blade(acc[rb][cb][0][0][v0], acc[rb][cb][0][1][v0], acc[rb][cb][0][0][v0 + 1],
-                         acc[rb][cb][0][1][v0 + 1], acc[rb][cb][1][0][v0], acc[rb][cb][1][1][v0],
-                         acc[rb][cb][1][0][v0 + 1], acc[rb][cb][1][1][v0 + 1], y);
-          if constexpr (!BIAS_IN_ACC) {
-#pragma unroll
-            for (int c = 0; c < 8; ++c) y[c] += bv[c];
-          }
-          activate_blade<ACT>(y);
-          if constexpr (OUT == kOutPauliRows) {
-            float c0[4], c1[4];
-            blade_to_pauli(y, c0, c1);
-            const pu32x2_t h0 = {pack2_bf16(c0[0], c0[1]), pack2_bf16(c0[2], c0[3])};
-            const pu32x2_t h1 = {pack2_bf16(c1[0], c1[1]), pack2_bf16(c1[2], c1[3])};
-            __builtin_amdgcn_raw_buffer_store_b64(h0, y_rsrc, v_off, s_off, 0);
-            __builtin_amdgcn_raw_buffer_store_b64(h1, y_rsrc, v_off + (uint32_t)d_out * 8, s_off, 0);
-          } else if constexpr (OUT_DT == kBF16) {
-            const pu32x4_t o = {pack2_bf16(y[0], y[1]), pack2_bf16(y[2], y[3]), pack2_bf16(y[4], y[5]),
-                                pack2_bf16(y[6], y[7])};
-            __builtin_amdgcn_raw_buffer_store_b128(o, y_rsrc, v_off, s_off, 0);
-          } else {
-            const pu32x4_t lo = {__builtin_bit_cast(unsigned, y[0]), __builtin_bit_cast(unsigned, y[1]),
-                                 __builtin_bit_cast(unsigned, y[2]), __builtin_bit_cast(unsigned, y[3])};
-            const pu32x4_t hi = {__builtin_bit_cast(unsigned, y[4]), __builtin_bit_cast(unsigned, y[5]),
-                                 __builtin_bit_cast(unsigned, y[6]), __builtin_bit_cast(unsigned, y[7])};
-            __builtin_amdgcn_raw_buffer_store_b128(lo, y_rsrc, v_off, s_off, 0);
-            __builtin_amdgcn_raw_buffer_store_b128(hi, y_rsrc, v_off + 16, s_off, 0);
-          }
-        }
-    }
-  }
-}
 
 // Epilogue of one tile of a split product (fp32 operands held as two fp16 parts,
 // scaled by powers of two per row and per output channel): the inverse Pauli map, the
@@ -271,29 +186,6 @@ __device__ __forceinline__ void pauli_split_epilogue(const pf32x4_t (&acc)[4][2]
         }
       }
     }
-  }
-}
-
-// The accumulators of a tile started from the bias: entry (a, b) of the halved
-// Pauli matrix of the lane's column bias, re and im (the weights hold W / 2, so
-// the products are half the Pauli matrices and pauli_to_blade needs no scale).
-template <int WR, int WC>
-__device__ __forceinline__ void pauli_acc_from_bias(pf32x16_t (&acc)[WR][WC][2][2], const float (&bvs)[WC][8]) {
-#pragma unroll
-  for (int cb = 0; cb < WC; ++cb) {
-    float c0[4], c1[4];
-    blade_to_pauli(bvs[cb], c0, c1);  // c0 = (M00, M10), c1 = (M01, M11)
-    // [a][re/im][b]
-    const float e[2][2][2] = {{{0.5f * c0[0], 0.5f * c1[0]}, {0.5f * c0[1], 0.5f * c1[1]}},
-                              {{0.5f * c0[2], 0.5f * c1[2]}, {0.5f * c0[3], 0.5f * c1[3]}}};
-#pragma unroll
-    for (int rb = 0; rb < WR; ++rb)
-#pragma unroll
-      for (int a = 0; a < 2; ++a)
-#pragma unroll
-        for (int ri = 0; ri < 2; ++ri)
-#pragma unroll
-          for (int v = 0; v < 16; ++v) acc[rb][cb][a][ri][v] = e[a][ri][v & 1];
   }
 }
 

@@ -1,37 +1,30 @@
 // pauli_small.hip -- bf16 Pauli expert products of few rows (decode and short prompts).
 //
-// The same products as pauli_gemm.hip (layouts there), cut for the case where the weights
-// are read once or a few times and set the time: its 64 x 64 tiles walk the whole
-// contraction in one workgroup, so a few tiles leave most of the chip idle behind a chain
-// of K / 8 steps (16 tokens, 64 experts, d = 256, F = 1024, k = 2: up 26, down 64 us for 105 MB
-// of weights each, 21 us at the rate of a large copy).
+// The products of pauli_gemm.hip (layouts there), cut for the case where the weights are
+// read once or a few times and set the time: the 64 x 64 tiles walk the whole contraction
+// in one workgroup of two per CU, so a few tiles leave most of the chip idle.
 //
-// A workgroup of 4 waves owns 16 tokens x 32 output multivectors; the waves split the
-// contraction, and gridDim.z splits it further into fp32 partial planes that the combine
-// adds.  Bound by the weight stream, so every wave runs its own: chunks of 32 columns x
-// 8 inputs (128 bytes a column, whole lines, eight columns per instruction) go straight
-// to LDS into a ring of four that no other wave touches -- no barrier in the loop, three
-// chunks (12 KiB) a wave in flight, 96 KiB a CU.  Loading the operands into registers
-// instead takes 16 bytes from each of 32 columns per instruction and reached 2.8-3.5 TB/s
-// of weights, this 4.5 TB/s over a whole layer call (64 tokens, 64 experts, d = 256,
-// F = 1024: 537 MB in 119 us, 153 with the 64 x 64 tiles; 16 tokens 67, 113 with them).  The activations of a wave's range (at most 8 chunks at a
-// time) are read into registers first; several row tiles of an expert read its weights
-// through the XCD's L2 (a column tile's row tiles run on one XCD when the column tiles are
-// a multiple of 8).
+// A wave owns 8 RB tokens x 16 CB output multivectors and is a workgroup of its own: nothing
+// is shared, so there is no barrier, and every wave runs its own stream of chunks of 8
+// inputs (weights 128 bytes a column, activations 64 bytes a half-row) straight to LDS into a
+// ring of RING; the operands of chunk c + 1 are read from LDS while chunk c is multiplied.
+// Bound by the chain of a wave's steps at the smallest sizes and by the weight stream above.
+// Several row tiles of an expert read its weights through the XCD's L2 (a column tile's row
+// tiles run on one XCD when the column tiles are a multiple of 8).
+//
+// An output element is the 64 x 64 tiles' chain of sums: the contraction is not cut, the
+// bias enters where theirs does, and a 16 x 16 x 32 MFMA gives the bits of their two chained
+// 32 x 32 x 16 ones (2^25 sums of random inputs over up to 60 binades compared, all the same).
+// So a row's outputs do not depend on which of the two kernels its batch takes.
 
 #include <algorithm>
+#include <type_traits>
 
-#include "pauli_common.h"
+#include "pauli_tile.h"
 #include "ygg_common.h"
 
 namespace ygg {
 namespace {
-
-constexpr int kSmWaves = 4, kSmTok = 16, kSmCols = 32;
-constexpr int kSmRing = 4;                 // chunks in a wave's ring
-constexpr int kSmChunk = kSmCols * 128;    // bytes: 8 inputs of 32 columns
-constexpr int kSmPhase = 8;                // chunks whose activations are held in registers
-enum SmallOut : int { kSmPauliRows = 0, kSmPlanes = 1 };
 
 // The tile-th tile of TOK rows over the experts' ranges: one lane per expert counts its
 // tiles, a scan finds the one that holds it.
@@ -56,217 +49,271 @@ __device__ __forceinline__ bool small_find_tile(const int32_t* __restrict__ offs
 }
 
 typedef __attribute__((address_space(3))) void sm_lds_t;
-// 16 bytes per lane from buffer `r` at byte `off` + `soff` to lds + 16 lane
-__device__ __forceinline__ void small_dma(__amdgpu_buffer_rsrc_t r, unsigned char* lds, uint32_t off, uint32_t soff) {
-  const uint32_t m0 = __builtin_amdgcn_readfirstlane((uint32_t)(uintptr_t)(sm_lds_t*)lds);
-  const uint32_t so = __builtin_amdgcn_readfirstlane(soff);
-  asm volatile("s_mov_b32 m0, %1\n\tbuffer_load_dwordx4 %0, %2, %3 offen lds" ::"v"(off), "s"(m0), "s"(r), "s"(so)
-               : "m0", "memory");
+__device__ __forceinline__ uint32_t small_lds(const unsigned char* p) { return (uint32_t)(uintptr_t)(const sm_lds_t*)p; }
+// 16 (or 4) bytes per lane from buffer `r` at byte `off` + `soff` to LDS address `lds` + 16 (4) lane
+template <int BYTES>
+__device__ __forceinline__ void small_dma(__amdgpu_buffer_rsrc_t r, uint32_t lds, uint32_t off, uint32_t soff) {
+  const uint32_t m0 = __builtin_amdgcn_readfirstlane(lds), so = __builtin_amdgcn_readfirstlane(soff);
+  if constexpr (BYTES == 4)
+    asm volatile("s_mov_b32 m0, %1\n\tbuffer_load_dword %0, %2, %3 offen lds" ::"v"(off), "s"(m0), "s"(r), "s"(so)
+                 : "m0", "memory");
+  else
+    asm volatile("s_mov_b32 m0, %1\n\tbuffer_load_dwordx4 %0, %2, %3 offen lds" ::"v"(off), "s"(m0), "s"(r), "s"(so)
+                 : "m0", "memory");
 }
 // at most N of this wave's loads outstanding, and every LDS read returned
 template <int N>
 __device__ __forceinline__ void small_wait() {
+  static_assert(N >= 0 && N < 64, "vmcnt field");
   asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"i"(N) : "memory");
 }
 __device__ __forceinline__ int small_swz(int c) { return (c ^ (c >> 3)) & 7; }
 
-template <int ACT, int OUT>
-__global__ __launch_bounds__(64 * kSmWaves, 2) void pauli_small_kernel(
+template <int ACT, int OUT, bool BIAS_FIRST, int RB, int CB, int RING>
+__global__ __launch_bounds__(64) void pauli_small_kernel(
     const uint16_t* __restrict__ X, uint32_t x_bytes, const int32_t* __restrict__ gather, const uint16_t* __restrict__ Wp,
     const float* __restrict__ bias, const int32_t* __restrict__ offsets, int E, int d_in, int d_out, int P_max,
     void* __restrict__ Y) {
-  constexpr int TOK = kSmTok;
-  constexpr int RING = kSmRing * kSmChunk;
-  __shared__ __attribute__((aligned(1024))) unsigned char smem[kSmWaves * RING];
-  typedef float4 part_t[2 * TOK][kSmCols + 1];  // (a0 re, a0 im, a1 re, a1 im) of two waves, over the rings
-  part_t* const part = reinterpret_cast<part_t*>(smem);
-  static_assert(2 * sizeof(part_t) <= sizeof(smem), "partial sums over the rings");
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int l32 = lane & 31, g = lane >> 5;
-  const int n_ct = (d_out + kSmCols - 1) / kSmCols;
+  constexpr int TOK = 8 * RB, COLS = 16 * CB;
+  constexpr int W_BYTES = COLS * 128, CHUNK = W_BYTES + TOK * 128;  // 8 inputs of the columns, then of the half-rows
+  constexpr int WL = W_BYTES / 1024, LOADS = CHUNK / 1024;          // direct loads of 64 x 16 bytes
+  __shared__ __attribute__((aligned(1024))) unsigned char smem[RING * CHUNK + 1024 + 256];
+  unsigned char* const s_bias = smem + RING * CHUNK;  // 32 bytes a column
+  unsigned char* const s_gather = s_bias + 1024;      // a row index per lane
+  const int lane = threadIdx.x, l16 = lane & 15, g = lane >> 4;
+  const int n_ct = (d_out + COLS - 1) / COLS;
   const int ct = blockIdx.x % n_ct, rt = blockIdx.x / n_ct;
   int e, row0, row_end;
   if (!small_find_tile<TOK>(offsets, E, rt, lane, e, row0, row_end)) return;
-  const int col0 = ct * kSmCols;
-  const int IP = d_in >> 1, chunks = (IP + 3) >> 2;
+  const int col0 = ct * COLS;
+  const int IP = d_in >> 1;
+  const int n = 2 * ((IP + 7) >> 3);  // chunks of four pairs: an even number, as the 64 x 64 tiles' steps
 
   const __amdgpu_buffer_rsrc_t x_rsrc =
       __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(X), (short)0, x_bytes, kBufferFlags);
   const __amdgpu_buffer_rsrc_t w_rsrc = __builtin_amdgcn_make_buffer_rsrc(
       const_cast<uint16_t*>(Wp) + (size_t)e * d_out * IP * 16, (short)0, (uint32_t)d_out * IP * 32, kBufferFlags);
-  // GEMM row l32 = (token, b): its half-row; rows past the expert's range repeat the last
-  const int m = min(row0 + (l32 >> 1), row_end - 1);
-  const int src = gather ? gather[m] : m;
-  const uint32_t a_row = (uint32_t)(2 * src + (l32 & 1)) * d_in * 8;
+  const __amdgpu_buffer_rsrc_t b_rsrc = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<float*>(bias), (short)0, bias ? (uint32_t)E * d_out * 32 : 0u, kBufferFlags);
+  const __amdgpu_buffer_rsrc_t g_rsrc = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<int32_t*>(gather), (short)0, gather ? (uint32_t)P_max * 4 : 0u, kBufferFlags);
 
-  // this (split, wave)'s chunks [c0, c0 + n)
-  const int per_split = (chunks + gridDim.z - 1) / gridDim.z;
-  const int c_beg = blockIdx.z * per_split, c_end = min(chunks, c_beg + per_split);
-  const int per_wave = (max(c_end - c_beg, 0) + kSmWaves - 1) / kSmWaves;
-  const int c0 = c_beg + wave * per_wave;
-  const int n = __builtin_amdgcn_readfirstlane(max(0, min(c_end, c0 + per_wave) - c0));
-
-  // W pieces of this lane: columns 8 u + lane / 8, piece (pair, a) lane % 8 through the
+  // Weights: piece u of this lane is column 8 u + lane / 8, (pair, a) lane % 8 through the
   // swizzle that keeps the operand reads free of bank conflicts.  A column past d_out lies
-  // past the expert's range and reads zero.
-  unsigned char* const ring = smem + wave * RING;
-  uint32_t w_off[4];
-  int w_lim[4];  // the piece is inside the contraction while its chunk's first pair is below this
+  // past the expert's range and reads zero; so does a pair past the contraction.
+  const uint32_t lds0 = small_lds(smem);
+  uint32_t w_off[WL], a_off[RB];
+  int w_lim[WL], a_lim[RB];  // the piece is inside the contraction while its chunk's first pair is below this
 #pragma unroll
-  for (int u = 0; u < 4; ++u) {
+  for (int u = 0; u < WL; ++u) {
     const int c = 8 * u + (lane >> 3), piece = (lane & 7) ^ small_swz(c);
     w_off[u] = (uint32_t)(col0 + c) * IP * 32 + piece * 16;
     w_lim[u] = IP - (piece >> 1);
   }
-  auto issue = [&](int i) __attribute__((always_inline)) {  // the i-th chunk of the range
-    const int p0 = (c0 + i) * 4;
-    unsigned char* st = ring + (i & (kSmRing - 1)) * kSmChunk;
-#pragma unroll
-    for (int u = 0; u < 4; ++u)
-      small_dma(w_rsrc, st + u * 1024, p0 < w_lim[u] ? w_off[u] : kBufferOff, (uint32_t)p0 * 32);
+  auto issue_w = [&](int c, int slot, int u) __attribute__((always_inline)) {  // piece u of chunk c to ring slot `slot`
+    small_dma<16>(w_rsrc, lds0 + slot * CHUNK + u * 1024, c * 4 < w_lim[u] ? w_off[u] : kBufferOff, (uint32_t)c * 128);
   };
-  // operand reads: column l32, pair 2 s + g, a
-  uint32_t w_rd[2][2];
+  // Activations: piece u is half-row 16 u + lane / 4 (token, b), pair lane % 4 through a swizzle
+  auto issue_a = [&](int c, int slot) __attribute__((always_inline)) {
 #pragma unroll
-  for (int s = 0; s < 2; ++s)
-#pragma unroll
-    for (int a = 0; a < 2; ++a) w_rd[s][a] = l32 * 128 + ((2 * (2 * s + g) + a) ^ small_swz(l32)) * 16;
+    for (int u = 0; u < RB; ++u)
+      small_dma<16>(x_rsrc, lds0 + slot * CHUNK + W_BYTES + u * 1024, c * 4 < a_lim[u] ? a_off[u] : kBufferOff, (uint32_t)c * 64);
+  };
 
-  pf32x16_t acc[2][2];
+  // The prologue asks for the row indices and the bias, then the weights of the first chunks,
+  // and, when the indices are here, those chunks' activations.
+  const int my_row = min(row0 + (lane & (TOK - 1)), row_end - 1);  // past the range: the last row again
+  small_dma<4>(g_rsrc, small_lds(s_gather), (uint32_t)my_row * 4, 0);
+  small_dma<16>(b_rsrc, small_lds(s_bias),
+                lane < 2 * COLS && col0 + (lane >> 1) < d_out ? (uint32_t)(e * d_out + col0) * 32 + lane * 16 : kBufferOff, 0);
 #pragma unroll
-  for (int a = 0; a < 2; ++a)
+  for (int c = 0; c < RING - 1; ++c)
 #pragma unroll
-    for (int q = 0; q < 2; ++q)
+    for (int u = 0; u < WL; ++u) issue_w(c, c, u);
+  small_wait<WL * (RING - 1) + 1>();
 #pragma unroll
-      for (int v = 0; v < 16; ++v) acc[a][q][v] = 0.f;
+  for (int u = 0; u < RB; ++u) {
+    const int r = 16 * u + (lane >> 2), piece = (lane & 3) ^ ((r >> 2) & 3), tok = r >> 1;
+    const int src = gather ? reinterpret_cast<const int*>(s_gather)[tok] : min(row0 + tok, row_end - 1);
+    a_off[u] = (uint32_t)(2 * src + (r & 1)) * d_in * 8 + piece * 16;
+    a_lim[u] = IP - piece;
+  }
+#pragma unroll
+  for (int c = 0; c < RING - 1; ++c) issue_a(c, c);
 
-  for (int ph = 0; ph < n; ph += kSmPhase) {
-    uint4 x[kSmPhase][2];
+  // operands of v_mfma_f32_16x16x32_bf16: lane column / half-row lane % 16, pair lane / 16
+  uint32_t w_rd[CB][2], a_rd[RB];
 #pragma unroll
-    for (int i = 0; i < kSmPhase; ++i)
+  for (int rb = 0; rb < RB; ++rb) a_rd[rb] = W_BYTES + (rb * 16 + l16) * 64 + (g ^ (l16 >> 2)) * 16;
 #pragma unroll
-      for (int s = 0; s < 2; ++s) {
-        const int p = (c0 + ph + i) * 4 + 2 * s + g;
-        x[i][s] = __builtin_bit_cast(
-            uint4, __builtin_amdgcn_raw_buffer_load_b128(x_rsrc, ph + i < n && p < IP ? a_row + (uint32_t)p * 16 : kBufferOff,
-                                                         0, 0));
+  for (int cb = 0; cb < CB; ++cb)
+#pragma unroll
+    for (int a = 0; a < 2; ++a) w_rd[cb][a] = (cb * 16 + l16) * 128 + ((2 * g + a) ^ small_swz(cb * 16 + l16)) * 16;
+  struct Ops {
+    uint4 x[RB], w[CB][2];
+  };
+  auto read_x = [&](const unsigned char* st, Ops& o) __attribute__((always_inline)) {
+#pragma unroll
+    for (int rb = 0; rb < RB; ++rb) o.x[rb] = *reinterpret_cast<const uint4*>(st + a_rd[rb]);
+  };
+  auto read_w = [&](const unsigned char* st, Ops& o, int cb) __attribute__((always_inline)) {
+#pragma unroll
+    for (int a = 0; a < 2; ++a) o.w[cb][a] = *reinterpret_cast<const uint4*>(st + w_rd[cb][a]);
+  };
+  pf32x4_t acc[RB][CB][2][2];
+  auto mma = [&](const Ops& o, int cb, int q) __attribute__((always_inline)) {  // q: real or imaginary part
+#pragma unroll
+    for (int rb = 0; rb < RB; ++rb) {
+      const uint4 v = o.x[rb];
+      const uint4 vr = q == 0 ? v : make_uint4(rot_conj(v.x), rot_conj(v.y), rot_conj(v.z), rot_conj(v.w));
+      const pbf16x8_t A = __builtin_bit_cast(pbf16x8_t, vr);
+#pragma unroll
+      for (int a = 0; a < 2; ++a)
+        acc[rb][cb][a][q] =
+            __builtin_amdgcn_mfma_f32_16x16x32_bf16(A, __builtin_bit_cast(pbf16x8_t, o.w[cb][a]), acc[rb][cb][a][q], 0, 0, 0);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  };
+
+  // The loads that may be outstanding when chunk k is needed, before chunk k + RING - 2 is
+  // asked for: those of the chunks after it -- of the prologue's chunks their activations
+  // only, since all its weights come first.
+  constexpr int kSteady = LOADS * (RING - 3);
+  static_assert(LOADS * (RING - 1) < 64, "the counter of outstanding loads");
+  // step c, in ring slot SLOT: chunk c + 1 has landed (and chunk c's operands are in registers),
+  // so the slot of chunk c - 1 is free and takes chunk c + RING - 1 (past the end: zeros,
+  // read by nobody).  A wave issues in order and an MFMA keeps its unit for 16 cycles: the other
+  // work goes between them.
+  auto step = [&](int c, auto slot_tag, const Ops& now, Ops& next) __attribute__((always_inline)) {
+    constexpr int slot = decltype(slot_tag)::value;
+    constexpr int to = (slot + RING - 1) % RING;
+    const unsigned char* st = smem + (slot + 1) % RING * CHUNK;
+    if (slot + 1 < RING - 2 && c < RING) small_wait<RB * (slot + 1 < RING - 2 ? RING - 3 - slot : 0) + LOADS * (slot < RING - 3 ? slot : 0)>();
+    else small_wait<kSteady>();
+    read_x(st, next);
+    mma(now, 0, 0);
+#pragma unroll
+    for (int cb = 0; cb < CB; ++cb) read_w(st, next, cb);
+    mma(now, 0, 1);
+#pragma unroll
+    for (int u = 0; u < 2; ++u) issue_w(c + RING - 1, to, u);
+    if constexpr (CB == 2) {
+      mma(now, 1, 0);
+#pragma unroll
+      for (int u = 2; u < 4; ++u) issue_w(c + RING - 1, to, u);
+      mma(now, 1, 1);
+    }
+    issue_a(c + RING - 1, to);
+  };
+  small_wait<RB * (RING - 2)>();  // chunk 0, and with it the bias
+  Ops o0, o1;
+  read_x(smem, o0);
+  float bvs[CB][8];
+#pragma unroll
+  for (int cb = 0; cb < CB; ++cb) {
+    read_w(smem, o0, cb);
+    const unsigned char* bp = s_bias + (cb * 16 + l16) * 32;
+    const uint4 lo = *reinterpret_cast<const uint4*>(bp), hi = *reinterpret_cast<const uint4*>(bp + 16);
+    const uint32_t mk[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};  // mask order
+#pragma unroll
+    for (int c = 0; c < 8; ++c) bvs[cb][c] = __builtin_bit_cast(float, mk[blade_to_mask(c)]);
+    float b[2][2][2] = {};
+    if constexpr (BIAS_FIRST) pauli_bias_entries(bvs[cb], b);
+#pragma unroll
+    for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+      for (int a = 0; a < 2; ++a)
+#pragma unroll
+        for (int q = 0; q < 2; ++q) acc[rb][cb][a][q] = pf32x4_t{b[a][q][0], b[a][q][1], b[a][q][0], b[a][q][1]};
+  }
+#pragma unroll 1
+  for (int c = 0;; c += RING) {  // (n is even)
+    static_assert(RING == 6 || RING == 8, "the steps of one round of the ring");
+#define YGG_TWO(S)                                        \
+  step(c + S, std::integral_constant<int, S>{}, o0, o1);         \
+  step(c + S + 1, std::integral_constant<int, S + 1>{}, o1, o0); \
+  if (c + S + 2 >= n) break
+    YGG_TWO(0);
+    YGG_TWO(2);
+    YGG_TWO(4);
+    if constexpr (RING == 8) {
+      YGG_TWO(6);
+    }
+#undef YGG_TWO
+  }
+  small_wait<0>();  // nothing may land in LDS after the wave has ended
+
+  const uint64_t y_bytes = (uint64_t)P_max * d_out * 16, first = (uint64_t)row0 * d_out * 16;
+  const __amdgpu_buffer_rsrc_t y_rsrc = __builtin_amdgcn_make_buffer_rsrc(
+      static_cast<char*>(Y) + first, (short)0, (uint32_t)(y_bytes - first), kBufferFlags);
+#pragma unroll
+  for (int cb = 0; cb < CB; ++cb) {
+    const int j = col0 + cb * 16 + l16;
+    if (j >= d_out) continue;
+#pragma unroll
+    for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const int rl = rb * 8 + 2 * g + h;  // row of the tile; its halves b = 0, 1 are sums 2 h, 2 h + 1
+        if (row0 + rl >= row_end) continue;
+        const auto& s = acc[rb][cb];
+        const uint32_t off = OUT == kOutPauliRows ? ((uint32_t)rl * 2 * d_out + j) * 8 : ((uint32_t)rl * d_out + j) * 16;
+        pauli_store_mv<ACT, OUT, kBF16, BIAS_FIRST>(s[0][0][2 * h], s[0][1][2 * h], s[0][0][2 * h + 1], s[0][1][2 * h + 1],
+                                                    s[1][0][2 * h], s[1][1][2 * h], s[1][0][2 * h + 1], s[1][1][2 * h + 1],
+                                                    bvs[cb], y_rsrc, off, 0, d_out);
       }
-    if (ph == 0) {
-      if (n > 0) issue(0);
-      if (n > 1) issue(1);
-      if (n > 2) issue(2);
-    }
-#pragma unroll
-    for (int i = 0; i < kSmPhase; ++i) {
-      const int c = ph + i;
-      if (c < n) {
-        // chunk c has landed (later ones stay in flight); the slot of chunk c - 1 has been
-        // read by this wave and takes chunk c + 3
-        if (n - 1 - c >= 2) small_wait<8>();
-        else if (n - 1 - c == 1) small_wait<4>();
-        else small_wait<0>();
-        if (c + 3 < n) issue(c + 3);
-        const unsigned char* st = ring + (c & (kSmRing - 1)) * kSmChunk;
-#pragma unroll
-        for (int s = 0; s < 2; ++s) {
-          const uint4 v = x[i][s];
-          const uint4 vr = make_uint4(rot_conj(v.x), rot_conj(v.y), rot_conj(v.z), rot_conj(v.w));
-          const pbf16x8_t A0 = __builtin_bit_cast(pbf16x8_t, v), A1 = __builtin_bit_cast(pbf16x8_t, vr);
-#pragma unroll
-          for (int a = 0; a < 2; ++a) {
-            const pbf16x8_t B = __builtin_bit_cast(pbf16x8_t, *reinterpret_cast<const uint4*>(st + w_rd[s][a]));
-            acc[a][0] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(A0, B, acc[a][0], 0, 0, 0);
-            acc[a][1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(A1, B, acc[a][1], 0, 0, 0);
-          }
-        }
-      }
-    }
-  }
-  __syncthreads();  // every wave is through with its ring
-
-  // the waves' sums: 2 and 3 into 0 and 1, then both from LDS
-  auto row_of = [&](int v) { return 8 * (v >> 2) + 4 * g + (v & 3); };
-  if (wave >= 2) {
-#pragma unroll
-    for (int v = 0; v < 16; ++v)
-      part[wave - 2][row_of(v)][l32] = make_float4(acc[0][0][v], acc[0][1][v], acc[1][0][v], acc[1][1][v]);
-  }
-  __syncthreads();
-  if (wave < 2) {
-#pragma unroll
-    for (int v = 0; v < 16; ++v) {
-      float4* q = &part[wave][row_of(v)][l32];
-      const float4 o = *q;
-      *q = make_float4(acc[0][0][v] + o.x, acc[0][1][v] + o.y, acc[1][0][v] + o.z, acc[1][1][v] + o.w);
-    }
-  }
-  __syncthreads();
-#pragma unroll
-  for (int h = 0; h < TOK * kSmCols / (64 * kSmWaves); ++h) {
-    const int o = tid + h * 64 * kSmWaves, t = o / kSmCols, jj = o % kSmCols;
-    const int row = row0 + t, j = col0 + jj;
-    if (row >= row_end || j >= d_out) continue;
-    float4 u0 = part[0][2 * t][jj], u1 = part[0][2 * t + 1][jj];
-    const float4 w0 = part[1][2 * t][jj], w1 = part[1][2 * t + 1][jj];
-    u0.x += w0.x; u0.y += w0.y; u0.z += w0.z; u0.w += w0.w;
-    u1.x += w1.x; u1.y += w1.y; u1.z += w1.z; u1.w += w1.w;
-    float y[8];
-    pauli_to_blade(u0.x, u0.y, u1.x, u1.y, u0.z, u0.w, u1.z, u1.w, y);
-    if (bias != nullptr && (OUT != kSmPlanes || blockIdx.z == 0)) {
-#pragma unroll
-      for (int c = 0; c < 8; ++c) y[c] += bias[((size_t)e * d_out + j) * 8 + blade_to_mask(c)];
-    }
-    if constexpr (OUT == kSmPauliRows) {
-      activate_blade<ACT>(y);
-      float c0[4], c1[4];
-      blade_to_pauli(y, c0, c1);
-      uint16_t* q = static_cast<uint16_t*>(Y) + ((size_t)row * 2 * d_out + j) * 4;
-      *reinterpret_cast<uint2*>(q) = make_uint2(pack2_bf16(c0[0], c0[1]), pack2_bf16(c0[2], c0[3]));
-      *reinterpret_cast<uint2*>(q + (size_t)d_out * 4) = make_uint2(pack2_bf16(c1[0], c1[1]), pack2_bf16(c1[2], c1[3]));
-    } else {
-      float4* q = reinterpret_cast<float4*>(static_cast<float*>(Y) +
-                                            (((size_t)blockIdx.z * P_max + row) * d_out + j) * 8);
-      q[0] = make_float4(y[0], y[1], y[2], y[3]);
-      q[1] = make_float4(y[4], y[5], y[6], y[7]);
-    }
   }
 }
 
-long long small_row_tiles(int P, int E) { return std::min<long long>(P, (P + kSmTok - 1) / kSmTok + E); }  // at most
+// at most this many tiles of `tok` rows
+long long small_row_tiles(int P, int E, int tok) { return std::min<long long>(P, (P + tok - 1) / tok + E); }
 
 template <int ACT, int OUT>
 int launch_small(const void* x, int x_rows, const int32_t* gather, int P, const void* w, const float* bias,
-                 const int32_t* offsets, int E, int d_in, int d_out, int splits, void* y, hipStream_t st) {
-  const dim3 grid((unsigned)(small_row_tiles(P, E) * ((d_out + kSmCols - 1) / kSmCols)), 1, splits);
+                 const int32_t* offsets, int E, int d_in, int d_out, void* y, hipStream_t st) {
   const uint16_t* X = static_cast<const uint16_t*>(x);
   const uint16_t* W = static_cast<const uint16_t*>(w);
   const uint32_t xb = (uint32_t)((size_t)x_rows * d_in * 16);
-  pauli_small_kernel<ACT, OUT><<<grid, 64 * kSmWaves, 0, st>>>(X, xb, gather, W, bias, offsets, E, d_in, d_out, P, y);
+  const bool bias_first = pauli_uses_dma(kInPauliRows, d_in);  // (the register-staged 64 x 64 tiles add it at the end)
+#define YGG_PSL(RB, CB, RING)                                                                                          \
+  do {                                                                                                                  \
+    const unsigned grid = (unsigned)(small_row_tiles(P, E, 8 * RB) * ((d_out + 16 * CB - 1) / (16 * CB)));              \
+    if (bias_first)                                                                                                     \
+      pauli_small_kernel<ACT, OUT, true, RB, CB, RING><<<grid, 64, 0, st>>>(X, xb, gather, W, bias, offsets, E, d_in,  \
+                                                                            d_out, P, y);                               \
+    else                                                                                                                \
+      pauli_small_kernel<ACT, OUT, false, RB, CB, RING><<<grid, 64, 0, st>>>(X, xb, gather, W, bias, offsets, E, d_in, \
+                                                                             d_out, P, y);                              \
+  } while (0)
+  // 8 tokens x 16 columns a wave, six waves a CU, while the products are small: a wave's step is
+  // four MFMAs.  Above, every row tile reads its expert's weights once more, and 16 x 32 a wave
+  // are faster (layer calls, 8 x 16 / 16 x 32, us: d = 128, F = 512, E = 32: 2 rows 21 / 34, 512 39 / 46, 1024
+  // 51 / 53, 2048 75 / 65; d = 256, F = 1024, E = 64: 32 52 / 69, 512 142 / 149, 1024 185 / 173; d = 200,
+  // F = 800, E = 4: 128 34 / 51, 512 60 / 61, 1024 91 / 76; d = 64, F = 512, E = 64: 1024 48 / 50, 2048 64 / 59)
+  if (P <= 1024 && (double)P * d_in * d_out <= 8e7) YGG_PSL(1, 1, 8);
+  else YGG_PSL(2, 2, 6);
+#undef YGG_PSL
   return check_launch("pauli_small");
 }
 
 }  // namespace
 
-// splits of the down product's contraction: as many as leave a wave eight chunks (64
-// inputs), planes of at most 16 MiB
-int pauli_small_splits(int P, int E, int d_in, int d_out) {
-  (void)E;
-  long long s = (d_in + 8 * kSmPhase * kSmWaves - 1) / (8 * kSmPhase * kSmWaves);
-  s = std::min<long long>(s, ((long long)16 << 20) / std::max<long long>(1, (long long)P * d_out * 32));
-  return (int)std::max<long long>(1, std::min<long long>(s, 8));
-}
-
-bool pauli_small_pays(int N, int P, int E, int d, int F) {
-  const uint64_t lim = (uint64_t)1 << 31;
-  return P >= 1 && P <= kPauliSmallRows && (uint64_t)(std::max(d, F) + 64) * std::min(d, F) * 16 < lim &&
-         (uint64_t)P * std::max(d, F) * 16 < lim && (uint64_t)N * d * 16 < lim;
+// From these sizes on the 64 x 64 tiles are faster (layer calls, few rows / tiles, us: d = 128,
+// F = 512, E = 32: 2 rows 21 / 53, 512 39 / 64, 2048 65 / 74, 3072 80 / 81, 4096 105 / 89; d = 128, F = 1024,
+// E = 16: 1 27 / 78, 1536 87 / 99; d = 256, F = 1024, E = 64: 2 31 / 92, 128 109 / 147, 512 142 / 169, 1024
+// 173 / 178, 2048 249 / 202; d = 256, F = 512, E = 8: 1536 70 / 76, 2048 101 / 85; d = 200, F = 800, E = 4: 1024
+// 76 / 86, 1536 92 / 92; d = 100, F = 302, E = 12: 1536 41 / 54, 3072 57 / 56; d = 64, F = 512, E = 64: 2048
+// 59 / 73, 4096 82 / 81).
+bool pauli_small_pays(long long N, long long P, int E, int d, int F) {
+  if (P < 1 || P > 2048 || (double)P * d * F > 2e8) return false;
+  const uint64_t lim = (uint64_t)1 << 31;  // the kernel's 32-bit offsets
+  return (uint64_t)(std::max(d, F) + 64) * std::min(d, F) * 16 < lim && (uint64_t)P * std::max(d, F) * 16 < lim &&
+         (uint64_t)N * d * 16 < lim && (uint64_t)E * std::max(d, F) * 32 < lim;
 }
 
 int pauli_small_up(const void* x, int x_rows, const int32_t* gather, int P, const void* w, const float* bias,
                    const int32_t* offsets, int E, int d_in, int d_out, int act, void* h, hipStream_t stream) {
-#define YGG_PS(A) \
-  return launch_small<A, kSmPauliRows>(x, x_rows, gather, P, w, bias, offsets, E, d_in, d_out, 1, h, stream)
+#define YGG_PS(A) return launch_small<A, kOutPauliRows>(x, x_rows, gather, P, w, bias, offsets, E, d_in, d_out, h, stream)
   switch (act) {
     case kActNone: YGG_PS(kActNone);
     case kActGelu: YGG_PS(kActGelu);
@@ -277,8 +324,8 @@ int pauli_small_up(const void* x, int x_rows, const int32_t* gather, int P, cons
 }
 
 int pauli_small_down(const void* h, int P, const void* w, const float* bias, const int32_t* offsets, int E, int d_in,
-                     int d_out, int splits, float* planes, hipStream_t stream) {
-  return launch_small<kActNone, kSmPlanes>(h, P, nullptr, P, w, bias, offsets, E, d_in, d_out, splits, planes, stream);
+                     int d_out, void* y, hipStream_t stream) {
+  return launch_small<kActNone, kOutBlade>(h, P, nullptr, P, w, bias, offsets, E, d_in, d_out, y, stream);
 }
 
 }  // namespace ygg

@@ -117,20 +117,13 @@ const char* pauli_size_limit(int x_layout, int x_rows, bool gathered, int P_max,
                              int y_layout, int y_dtype);
 
 // bf16 Pauli products of few rows (pauli_small.hip): whether a layer's products take them,
-// the up product (Pauli half-rows in, h as Pauli half-rows), and the down product in
-// `splits` K ranges to fp32 blade planes (splits, P, d_out, 8) by product row
-// up to this many (token, expert) rows: every row tile of 16 reads its expert's weights
-// again, and from some 1500 rows on the 64 x 64 tiles are faster (layer calls, few-rows /
-// tiles, us: d = 128, F = 512, E = 32, k = 2: 128 rows 32 / 59, 512 45 / 65, 1024 66 / 75, 3072
-// 101 / 81; d = 128, F = 1024, E = 16, k = 1: 64 rows 30 / 83, 512 58 / 94, 2048 125 / 116; d = 256,
-// F = 1024, E = 64, k = 2: 1024 182 / 195, 2048 257 / 242)
-constexpr int kPauliSmallRows = 1280;
-bool pauli_small_pays(int N, int P, int E, int d, int F);
-int pauli_small_splits(int P, int E, int d_in, int d_out);
+// the up product (Pauli half-rows in, h as Pauli half-rows) and the down product (bf16
+// blade rows).  Their outputs are those of ygg_pauli_grouped_linear, bit for bit.
+bool pauli_small_pays(long long N, long long P, int E, int d, int F);
 int pauli_small_up(const void* x, int x_rows, const int32_t* gather, int P, const void* w, const float* bias,
                    const int32_t* offsets, int E, int d_in, int d_out, int act, void* h, hipStream_t stream);
 int pauli_small_down(const void* h, int P, const void* w, const float* bias, const int32_t* offsets, int E, int d_in,
-                     int d_out, int splits, float* planes, hipStream_t stream);
+                     int d_out, void* y, hipStream_t stream);
 
 // Blade rows -> Pauli rows carried by the workgroups of another launch (the routing
 // kernels append them to their own): n multivectors of x, rows of d, bf16 -> bf16

@@ -90,3 +90,54 @@ def test_bf16_rows_do_not_depend_on_the_batch(d, F, E, k):
     full = layer.moe_forward(x, logits=lg)
     for n in (1, 7, 500, 900):
         assert torch.equal(layer.moe_forward(x[:, :n].contiguous(), logits=lg[:n].contiguous()), full[:, :n])
+
+
+@pytest.mark.parametrize("N,d,E,k", [(64, 256, 8, 2), (256, 64, 8, 2), (1024, 40, 64, 4)])
+def test_route_energy_needs_no_scratch_up_to_1024_tokens(N, d, E, k):
+    """The C entry up to 1024 tokens: no workspace, a scratch that it does not touch, the outputs of the
+    same call in two steps."""
+    from yggdrasil_amd import ops
+    from yggdrasil_amd._native import check, lib, ptr, stream_handle
+
+    torch.manual_seed(N)
+    x = torch.randn(N, d, 8, device="cuda")
+    rw, rb = torch.randn(E, 4, device="cuda"), torch.randn(E, device="cuda")
+    out = {n: torch.empty(s, device="cuda", dtype=t) for n, s, t in (
+        ("idx", (N, k), torch.int32), ("w", (N, k), torch.float32), ("counts", (E,), torch.int32),
+        ("offsets", (E + 1,), torch.int32), ("perm", (N * k,), torch.int32), ("slot", (N, k), torch.int32))}
+    scratch = torch.full((N * E,), -7.0, device="cuda")
+    say(f"route_energy without workspace N={N} d={d} E={E}")
+    check(lib().ygg_route_energy(ptr(x), 0, N, d, ptr(rw), ptr(rb), E, k, ptr(out["idx"]), ptr(out["w"]),
+                                 ptr(out["counts"]), ptr(out["offsets"]), ptr(out["perm"]), ptr(out["slot"]),
+                                 ptr(scratch), None, 0, stream_handle(x.device)), "route_energy")
+    assert (scratch == -7.0).all()
+    ref = ops.route(ops.router_energy_logits(x, rw, rb), k)
+    same = (out["idx"] == ref.topk_idx).all(dim=1)  # (the two sum in another order: ties may differ)
+    assert same.float().mean().item() > 0.98
+    assert (out["w"] - ref.topk_w)[same].abs().max().item() < 1e-5
+    assert int(out["counts"].sum()) == N * k and torch.equal(out["offsets"][1:], out["counts"].cumsum(0).int())
+    tok = torch.arange(N, device="cuda").repeat_interleave(k)
+    assert torch.equal(out["perm"][out["slot"].flatten().long()].long(), tok)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("N,d,E,k", [(63, 256, 8, 2), (203, 66, 8, 3), (256, 64, 64, 2), (1024, 40, 33, 4)])
+def test_energy_logits_of_the_layer_and_the_entry_are_the_same(N, d, E, k, dtype):
+    """From these sizes on a layer takes the grade-energy logits in a launch of its own, the entry never does:
+    the same sums in the same order, so the same weights bit for bit, every token."""
+    import yggdrasil_amd
+    from yggdrasil_amd import ops
+
+    cfg = yggdrasil_amd.MoEHLMConfig(d_model=d, d_ff=16, n_experts=E, top_k=k, dtype=dtype, router="energy")
+    layer = yggdrasil_amd.CliffordMoELayer(cfg, device="cuda")
+    with torch.no_grad():
+        layer.router_weight.normal_()
+        layer.router_bias.normal_()
+    x = torch.randn(1, N, d, 8, device="cuda").to(dtype)
+    say(f"energy logits N={N} d={d} E={E} {dtype}")
+    with torch.no_grad():
+        layer.moe_forward(x)
+    r = ops.route_energy(x[0], layer.router_weight.detach(), layer.router_bias.detach(), k)
+    got = layer.last_routing
+    assert torch.equal(got["topk_idx"], r.topk_idx) and torch.equal(got["topk_w"], r.topk_w)
+    assert torch.equal(got["counts"], r.counts) and torch.equal(got["offsets"], r.offsets)

@@ -613,16 +613,19 @@ YGG_API int ygg_router_energy_logits(const void* x, int x_dtype, int N, int d, c
 // CliffordRouter.forward end to end (clifford_router.py:54-104) plus the expert
 // counting sort (hlm_block.py:165-177): grade energies of x, the (E, 4) map and
 // bias, softmax, top-k, renormalisation, counts, offsets, perm and slot rows.
-// Up to 1024 tokens it is one launch (the logits never leave the chip); beyond,
-// the logits go through `logits_scratch` (N x E fp32) and ygg_route.
+// Up to 1024 tokens it is one launch (the logits never leave the chip, so the caller
+// needs neither scratch nor workspace); beyond, the logits go through
+// `logits_scratch` (N x E fp32) and ygg_route.
 YGG_API int ygg_route_energy(const void* x, int x_dtype, int N, int d, const float* router_w, const float* router_b,
                              int E, int k, int32_t* topk_idx, float* topk_w, int32_t* counts, int32_t* offsets,
                              int32_t* perm, int32_t* slot_pos, float* logits_scratch, void* workspace,
                              size_t workspace_bytes, hipStream_t stream) {
   return ygg::route_energy_convert(x, x_dtype, N, d, router_w, router_b, E, k, topk_idx, topk_w, counts, offsets, perm,
-                                   slot_pos, logits_scratch, workspace, workspace_bytes, RowConvert{}, stream);
+                                   slot_pos, N <= kSmallMaxN ? nullptr : logits_scratch, workspace, workspace_bytes,
+                                   RowConvert{}, stream);
 }
 
+// With logits_scratch (and the workspace of ygg_route) smaller batches too may go through it.
 int ygg::route_energy_convert(const void* x, int x_dtype, int N, int d, const float* router_w, const float* router_b,
                               int E, int k, int32_t* topk_idx, float* topk_w, int32_t* counts, int32_t* offsets,
                               int32_t* perm, int32_t* slot_pos, float* logits_scratch, void* workspace,

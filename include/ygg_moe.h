@@ -28,7 +28,7 @@
  *  - dtype codes: 0 = fp32, 1 = bf16 (activations); weight formats:
  *    0 = fp32, 1 = bf16 (dual, sign-folded), 2 = int8 per-output-channel,
  *    3 = bf16 Pauli (the weights as 2x2 complex matrices; even d_in),
- *    4 = fp32 Pauli (fp32 layers on the fp32 MFMA units),
+ *    4 = fp32 Pauli (fp32 layers; ygg_f32_layer_split says on which MFMA units),
  *    5 = int8 Pauli (the entries of each weight's 2x2 complex matrix, int8 per
  *        output channel; bf16 decode layers of at most 128 tokens, d <= 128).
  *    activation codes: 0 none, 1 gelu, 2 relu, 3 sigmoid
@@ -59,7 +59,7 @@ int ygg_version(void);
  * cl3_geom_matmul_flat (mjolnir/src/cpu/batch_ops.c:165-172, declared
  * mjolnir/include/cl3_ops.h:210, bound at rune/bindings/mjolnir_ffi.py:208-209).
  * Unlike those, it reports errors and takes the stream explicitly.  Computed as
- * one fp32 Pauli MFMA product (a as the weight of a single expert, the columns
+ * one fp32 Pauli product (a as the weight of a single expert, the columns
  * of b as its rows); its scratch (the converted operands) is taken from the
  * device's stream-ordered pool for the call. */
 int ygg_geom_matmul_f32(const float* a, const float* b, float* out, int M, int K, int N, ygg_stream_t stream);
@@ -217,6 +217,12 @@ int ygg_pauli_grouped_linear_f32(const float* x, const int32_t* gather, int P_ma
 size_t ygg_clifford_linear_workspace_bytes(int dtype, int rows, int d_in, int d_out);
 int ygg_clifford_linear(const void* x, int dtype, int rows, const void* w, const float* bias, int d_in, int d_out,
                         void* y, void* workspace, size_t workspace_bytes, ygg_stream_t stream);
+
+/* 1 where fp32 work runs on the bf16 MFMA units, every value as three bf16 parts (24 bits), and 0
+ * where it runs on the fp32 ones: a product of `rows` rows (ygg_geom_matmul_f32's columns of b,
+ * ygg_clifford_linear's rows), and the products and weight gradients of a format 4 layer. */
+int ygg_f32_product_split(int rows, int d_in, int d_out);
+int ygg_f32_layer_split(int N, int d, int F, int E, int k);
 
 /* Blade-order fp32 rows (rows, d, 8) -> fp32 Pauli rows (rows, d, 2, 2, 2): element
  * [m][i][b][k][c] is the real (k = 0) or imaginary (k = 1) part of entry (c, b) of

@@ -141,3 +141,124 @@ def test_energy_logits_of_the_layer_and_the_entry_are_the_same(N, d, E, k, dtype
     got = layer.last_routing
     assert torch.equal(got["topk_idx"], r.topk_idx) and torch.equal(got["topk_w"], r.topk_w)
     assert torch.equal(got["counts"], r.counts) and torch.equal(got["offsets"], r.offsets)
+
+
+def _split(*sizes):
+    """The case runs on the units it means to test."""
+    from yggdrasil_amd._native import lib
+
+    assert (lib().ygg_f32_product_split if len(sizes) == 3 else lib().ygg_f32_layer_split)(*sizes) == 1
+
+
+def _rows_rel(got, ref):
+    """The largest relative 2-norm error of a row."""
+    got, ref = np.asarray(got, np.float64), np.asarray(ref, np.float64)
+    got, ref = got.reshape(got.shape[0], -1), ref.reshape(ref.shape[0], -1)
+    return float((np.linalg.norm(got - ref, axis=1) / np.linalg.norm(ref, axis=1)).max())
+
+
+# 24 bits of each operand, sums of up to 1000 fp32 terms of random sign: 2^-24 sqrt(1000) of a row's norm at most
+FP32_ROW = 2e-6
+
+
+@pytest.mark.parametrize("M,K,N", [(64, 128, 6400), (70, 130, 6000), (129, 33, 3300)])
+def test_geom_matmul_keeps_small_inputs_beside_large_ones(M, K, N):
+    """Output rows whose weights are zero on the large inputs depend on the small ones, 2^-28 below, alone."""
+    from yggdrasil_amd import ops
+
+    _split(N, K, M)
+    g = np.random.default_rng(M)
+    a = g.standard_normal((M, K, 8)).astype(np.float32)
+    b = g.standard_normal((K, N, 8)).astype(np.float32)
+    a[::2, :K // 2] = 0.0
+    b[:K // 2] *= np.float32(2.0 ** 28)
+    say(f"geom_matmul, small inputs beside large ones M={M} K={K} N={N}")
+    out = ops.geom_matmul(torch.from_numpy(a).cuda(), torch.from_numpy(b).cuda()).cpu().numpy()
+    ref = np.transpose(dense.linear(np.transpose(b, (1, 0, 2)), a), (1, 0, 2))
+    assert _rows_rel(out, ref) < FP32_ROW
+
+
+def _lopsided(N, d, F, E, scale):
+    """An expert's first token is `scale` times the others and lies in the first half of the inputs, from which the
+    second half of the hidden channels has no weights."""
+    g = np.random.default_rng(N + F)
+    x = g.standard_normal((N, d, 8)).astype(np.float32)
+    lg = g.standard_normal((N, E)).astype(np.float32)
+    big = [int(np.flatnonzero(lg.argmax(1) == e)[0]) for e in range(E)]
+    x[big] *= np.float32(scale)
+    x[big, d // 2:] = 0.0
+    wu = (g.standard_normal((E, F, d, 8)) / np.sqrt(8 * d)).astype(np.float32)
+    wu[:, F // 2:, :d // 2] = 0.0
+    wd = (g.standard_normal((E, d, F, 8)) / np.sqrt(8 * F)).astype(np.float32)
+    return g, x, lg, big, wu, wd, np.zeros((E, F, 8), np.float32), np.zeros((E, d, 8), np.float32)
+
+
+@pytest.mark.parametrize("N,F", [(4096, 128), (20000, 250)])
+def test_layer_and_gradients_keep_small_rows_beside_large_ones(N, F):
+    """A token 2^25 times the others, in x and in the output's gradient: weight gradients to which it adds exact
+    zeros keep the other tokens' to fp32, and the other tokens' outputs and gradients theirs.  (The weight gradients
+    take the fp32 units in the smaller case, the bf16 ones in the larger.)"""
+    import yggdrasil_amd
+
+    d, E = 128, 2
+    _split(N, d, F, E, 1)
+    g, x, lg, big, wu, wd, bu, bd = _lopsided(N, d, F, E, 2.0 ** 25)
+    dout = g.standard_normal((N, d, 8)).astype(np.float32)
+    dout[big] *= np.float32(2.0 ** 25)
+    cfg = yggdrasil_amd.MoEHLMConfig(d_model=d, d_ff=F, n_experts=E, top_k=1, activation="gelu", router="logits")
+    layer = yggdrasil_amd.CliffordMoELayer(cfg, device="cuda")
+    layer.load_reference_weights(w_up=wu, b_up=bu, w_down=wd, b_down=bd)
+    say("fp32 layer, one token 2^25 times the others")
+    xt = torch.from_numpy(x).cuda()[None].requires_grad_(True)
+    out = layer.moe_forward(xt, logits=torch.from_numpy(lg).cuda())
+    grads = torch.autograd.grad(out, (xt, layer.w_up, layer.w_down), torch.from_numpy(dout).cuda()[None])
+    dx, dwu, dwd = (t.cpu().numpy() for t in grads)
+    idx = layer.last_routing["topk_idx"].cpu().numpy()
+    w = layer.last_routing["topk_w"].cpu().numpy()
+    ref = dense.moe_layer(x, idx, w, wu, bu, wd, bd, "gelu")
+    rdx, rwu, _, rwd, _ = dense.moe_layer_backward(x, idx, w, wu, bu, wd, bd, dout, "gelu")
+    # two products in turn and the activation's fast exponential (2^-21 of a component)
+    assert _rows_rel(out[0].detach().cpu().numpy(), ref) < 2 * FP32_ROW
+    assert _rows_rel(dx[0], rdx) < 2 * FP32_ROW
+    for e in range(E):
+        # sums over 10000 tokens of terms of random sign, 384 at a time: below 2^-24 sqrt(1000) of a row's norm, and
+        # the products' errors
+        assert _rows_rel(dwd[e][:, F // 2:], rwd[e][:, F // 2:]) < 2 * FP32_ROW  # (the large token's h is zero there)
+        assert _rows_rel(dwu[e][:, d // 2:], rwu[e][:, d // 2:]) < 2 * FP32_ROW  # (and its x there)
+        assert _rows_rel(dwd[e][:, :F // 2], rwd[e][:, :F // 2]) < 2 * FP32_ROW
+
+
+@pytest.mark.parametrize("k", [1, 2])
+def test_layer_with_non_finite_rows(k):
+    """Tokens with a NaN or an infinity: their rows are not finite, every other row is as without them."""
+    import yggdrasil_amd
+
+    N, d, F, E = 3000, 100, 130, 3
+    _split(N, d, F, E, k)
+    torch.manual_seed(k)
+    layer = yggdrasil_amd.CliffordMoELayer(
+        yggdrasil_amd.MoEHLMConfig(d_model=d, d_ff=F, n_experts=E, top_k=k, router="logits"), device="cuda")
+    x, lg = torch.randn(1, N, d, 8, device="cuda"), torch.randn(N, E, device="cuda")
+    x[0, 11] = 0.0
+    bad = x.clone()
+    bad[0, 7, 3, 2] = float("nan")
+    bad[0, 2222, 99, 0] = float("inf")
+    say(f"fp32 layer, non-finite tokens, k={k}")
+    with torch.no_grad():
+        out, out_bad = layer.moe_forward(x, logits=lg), layer.moe_forward(bad, logits=lg)
+    keep = torch.ones(N, dtype=torch.bool, device="cuda")
+    keep[[7, 2222]] = False
+    assert torch.isfinite(out).all() and torch.equal(out[0][keep], out_bad[0][keep])
+    assert not torch.isfinite(out_bad[0, [7, 2222]]).flatten(1).all(dim=1).any()
+    # a NaN in one token's gradient reaches the weights of its experts only
+    xt = x.clone().requires_grad_(True)
+    go = torch.randn_like(x)
+    params = (layer.w_up, layer.b_up, layer.w_down, layer.b_down)
+    ref = torch.autograd.grad(layer.moe_forward(xt, logits=lg), params, go)
+    go[0, 7, 5, 1] = float("nan")
+    got = torch.autograd.grad(layer.moe_forward(xt, logits=lg), params, go)
+    hit = set(layer.last_routing["topk_idx"][7].tolist())
+    for a, b in zip(ref, got):
+        for e in range(E):
+            assert torch.isfinite(b[e]).all() == (e not in hit)
+            assert e in hit or torch.equal(a[e], b[e])

@@ -48,6 +48,8 @@ SIGNATURES = {
                                               _c_int, _vp]),
     "ygg_clifford_linear_workspace_bytes": (_c_size, [_c_int, _c_int, _c_int, _c_int]),
     "ygg_clifford_linear": (_c_int, [_vp, _c_int, _c_int, _vp, _vp, _c_int, _c_int, _vp, _vp, _c_size, _vp]),
+    "ygg_f32_product_split": (_c_int, [_c_int, _c_int, _c_int]),
+    "ygg_f32_layer_split": (_c_int, [_c_int, _c_int, _c_int, _c_int, _c_int]),
     "ygg_pauli_rows_from_blade_f32": (_c_int, [_vp, _c_int, _c_int, _vp, _vp]),
     "ygg_moe_workspace_bytes": (_c_size, [_c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int]),
     "ygg_moe_forward": (_c_int, [_vp, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _vp, _vp, _vp,

@@ -21,7 +21,7 @@
 
 #include <algorithm>
 
-#include "pauli_common.h"
+#include "pauli_split.h"
 #include "ygg_common.h"
 
 namespace ygg {
@@ -116,73 +116,6 @@ __global__ __launch_bounds__(256) void act_backward_kernel(const float* __restri
   if (out_pauli != nullptr) store_pauli_f32(out_pauli + n * 8, o);
 }
 
-// Row-wise: the activation of h (BWD false) or its backward of g at h, as split rows.  One
-// workgroup per row; with U > 0 a thread keeps its U multivectors between the row's
-// maximum and the store (d <= 256 U), with U = 0 it computes them twice.
-template <int ACT, bool BWD, int U>
-__global__ __launch_bounds__(256) void act_split_kernel(const float* __restrict__ h, const float* __restrict__ g, int d,
-                                                        unsigned char* __restrict__ out, int32_t* __restrict__ row_exp) {
-  __shared__ uint32_t wm[4];
-  const size_t r = blockIdx.x;
-  const int t = threadIdx.x, d_pad = (d + 7) & ~7;
-  const float* hr = h + r * d * 8;
-  const float* gr = BWD ? g + r * d * 8 : nullptr;
-  auto value = [&](int i, float* o) __attribute__((always_inline)) {
-    if (i >= d) {
-#pragma unroll
-      for (int c = 0; c < 8; ++c) o[c] = 0.f;
-      return;
-    }
-    float x[8];
-    const float4* hp = reinterpret_cast<const float4*>(hr + (size_t)i * 8);
-    const float4 h0 = hp[0], h1 = hp[1];
-    x[0] = h0.x; x[1] = h0.y; x[2] = h0.z; x[3] = h0.w; x[4] = h1.x; x[5] = h1.y; x[6] = h1.z; x[7] = h1.w;
-    if constexpr (BWD) {
-      float gv[8];
-      const float4* gp = reinterpret_cast<const float4*>(gr + (size_t)i * 8);
-      const float4 g0 = gp[0], g1 = gp[1];
-      gv[0] = g0.x; gv[1] = g0.y; gv[2] = g0.z; gv[3] = g0.w; gv[4] = g1.x; gv[5] = g1.y; gv[6] = g1.z; gv[7] = g1.w;
-      act_backward_mv<ACT>(x, gv, o);
-    } else {
-#pragma unroll
-      for (int c = 0; c < 8; ++c) o[c] = x[c];
-      activate_blade<ACT>(o);
-    }
-  };
-  constexpr int UC = U > 0 ? U : 1;
-  float o[UC][8];
-  uint32_t m = 0;
-  if constexpr (U > 0) {
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      value(t + 256 * u, o[u]);
-      m = max(m, pauli_mag(o[u]));
-    }
-  } else {
-    for (int i = t; i < d; i += 256) {
-      value(i, o[0]);
-      m = max(m, pauli_mag(o[0]));
-    }
-  }
-  m = wave_max_u32(m);
-  if ((t & 63) == 0) wm[t >> 6] = m;
-  __syncthreads();
-  m = max(max(wm[0], wm[1]), max(wm[2], wm[3]));
-  const int s = split_exp(__builtin_bit_cast(float, m));
-  if (t == 0) row_exp[r] = s;
-  unsigned char* row = out + r * pauli_split_row_bytes(d);
-  if constexpr (U > 0) {
-#pragma unroll
-    for (int u = 0; u < U; ++u)
-      if (t + 256 * u < d_pad) store_split_mv(row, d_pad, t + 256 * u, o[u], s);
-  } else {
-    for (int i = t; i < d_pad; i += 256) {
-      value(i, o[0]);
-      store_split_mv(row, d_pad, i, o[0], s);
-    }
-  }
-}
-
 // The forward activation of blade-order rows (the same activate_blade the fused
 // epilogues apply), for the backward's recompute of h from h before the activation.
 template <int ACT>
@@ -205,74 +138,21 @@ __global__ __launch_bounds__(256) void act_forward_kernel(const float* __restric
 // ---- combine backward: dy[slot] = w dout_t; dw[t, s] = <dout_t, y[slot]> ----------
 // One wave per token, a multivector per lane; dy goes out in blade order and/or as
 // fp32 Pauli rows (whichever is not NULL).
-constexpr int kCbU = 4;  // multivectors of a token's row per lane that stay in registers
 __global__ __launch_bounds__(256) void combine_backward_kernel(const float* __restrict__ dout,
                                                                const float* __restrict__ y_sorted, int N, int k,
                                                                int d, const float* __restrict__ topk_w,
                                                                const int32_t* __restrict__ slot_pos,
                                                                float* __restrict__ dy_sorted,
                                                                float* __restrict__ dy_pauli,
-                                                               float* __restrict__ dtopk_w,
-                                                               unsigned char* __restrict__ dy_split,
-                                                               int32_t* __restrict__ dy_exp) {
+                                                               float* __restrict__ dtopk_w) {
   const int lane = threadIdx.x & 63;
   const int t = blockIdx.x * 4 + (threadIdx.x >> 6);
   if (t >= N) return;
   const float* go = dout + (size_t)t * d * 8;
-  float gr[kCbU][8];  // split rows: the token's row, read once for its k slots
-  if (dy_split && d <= 64 * kCbU) {
-#pragma unroll
-    for (int u = 0; u < kCbU; ++u) {
-      const int i = lane + 64 * u;
-      const float4* gp = reinterpret_cast<const float4*>(go + (size_t)min(i, d - 1) * 8);
-      const float4 a = gp[0], b = gp[1];
-      const float v[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
-#pragma unroll
-      for (int c = 0; c < 8; ++c) gr[u][c] = i < d ? v[c] : 0.f;
-    }
-  }
   for (int s = 0; s < k; ++s) {
     const size_t row = (size_t)slot_pos[(size_t)t * k + s];
     const float w = topk_w[(size_t)t * k + s];
     float acc = 0.f;
-    if (dy_split) {  // the row's largest entry, then its split parts
-      const int d_pad = (d + 7) & ~7;
-      unsigned char* dst = dy_split + row * pauli_split_row_bytes(d);
-      uint32_t m = 0;
-      if (d <= 64 * kCbU) {  // the token's row is in registers
-#pragma unroll
-        for (int u = 0; u < kCbU; ++u) {
-          float o[8];
-#pragma unroll
-          for (int c = 0; c < 8; ++c) o[c] = lane + 64 * u < d ? w * gr[u][c] : 0.f;  // (w may be infinite)
-          m = max(m, pauli_mag(o));
-        }
-      } else {
-        for (int i = lane; i < d; i += 64) {
-          float o[8];
-          for (int c = 0; c < 8; ++c) o[c] = w * go[(size_t)i * 8 + c];
-          m = max(m, pauli_mag(o));
-        }
-      }
-      const int sx = split_exp(__builtin_bit_cast(float, wave_max_u32(m)));
-      if (lane == 0) dy_exp[row] = sx;
-      if (d <= 64 * kCbU) {
-#pragma unroll
-        for (int u = 0; u < kCbU; ++u) {
-          float o[8];
-#pragma unroll
-          for (int c = 0; c < 8; ++c) o[c] = lane + 64 * u < d ? w * gr[u][c] : 0.f;
-          if (lane + 64 * u < d_pad) store_split_mv(dst, d_pad, lane + 64 * u, o, sx);
-        }
-      } else {
-        for (int i = lane; i < d_pad; i += 64) {
-          float o[8];
-          for (int c = 0; c < 8; ++c) o[c] = i < d ? w * go[(size_t)i * 8 + c] : 0.f;
-          store_split_mv(dst, d_pad, i, o, sx);
-        }
-      }
-      if (!dtopk_w) continue;
-    }
     for (int i = lane; i < d; i += 64) {
       const float4* gp = reinterpret_cast<const float4*>(go + (size_t)i * 8);
       const float4 g0 = gp[0], g1 = gp[1];
@@ -708,30 +588,23 @@ __global__ __launch_bounds__(256, 2) void weight_grad_mfma_kernel(const float* _
   }
 }
 
-// The same from split rows (two fp16 parts per Pauli entry, each row scaled by its own
-// power of two) on v_mfma_f32_32x32x16_f16: K = 16 holds four rows x b x (re, im), a lane
-// two rows of them.  A lane loads (entry 0, entry 1) of its column -- 8 bytes, hi and lo
-// apart -- for each of its four half-rows; entry 0's four dwords are one operand, entry
-// 1's another.  Im(D conj(A)) takes the D operand rotated, (re, im) -> (im, -re).  Rows
-// enter a sum with one common scale, 2^-(exponent of D + exponent of A) of the row that
-// is the largest of the chunk: D is multiplied by the ratio (a power of two, at most 1).
-// Three products (hi hi, lo hi, hi lo) as in pauli_gemm.hip.  The fp32 kernel above ran at
-// 64 % of its units' rate (1290-1310 us at 32768 rows, 512 x 128, 32 experts); this one
-// takes 551 us (750 TFLOP/s issued), bound by the loads' latency and the vector work beside the MFMAs (rotation,
-// scale).  All tiles of a chunk run on one XCD, so its rows are read into one L2.
+// The same on the bf16 MFMA units (the sums: pauli_split.h), for batches whose products run there: a
+// step is eight rows, as pauli_split.hip's is eight inputs -- the operands (16 KiB of D, 16 KiB of
+// the gathered rows of A) direct to LDS, double buffered, a wave 32 j x 32 i of the workgroup's
+// 64 x 64, every value cut into parts on its way to the MFMA.  Bound by the MFMAs: 32768 rows, 512 x
+// 128, 32 experts 758 us, 1.09 PFLOP/s issued (1290-1310 us on the fp32 units), error against float64
+// 2.0e-7 (7.2e-7).  All tiles of a chunk run on one XCD, so its rows are read into one L2;
+// the workgroups behind the chunk's tiles add its rows of D, in fp32, for the bias gradient.
 __global__ __launch_bounds__(256, 2) void weight_grad_split_kernel(
-    const unsigned char* __restrict__ Ds, const int32_t* __restrict__ d_exp, const unsigned char* __restrict__ As,
-    uint32_t a_bytes, const int32_t* __restrict__ a_exp, const int32_t* __restrict__ gather,
-    const int32_t* __restrict__ offsets, int E, int d_in, int d_out, int n_chunks, int n_xcd,
-    float* __restrict__ part, float* __restrict__ dbpart, float* __restrict__ dW, float* __restrict__ db) {
-  typedef unsigned int u32x2_t __attribute__((ext_vector_type(2)));
-  __shared__ alignas(8) uint32_t s_delta[kWgmChunk];  // the row's ratio, twice, as fp16
-  __shared__ alignas(8) uint32_t s_src[kWgmChunk];    // byte offset of the row of A
-  __shared__ int s_q[kWgmChunk];
-  __shared__ int s_min[4];
-  const int nj = (d_out + kWgmTile - 1) / kWgmTile, ni = (d_in + kWgmTile - 1) / kWgmTile, nt = nj * ni;
-  const int xcd = blockIdx.x % n_xcd, bq = blockIdx.x / n_xcd;
-  const int chunk = bq / nt * n_xcd + xcd, tile = bq % nt;
+    const float* __restrict__ Dp, const float* __restrict__ Ap, uint32_t a_bytes, const int32_t* __restrict__ gather,
+    const int32_t* __restrict__ offsets, int E, int d_in, int d_out, int n_chunks, int n_xcd, float* __restrict__ part,
+    float* __restrict__ dbpart, float* __restrict__ dW, float* __restrict__ db) {
+  constexpr int kRows = 8, kStage = kRows * kWgmTile * 32;  // rows of a step; bytes of one operand of it
+  __shared__ __attribute__((aligned(1024))) unsigned char smem[4 * kStage];
+  __shared__ int s_src[kWgmChunk];  // the chunk's rows of A
+  const int nj = (d_out + kWgmTile - 1) / kWgmTile, ni = (d_in + kWgmTile - 1) / kWgmTile;
+  const int nt = nj * ni + (db != nullptr ? nj : 0);
+  const int bq = blockIdx.x / n_xcd, chunk = bq / nt * n_xcd + (blockIdx.x - bq * n_xcd), tile = bq % nt;
   const int tid = threadIdx.x, lane = tid & 63;
   int e, r0, r1;
   bool only;
@@ -739,171 +612,133 @@ __global__ __launch_bounds__(256, 2) void weight_grad_split_kernel(
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   r0 = __builtin_amdgcn_readfirstlane(r0);
   r1 = __builtin_amdgcn_readfirstlane(r1);
-  const int l32 = lane & 31, g = lane >> 5, rows = r1 - r0;
-  const uint32_t half_d = (uint32_t)pauli_split_row_bytes(d_out) / 2, half_a = (uint32_t)pauli_split_row_bytes(d_in) / 2;
-  int qmin = 0x7fffffff;
-  for (int i = tid; i < kWgmChunk; i += 256) {
-    if (i < rows) {
-      const int src = gather ? gather[r0 + i] : r0 + i;
-      const int q = d_exp[r0 + i] + a_exp[src];
-      s_q[i] = q;
-      s_src[i] = (uint32_t)(gather ? src : i) * 2 * half_a;
-      qmin = min(qmin, q);
-    } else {
-      s_src[i] = kBufferOff;
-    }
-  }
+  const int rows = r1 - r0;
+  if (tile >= nj * ni) {  // the bias gradient of 64 channels: every fourth row a wave, added in wave order
+    const int j = (tile - nj * ni) * kWgmTile + lane;
+    float t[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};  // [b][k][a]
+    if (j < d_out)
+      for (int r = r0 + wave; r < r1; r += 4) {
+        const float4* q = reinterpret_cast<const float4*>(Dp + ((size_t)r * d_out + j) * 8);
+        const float4 u = q[0], w = q[1];
+        t[0] += u.x; t[1] += u.y; t[2] += u.z; t[3] += u.w;
+        t[4] += w.x; t[5] += w.y; t[6] += w.z; t[7] += w.w;
+      }
+    float* const red = reinterpret_cast<float*>(smem);  // [wave][value][lane]
 #pragma unroll
-  for (int o = 32; o > 0; o >>= 1) qmin = min(qmin, __shfl_xor(qmin, o));
-  if (lane == 0) s_min[wave] = qmin;
-  __syncthreads();
-  const int Q = min(min(s_min[0], s_min[1]), min(s_min[2], s_min[3]));
-  for (int i = tid; i < kWgmChunk; i += 256) {
-    const int sh = i < rows ? Q - s_q[i] : -100;
-    const _Float16 f = (_Float16)__builtin_ldexpf(1.f, max(sh, -100));  // below 2^-24 of the largest row: 0
-    s_delta[i] = (uint32_t)__builtin_bit_cast(uint16_t, f) * 0x10001u;
+    for (int c = 0; c < 8; ++c) red[(wave * 8 + c) * 64 + lane] = t[c];
+    __syncthreads();
+    if (wave > 0 || j >= d_out) return;
+#pragma unroll
+    for (int w = 1; w < 4; ++w)
+#pragma unroll
+      for (int c = 0; c < 8; ++c) t[c] += red[(w * 8 + c) * 64 + lane];
+    if (only) {
+      store_db(db + ((size_t)e * d_out + j) * 8, t);
+    } else {
+      float4* q = reinterpret_cast<float4*>(dbpart + ((size_t)chunk * d_out + j) * 8);
+      q[0] = make_float4(t[0], t[1], t[2], t[3]);
+      q[1] = make_float4(t[4], t[5], t[6], t[7]);
+    }
+    return;
   }
-  __syncthreads();
-
-  const int jt = tile % nj, it = tile / nj;
-  const int j0 = jt * kWgmTile + (wave & 1) * 32, i0 = it * kWgmTile + (wave >> 1) * 32;
-  const int jc = min(j0 + l32, d_out - 1), ic = min(i0 + l32, d_in - 1);  // clamped loads, not stored
+  for (int i = tid; i < rows; i += 256) s_src[i] = gather ? gather[r0 + i] : i;
+  const int jt = tile % nj, it = tile / nj, j0 = jt * kWgmTile, i0 = it * kWgmTile;
   // rows of the chunk in D; rows of A: the chunk's, or the whole of A through `gather`
   const __amdgpu_buffer_rsrc_t d_rsrc = __builtin_amdgcn_make_buffer_rsrc(
-      const_cast<unsigned char*>(Ds) + (size_t)r0 * 2 * half_d, (short)0, (uint32_t)rows * 2 * half_d, kBufferFlags);
-  const __amdgpu_buffer_rsrc_t a_rsrc = __builtin_amdgcn_make_buffer_rsrc(
-      const_cast<unsigned char*>(As) + (gather ? 0 : (size_t)r0 * 2 * half_a), (short)0,
-      gather ? a_bytes : (uint32_t)rows * 2 * half_a, kBufferFlags);
-  const uint32_t d_col = (uint32_t)(jc >> 3) * 128 + (jc & 7) * 8 + (uint32_t)(2 * g) * 2 * half_d;
-  const uint32_t a_col = (uint32_t)(ic >> 3) * 128 + (ic & 7) * 8;
-  const bool bias_wave = dbpart != nullptr && it == 0 && (wave >> 1) == 0;
-
-  pf32x16_t acc[2][2][2];
+      const_cast<float*>(Dp) + (size_t)r0 * d_out * 8, (short)0, (uint32_t)rows * d_out * 32, kBufferFlags);
+  const __amdgpu_buffer_rsrc_t a_rsrc =
+      __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(Ap) + (gather ? 0 : (size_t)r0 * d_in * 8), (short)0,
+                                        gather ? a_bytes : (uint32_t)rows * d_in * 32, kBufferFlags);
+  // This lane's pieces (16 bytes): load u covers row 2 wave + u / 2 of the step and 32 columns
+  // (u % 2); slot 2 j + s of a row's run holds (column j, b = s ^ (j / 8 % 2)), which keeps the
+  // operand reads free of conflicts.
+  uint32_t d_off[2], a_off[2];
 #pragma unroll
-  for (int a = 0; a < 2; ++a)
+  for (int u = 0; u < 2; ++u) {
+    const int c = u * 32 + (lane >> 1), b = (lane & 1) ^ ((c >> 3) & 1);
+    d_off[u] = j0 + c < d_out ? (uint32_t)(j0 + c) * 32 + b * 16 : kBufferOff;
+    a_off[u] = i0 + c < d_in ? (uint32_t)(i0 + c) * 32 + b * 16 : kBufferOff;
+  }
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(sp_lds_t*)smem;
+  auto issue = [&](int f) __attribute__((always_inline)) {  // step f's rows to stage f % 2; past the chunk: zeros
+    const uint32_t st = lds0 + (f & 1) * 2 * kStage + 4 * wave * 1024;
 #pragma unroll
-    for (int c = 0; c < 2; ++c)
-#pragma unroll
-      for (int q = 0; q < 2; ++q)
-#pragma unroll
-        for (int v = 0; v < 16; ++v) acc[a][c][q][v] = 0.f;
-  float bs[2][2][2] = {};  // [b][re, im][a]
-
-  struct Ops {
-    u32x2_t d[2][4], x[2][4];  // [hi, lo][half-row: row of the lane's two, b]; (entry 0, entry 1)
-  };
-  auto load_rows = [&](int r, Ops& o) __attribute__((always_inline)) {  // rows r .. r + 3 of the chunk
-    // the row in the vector offset, which the range check covers: a row past the end reads zero
-    const uint32_t dv[2] = {(uint32_t)r * 2 * half_d + d_col, (uint32_t)(r + 1) * 2 * half_d + d_col};
-    const uint2 src = *reinterpret_cast<const uint2*>(&s_src[r + 2 * g]);
-#pragma unroll
-    for (int p = 0; p < 2; ++p)
-#pragma unroll
-      for (int hr = 0; hr < 4; ++hr) {
-        o.d[p][hr] = __builtin_amdgcn_raw_buffer_load_b64(d_rsrc, dv[hr >> 1] + p * 64, (hr & 1) * half_d, 0);
-        o.x[p][hr] = __builtin_amdgcn_raw_buffer_load_b64(a_rsrc, (hr < 2 ? src.x : src.y) + a_col + p * 64,
-                                                          (hr & 1) * half_a, 0);
-      }
-  };
-  auto mma_rows = [&](int r, const Ops& o) __attribute__((always_inline)) {
-    const uint2 dl = *reinterpret_cast<const uint2*>(&s_delta[r + 2 * g]);
-    pf16x8_t X[2][2];  // [hi, lo][c]
-#pragma unroll
-    for (int p = 0; p < 2; ++p)
-#pragma unroll
-      for (int c = 0; c < 2; ++c)
-        X[p][c] = __builtin_bit_cast(pf16x8_t, make_uint4(o.x[p][0][c], o.x[p][1][c], o.x[p][2][c], o.x[p][3][c]));
-#pragma unroll
-    for (int a = 0; a < 2; ++a)
-#pragma unroll
-      for (int p = 0; p < 2; ++p) {
-        uint32_t w[4];
-#pragma unroll
-        for (int hr = 0; hr < 4; ++hr) {
-          const uint32_t v = o.d[p][hr][a], f = hr < 2 ? dl.x : dl.y;
-          w[hr] = __builtin_bit_cast(uint32_t, __builtin_bit_cast(pf16x2_t, v) * __builtin_bit_cast(pf16x2_t, f));
-        }
-        const pf16x8_t D0 = __builtin_bit_cast(pf16x8_t, make_uint4(w[0], w[1], w[2], w[3]));
-        const pf16x8_t D1 =
-            __builtin_bit_cast(pf16x8_t, make_uint4(rot_conj(w[0]), rot_conj(w[1]), rot_conj(w[2]), rot_conj(w[3])));
-#pragma unroll
-        for (int px = 0; px < 2 - p; ++px)  // hi with both parts of x, lo with its hi part
-#pragma unroll
-          for (int c = 0; c < 2; ++c) {
-            acc[a][c][0] = __builtin_amdgcn_mfma_f32_32x32x16_f16(D0, X[px][c], acc[a][c][0], 0, 0, 0);
-            acc[a][c][1] = __builtin_amdgcn_mfma_f32_32x32x16_f16(D1, X[px][c], acc[a][c][1], 0, 0, 0);
-          }
-      }
-    if (bias_wave) {  // the rows themselves, each with its own exponent
-#pragma unroll
-      for (int rr = 0; rr < 2; ++rr) {
-        const int ri = min(r + 2 * g + rr, rows - 1);  // (a row past the end was read as zero)
-        const float sc = __builtin_ldexpf(1.f, -d_exp[r0 + ri]);
-#pragma unroll
-        for (int b = 0; b < 2; ++b)
-#pragma unroll
-          for (int a = 0; a < 2; ++a) {
-            const uint32_t vh = o.d[0][2 * rr + b][a], vl = o.d[1][2 * rr + b][a];
-            const pf16x2_t hi = __builtin_bit_cast(pf16x2_t, vh), lo = __builtin_bit_cast(pf16x2_t, vl);
-#pragma unroll
-            for (int ri2 = 0; ri2 < 2; ++ri2) bs[b][ri2][a] += ((float)hi[ri2] + (float)lo[ri2]) * sc;
-          }
-      }
+    for (int u = 0; u < 4; ++u) {
+      const int r = f * kRows + 2 * wave + (u >> 1);
+      const int src = __builtin_amdgcn_readfirstlane(s_src[min(r, rows - 1)]);
+      split_dma(d_rsrc, st + u * 1024, r < rows ? d_off[u & 1] : kBufferOff, r < rows ? (uint32_t)r * d_out * 32 : 0u);
+      split_dma(a_rsrc, st + kStage + u * 1024, r < rows ? a_off[u & 1] : kBufferOff, r < rows ? (uint32_t)src * d_in * 32 : 0u);
     }
   };
-  // four rows at a time, double buffered in registers; rows past the end read zero
-  const int nblk = (rows + 3) / 4;
-  Ops b0, b1;
-  load_rows(0, b0);
-  for (int b = 0; b < nblk; b += 2) {
-    if (b + 1 < nblk) load_rows((b + 1) * 4, b1);
-    mma_rows(b * 4, b0);
-    if (b + 1 < nblk) {
-      if (b + 2 < nblk) load_rows((b + 2) * 4, b0);
-      mma_rows((b + 1) * 4, b1);
+  // operands of v_mfma_f32_16x16x32_bf16: lane column lane % 16 of a block of 16, rows 2 g and 2 g + 1
+  const int wj = wave & 1, wi = wave >> 1, l16 = lane & 15, g = lane >> 4;
+  const uint32_t swz = ((l16 >> 3) & 1) * 16;  // (b = 0; b = 1 at ^ 16)
+  const uint32_t d_rd = 2 * g * 2048 + (wj * 32 + l16) * 32 + swz, a_rd = kStage + 2 * g * 2048 + (wi * 32 + l16) * 32 + swz;
+
+  pf32x4_t acc[4][4][2];  // [block of 16 j, a][block of 16 i, c][re, im]
+#pragma unroll
+  for (int r = 0; r < 4; ++r)
+#pragma unroll
+    for (int c = 0; c < 4; ++c)
+#pragma unroll
+      for (int q = 0; q < 2; ++q) acc[r][c][q] = pf32x4_t{0.f, 0.f, 0.f, 0.f};
+  __syncthreads();
+  const int n = (rows + kRows - 1) / kRows;
+  issue(0);
+  for (int f = 0; f < n; ++f) {
+    split_wait();  // step f may be read and the other stage, read by step f - 1, overwritten
+    if (f + 1 < n) issue(f + 1);
+    const unsigned char* st = smem + (f & 1) * 2 * kStage;
+    const uint32_t neg = (f & 1) << 31;
+    uint4 D[4][3];  // (re b0, re b1), (im b0, im b1) of two rows
+#pragma unroll
+    for (int jb = 0; jb < 2; ++jb)
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const float4 b0 = *reinterpret_cast<const float4*>(st + d_rd + h * 2048 + jb * 512);
+        const float4 b1 = *reinterpret_cast<const float4*>(st + (d_rd ^ 16) + h * 2048 + jb * 512);
+        split_operand(D[2 * jb], h, b0.x, b1.x, b0.z, b1.z);
+        split_operand(D[2 * jb + 1], h, b0.y, b1.y, b0.w, b1.w);
+      }
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      __builtin_amdgcn_sched_barrier(0);
+      uint4 X[2][3];  // D conj(A): (re, im) for the real part, (-im, re) for the imaginary one
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const uint32_t off = h * 2048 + (c >> 1) * 512;
+        const float4 b0 = *reinterpret_cast<const float4*>(st + a_rd + off);
+        const float4 b1 = *reinterpret_cast<const float4*>(st + (a_rd ^ 16) + off);
+        const float re0 = c & 1 ? b0.y : b0.x, re1 = c & 1 ? b1.y : b1.x, im0 = c & 1 ? b0.w : b0.z, im1 = c & 1 ? b1.w : b1.z;
+        split_operands<0u, 0x80008000u>(X, h, split_flip(re0, neg), split_flip(re1, neg), split_flip(im0, neg),
+                                        split_flip(im1, neg));
+      }
+      split_accumulate(acc, c, D, X, f & 1 ? -1.f : 1.f);
     }
   }
 
-  // lane holds column i0 + l32, rows j0 + 8 (v / 4) + 4 g + v % 4
-  const int i = i0 + l32;
   float* pc = only ? dW + (size_t)e * d_out * d_in * 8 : part + (size_t)chunk * d_out * d_in * 8;
-  if (i < d_in) {
 #pragma unroll
-    for (int v = 0; v < 16; ++v) {
-      const int j = j0 + 8 * (v >> 2) + 4 * g + (v & 3);
-      if (j >= d_out) continue;
-      float o[8];
+  for (int ib = 0; ib < 2; ++ib) {
+    const int i = i0 + wi * 32 + ib * 16 + l16;
+    if (i >= d_in) continue;
 #pragma unroll
-      for (int a = 0; a < 2; ++a)
+    for (int jb = 0; jb < 2; ++jb)
 #pragma unroll
-        for (int c = 0; c < 2; ++c)
+      for (int v = 0; v < 4; ++v) {
+        const int j = j0 + wj * 32 + jb * 16 + 4 * g + v;
+        if (j >= d_out) continue;
+        float o[8];  // [a][c][re, im]
 #pragma unroll
-          for (int q = 0; q < 2; ++q) o[a * 4 + c * 2 + q] = __builtin_ldexpf(acc[a][c][q][v], -Q);
-      float* dst = pc + ((size_t)j * d_in + i) * 8;
-      if (only) {
-        store_dw(dst, o);
-      } else {
-        reinterpret_cast<float4*>(dst)[0] = make_float4(o[0], o[1], o[2], o[3]);
-        reinterpret_cast<float4*>(dst)[1] = make_float4(o[4], o[5], o[6], o[7]);
+        for (int q = 0; q < 8; ++q) o[q] = acc[2 * jb + (q >> 2)][2 * ib + ((q >> 1) & 1)][q & 1][v];
+        float* dst = pc + ((size_t)j * d_in + i) * 8;
+        if (only) {
+          store_dw(dst, o);
+        } else {
+          reinterpret_cast<float4*>(dst)[0] = make_float4(o[0], o[1], o[2], o[3]);
+          reinterpret_cast<float4*>(dst)[1] = make_float4(o[4], o[5], o[6], o[7]);
+        }
       }
-    }
-  }
-  if (bias_wave) {
-    float t[8];  // [b][k][a]
-#pragma unroll
-    for (int q = 0; q < 8; ++q) {
-      t[q] = bs[q >> 2][(q >> 1) & 1][q & 1];
-      t[q] += __shfl_xor(t[q], 32);
-    }
-    if (g == 0 && j0 + l32 < d_out) {
-      if (only) {
-        store_db(db + ((size_t)e * d_out + j0 + l32) * 8, t);
-      } else {
-        float4* q = reinterpret_cast<float4*>(dbpart + ((size_t)chunk * d_out + j0 + l32) * 8);
-        q[0] = make_float4(t[0], t[1], t[2], t[3]);
-        q[1] = make_float4(t[4], t[5], t[6], t[7]);
-      }
-    }
   }
 }
 
@@ -982,62 +817,37 @@ int weight_grad_pauli(const float* dy_pauli, const float* a_pauli, const int32_t
   return check_launch("weight gradient (reduction)");
 }
 
-bool weight_grad_split_fits(int a_rows, bool gathered, int d_in, int d_out) {
+// Where the sizes fit the kernel's 32-bit offsets, and from some 320 workgroups on: a chunk of 384 rows
+// is a chain of 48 steps of 2.9 us, and fewer chunks leave CUs idle that the fp32 MFMA kernels use
+// (training steps, us, split / fp32 MFMA weight gradients, by workgroups: d = F = 128, E = 4: 56 592 / 435, 104 738 /
+// 671; d = 64, F = 256, E = 8: 120 752 / 686, 204 1069 / 1147; d = 100, F = 300, E = 12: 230 724 / 653, 340 1121 / 1151;
+// d = 64, F = 256, E = 32: 216 689 / 632, 300 1161 / 1144; d = 128, F = 512, E = 32: 608 720 / 782, 1872 4836 / 5864;
+// d = 256, F = 512, E = 16: 608 743 / 849).
+bool weight_grad_split_pays(long long P, int E, long long a_rows, bool gathered, int d_in, int d_out) {
   const uint64_t lim = (uint64_t)1 << 31;
-  return (uint64_t)kWgmChunk * pauli_split_row_bytes(d_out) < lim && (uint64_t)kWgmChunk * pauli_split_row_bytes(d_in) < lim &&
-         (!gathered || (uint64_t)a_rows * pauli_split_row_bytes(d_in) < lim);
+  const long long chunks = (P + kWgmChunk - 1) / kWgmChunk + E;
+  return chunks * ((d_out + kWgmTile - 1) / kWgmTile) * ((d_in + kWgmTile - 1) / kWgmTile) >= 320 &&
+         (uint64_t)kWgmChunk * std::max(d_in, d_out) * 32 < lim && (!gathered || (uint64_t)a_rows * d_in * 32 < lim);
 }
 
-int weight_grad_split(const void* dy, const int32_t* dy_exp, const void* a, int a_rows, const int32_t* a_exp,
-                      const int32_t* gather, const int32_t* offsets, int P_max, int E, int d_in, int d_out, float* dW,
-                      float* db, void* workspace, hipStream_t stream) {
+int weight_grad_split(const float* dy_pauli, const float* a_pauli, int a_rows, const int32_t* gather,
+                      const int32_t* offsets, int P_max, int E, int d_in, int d_out, float* dW, float* db, void* workspace,
+                      hipStream_t stream) {
   if (E == 0) return 0;
   const size_t chunks = (size_t)(P_max + kWgmChunk - 1) / kWgmChunk + E;
   float* part = static_cast<float*>(workspace);
   float* dbpart = db ? part + chunks * d_out * d_in * 8 : nullptr;
   const int n_xcd = 8;  // workgroups go to the XCDs round robin (8 on MI355X)
-  const size_t tiles = (size_t)((d_out + kWgmTile - 1) / kWgmTile) * ((d_in + kWgmTile - 1) / kWgmTile);
+  const size_t nj = (d_out + kWgmTile - 1) / kWgmTile, ni = (d_in + kWgmTile - 1) / kWgmTile, nt = nj * ni + (db ? nj : 0);
   if (P_max > 0) {
-    hipLaunchKernelGGL(weight_grad_split_kernel, dim3((unsigned)((chunks + n_xcd - 1) / n_xcd * n_xcd * tiles)),
-                       dim3(256), 0, stream, static_cast<const unsigned char*>(dy), dy_exp,
-                       static_cast<const unsigned char*>(a),
-                       gather ? (uint32_t)((size_t)a_rows * pauli_split_row_bytes(d_in)) : 0u, a_exp, gather, offsets, E,
+    hipLaunchKernelGGL(weight_grad_split_kernel, dim3((unsigned)((chunks + n_xcd - 1) / n_xcd * n_xcd * nt)), dim3(256), 0,
+                       stream, dy_pauli, a_pauli, gather ? (uint32_t)((size_t)a_rows * d_in * 32) : 0u, gather, offsets, E,
                        d_in, d_out, (int)chunks, n_xcd, part, dbpart, dW, db);
     if (check_launch("weight gradient (split)")) return -1;
   }
   hipLaunchKernelGGL(weight_grad_reduce_kernel, dim3((unsigned)(((size_t)d_out * d_in + 255) / 256), E), dim3(256), 0,
                      stream, part, dbpart, offsets, E, d_in, d_out, dW, db);
   return check_launch("weight gradient (reduction)");
-}
-
-namespace {
-template <int ACT, bool BWD>
-void launch_act_split(const float* h, const float* g, unsigned P, int d, unsigned char* out, int32_t* row_exp,
-                      hipStream_t st) {
-  const dim3 grid(P), blk(256);
-  if (d <= 256) hipLaunchKernelGGL((act_split_kernel<ACT, BWD, 1>), grid, blk, 0, st, h, g, d, out, row_exp);
-  else if (d <= 512) hipLaunchKernelGGL((act_split_kernel<ACT, BWD, 2>), grid, blk, 0, st, h, g, d, out, row_exp);
-  else if (d <= 1024) hipLaunchKernelGGL((act_split_kernel<ACT, BWD, 4>), grid, blk, 0, st, h, g, d, out, row_exp);
-  else hipLaunchKernelGGL((act_split_kernel<ACT, BWD, 0>), grid, blk, 0, st, h, g, d, out, row_exp);
-}
-}  // namespace
-
-int activation_split_rows(const float* h, const float* g, size_t P, int d, int act, void* out, int32_t* row_exp,
-                          hipStream_t stream) {
-  if (P == 0) return 0;
-  unsigned char* o = static_cast<unsigned char*>(out);
-#define YGG_AS(A)                                                                     \
-  if (g) launch_act_split<A, true>(h, g, (unsigned)P, d, o, row_exp, stream);        \
-  else launch_act_split<A, false>(h, nullptr, (unsigned)P, d, o, row_exp, stream);   \
-  break
-  switch (act) {
-    case kActNone: YGG_AS(kActNone);
-    case kActGelu: YGG_AS(kActGelu);
-    case kActRelu: YGG_AS(kActRelu);
-    default: YGG_AS(kActSigmoid);
-  }
-#undef YGG_AS
-  return check_launch("activation (split rows)");
 }
 
 int activation_backward(const float* h, const float* g, size_t n_mv, int act, float* out, float* out_pauli,
@@ -1082,11 +892,10 @@ int fill_zero_f32(float* p, size_t n, hipStream_t stream) {
 }
 
 int combine_backward(const float* dout, const float* y_sorted, int N, int k, int d, const float* topk_w,
-                     const int32_t* slot_pos, float* dy_sorted, float* dy_pauli, float* dtopk_w, hipStream_t stream,
-                     void* dy_split, int32_t* dy_exp) {
+                     const int32_t* slot_pos, float* dy_sorted, float* dy_pauli, float* dtopk_w, hipStream_t stream) {
   if (N == 0) return 0;
   hipLaunchKernelGGL(combine_backward_kernel, dim3((N + 3) / 4), dim3(256), 0, stream, dout, y_sorted, N, k, d, topk_w,
-                     slot_pos, dy_sorted, dy_pauli, dtopk_w, static_cast<unsigned char*>(dy_split), dy_exp);
+                     slot_pos, dy_sorted, dy_pauli, dtopk_w);
   return check_launch("combine backward");
 }
 

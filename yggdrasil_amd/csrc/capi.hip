@@ -81,45 +81,29 @@ static size_t ys_bytes(size_t P, int E, int d, int F, int dtype, int w_format) {
   return P * d * 8 * es;
 }
 
-// Whether a layer's two fp32 Pauli products run as split products (fp32 operands as two
-// fp16 parts), and the regions of its workspace that this enlarges or adds.
+// Whether a layer's two fp32 Pauli products (and their adjoints) run on the bf16 MFMA units
 static bool f32_split(int N, int d, int F, int E, int k, int w_format) {
   const long long P = (long long)N * k;
-  return w_format == kWPauliF32 && N > 0 && P <= 0x7fffffffLL && ygg::pauli_split_pays(P, E, d, F) &&
-         ygg::pauli_split_pays(P, E, F, d) && ygg::pauli_split_fits(E, (int)P, N, true, d, F, false) &&
-         ygg::pauli_split_fits(E, (int)P, (int)P, false, F, d, false);
-}
-struct SplitSizes {
-  size_t x, h, w, col_exp, norms;
-};
-static SplitSizes split_sizes(size_t N, size_t P, int d, int F, int E) {
-  SplitSizes z;
-  z.x = N * pauli_split_row_bytes(d);
-  z.h = P * pauli_split_row_bytes(F);
-  z.w = std::max((size_t)F * pauli_split_row_bytes(d), (size_t)d * pauli_split_row_bytes(F)) * E;  // both products, in turn
-  z.col_exp = (size_t)E * std::max(d, F) * 4;
-  z.norms = (size_t)E * 2 * pauli_split_norm_blocks(F) * 4;
-  return z;
+  return w_format == kWPauliF32 && N > 0 && P <= 0x7fffffffLL && ygg::pauli_split_layer_pays(P, E, d, F) &&
+         ygg::pauli_split_fits(E, N, true, d, F) && ygg::pauli_split_fits(E, P, false, F, d);
 }
 
-static size_t moe_workspace(int N, int d, int F, int E, int k, int dtype, int w_format, bool allow_split) {
+YGG_API int ygg_f32_layer_split(int N, int d, int F, int E, int k) {
+  return d >= 1 && F >= 1 && E >= 1 && k >= 1 && f32_split(N, d, F, E, k, kWPauliF32);
+}
+
+YGG_API size_t ygg_moe_workspace_bytes(int N, int d, int F, int E, int k, int dtype, int w_format) {
   const size_t P = (size_t)N * k;
   const size_t es = (dtype == kF32) ? 4 : 2;
   size_t b = 0;
-  const bool split = allow_split && f32_split(N, d, F, E, k, w_format);
-  const SplitSizes z = split_sizes(N, P, d, F, E);
   b += align256((size_t)N * E * 4);       // logits
   b += align256(P * 4) * 2;               // perm, slot_pos
   b += align256(ygg_route_workspace_bytes(N, E, k));
-  b += align256(std::max(P * d * 8 * es, split ? z.x : 0));  // x_sorted (Pauli half-rows of x for format 3, split rows)
-  b += align256(std::max(P * F * 8 * es, split ? z.h : 0));  // h
+  b += align256(P * d * 8 * es);          // x_sorted (Pauli rows of x for formats 3 and 4)
+  b += align256(P * F * 8 * es);          // h
   b += align256(ys_bytes(P, E, d, F, dtype, w_format));  // y_sorted
   if (w_format == kWPauliF32) b += align256(P * 4);       // row_slot: each row's slot, for the partial planes
-  if (split) b += align256(z.w) + align256(z.col_exp) + align256(z.norms) + 2 * align256(P * 4);  // row and h exponents
   return b;
-}
-YGG_API size_t ygg_moe_workspace_bytes(int N, int d, int F, int E, int k, int dtype, int w_format) {
-  return moe_workspace(N, d, F, E, k, dtype, w_format, true);
 }
 
 // Sizes the layer's kernels cannot address, refused before the first launch: more
@@ -147,7 +131,7 @@ static int moe_forward_impl(const void* x, int dtype, int N, int d, int F, int E
                             const float* b_down, int w_format, const void* residual, void* out, int32_t* topk_idx,
                             float* topk_w, int32_t* counts, int32_t* offsets, void* workspace,
                             size_t workspace_bytes, hipStream_t stream,
-                            float* h_pre_out, bool allow_split = true) {
+                            float* h_pre_out) {
   // every path checks the sizes here, also those that route inside a product
   YGG_CHECK_ARG(N >= 0 && d >= 1 && F >= 1, "ygg_moe_forward: bad sizes N=%d d=%d F=%d", N, d, F);
   YGG_CHECK_ARG(E >= 1 && E <= kMaxExperts, "ygg_moe_forward: E=%d out of range [1, %d]", E, kMaxExperts);
@@ -170,9 +154,9 @@ static int moe_forward_impl(const void* x, int dtype, int N, int d, int F, int E
   YGG_CHECK_ARG(w_format != kWPauli || (d % 2 == 0 && F % 2 == 0),
                 "ygg_moe_forward: the Pauli weight format needs even d and F (d=%d F=%d)", d, F);
   if (layer_size_check("ygg_moe_forward", N, d, F, E, k, w_format)) return -1;
-  const size_t ws_need = moe_workspace(N, d, F, E, k, dtype, w_format, allow_split);
-  YGG_CHECK_ARG(workspace_bytes >= ws_need, "ygg_moe_forward: workspace of %zu bytes, need %zu", workspace_bytes,
-                ws_need);
+  YGG_CHECK_ARG(workspace_bytes >= ygg_moe_workspace_bytes(N, d, F, E, k, dtype, w_format),
+                "ygg_moe_forward: workspace of %zu bytes, need %zu", workspace_bytes,
+                ygg_moe_workspace_bytes(N, d, F, E, k, dtype, w_format));
   YGG_CHECK_ARG(N == 0 || logits || (router_w && router_b), "ygg_moe_forward: need logits or router parameters");
   if (N == 0)  // no tokens: every expert's count and offset is zero, as ygg_route writes them
     return (counts && offsets) ? ygg_route(nullptr, 0, E, k, nullptr, nullptr, counts, offsets, nullptr, nullptr,
@@ -190,12 +174,10 @@ static int moe_forward_impl(const void* x, int dtype, int N, int d, int F, int E
   void* rws = p;
   const size_t rws_bytes = align256(ygg_route_workspace_bytes(N, E, k));
   p += rws_bytes;
-  const bool split = allow_split && f32_split(N, d, F, E, k, w_format);
-  const SplitSizes z = split_sizes(N, P, d, F, E);
   void* xs = p;
-  p += align256(std::max(P * d * 8 * es, split ? z.x : 0));
+  p += align256(P * d * 8 * es);
   void* h = p;
-  p += align256(std::max(P * F * 8 * es, split ? z.h : 0));
+  p += align256(P * F * 8 * es);
   void* ys = p;
 
   if (w_format == kWPauliI8) {
@@ -229,13 +211,14 @@ static int moe_forward_impl(const void* x, int dtype, int N, int d, int F, int E
                           slot_pos, residual, out, dtype, stream);
   }
   // fp32 Pauli weights, logits given, a batch of at most 256 tokens of at most 64
-  // multivectors: the up product routes the batch itself and reads x's blade rows, so
-  // no routing launch runs
-  const bool f32_routed_up = w_format == kWPauliF32 && logits && pauli_f32_route_fusable(N, E, k, d);
+  // multivectors: the fp32 MFMA up product routes the batch itself and reads x's blade
+  // rows, so no routing launch runs (the split products need one)
+  const bool split = f32_split(N, d, F, E, k, w_format);
+  const bool f32_routed_up = w_format == kWPauliF32 && !split && logits && pauli_f32_route_fusable(N, E, k, d);
   // the Pauli formats' conversion of x to Pauli rows (into the x_sorted region: N <= P
   // rows) runs as extra workgroups of the routing's first launch
   ygg::RowConvert cv;
-  if ((w_format == kWPauli || w_format == kWPauliF32) && !f32_routed_up && !split) {
+  if ((w_format == kWPauli || w_format == kWPauliF32) && !f32_routed_up) {
     cv.x = x;
     cv.out = xs;
     cv.n = (long long)N * d;
@@ -246,7 +229,7 @@ static int moe_forward_impl(const void* x, int dtype, int N, int d, int F, int E
   // partial planes at slot rows t k + s (the combine's plane loads then need no
   // routing array)
   int32_t* row_slot = nullptr;
-  if (w_format == kWPauliF32 && !split) {
+  if (w_format == kWPauliF32) {
     row_slot = reinterpret_cast<int32_t*>(static_cast<char*>(ys) + align256(ys_bytes(P, E, d, F, dtype, w_format)));
     cv.row_slot = row_slot;
   }
@@ -260,34 +243,11 @@ static int moe_forward_impl(const void* x, int dtype, int N, int d, int F, int E
                                 cv, stream)) {
     return -1;
   }
-  if (split) {
-    // fp32 Pauli, enough rows: both operands of each product as two fp16 parts.  The up
-    // product gathers x's split rows and writes h as split rows, whose exponents come
-    // from a bound taken with x's; the weights are split into one region in turn.
-    char* q = static_cast<char*>(ys) + align256(ys_bytes(P, E, d, F, dtype, w_format)) + align256(P * 4);
-    auto take = [&](size_t bytes) {
-      char* r = q;
-      q += align256(bytes);
-      return r;
-    };
-    void* ws = take(z.w);
-    int32_t* col_exp = reinterpret_cast<int32_t*>(take(z.col_exp));
-    float* norms = reinterpret_cast<float*>(take(z.norms));
-    int32_t* row_exp = reinterpret_cast<int32_t*>(take(P * 4));
-    ygg::SplitHidden hid;
-    hid.k = k;
-    hid.d_ff = F;
-    hid.act = act;
-    hid.slot_pos = slot_pos;
-    hid.topk_idx = topk_idx;
-    hid.norms = norms;
-    hid.h_exp = reinterpret_cast<int32_t*>(take(P * 4));
-    if (pauli_split_weights(static_cast<const float*>(w_up), E, F, d, b_up, ws, col_exp, norms, stream) ||
-        pauli_split_rows(static_cast<const float*>(x), N, d, xs, row_exp, hid, stream) ||
-        pauli_split_up(xs, N, row_exp, perm, (int)P, ws, col_exp, b_up, offsets, E, d, F, act, h, hid.h_exp, h_pre_out,
-                       stream) ||
-        pauli_split_weights(static_cast<const float*>(w_down), E, d, F, nullptr, ws, col_exp, nullptr, stream) ||
-        pauli_split_linear(h, hid.h_exp, (int)P, ws, col_exp, b_down, offsets, E, F, d, static_cast<float*>(ys), stream))
+  if (split) {  // fp32 Pauli, enough rows
+    if (pauli_split_linear(static_cast<const float*>(xs), N, perm, (int)P, static_cast<const float*>(w_up), b_up, offsets, E,
+                           d, F, act, static_cast<float*>(h), /*Pauli rows*/ 0, h_pre_out, stream) ||
+        pauli_split_linear(static_cast<const float*>(h), (int)P, nullptr, (int)P, static_cast<const float*>(w_down), b_down,
+                           offsets, E, F, d, kActNone, static_cast<float*>(ys), /*blade*/ 1, nullptr, stream))
       return -1;
     return ygg_combine(ys, kF32, /*y_mask=*/0, N, k, d, topk_idx, topk_w, slot_pos, residual, out, dtype, stream);
   }
@@ -431,10 +391,7 @@ YGG_API int ygg_moe_forward_noalloc(const void* x, int dtype, int N, int d, int 
                                     hipStream_t stream) {
   YGG_CHECK_ARG(N >= 0 && d >= 1 && F >= 1 && k >= 1, "ygg_moe_forward_noalloc: bad sizes N=%d d=%d F=%d k=%d", N, d,
                 F, k);
-  // the split fp32 products, which need a larger workspace, only where it fits the scratch, so
-  // that they refuse no call
-  const bool allow = moe_workspace(N, d, F, E, k, dtype, w_format, true) <= kNoAllocScratchBytes;
-  const size_t need = moe_workspace(N, d, F, E, k, dtype, w_format, allow);
+  const size_t need = ygg_moe_workspace_bytes(N, d, F, E, k, dtype, w_format);
   YGG_CHECK_ARG(need <= kNoAllocScratchBytes,
                 "ygg_moe_forward_noalloc: this layer call needs %zu bytes of scratch, more than the %zu the library "
                 "holds per device; use ygg_moe_forward with a workspace",
@@ -443,7 +400,7 @@ YGG_API int ygg_moe_forward_noalloc(const void* x, int dtype, int N, int d, int 
   if (N > 0 && device_scratch(stream, &ws)) return -1;
   return moe_forward_impl(x, dtype, N, d, F, E, k, act, logits, router_w, router_b, w_up, s_up, b_up, w_down, s_down,
                           b_down, w_format, residual, out, topk_idx, topk_w, counts, offsets, ws,
-                          kNoAllocScratchBytes, stream, nullptr, allow);
+                          kNoAllocScratchBytes, stream, nullptr);
 }
 
 // The forward of a training step (fp32 Pauli weights): ygg_moe_forward, and the
@@ -501,29 +458,20 @@ static int bw_regions(int N, int d, int F, int E, int k, size_t* r) {
   r[n++] = P * 4;              // slot_pos
   r[n++] = (size_t)N * E * 4;  // logits scratch
   r[n++] = ygg_route_workspace_bytes(N, E, k);
-  const bool split = f32_split(N, d, F, E, k, kWPauliF32);  // (split rows are padded to blocks of 8 multivectors)
-  const size_t row_d = split ? pauli_split_row_bytes(d) : (size_t)d * 32;
-  const size_t row_f = split ? pauli_split_row_bytes(F) : (size_t)F * 32;
-  r[n++] = N * row_d;  // x in Pauli rows
-  for (int q = 0; q < 4; ++q) r[n++] = P * row_f;  // h_pre, h, Pauli rows of h / dh_pre, dh / dh_pre
-  for (int q = 0; q < 3; ++q) r[n++] = P * row_d;  // y / dx rows, dy, Pauli rows of dy
+  r[n++] = (size_t)N * d * 32;  // x in Pauli rows
+  for (int q = 0; q < 4; ++q) r[n++] = P * F * 32;  // h_pre, h, Pauli rows of h / dh_pre, dh / dh_pre
+  for (int q = 0; q < 3; ++q) r[n++] = P * d * 32;  // y / dx rows, dy, Pauli rows of dy
   // weight-gradient partial sums, reused by both products: the up product's
   // (d_in = d, d_out = F) and the down product's (d_in = F, d_out = d, whose
   // bias planes are d-wide), so the larger of the two
   const size_t wg_up = weight_grad_pauli_workspace_bytes((int)P, E, d, F);
   const size_t wg_down = weight_grad_pauli_workspace_bytes((int)P, E, F, d);
   r[n++] = wg_up > wg_down ? wg_up : wg_down;
-  if (split) {
-    const SplitSizes z = split_sizes(N, P, d, F, E);
-    r[n++] = z.w;        // split weights of one product at a time
-    r[n++] = z.col_exp;
-    for (int q = 0; q < 4; ++q) r[n++] = P * 4;  // exponents of the rows of x (N), h, dy, dh_pre
-  }
   return n;
 }
 
 YGG_API size_t ygg_moe_backward_workspace_bytes(int N, int d, int F, int E, int k) {
-  size_t r[32], b = 0;
+  size_t r[24], b = 0;
   const int n = bw_regions(N, d, F, E, k, r);
   for (int q = 0; q < n; ++q) b += align256(r[q]);
   return b;
@@ -551,7 +499,7 @@ YGG_API int ygg_moe_backward(const float* x, int N, int d, int F, int E, int k, 
   }
   YGG_CHECK_ARG(x && dout && dx, "ygg_moe_backward: null x, dout or dx");
   const size_t P = (size_t)N * k;
-  size_t sz[32];
+  size_t sz[24];
   bw_regions(N, d, F, E, k, sz);
   char* base = static_cast<char*>(workspace);
   int next = 0;
@@ -579,20 +527,13 @@ YGG_API int ygg_moe_backward(const float* x, int N, int d, int F, int E, int k, 
   float* dp = static_cast<float*>(take());  // Pauli rows of dy
   void* wg = take();                        // weight-gradient partial sums
 
-  // forward recompute: h_pre (unless the forward kept it), h (Pauli rows), y (blade, for dtopk_w)
-  const float* hp_in = h_pre_saved;
-  // split products and weight gradients, where the forward's products were split
-  const bool split = hp_in && f32_split(N, d, F, E, k, kWPauliF32) && weight_grad_split_fits(N, true, d, F) &&
-                     weight_grad_split_fits((int)P, false, F, d);
   // x's Pauli rows are converted by extra workgroups of the routing launch
   ygg::RowConvert cv;
-  if (!split) {
-    cv.x = x;
-    cv.out = xp;
-    cv.n = (long long)N * d;
-    cv.d = d;
-    cv.kind = ygg::kConvF32Pauli;
-  }
+  cv.x = x;
+  cv.out = xp;
+  cv.n = (long long)N * d;
+  cv.d = d;
+  cv.kind = ygg::kConvF32Pauli;
   if (logits) {
     if (ygg::route_convert(logits, N, E, k, idx, tw, counts, offsets, perm, slot_pos, rws, rws_bytes, cv, stream))
       return -1;
@@ -600,53 +541,39 @@ YGG_API int ygg_moe_backward(const float* x, int N, int d, int F, int E, int k, 
                                        slot_pos, lg, rws, rws_bytes, cv, stream)) {
     return -1;
   }
-  if (split) {
-    void* ws = take();
-    int32_t* col_exp = static_cast<int32_t*>(take());
-    int32_t* x_exp = static_cast<int32_t*>(take());
-    int32_t* h_exp = static_cast<int32_t*>(take());
-    int32_t* dy_exp = static_cast<int32_t*>(take());
-    int32_t* dh_exp = static_cast<int32_t*>(take());
-    // split rows of x, h (from h before the activation) and, by the combine's backward, dy
-    if (pauli_split_rows(x, N, d, xp, x_exp, ygg::SplitHidden{}, stream) ||
-        activation_split_rows(hp_in, nullptr, P, F, act, h, h_exp, stream))
-      return -1;
-    if (dtopk_w && (pauli_split_weights(w_down, E, d, F, nullptr, ws, col_exp, nullptr, stream) ||
-                    pauli_split_linear(h, h_exp, (int)P, ws, col_exp, b_down, offsets, E, F, d, y, stream)))
-      return -1;
-    if (combine_backward(dout, dtopk_w ? y : nullptr, N, k, d, tw, slot_pos, nullptr, nullptr, dtopk_w, stream, dp,
-                         dy_exp) ||
-        pauli_split_weights(w_down_adj, E, F, d, nullptr, ws, col_exp, nullptr, stream) ||
-        pauli_split_linear(dp, dy_exp, (int)P, ws, col_exp, nullptr, offsets, E, d, F, dh, stream) ||
-        weight_grad_split(dp, dy_exp, h, (int)P, h_exp, nullptr, offsets, (int)P, E, F, d, dw_down, db_down, wg, stream) ||
-        activation_split_rows(hp_in, dh, P, F, act, fp, dh_exp, stream) ||
-        pauli_split_weights(w_up_adj, E, d, F, nullptr, ws, col_exp, nullptr, stream) ||
-        pauli_split_linear(fp, dh_exp, (int)P, ws, col_exp, nullptr, offsets, E, F, d, y, stream) ||
-        weight_grad_split(fp, dh_exp, xp, N, x_exp, perm, offsets, (int)P, E, d, F, dw_up, db_up, wg, stream))
-      return -1;
-    return dispatch_backward(y, N, k, d, slot_pos, residual ? dout : nullptr, dx, stream);
-  }
+  // the products run on the units that the forward's ran on
+  const bool split = f32_split(N, d, F, E, k, kWPauliF32);
+  auto product = [&](const float* in, const int32_t* gather, const float* w, const float* b, int d_in, int d_out,
+                     float* out) {
+    if (split)
+      return pauli_split_linear(in, gather ? N : (int)P, gather, (int)P, w, b, offsets, E, d_in, d_out, kActNone, out,
+                                /*blade*/ 1, nullptr, stream);
+    return ygg_pauli_grouped_linear_f32(in, gather, (int)P, w, b, offsets, E, d_in, d_out, kActNone, out, 1, stream);
+  };
+  const bool split_wg = split && weight_grad_split_pays(P, E, N, true, d, F) &&
+                        weight_grad_split_pays(P, E, P, false, F, d);
+  auto weight_grad = [&](const float* dr, const float* a, const int32_t* gather, int d_in, int d_out, float* dw, float* db) {
+    if (split_wg)
+      return weight_grad_split(dr, a, gather ? N : (int)P, gather, offsets, (int)P, E, d_in, d_out, dw, db, wg, stream);
+    return weight_grad_pauli(dr, a, gather, offsets, (int)P, E, d_in, d_out, dw, db, wg, stream);
+  };
+  // forward recompute: h_pre (unless the forward kept it), h (Pauli rows), y (blade, for dtopk_w)
+  const float* hp_in = h_pre_saved;
   if (!hp_in) {
-    if (ygg_pauli_grouped_linear_f32(xp, perm, (int)P, w_up, b_up, offsets, E, d, F, kActNone, h_pre, 1, stream))
-      return -1;
+    if (product(xp, perm, w_up, b_up, d, F, h_pre)) return -1;
     hp_in = h_pre;
   }
   // h as Pauli rows for the down product and its weight gradient
   if (activation_forward(hp_in, P * F, act, nullptr, fp, stream)) return -1;
-  if (dtopk_w &&
-      ygg_pauli_grouped_linear_f32(fp, nullptr, (int)P, w_down, b_down, offsets, E, F, d, kActNone, y, 1, stream))
-    return -1;
+  if (dtopk_w && product(fp, nullptr, w_down, b_down, F, d, y)) return -1;
   // combine backward -> dy; down backward -> dh, dW_down, db_down
-  if (combine_backward(dout, dtopk_w ? y : nullptr, N, k, d, tw, slot_pos, nullptr, dp, dtopk_w, stream))
-    return -1;
-  if (ygg_pauli_grouped_linear_f32(dp, nullptr, (int)P, w_down_adj, nullptr, offsets, E, d, F, kActNone, dh, 1, stream))
-    return -1;
-  if (weight_grad_pauli(dp, fp, nullptr, offsets, (int)P, E, F, d, dw_down, db_down, wg, stream)) return -1;
+  if (combine_backward(dout, dtopk_w ? y : nullptr, N, k, d, tw, slot_pos, nullptr, dp, dtopk_w, stream)) return -1;
+  if (product(dp, nullptr, w_down_adj, nullptr, d, F, dh)) return -1;
+  if (weight_grad(dp, fp, nullptr, F, d, dw_down, db_down)) return -1;
   // activation backward -> Pauli rows of dh before the activation; up backward -> dx rows, dW_up, db_up
   if (activation_backward(hp_in, dh, P * F, act, nullptr, fp, stream)) return -1;
-  if (ygg_pauli_grouped_linear_f32(fp, nullptr, (int)P, w_up_adj, nullptr, offsets, E, F, d, kActNone, y, 1, stream))
-    return -1;
-  if (weight_grad_pauli(fp, xp, perm, offsets, (int)P, E, d, F, dw_up, db_up, wg, stream)) return -1;
+  if (product(fp, nullptr, w_up_adj, nullptr, F, d, y)) return -1;
+  if (weight_grad(fp, xp, perm, d, F, dw_up, db_up)) return -1;
   // dispatch backward: each token's rows summed, plus dout when the forward added x
   return dispatch_backward(y, N, k, d, slot_pos, residual ? dout : nullptr, dx, stream);
 }

@@ -15,7 +15,6 @@
 namespace ygg {
 
 typedef __bf16 pbf16x8_t __attribute__((ext_vector_type(8)));
-typedef _Float16 pf16x8_t __attribute__((ext_vector_type(8)));
 typedef __bf16 pbf16x2_t __attribute__((ext_vector_type(2)));
 typedef float pf32x2_t __attribute__((ext_vector_type(2)));
 typedef float pf32x4_t __attribute__((ext_vector_type(4)));
@@ -116,66 +115,24 @@ __device__ inline void store_pauli_f32(float* dst, const float* x) {
   q[1] = make_float4(c1[0], c1[2], c1[1], c1[3]);
 }
 
-// ---- fp32 values as two fp16 parts (the split products of pauli_gemm.hip) ----------
-typedef _Float16 pf16x2_t __attribute__((ext_vector_type(2)));
-typedef _Float16 pf16x4_t __attribute__((ext_vector_type(4)));
-// the scale exponent of values whose largest magnitude is m: it brings them below 2^15
-// (m not finite: unscaled; m zero: as if they were small, so that a row of zeros does
-// not set the common scale of the rows summed with it)
-constexpr int kSplitExpZero = 100;
-__device__ __forceinline__ int split_exp(float m) {
-  if (m == 0.f) return kSplitExpZero;
-  if (!(m < INFINITY)) return 0;
-  return 15 - __builtin_amdgcn_frexp_expf(m);
-}
-// magnitudes compared as integers, which orders a NaN above every number
-__device__ __forceinline__ uint32_t mag_bits(float v) { return __builtin_bit_cast(uint32_t, v) & 0x7fffffffu; }
-__device__ __forceinline__ uint32_t wave_max_u32(uint32_t v) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v = max(v, (uint32_t)__shfl_xor((int)v, o));
-  return v;
-}
-// the largest magnitude of a multivector's Pauli entries (as bits)
-__device__ __forceinline__ uint32_t pauli_mag(const float* x) {
-  float c0[4], c1[4];
-  uint32_t m = 0;
-  blade_to_pauli(x, c0, c1);
-#pragma unroll
-  for (int c = 0; c < 4; ++c) m = max(m, max(mag_bits(c0[c]), mag_bits(c1[c])));
-  return m;
-}
-// four values scaled by 2^s -> their hi and lo parts, 8 bytes each, rounded to nearest
-__device__ __forceinline__ void split4_f16(const float* v, int s, uint2& hi, uint2& lo) {
-  pf16x4_t h, l;
-#pragma unroll
-  for (int q = 0; q < 4; ++q) {
-    const float x = __builtin_ldexpf(v[q], s);
-    h[q] = (_Float16)x;
-    l[q] = (_Float16)(x - (float)h[q]);
-  }
-  hi = __builtin_bit_cast(uint2, h);
-  lo = __builtin_bit_cast(uint2, l);
-}
-
-// multivector i of a split row (`row` its start, d_pad multivectors per half-row)
-__device__ __forceinline__ void store_split_mv(unsigned char* row, int d_pad, int i, const float* x, int s) {
-  float c0[4], c1[4];
-  blade_to_pauli(x, c0, c1);
-  uint2 h0, l0, h1, l1;
-  split4_f16(c0, s, h0, l0);
-  split4_f16(c1, s, h1, l1);
-  unsigned char* p = row + (size_t)(i >> 3) * 128 + (i & 7) * 8;
-  *reinterpret_cast<uint2*>(p) = h0;
-  *reinterpret_cast<uint2*>(p + 64) = l0;
-  *reinterpret_cast<uint2*>(p + (size_t)d_pad * 16) = h1;
-  *reinterpret_cast<uint2*>(p + (size_t)d_pad * 16 + 64) = l1;
-}
-
 // two floats -> packed bf16 pair (v_cvt_pk_bf16_f32, round to nearest even)
 __device__ inline uint32_t pack2_bf16(float lo, float hi) {
   const pf32x2_t f = {lo, hi};
   return __builtin_bit_cast(uint32_t, __builtin_convertvector(f, pbf16x2_t));
 }
+
+// ---- fp32 values as three bf16 parts (the split products) ----------------------------
+// hi is v's upper 16 bits, mid the rest rounded to bf16, lo what is left: 8 bits each, so
+// their sum is v itself (above 2^-110: below, lo runs out of exponents).  bf16 has fp32's
+// range, so no part needs a scale.
+__device__ __forceinline__ void split_pair(float x, float y, uint32_t& hi, uint32_t& mid, uint32_t& lo) {
+  const uint32_t ux = __builtin_bit_cast(uint32_t, x), uy = __builtin_bit_cast(uint32_t, y);
+  hi = __builtin_amdgcn_perm(uy, ux, 0x07060302u);  // packed (x, y)
+  const float mx = x - __builtin_bit_cast(float, ux & 0xffff0000u), my = y - __builtin_bit_cast(float, uy & 0xffff0000u);
+  mid = pack2_bf16(mx, my);
+  lo = pack2_bf16(mx - __builtin_bit_cast(float, mid << 16), my - __builtin_bit_cast(float, mid & 0xffff0000u));
+}
+
 __device__ inline float bf_lo(uint32_t w) { return __builtin_bit_cast(float, w << 16); }
 __device__ inline float bf_hi(uint32_t w) { return __builtin_bit_cast(float, w & 0xffff0000u); }
 

@@ -36,7 +36,7 @@
 
 #include <algorithm>
 
-#include "pauli_common.h"
+#include "pauli_f32.h"
 #include "route_select.h"
 
 namespace ygg {
@@ -52,7 +52,6 @@ constexpr long long kF32TwoBlockMinGroups = 2048;  // 32-token tiles from this m
 // output layouts: Pauli rows (for the next product), blade rows (row, d_out), fp32
 // partial planes, and blade columns (d_out, rows) -- the transposed product geom_matmul
 // returns
-enum PauliF32Out : int { kF32OutPauliRows = 0, kF32OutBlade = 1, kF32OutPartial = 2, kF32OutBladeT = 3 };
 
 template <int TOK>  // tokens per tile
 __device__ inline bool f32_find_tile(const int32_t* __restrict__ offsets, int E, int tile, int& e, int& row0,
@@ -146,43 +145,6 @@ __device__ inline void f32_kloop(f32x16v_t (&acc)[WR][2][2], const float* const 
     Ops o;
     load_op(i, o);
     mma(o);
-  }
-}
-
-// One output multivector (token row, column j) from its Pauli sums Y[a][b] = (re, im):
-// blade map, bias (split 0 only for partial planes), the pre-activation rows when
-// Ypre is set, activation, and the store in the OUT layout.
-template <int ACT, int OUT>
-__device__ inline void f32_store_mv(float y00r, float y00i, float y01r, float y01i, float y10r, float y10i, float y11r,
-                                    float y11i, const float* __restrict__ bias, int e, int row, int j, int d_out,
-                                    int split, int P_max, float* __restrict__ Y, float* __restrict__ Ypre,
-                                    const int32_t* __restrict__ row_map) {
-  float y[8];
-  pauli_to_blade(y00r, y00i, y01r, y01i, y10r, y10i, y11r, y11i, y);
-  if (bias != nullptr && (OUT != kF32OutPartial || split == 0)) {
-#pragma unroll
-    for (int c = 0; c < 8; ++c) y[c] += bias[((size_t)e * d_out + j) * 8 + blade_to_mask(c)];
-  }
-  if constexpr (OUT == kF32OutPauliRows) {
-    if (Ypre != nullptr) {  // the pre-activation rows, blade order (kept for the backward)
-      float4* q = reinterpret_cast<float4*>(Ypre + ((size_t)row * d_out + j) * 8);
-      q[0] = make_float4(y[0], y[1], y[2], y[3]);
-      q[1] = make_float4(y[4], y[5], y[6], y[7]);
-    }
-    activate_blade<ACT>(y);
-    float c0[4], c1[4];
-    blade_to_pauli(y, c0, c1);  // c0 = (M00, M10), c1 = (M01, M11)
-    float4* q = reinterpret_cast<float4*>(Y + ((size_t)row * d_out + j) * 8);  // [b][k][c]
-    q[0] = make_float4(c0[0], c0[2], c0[1], c0[3]);
-    q[1] = make_float4(c1[0], c1[2], c1[1], c1[3]);
-  } else {
-    size_t mv = OUT == kF32OutBladeT ? (size_t)j * P_max + row : (size_t)row * d_out + j;
-    if constexpr (OUT == kF32OutPartial)  // partial planes: at row_map[row] when given (slot rows)
-      mv = (size_t)split * P_max * d_out + (size_t)(row_map != nullptr ? row_map[row] : row) * d_out + j;
-    else activate_blade<ACT>(y);
-    float4* p = reinterpret_cast<float4*>(Y + mv * 8);
-    p[0] = make_float4(y[0], y[1], y[2], y[3]);
-    p[1] = make_float4(y[4], y[5], y[6], y[7]);
   }
 }
 
@@ -755,32 +717,14 @@ size_t gm_w_bytes(int M, int K) { return gm_align((size_t)M * K * 2 * 8 * sizeof
 size_t gm_x_bytes(int K, int N) { return gm_align((size_t)N * K * 8 * sizeof(float)); }
 }  // namespace
 
+YGG_API int ygg_f32_product_split(int rows, int d_in, int d_out) {
+  return pauli_split_pays(rows, d_in, d_out) && pauli_split_fits(1, rows, false, d_in, d_out);
+}
+
 YGG_API size_t ygg_geom_matmul_f32_workspace_bytes(int M, int K, int N) {
   if (M <= 0 || K <= 0 || N <= 0) return 0;
   return gm_w_bytes(M, K) + gm_x_bytes(K, N) + kGmAlign;
 }
-
-namespace {
-// The split product's operands in the workspace: split weights at 0, then these offsets.
-struct GmSplit {
-  size_t x, col_exp, row_exp, partial, offsets, end;
-};
-GmSplit gm_split_layout(int M, int K, int N) {
-  GmSplit g;
-  g.x = gm_align((size_t)M * pauli_split_row_bytes(K));
-  g.col_exp = g.x + gm_align((size_t)N * pauli_split_row_bytes(K));
-  g.row_exp = g.col_exp + gm_align((size_t)M * 4);
-  g.partial = g.row_exp + gm_align((size_t)N * 4);
-  g.offsets = g.partial + gm_align(pauli_split_gm_partials(K, N) * 4);
-  g.end = g.offsets + kGmAlign;
-  return g;
-}
-// geom_matmul through the split product, within the workspace of the fp32 MFMA one.
-bool gm_split(int M, int K, int N) {
-  return pauli_split_pays((long long)N, 1, K, M) && pauli_split_fits(1, N, N, false, K, M, true) &&
-         gm_split_layout(M, K, N).end <= ygg_geom_matmul_f32_workspace_bytes(M, K, N);
-}
-}  // namespace
 
 YGG_API int ygg_geom_matmul_f32_ws(const float* a, const float* b, float* out, int M, int K, int N, void* workspace,
                                    size_t workspace_bytes, hipStream_t stream) {
@@ -799,16 +743,6 @@ YGG_API int ygg_geom_matmul_f32_ws(const float* a, const float* b, float* out, i
   YGG_CHECK_ARG(workspace != nullptr && workspace_bytes >= need,
                 "ygg_geom_matmul_f32: workspace of %zu bytes, %zu needed", workspace_bytes, need);
   char* ws = static_cast<char*>(workspace);
-  if (gm_split(M, K, N)) {
-    const GmSplit g = gm_split_layout(M, K, N);
-    int32_t* off = reinterpret_cast<int32_t*>(ws + g.offsets);
-    int32_t* ce = reinterpret_cast<int32_t*>(ws + g.col_exp);
-    int32_t* re = reinterpret_cast<int32_t*>(ws + g.row_exp);
-    if (pauli_split_gm_operands(a, b, M, K, N, ws, ce, ws + g.x, re, reinterpret_cast<float*>(ws + g.partial), off,
-                                stream))
-      return -1;
-    return pauli_split_linear_t(ws + g.x, re, N, ws, ce, off, K, M, out, stream);
-  }
   float* wp = reinterpret_cast<float*>(ws);
   float* xp = reinterpret_cast<float*>(ws + gm_w_bytes(M, K));
   int32_t* off = reinterpret_cast<int32_t*>(ws + gm_w_bytes(M, K) + gm_x_bytes(K, N));
@@ -816,6 +750,8 @@ YGG_API int ygg_geom_matmul_f32_ws(const float* a, const float* b, float* out, i
   const dim3 tgrid((unsigned)((N + 31) / 32), (unsigned)((K + 7) / 8));
   pauli_f32_rows_t_kernel<<<tgrid, 256, 0, stream>>>(b, K, N, xp, off);
   if (check_launch("pauli_f32_rows_t")) return -1;
+  if (ygg_f32_product_split(N, K, M))
+    return pauli_split_linear(xp, N, nullptr, N, wp, nullptr, off, 1, K, M, kActNone, out, kF32OutBladeT, nullptr, stream);
   return launch_f32_act<kF32OutBladeT>(kActNone, 1, stream, xp, nullptr, wp, nullptr, off, 1, K, M, N, out);
 }
 
@@ -858,22 +794,7 @@ __global__ __launch_bounds__(256) void linear_rows_kernel(const void* __restrict
   }
 }
 
-struct LinearLayout {
-  bool split;
-  size_t x, w, col_exp, row_exp, offsets, end;
-};
-LinearLayout linear_layout(int dtype, int rows, int d_in, int d_out) {
-  LinearLayout l;
-  l.split = dtype == kF32 && pauli_split_pays(rows, 1, d_in, d_out) &&
-            pauli_split_fits(1, rows, rows, false, d_in, d_out, false);
-  l.x = 0;
-  l.w = gm_align(l.split ? (size_t)rows * pauli_split_row_bytes(d_in) : (size_t)rows * d_in * (dtype == kF32 ? 32 : 16));
-  l.col_exp = l.w + gm_align(l.split ? (size_t)d_out * pauli_split_row_bytes(d_in) : 0);
-  l.row_exp = l.col_exp + gm_align(l.split ? (size_t)d_out * 4 : 0);
-  l.offsets = l.row_exp + gm_align(l.split ? (size_t)rows * 4 : 0);
-  l.end = l.offsets + kGmAlign;
-  return l;
-}
+size_t linear_x_bytes(int dtype, int rows, int d_in) { return gm_align((size_t)rows * d_in * (dtype == kF32 ? 32 : 16)); }
 }  // namespace
 
 extern "C" int ygg_grouped_clifford_linear(const void*, int, const void*, int, const float*, const float*,
@@ -881,13 +802,12 @@ extern "C" int ygg_grouped_clifford_linear(const void*, int, const void*, int, c
 
 YGG_API size_t ygg_clifford_linear_workspace_bytes(int dtype, int rows, int d_in, int d_out) {
   if (rows <= 0 || d_in <= 0 || d_out <= 0) return 0;
-  return linear_layout(dtype, rows, d_in, d_out).end;
+  return linear_x_bytes(dtype, rows, d_in) + kGmAlign;  // the converted rows, then the one-expert offsets
 }
 
-// fp32: the split product from the sizes where it pays (4096 x 128 -> 512: 71 us a call;
-// the L(w) blocks on the vector units, 64 multiply-adds a pair, took 363 of the 398 us of a
-// call that also copied its row range from the host and waited for it), the fp32
-// MFMA product below; bf16: the L(w) blocks.
+// fp32: the split product or the fp32 MFMA one; bf16: the L(w) blocks.  (4096 x 128 -> 512, fp32:
+// 95-105 us; the L(w) blocks on the vector units, 64 multiply-adds a pair, took 363 of the 398 us of a
+// call that also copied its row range from the host and waited for it.)
 YGG_API int ygg_clifford_linear(const void* x, int dtype, int rows, const void* w, const float* bias, int d_in,
                                 int d_out, void* y, void* workspace, size_t workspace_bytes, hipStream_t stream) {
   YGG_CHECK_ARG(dtype == kF32 || dtype == kBF16, "ygg_clifford_linear: dtype %d", dtype);
@@ -895,26 +815,18 @@ YGG_API int ygg_clifford_linear(const void* x, int dtype, int rows, const void* 
                 d_in, d_out);
   if (rows == 0) return 0;
   YGG_CHECK_ARG(x && w && y && workspace, "ygg_clifford_linear: null pointer");
-  const LinearLayout l = linear_layout(dtype, rows, d_in, d_out);
-  YGG_CHECK_ARG(workspace_bytes >= l.end, "ygg_clifford_linear: workspace of %zu bytes, need %zu", workspace_bytes, l.end);
+  const size_t x_bytes = linear_x_bytes(dtype, rows, d_in), need = x_bytes + kGmAlign;
+  YGG_CHECK_ARG(workspace_bytes >= need, "ygg_clifford_linear: workspace of %zu bytes, need %zu", workspace_bytes, need);
   char* ws = static_cast<char*>(workspace);
-  int32_t* off = reinterpret_cast<int32_t*>(ws + l.offsets);
-  if (l.split) {
-    int32_t* ce = reinterpret_cast<int32_t*>(ws + l.col_exp);
-    int32_t* re = reinterpret_cast<int32_t*>(ws + l.row_exp);
-    SplitHidden none;
-    none.one_offsets = off;
-    if (pauli_split_weights(static_cast<const float*>(w), 1, d_out, d_in, nullptr, ws + l.w, ce, nullptr, stream) ||
-        pauli_split_rows(static_cast<const float*>(x), rows, d_in, ws + l.x, re, none, stream))
-      return -1;
-    return pauli_split_linear(ws + l.x, re, rows, ws + l.w, ce, bias, off, 1, d_in, d_out, static_cast<float*>(y),
-                              stream);
-  }
+  int32_t* off = reinterpret_cast<int32_t*>(ws + x_bytes);
   const size_t n = (size_t)rows * d_in;
   const unsigned grid = (unsigned)((n + 255) / 256);
   if (dtype == kF32) linear_rows_kernel<kF32><<<grid, 256, 0, stream>>>(x, rows, n, ws, off);
   else linear_rows_kernel<kBF16><<<grid, 256, 0, stream>>>(x, rows, n, ws, off);
   if (check_launch("linear_rows")) return -1;
+  if (dtype == kF32 && ygg_f32_product_split(rows, d_in, d_out))
+    return pauli_split_linear(reinterpret_cast<const float*>(ws), rows, nullptr, rows, static_cast<const float*>(w), bias,
+                              off, 1, d_in, d_out, kActNone, static_cast<float*>(y), kF32OutBlade, nullptr, stream);
   if (dtype == kF32)
     return launch_f32_act<kF32OutBlade>(kActNone, 1, stream, reinterpret_cast<const float*>(ws), nullptr,
                                         static_cast<const float*>(w), bias, off, 1, d_in, d_out, rows,

@@ -81,114 +81,6 @@ struct PauliTile {
   static_assert(A_ITEMS_ROWS % NT == 0 && W_ITEMS % NT == 0, "staging split");
 };
 
-// Epilogue of one tile of a split product (fp32 operands held as two fp16 parts,
-// scaled by powers of two per row and per output channel): the inverse Pauli map, the
-// scales taken back (exactly, one ldexp per value), bias, activation, and fp32 blade
-// output or the next product's split rows (scaled by 2^out_e).  row_e / col_e: the
-// tile's row and column scale exponents; y_rsrc starts at the tile's first row, or at
-// (column col0, row row0) of the transposed output; pre_rsrc (split rows out) takes the
-// fp32 blade rows before the activation, or is empty.
-// FLUSH: the first half of the contraction goes out as it is, without bias and
-// activation; the last call adds it back.  (With split rows out it waits, as fp32, in
-// the 32 bytes that the same lane writes at the end.)
-template <int ACT, int OUT, bool FLUSH>
-__device__ __forceinline__ void pauli_split_epilogue(const pf32x4_t (&acc)[4][2][2][2], const float (&bvs)[2][8],
-                                                     const PauliTileInfo& ti, int wave, int lane, int d_out,
-                                                     const int* row_e, const int* col_e, const int32_t* out_e,
-                                                     __amdgpu_buffer_rsrc_t y_rsrc, __amdgpu_buffer_rsrc_t pre_rsrc,
-                                                     uint32_t t_stride) {
-  typedef unsigned int pu32x2_t __attribute__((ext_vector_type(2)));
-  typedef unsigned int pu32x4_t __attribute__((ext_vector_type(4)));
-  const int wt = wave & 1, wj = wave >> 1, g = lane >> 4;
-  const int d_pad = (d_out + 7) & ~7;
-#pragma unroll
-  for (int cb = 0; cb < 2; ++cb) {
-    const int jl = wj * 32 + cb * 16 + (lane & 15), j = ti.col0 + jl;
-    // split rows: the padding columns are written as zeros
-    if (j >= (OUT == kOutSplitRows && !FLUSH ? d_pad : d_out)) continue;
-    const int ce = col_e[jl];
-#pragma unroll
-    for (int rb = 0; rb < 4; ++rb) {
-      if (ti.half >= 0 && rb > 1) break;  // a half tile: the first accumulators hold block `half`
-#pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        // row of the tile: the wave's 16 or 32 tokens, eight per 16-row block, two per lane
-        const int rl = (ti.compact ? wt * 16 : wt * 32 + (ti.half > 0 ? 16 : 0)) + rb * 8 + 2 * g + h;
-        if (ti.row0 + rl >= ti.row_end) continue;
-        const int v0 = 2 * h;  // b = 0 at v0, b = 1 at v0 + 1
-        float y[8];
-        pauli_to_blade(acc[rb][cb][0][0][v0], acc[rb][cb][0][1][v0], acc[rb][cb][0][0][v0 + 1],
-                       acc[rb][cb][0][1][v0 + 1], acc[rb][cb][1][0][v0], acc[rb][cb][1][1][v0],
-                       acc[rb][cb][1][0][v0 + 1], acc[rb][cb][1][1][v0 + 1], y);
-        const int ex = -(ce + row_e[rl]);
-#pragma unroll
-        for (int c = 0; c < 8; ++c) y[c] = __builtin_ldexpf(y[c], ex);
-        // split rows: hi at off, lo at off + 64 of half-row b = 0; half-row b = 1 follows
-        const uint32_t half_row = (uint32_t)d_pad * 16;
-        const uint32_t off = OUT == kOutBladeT     ? (uint32_t)jl * t_stride + (uint32_t)rl * 32
-                             : OUT == kOutSplitRows ? (uint32_t)rl * 2 * half_row + (uint32_t)(j >> 3) * 128 + (j & 7) * 8
-                                                    : ((uint32_t)rl * d_out + j) * 32;
-        if constexpr (!FLUSH) {
-          pu32x4_t p0, p1;
-          if constexpr (OUT == kOutSplitRows) {
-            const pu32x2_t q0 = __builtin_amdgcn_raw_buffer_load_b64(y_rsrc, off, 0, 0);
-            const pu32x2_t q1 = __builtin_amdgcn_raw_buffer_load_b64(y_rsrc, off + 64, 0, 0);
-            const pu32x2_t q2 = __builtin_amdgcn_raw_buffer_load_b64(y_rsrc, off + half_row, 0, 0);
-            const pu32x2_t q3 = __builtin_amdgcn_raw_buffer_load_b64(y_rsrc, off + half_row + 64, 0, 0);
-            p0 = {q0[0], q0[1], q1[0], q1[1]};
-            p1 = {q2[0], q2[1], q3[0], q3[1]};
-          } else {
-            p0 = __builtin_amdgcn_raw_buffer_load_b128(y_rsrc, off, 0, 0);
-            p1 = __builtin_amdgcn_raw_buffer_load_b128(y_rsrc, off + 16, 0, 0);
-          }
-#pragma unroll
-          for (int c = 0; c < 8; ++c) y[c] = (y[c] + __builtin_bit_cast(float, c < 4 ? p0[c & 3] : p1[c & 3])) + bvs[cb][c];
-          if constexpr (OUT == kOutSplitRows) {
-            const uint32_t po = j < d_out ? ((uint32_t)rl * d_out + j) * 32 : kBufferOff;
-            const pu32x4_t lo = {__builtin_bit_cast(unsigned, y[0]), __builtin_bit_cast(unsigned, y[1]),
-                                 __builtin_bit_cast(unsigned, y[2]), __builtin_bit_cast(unsigned, y[3])};
-            const pu32x4_t hi = {__builtin_bit_cast(unsigned, y[4]), __builtin_bit_cast(unsigned, y[5]),
-                                 __builtin_bit_cast(unsigned, y[6]), __builtin_bit_cast(unsigned, y[7])};
-            __builtin_amdgcn_raw_buffer_store_b128(lo, pre_rsrc, po, 0, 0);
-            __builtin_amdgcn_raw_buffer_store_b128(hi, pre_rsrc, po + 16, 0, 0);
-          }
-          activate_blade<ACT>(y);
-        }
-        if constexpr (OUT == kOutSplitRows && !FLUSH) {
-          float c0[4], c1[4];
-          if (j >= d_out) {
-#pragma unroll
-            for (int c = 0; c < 8; ++c) y[c] = 0.f;
-          }
-          blade_to_pauli(y, c0, c1);
-          const int oe = out_e[min(rl, ti.row_end - 1 - ti.row0)];
-          uint2 h0, l0, h1, l1;
-          split4_f16(c0, oe, h0, l0);
-          split4_f16(c1, oe, h1, l1);
-          __builtin_amdgcn_raw_buffer_store_b64(pu32x2_t{h0.x, h0.y}, y_rsrc, off, 0, 0);
-          __builtin_amdgcn_raw_buffer_store_b64(pu32x2_t{l0.x, l0.y}, y_rsrc, off + 64, 0, 0);
-          __builtin_amdgcn_raw_buffer_store_b64(pu32x2_t{h1.x, h1.y}, y_rsrc, off + half_row, 0, 0);
-          __builtin_amdgcn_raw_buffer_store_b64(pu32x2_t{l1.x, l1.y}, y_rsrc, off + half_row + 64, 0, 0);
-        } else {
-          const pu32x4_t lo = {__builtin_bit_cast(unsigned, y[0]), __builtin_bit_cast(unsigned, y[1]),
-                               __builtin_bit_cast(unsigned, y[2]), __builtin_bit_cast(unsigned, y[3])};
-          const pu32x4_t hi = {__builtin_bit_cast(unsigned, y[4]), __builtin_bit_cast(unsigned, y[5]),
-                               __builtin_bit_cast(unsigned, y[6]), __builtin_bit_cast(unsigned, y[7])};
-          if constexpr (OUT == kOutSplitRows) {
-            __builtin_amdgcn_raw_buffer_store_b64(pu32x2_t{lo[0], lo[1]}, y_rsrc, off, 0, 0);
-            __builtin_amdgcn_raw_buffer_store_b64(pu32x2_t{lo[2], lo[3]}, y_rsrc, off + 64, 0, 0);
-            __builtin_amdgcn_raw_buffer_store_b64(pu32x2_t{hi[0], hi[1]}, y_rsrc, off + half_row, 0, 0);
-            __builtin_amdgcn_raw_buffer_store_b64(pu32x2_t{hi[2], hi[3]}, y_rsrc, off + half_row + 64, 0, 0);
-          } else {
-            __builtin_amdgcn_raw_buffer_store_b128(lo, y_rsrc, off, 0, 0);
-            __builtin_amdgcn_raw_buffer_store_b128(hi, y_rsrc, off + 16, 0, 0);
-          }
-        }
-      }
-    }
-  }
-}
-
 template <int ACT, int IN, int OUT, int OUT_DT, class TL>
 __global__ __launch_bounds__(TL::NT) __attribute__((amdgpu_waves_per_eu(2))) void pauli_gemm_kernel(
     const uint16_t* __restrict__ X, const int32_t* __restrict__ gather, const uint16_t* __restrict__ Wp,
@@ -486,8 +378,6 @@ struct PauliDmaTile {
   static constexpr int G_OFF = W_OFF + NW * W_SLOT;         // 2 x 64 row indices (tile parity)
   static constexpr int B_OFF = G_OFF + 2 * T * 4;           // 2 x 64 columns x 32 B of bias
   static constexpr int LDS = B_OFF + 2 * BN * 32;           // 78336 B: two workgroups per CU
-  static constexpr int S_OFF = LDS;                         // split products: 2 x (64 row, 64 column) exponents
-  static constexpr int LDS_SPLIT = S_OFF + 2 * (T + BN) * 4;
   static constexpr int A_AHEAD = 2, W_AHEAD = 2;            // chunks issued ahead of use
 };
 
@@ -530,40 +420,19 @@ __device__ __forceinline__ void wait_vmcnt() {
 // the staged LDS contents ready are the explicit ones above
 __device__ __forceinline__ void lds_barrier() { asm volatile("s_barrier" ::: "memory"); }
 
-// SPLIT products: fp32 operands as two fp16 parts.  A row of x (scaled by 2^row_exp) and
-// a column of W (by 2^col_exp) are stored as hi = fp16(v), lo = fp16(v - hi), every
-// block of eight multivectors as its hi parts and then its lo parts, so d_in here is
-// twice the padded number of inputs: an A chunk holds both parts of eight inputs, and
-// the W chunks are hi and lo in turn.  The even step adds hi hi and lo hi, the odd one
-// hi lo (lo lo is below 2^-22 of a product of full-size parts): three fp16 MFMAs in the
-// place of the sixteen times slower fp32 ones.  The MFMA units round their fp32 sums
-// every eight terms, so one accumulator over the whole contraction would round more
-// than the fp32 kernel's four K ranges do (geom_matmul 512 x 128 x 8192: 2.7e-7 off
-// float64 against 2.1e-7): half way the sums go out to the output, and the second half
-// starts from zero (2.0e-7; 147 -> 166 us with the conversions, 411 us on the fp32
-// units).  Bound by staging and the steps' chain, as the bf16 product: the MFMAs alone
-// would take 41 us at the rate of a large library product.
-//
 // Sizes: x_bytes and y_bytes are the operands' whole sizes (64-bit).  Gathered rows
 // (token ids through `gather`) index the whole of x, which the host keeps below
 // 2 GiB; rows taken in place, and the output, are addressed from buffer resources
 // whose 64-bit base is the tile's first row, so only one tile's span needs 32-bit
 // offsets and the number of rows is not limited by them.
-struct PauliSplitExps {
-  const int32_t* row = nullptr;  // per product row
-  const int32_t* col = nullptr;  // per (expert, output channel)
-  int n_rows = 0;                // rows of `row` (and of the transposed output)
-  const int32_t* out = nullptr;  // split rows out: the exponents to write them with, per product row
-  float* pre = nullptr;          // split rows out: when set, takes the blade rows before the activation
-};
-template <int ACT, int OUT, int OUT_DT, bool SPLIT = false>
+template <int ACT, int OUT, int OUT_DT>
 __global__ __launch_bounds__(PauliDmaTile::NT) __attribute__((amdgpu_waves_per_eu(2))) void pauli_gemm_dma_kernel(
     const uint16_t* __restrict__ X, const int32_t* __restrict__ gather, const uint16_t* __restrict__ Wp,
     const float* __restrict__ bias, const int32_t* __restrict__ offsets, int E, int d_in, int d_out,
-    void* __restrict__ Y, int n_xcd, uint64_t x_bytes, uint64_t y_bytes, PauliSplitExps exps = PauliSplitExps{}) {
+    void* __restrict__ Y, int n_xcd, uint64_t x_bytes, uint64_t y_bytes) {
   using C = PauliDmaTile;
   constexpr int NT = C::NT, T = C::T, BN = C::BN, KC = C::KC, WR = C::WR, WC = C::WC, BWT = C::BWT;
-  __shared__ __attribute__((aligned(1024))) unsigned char smem[SPLIT ? C::LDS_SPLIT : C::LDS];
+  __shared__ __attribute__((aligned(1024))) unsigned char smem[C::LDS];
   __shared__ int s_off[kPauliMaxExperts + 1];   // expert row offsets
   __shared__ int s_tbeg[kPauliMaxExperts + 1];  // first whole row tile of each expert
   __shared__ int s_cbeg[kPauliMaxExperts + 1];  // first compact row tile of each expert
@@ -678,10 +547,6 @@ __global__ __launch_bounds__(PauliDmaTile::NT) __attribute__((amdgpu_waves_per_e
   const __amdgpu_buffer_rsrc_t b_rsrc = __builtin_amdgcn_make_buffer_rsrc(
       const_cast<float*>(bias), (short)0, bias ? (uint32_t)E * d_out * 32 : 0u, kBufferFlags);
   __amdgpu_buffer_rsrc_t w_rsrc = x_rsrc;
-  const __amdgpu_buffer_rsrc_t re_rsrc = __builtin_amdgcn_make_buffer_rsrc(
-      const_cast<int32_t*>(exps.row), (short)0, SPLIT ? (uint32_t)exps.n_rows * 4 : 0u, kBufferFlags);
-  const __amdgpu_buffer_rsrc_t ce_rsrc = __builtin_amdgcn_make_buffer_rsrc(
-      const_cast<int32_t*>(exps.col), (short)0, SPLIT ? (uint32_t)E * d_out * 4 : 0u, kBufferFlags);
 
   // this lane's pieces: A loads 4 w .. 4 w + 3 (half-rows 8 q .. 8 q + 7, one
   // 128-byte line each), W loads 2 w and 2 w + 1 (columns 8 q .. 8 q + 7)
@@ -760,15 +625,6 @@ __global__ __launch_bounds__(PauliDmaTile::NT) __attribute__((amdgpu_waves_per_e
         const int j = t.col0 + 32 * wave + (lane >> 1);
         dma_to_lds<16>(b_rsrc, smem + C::B_OFF + (iwm & 1) * BN * 32 + wave * 1024,
                        j < d_out ? (uint32_t)(t.e * d_out + j) * 32 + (lane & 1) * 16 : kOff);
-      }
-      if constexpr (SPLIT) {  // the tile's scale exponents: rows (wave 2), columns (wave 3)
-        unsigned char* es = smem + C::S_OFF + (iwm & 1) * (T + BN) * 4;
-        if (wave == 2) {
-          dma_to_lds<4>(re_rsrc, es, (uint32_t)min(t.row0 + lane, t.row_end - 1) * 4);
-        } else if (wave == 3) {
-          const int j = t.col0 + lane;
-          dma_to_lds<4>(ce_rsrc, es + T * 4, j < d_out ? (uint32_t)(t.e * d_out + j) * 4 : kOff);
-        }
       }
 #pragma unroll
       for (int u = 0; u < 2; ++u) {
@@ -865,107 +721,26 @@ __global__ __launch_bounds__(PauliDmaTile::NT) __attribute__((amdgpu_waves_per_e
     __builtin_amdgcn_s_setprio(0);
   };
 
-  // Split products: the operands of 16 x 16 x 32 MFMAs, lane row / column lane % 16,
-  // pair lane / 16 of the chunk's four; row block rb of four 16-row blocks, part 0 / 1
-  // the hi / lo half of the A chunk.
-  const int l16 = lane & 15, g4 = lane >> 4;
-  pf32x4_t sacc[4][2][2][2];
-  auto split_step = [&](int as, int ws, int par, auto nr_tag, int rb0) __attribute__((always_inline)) {
-    constexpr int NB = 2 * decltype(nr_tag)::value;  // 16-row blocks of this tile's share
-    const unsigned char* As = smem + as * C::A_SLOT;
-    const unsigned char* Ws = smem + C::W_OFF + ws * C::W_SLOT;
-    uint4 w[2][2];
-#pragma unroll
-    for (int cb = 0; cb < 2; ++cb) {
-      const int col = wj * 32 + cb * 16 + l16;
-#pragma unroll
-      for (int a = 0; a < 2; ++a)
-        w[cb][a] = *reinterpret_cast<const uint4*>(Ws + col * 128 + (((2 * g4 + a) ^ swz8(col)) * 16));
-    }
-    uint4 x[2][NB];
-    auto read_part = [&](int part) __attribute__((always_inline)) {
-#pragma unroll
-      for (int rb = 0; rb < NB; ++rb) {
-        const int row = wt * 64 + rb0 * 32 + rb * 16 + l16;
-        x[part][rb] = *reinterpret_cast<const uint4*>(As + row * 128 + (((4 * part + g4) ^ swz8(row)) * 16));
-      }
-    };
-    auto mma_part = [&](int part) __attribute__((always_inline)) {
-#pragma unroll
-      for (int rb = 0; rb < NB; ++rb) {
-        const uint4 v = x[part][rb];
-        const uint4 vp = make_uint4(rot_conj(v.x), rot_conj(v.y), rot_conj(v.z), rot_conj(v.w));
-        const pf16x8_t A0 = __builtin_bit_cast(pf16x8_t, v), A1 = __builtin_bit_cast(pf16x8_t, vp);
-#pragma unroll
-        for (int cb = 0; cb < 2; ++cb)
-#pragma unroll
-          for (int a = 0; a < 2; ++a) {
-            const pf16x8_t B = __builtin_bit_cast(pf16x8_t, w[cb][a]);
-            sacc[rb][cb][a][0] = __builtin_amdgcn_mfma_f32_16x16x32_f16(A0, B, sacc[rb][cb][a][0], 0, 0, 0);
-            sacc[rb][cb][a][1] = __builtin_amdgcn_mfma_f32_16x16x32_f16(A1, B, sacc[rb][cb][a][1], 0, 0, 0);
-          }
-      }
-    };
-    read_part(0);
-    if (par == 0) read_part(1);
-    if (par == 0 && ia < total_a) issue_a();
-    if (iw < total) issue_w();
-    __builtin_amdgcn_s_setprio(1);
-    mma_part(0);
-    if (par == 0) mma_part(1);
-    __builtin_amdgcn_s_setprio(0);
-  };
-
   // a tile's accumulators start from its bias (slot m % 2, complete by the tile's first step)
-  // (split products: from zero, their scales come off before the bias)
-  constexpr int NBV = SPLIT ? 2 : WC;  // columns per lane
-  float bvs[NBV][8];
-  auto load_bias = [&](int m) __attribute__((always_inline)) {
+  float bvs[WC][8];
+  auto acc_from_bias = [&](int m) __attribute__((always_inline)) {
     const unsigned char* bs = smem + C::B_OFF + (m & 1) * BN * 32;
 #pragma unroll
-    for (int cb = 0; cb < NBV; ++cb) {
-      const int jl = SPLIT ? wj * 32 + cb * 16 + l16 : (wj * WC + cb) * 32 + l32;
+    for (int cb = 0; cb < WC; ++cb) {
+      const int jl = (wj * WC + cb) * 32 + l32;
       const uint4 lo4 = *reinterpret_cast<const uint4*>(bs + jl * 32);
       const uint4 hi4 = *reinterpret_cast<const uint4*>(bs + jl * 32 + 16);
       const uint32_t mk[8] = {lo4.x, lo4.y, lo4.z, lo4.w, hi4.x, hi4.y, hi4.z, hi4.w};  // mask order
 #pragma unroll
       for (int c = 0; c < 8; ++c) bvs[cb][c] = __builtin_bit_cast(float, mk[blade_to_mask(c)]);
     }
-  };
-  auto start_acc = [&](int m) __attribute__((always_inline)) {
-    if constexpr (SPLIT) {
-#pragma unroll
-      for (int rb = 0; rb < 4; ++rb)
-#pragma unroll
-        for (int cb = 0; cb < 2; ++cb)
-#pragma unroll
-          for (int a = 0; a < 2; ++a)
-#pragma unroll
-            for (int ri = 0; ri < 2; ++ri) sacc[rb][cb][a][ri] = pf32x4_t{0.f, 0.f, 0.f, 0.f};
-    } else {
-      load_bias(m);
-      pauli_acc_from_bias<WR, WC>(acc, bvs);
-    }
+    pauli_acc_from_bias<WR, WC>(acc, bvs);
   };
   // the output from the tile's first row on (64-bit base)
   constexpr uint64_t Y_MV_BYTES = (OUT == kOutPauliRows || OUT_DT == kBF16) ? 16 : 32;
-  auto epilogue = [&](const PauliTileInfo& ti, int m, auto flush) __attribute__((always_inline)) {
-    if constexpr (SPLIT) {
-      if (!decltype(flush)::value) load_bias(m);
-      const int* es = reinterpret_cast<const int*>(smem + C::S_OFF + (m & 1) * (T + BN) * 4);
-      const uint64_t first = OUT == kOutBladeT      ? ((uint64_t)ti.col0 * exps.n_rows + ti.row0) * 32
-                             : OUT == kOutSplitRows ? (uint64_t)ti.row0 * pauli_split_row_bytes(d_out)
-                                                    : (uint64_t)ti.row0 * d_out * 32;
-      const uint64_t pre_bytes = OUT == kOutSplitRows && exps.pre != nullptr ? (uint64_t)exps.n_rows * d_out * 32 : 0;
-      pauli_split_epilogue<ACT, OUT, decltype(flush)::value>(
-          sacc, bvs, ti, wave, lane, d_out, es, es + T, OUT == kOutSplitRows ? exps.out + ti.row0 : nullptr,
-          rsrc_from(Y, y_bytes, first), rsrc_from(exps.pre, pre_bytes, (uint64_t)ti.row0 * d_out * 32),
-          (uint32_t)exps.n_rows * 32);
-    }
-    if constexpr (!SPLIT) {
-      const __amdgpu_buffer_rsrc_t y_rsrc = rsrc_from(Y, y_bytes, (uint64_t)ti.row0 * d_out * Y_MV_BYTES);
-      pauli_tile_epilogue<ACT, OUT, OUT_DT, WR, WC, BWT, true>(acc, bvs, ti, wave, g, l32, d_out, y_rsrc, ti.row0);
-    }
+  auto epilogue = [&](const PauliTileInfo& ti) __attribute__((always_inline)) {
+    const __amdgpu_buffer_rsrc_t y_rsrc = rsrc_from(Y, y_bytes, (uint64_t)ti.row0 * d_out * Y_MV_BYTES);
+    pauli_tile_epilogue<ACT, OUT, OUT_DT, WR, WC, BWT, true>(acc, bvs, ti, wave, g, l32, d_out, y_rsrc, ti.row0);
   };
 
   // prologue: the first tile's gather indices; then what steps -4 .. -1 would
@@ -989,7 +764,6 @@ __global__ __launch_bounds__(PauliDmaTile::NT) __attribute__((amdgpu_waves_per_e
   // before those, only make the wait stricter); near the end, none.
   PauliTileInfo cur = {0, 0, 1, 0, -1};
   int fm = 0, fkc = 0;   // tile and K chunk of the step computed
-  const int mid = nka / 2 * 2 - 1;  // split products: the step after which the first half goes out
   int fas = 0, fws = 0;  // its A and W slots
   auto step = [&](int f, auto nr_tag) __attribute__((always_inline)) {
     constexpr int NR = decltype(nr_tag)::value;
@@ -1003,24 +777,14 @@ __global__ __launch_bounds__(PauliDmaTile::NT) __attribute__((amdgpu_waves_per_e
     lds_barrier();
     if (fkc == 0) {
       cur = decode(fm);
-      start_acc(fm);
+      acc_from_bias(fm);
     }
-    if constexpr (SPLIT) {
-      split_step(fas, fws, odd ? 1 : 0, nr_tag, cur.half < 0 ? 0 : cur.half);
-    } else {
-      read_operands(fas, fws, odd ? 1 : 0, nr_tag, cur.half < 0 ? 0 : cur.half);
-      if (!odd && ia < total_a) issue_a();
-      if (iw < total) issue_w();
-      mfmas(nr_tag);
-    }
+    read_operands(fas, fws, odd ? 1 : 0, nr_tag, cur.half < 0 ? 0 : cur.half);
+    if (!odd && ia < total_a) issue_a();
+    if (iw < total) issue_w();
+    mfmas(nr_tag);
     const bool last = fkc == nk - 1;
-    if constexpr (SPLIT) {
-      if (odd && fkc == mid) {
-        epilogue(cur, fm, std::true_type{});
-        start_acc(fm);
-      }
-    }
-    if (last) epilogue(cur, fm, std::false_type{});
+    if (last) epilogue(cur);
     fm += last ? 1 : 0;
     fkc = last ? 0 : fkc + 1;
     fas = odd ? (fas == C::NA - 1 ? 0 : fas + 1) : fas;
@@ -1113,16 +877,13 @@ namespace {
 // 512-thread 64 x 128 workgroup per CU.)
 using Tile = PauliTile</*WR*/ 2, /*WC*/ 1, /*BWT*/ 2, /*BWJ*/ 2, /*KC*/ 16>;
 constexpr int kWgPerCu = 2;
+
 // Fewer tiles than workgroups: one workgroup per tile -- unless every tile cut in halves
-// still gets a CU of its own (a split product: a workgroup's place): then the whole grid
-// runs and the kernel cuts them, which shortens a workgroup's steps.  Half tiles stage as
-// much as whole ones, so two to a CU are no faster where a staged operand feeds one MFMA
-// instead of three.  (geom_matmul 512 x 128 x 1024, 128 tiles: 57 -> 46 us, 512 x 512 x 1024 138 -> 106;
-// bf16 layer of 1024 tokens, d = 64, F = 128, E = 4, 36 and 72 tiles: 39 -> 34; of 1500 tokens,
-// 144 tiles in the down product: 65 -> 66, left as it was.)
-bool clip_grid(long long tiles, int grid, int halves_per_place) {
-  return tiles < grid && halves_per_place * tiles > grid;
-}
+// still gets a CU of its own: then the whole grid runs and the kernel cuts them, which
+// shortens a workgroup's steps.  Half tiles stage as much as whole ones, so two to a CU are
+// no faster.  (Layer of 1024 tokens, d = 64, F = 128, E = 4, 36 and 72 tiles: 39 -> 34 us; of 1500
+// tokens, 144 tiles in the down product: 65 -> 66, left as it was.)
+bool clip_grid(long long tiles, int grid) { return tiles < grid && 4 * tiles > grid; }
 
 // persistent grid: as many workgroups as fit on the chip at once
 struct DeviceShape {
@@ -1155,7 +916,7 @@ int launch_pauli(hipStream_t st, const uint16_t* X, uint64_t x_bytes, const int3
       ((long long)(P_max + Tile::T - 1) / Tile::T + E) * ((d_out + Tile::BN - 1) / Tile::BN);
   int grid = ds.cus * kWgPerCu;
   int xcds = ds.xcds;
-  if (clip_grid(max_tiles, grid, 4)) {
+  if (clip_grid(max_tiles, grid)) {
     grid = (int)max_tiles;
     xcds = 1;
   }
@@ -1185,89 +946,6 @@ int launch_pauli_act(hipStream_t st, int in_layout, int out_layout, int y_dtype,
 #undef YGG_PL
 }
 }  // namespace
-
-// ---- split products: launcher ------------------------------------------------------
-// From 128 inputs on: below, the parts' own rounding (7.5e-8 of a result) shows beside
-// that of the sums (geom_matmul against float64, split / fp32 MFMA: 3.7e-7 / 4.1e-7 at
-// K = 512, 2.04e-7 / 2.13e-7 at 128, 1.62e-7 / 1.57e-7 at 64).  From about 100 tiles
-// of 64 rows x 64 channels on: a tile's steps are a chain of some 1.4 us per eight
-// inputs, and fewer tiles leave CUs idle that the fp32 MFMA kernel's 16 x 32 tiles use
-// (one expert, K = 128: 64 tiles 60 us against 50-51, 128 tiles 57-60 against 77-80, 512
-// tiles 94 against 218).  And from 32 rows per expert on, where half a tile is filled.
-bool ygg::pauli_split_pays(long long P, int E, int d_in, int d_out) {
-  return d_in >= 128 && P * d_out >= 100LL * 64 * 64 && P >= 32LL * E;
-}
-
-bool ygg::pauli_split_fits(int E, int P_max, int x_rows, bool gathered, int d_in, int d_out, bool transposed) {
-  const uint64_t dv = pauli_split_width(d_in), lim = (uint64_t)1 << 31;
-  return E >= 1 && E <= kPauliMaxExperts && dv > 2 * PauliDmaTile::KC && (uint64_t)P_max * 4 < lim &&
-         (uint64_t)(d_out + 64) * dv * 16 < lim && (uint64_t)E * d_out * 32 < lim &&
-         (uint64_t)PauliDmaTile::T * dv * 16 < lim && (uint64_t)PauliDmaTile::T * d_out * 32 < lim &&
-         (!gathered || (uint64_t)x_rows * dv * 16 < lim) && (!transposed || (uint64_t)PauliDmaTile::BN * P_max * 32 < lim);
-}
-
-namespace {
-template <int ACT, int OUT>
-int launch_split(const void* x, int x_rows, int P_max, const void* w, const float* bias, const int32_t* gather,
-                 const int32_t* offsets, int E, int d_in, int d_out, void* y, const PauliSplitExps& ex,
-                 hipStream_t st) {
-  const DeviceShape ds = device_shape();
-  const int dv = pauli_split_width(d_in);
-  const uint64_t y_row = OUT == kOutSplitRows ? pauli_split_row_bytes(d_out) : (uint64_t)d_out * 32;
-  const long long max_tiles = ((long long)(P_max + PauliDmaTile::T - 1) / PauliDmaTile::T + E) *
-                              ((d_out + PauliDmaTile::BN - 1) / PauliDmaTile::BN);
-  int grid = ds.cus * kWgPerCu, xcds = ds.xcds;
-  if (clip_grid(max_tiles, grid, 2)) {
-    grid = (int)max_tiles;
-    xcds = 1;
-  }
-  pauli_gemm_dma_kernel<ACT, OUT, kF32, true><<<grid, PauliDmaTile::NT, 0, st>>>(
-      static_cast<const uint16_t*>(x), gather, static_cast<const uint16_t*>(w), bias, offsets, E, dv, d_out, y, xcds,
-      (uint64_t)x_rows * dv * 16, (uint64_t)P_max * y_row, ex);
-  return check_launch("pauli_split");
-}
-}  // namespace
-
-int ygg::pauli_split_linear_t(const void* x, const int32_t* row_exp, int P_max, const void* w, const int32_t* col_exp,
-                              const int32_t* offsets, int d_in, int d_out, float* y_t, hipStream_t stream) {
-  PauliSplitExps ex;
-  ex.row = row_exp;
-  ex.col = col_exp;
-  ex.n_rows = P_max;
-  return launch_split<kActNone, kOutBladeT>(x, P_max, P_max, w, nullptr, nullptr, offsets, 1, d_in, d_out, y_t, ex,
-                                            stream);
-}
-
-int ygg::pauli_split_linear(const void* x, const int32_t* row_exp, int P_max, const void* w, const int32_t* col_exp,
-                            const float* bias, const int32_t* offsets, int E, int d_in, int d_out, float* y,
-                            hipStream_t stream) {
-  PauliSplitExps ex;
-  ex.row = row_exp;
-  ex.col = col_exp;
-  ex.n_rows = P_max;
-  return launch_split<kActNone, kOutBlade>(x, P_max, P_max, w, bias, nullptr, offsets, E, d_in, d_out, y, ex, stream);
-}
-
-int ygg::pauli_split_up(const void* x, int x_rows, const int32_t* row_exp, const int32_t* gather, int P_max,
-                        const void* w, const int32_t* col_exp, const float* bias, const int32_t* offsets, int E,
-                        int d_in, int d_out, int act, void* h, const int32_t* h_exp, float* h_pre,
-                        hipStream_t stream) {
-  PauliSplitExps ex;
-  ex.row = row_exp;
-  ex.col = col_exp;
-  ex.n_rows = P_max;
-  ex.out = h_exp;
-  ex.pre = h_pre;
-#define YGG_SU(A) \
-  return launch_split<A, kOutSplitRows>(x, x_rows, P_max, w, bias, gather, offsets, E, d_in, d_out, h, ex, stream)
-  switch (act) {
-    case kActNone: YGG_SU(kActNone);
-    case kActGelu: YGG_SU(kActGelu);
-    case kActRelu: YGG_SU(kActRelu);
-    default: YGG_SU(kActSigmoid);
-  }
-#undef YGG_SU
-}
 
 // Pauli weight preparation, called by ygg_prepare_weights (format 3).
 int ygg::pauli_prepare_weights(const float* W, int E, int d_out, int d_in, void* out, hipStream_t stream) {

@@ -1,345 +1,227 @@
-// pauli_split.hip -- fp32 operands of the Pauli products as two fp16 parts, for the
-// split products of pauli_gemm.hip.
+// pauli_split.hip -- fp32 Pauli products of enough rows on the bf16 MFMA units (the sums:
+// pauli_split.h), from the operands of pauli_f32.hip: Pauli rows and weights in format 4.
 //
-// A Pauli entry v of a row whose largest entry lies in [2^m, 2^(m+1)) is scaled by 2^s,
-// s = 14 - m, and stored as hi = fp16(2^s v) and lo = fp16(2^s v - hi), each rounded to
-// nearest even: together 22 bits, v (1 + 2^-23) or closer while |v| is within 2^-16 of
-// the row's largest, and within 2^-39 of that largest below.  (The entries of a row with
-// a non-finite value are stored unscaled: the row's outputs are then not finite either.)
-//
-// These kernels are bound by memory (they read fp32 operands once and write as many
-// bytes); the second pass over a row, after its maximum is known, hits the caches.
+// A workgroup of four waves owns 64 tokens x 64 output multivectors, a wave 32 x 32; a step is
+// eight inputs: 16 KiB of rows and 16 KiB of weights, direct to LDS, double buffered; the values
+// are cut into parts on their way from LDS to the MFMA.  Bound by the MFMAs, at the rate that a
+// large library product reaches on the card: 32768 rows, 128 -> 512, 32 experts 749 us, 1.10
+// PFLOP/s issued.  geom_matmul 512 x 128 x 8192: 412 us on the fp32 units, 205-225 here, error
+// against float64 2.1e-7 and 1.0e-7.
 
 #include <algorithm>
+#include <type_traits>
 
-#include "pauli_common.h"
+#include "pauli_f32.h"
+#include "pauli_split.h"
+#include "ygg_common.h"
 
 namespace ygg {
 namespace {
 
-// entries of a weight multivector as the product's B operand: per a, (c0 u, c0 -v,
-// c1 u, c1 -v) of W / 2 (the 1/2 makes the inverse map a plain sum)
-__device__ __forceinline__ void w_entries(const float* w8, float (&e0)[4], float (&e1)[4]) {
-  float x[8], c0[4], c1[4];
-#pragma unroll
-  for (int c = 0; c < 8; ++c) x[c] = 0.5f * w8[c];
-  blade_to_pauli(x, c0, c1);  // c0 = (M00, M10), c1 = (M01, M11)
-  e0[0] = c0[0]; e0[1] = -c0[1]; e0[2] = c1[0]; e0[3] = -c1[1];
-  e1[0] = c0[2]; e1[1] = -c0[3]; e1[2] = c1[2]; e1[3] = -c1[3];
-}
+constexpr int kSpT = 64, kSpN = 64, kSpK = 8;              // tokens, columns, inputs of a step
+constexpr int kSpA = kSpT * kSpK * 32, kSpW = kSpK * kSpN * 32;  // bytes of a stage: rows, weights
+constexpr int kSpMaxExperts = 64;
 
-__device__ __forceinline__ void load8(const float* p, float (&v)[8]) {
-  const float4 a = reinterpret_cast<const float4*>(p)[0], b = reinterpret_cast<const float4*>(p)[1];
-  v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w; v[4] = b.x; v[5] = b.y; v[6] = b.z; v[7] = b.w;
-}
+template <int ACT, int OUT>
+__global__ __launch_bounds__(256, 2) void pauli_split_kernel(
+    const float* __restrict__ X, uint64_t x_bytes, const int32_t* __restrict__ gather, const float* __restrict__ Wp,
+    const float* __restrict__ bias, const int32_t* __restrict__ offsets, int E, int d_in, int d_out, int P_max, int n_xcd,
+    float* __restrict__ Y, float* __restrict__ Ypre) {
+  __shared__ __attribute__((aligned(1024))) unsigned char smem[2 * (kSpA + kSpW)];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  // The tiles (row tile of an expert) x (column tile), column tiles first, in one contiguous
+  // range per XCD; one lane per expert counts its row tiles, a scan finds the one that holds
+  // this workgroup's.
+  const int beg = lane < E ? offsets[lane] : 0, end = lane < E ? offsets[lane + 1] : 0;
+  const int nt = (end - beg + kSpT - 1) / kSpT;
+  int incl = nt;
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const int v = __shfl_up(incl, o);
+    if (lane >= o) incl += v;
+  }
+  const int CT = (d_out + kSpN - 1) / kSpN;
+  const int n_tiles = __builtin_amdgcn_readlane(incl, 63) * CT, per = (n_tiles + n_xcd - 1) / n_xcd;
+  const int slot = blockIdx.x / n_xcd, tile = (blockIdx.x - slot * n_xcd) * per + slot;
+  if (slot >= per || tile >= n_tiles) return;
+  const int rt = tile / CT, col0 = (tile - rt * CT) * kSpN;
+  const int e = (int)__builtin_ctzll(__ballot(incl > rt));  // the first expert whose tiles reach past rt
+  const int row_end = __builtin_amdgcn_readlane(end, e);
+  const int row0 = __builtin_amdgcn_readlane(beg, e) +
+                   (rt - (__builtin_amdgcn_readlane(incl, e) - __builtin_amdgcn_readlane(nt, e))) * kSpT;
 
-// One output channel's weights, d_in blade multivectors at w, by one wave.
-__device__ void split_w_channel(const float* __restrict__ w, int d_in, int lane, unsigned char* __restrict__ out,
-                                int32_t* __restrict__ col_exp) {
-  uint32_t m = 0;
-  for (int i = lane; i < d_in; i += 64) {
-    float v[8], e0[4], e1[4];
-    load8(w + (size_t)i * 8, v);
-    w_entries(v, e0, e1);
+  // rows: gathered ones index the whole of x (below 2 GiB), rows in place start at the tile's first
+  const uint64_t x_first = gather ? 0 : (uint64_t)row0 * d_in * 32, x_left = x_bytes > x_first ? x_bytes - x_first : 0;
+  const __amdgpu_buffer_rsrc_t x_rsrc =
+      __builtin_amdgcn_make_buffer_rsrc(const_cast<char*>(reinterpret_cast<const char*>(X)) + x_first, (short)0,
+                                        (uint32_t)(x_left < 0x7fffffffull ? x_left : 0x7fffffffull), kBufferFlags);
+  const __amdgpu_buffer_rsrc_t w_rsrc =
+      __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(Wp) + (size_t)e * d_in * 2 * d_out * 8, (short)0,
+                                        (uint32_t)d_in * 2 * d_out * 32, kBufferFlags);
+  // This lane's pieces (16 bytes).  Rows: load u covers tokens 16 wave + 4 u .. + 3, 256 bytes
+  // each; LDS slot s of token t holds piece s ^ 2 (t % 8), piece 2 i + b being input i, half b.
+  // Weights: load u covers input 2 wave + u / 2 and 32 columns (u % 2); slot 2 j + s of an input's
+  // run holds (column j, c = s ^ (j / 8 % 2)).  Both orders keep the operand reads free of conflicts.
+  uint32_t a_off[4], w_off[2];
+  int a_lim[2];  // (by u % 2) the piece is inside the contraction while the step's first input is below this
 #pragma unroll
-    for (int q = 0; q < 4; ++q) m = max(m, max(mag_bits(e0[q]), mag_bits(e1[q])));
+  for (int u = 0; u < 4; ++u) {
+    const int t = 16 * wave + 4 * u + (lane >> 4), piece = (lane & 15) ^ ((t & 7) << 1);
+    const int r = min(row0 + t, row_end - 1);  // rows past the range: computed, not stored
+    const int src = gather ? gather[r] : r - row0;
+    a_off[u] = (uint32_t)src * d_in * 32 + piece * 16;
+    a_lim[u & 1] = d_in - (piece >> 1);
   }
-  const int s = split_exp(__builtin_bit_cast(float, wave_max_u32(m)));
-  if (lane == 0) *col_exp = s;
-  const int d_pad = (d_in + 7) / 8 * 8;
-  for (int i = lane; i < d_pad; i += 64) {
-    float v[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f}, e0[4], e1[4];
-    if (i < d_in) load8(w + (size_t)i * 8, v);
-    w_entries(v, e0, e1);
-    uint2 h0, l0, h1, l1;
-    split4_f16(e0, s, h0, l0);
-    split4_f16(e1, s, h1, l1);
-    unsigned char* p = out + (size_t)(i >> 3) * 256 + ((i >> 1) & 3) * 32 + (i & 1) * 8;
-    *reinterpret_cast<uint2*>(p) = h0;
-    *reinterpret_cast<uint2*>(p + 16) = h1;
-    *reinterpret_cast<uint2*>(p + 128) = l0;
-    *reinterpret_cast<uint2*>(p + 144) = l1;
+#pragma unroll
+  for (int u = 0; u < 2; ++u) {
+    const int j = u * 32 + (lane >> 1), c = (lane & 1) ^ ((j >> 3) & 1);
+    w_off[u] = col0 + j < d_out ? (uint32_t)(col0 + j) * 32 + c * 16 : kBufferOff;
   }
-}
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(sp_lds_t*)smem;
+  auto issue = [&](int f) __attribute__((always_inline)) {  // step f's operands to stage f % 2
+    const uint32_t st = lds0 + (f & 1) * (kSpA + kSpW);
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+      split_dma(x_rsrc, st + (4 * wave + u) * 1024, f * kSpK < a_lim[u & 1] ? a_off[u] : kBufferOff, (uint32_t)f * 256);
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int i = f * kSpK + 2 * wave + (u >> 1);  // uniform; past the contraction: zeros
+      split_dma(w_rsrc, st + kSpA + (4 * wave + u) * 1024, i < d_in ? w_off[u & 1] : kBufferOff,
+                i < d_in ? (uint32_t)i * 64 * d_out : 0u);
+    }
+  };
 
-// ---- prepared weights (format 4) -> split weights ------------------------------------
-// Workgroup: 8 channels of one expert, thread (input t / 8 of 32, channel t % 8); the
-// first pass takes each channel's largest entry, the second writes 32 inputs at a time
-// through LDS (the source is contiguous over channels, the result over inputs).
-__global__ __launch_bounds__(256) void split_weights_kernel(const float* __restrict__ w, int d_out, int d_in,
-                                                            const float* __restrict__ bias,
-                                                            unsigned char* __restrict__ out,
-                                                            int32_t* __restrict__ col_exp, float* __restrict__ norms) {
-  __shared__ uint32_t mx[32][8];
-  __shared__ float sq[32][8];
-  __shared__ int se[8];
-  __shared__ uint2 tile[8][4][32];  // [channel][block of 8 inputs][256 bytes]
-  const int nb = (d_out + 7) / 8, e = blockIdx.x / nb, jb = blockIdx.x - e * nb;
-  const int t = threadIdx.x, ii = t >> 3, jj = t & 7, j = jb * 8 + jj, jc = min(j, d_out - 1);
-  // (u, v) of every entry: the k = 0 record of (e, i, j)
-  const float* src = w + (((size_t)e * d_in * 2) * d_out + jc) * 8;
-  const size_t step = (size_t)2 * d_out * 8;
-  uint32_t m = 0;
-#pragma unroll 4
-  for (int i = ii; i < d_in; i += 32) {
-    float v[8];
-    load8(src + i * step, v);
+  // Operands of v_mfma_f32_16x16x32_bf16: lane row / column lane % 16, inputs 2 g and 2 g + 1 of
+  // the step, g = lane / 16.  A wave's row block rb is tokens 16 rb + 8 wt .. + 7, both halves.
+  const int wt = wave & 1, wj = wave >> 1, l16 = lane & 15, g = lane >> 4;
+  uint32_t a_rd[2];  // inputs 2 g, 2 g + 1 of token 8 wt + l16 / 2 (+ 4096 per row block)
 #pragma unroll
-    for (int c = 0; c < 8; ++c) m = max(m, mag_bits(v[c]));
+  for (int h = 0; h < 2; ++h) {
+    const int t = 8 * wt + (l16 >> 1);
+    a_rd[h] = t * 256 + (((2 * (2 * g + h) + (l16 & 1)) ^ ((t & 7) << 1)) * 16);
   }
-  mx[ii][jj] = m;
-  __syncthreads();
-  if (t < 8) {
-    for (int r = 1; r < 32; ++r) m = max(m, mx[r][t]);
-    se[t] = split_exp(__builtin_bit_cast(float, m));
-    if (jb * 8 + t < d_out) col_exp[(size_t)e * d_out + jb * 8 + t] = se[t];
-  }
-  __syncthreads();
-  const int s = se[jj];
-  float n2 = 0.f;
-  const size_t rec = pauli_split_row_bytes(d_in);  // bytes per channel
-  const int d_pad = (d_in + 7) & ~7;
-  float v[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-  if (ii < d_in) load8(src + ii * step, v);
-  for (int i0 = 0; i0 < d_pad; i0 += 32) {
-    // v: [c][a][(u, v)]; the operand is (u, -v) per (a, c)
-    const float e0[4] = {v[0], -v[1], v[4], -v[5]}, e1[4] = {v[2], -v[3], v[6], -v[7]};
-    if (norms != nullptr) {
+  const int jl = wj * 32 + l16;  // (+ 16 per column block: j / 8 % 2 stays)
+  const uint32_t w_rd = kSpA + 2 * g * 2048 + jl * 32 + ((jl >> 3) & 1) * 16;  // (c = 0; c = 1 at ^ 16; input 2 g + 1 at + 2048)
+
+  pf32x4_t acc[4][4][2];  // [row block][column block, a][re, im]
 #pragma unroll
-      for (int c = 0; c < 8; ++c) {
-        const float x = __builtin_ldexpf(v[c], s);
-        n2 += x * x;
+  for (int rb = 0; rb < 4; ++rb)
+#pragma unroll
+    for (int c = 0; c < 4; ++c)
+#pragma unroll
+      for (int q = 0; q < 2; ++q) acc[rb][c][q] = pf32x4_t{0.f, 0.f, 0.f, 0.f};
+
+  // A step of NP pairs of row blocks.  (The barriers keep the scheduler from holding more parts
+  // than the registers do: the other wave of the SIMD fills the gaps.)
+  auto compute = [&](int f, auto pairs_tag) __attribute__((always_inline)) {
+    constexpr int NP = decltype(pairs_tag)::value;
+    const unsigned char* st = smem + (f & 1) * (kSpA + kSpW);
+    const uint32_t neg = (f & 1) << 31;
+    uint4 A[2 * NP][3];  // (re c0, re c1), (im c0, im c1) of two inputs
+#pragma unroll
+    for (int r = 0; r < 2 * NP; ++r)
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const float4 x = *reinterpret_cast<const float4*>(st + a_rd[h] + r * 4096);
+        split_operand(A[r], h, x.x, x.y, x.z, x.w);
       }
-    }
-    uint2 h0, l0, h1, l1;
-    split4_f16(e0, s, h0, l0);
-    split4_f16(e1, s, h1, l1);
-    const int b8 = ii >> 3, p = ((ii >> 1) & 3) * 4 + (ii & 1);  // 8-byte pieces: pair record, input of the pair
-    tile[jj][b8][p] = h0;
-    tile[jj][b8][p + 2] = h1;
-    tile[jj][b8][p + 16] = l0;
-    tile[jj][b8][p + 18] = l1;
-    const int in = i0 + 32 + ii;  // the next inputs load while these are written
-#pragma unroll
-    for (int c = 0; c < 8; ++c) v[c] = 0.f;
-    if (in < d_in) load8(src + in * step, v);
-    __syncthreads();
-    const int oj = t >> 5, ob = (t >> 3) & 3, oq = (t & 7) * 4;  // 32 bytes per thread
-    if (jb * 8 + oj < d_out && i0 + ob * 8 < d_pad) {
-      const uint2* q = &tile[oj][ob][oq];
-      uint4* dst = reinterpret_cast<uint4*>(out + ((size_t)e * d_out + jb * 8 + oj) * rec + (size_t)(i0 / 8 + ob) * 256 + oq * 8);
-      dst[0] = make_uint4(q[0].x, q[0].y, q[1].x, q[1].y);
-      dst[1] = make_uint4(q[2].x, q[2].y, q[3].x, q[3].y);
-    }
-    __syncthreads();
-  }
-  if (norms == nullptr) return;
-  sq[ii][jj] = n2;
-  __syncthreads();
-  if (t < 8) {
-    float a = 0.f, b = 0.f;
-    for (int r = 0; r < 32; ++r) a += sq[r][t];
-    // Frobenius norm of the matrices of W (its halves are stored: 2 |W / 2|)
-    a = __builtin_ldexpf(2.f * __builtin_sqrtf(a), -se[t]);
-    if (bias != nullptr) {
-      const float* bp = bias + ((size_t)e * d_out + min(jb * 8 + t, d_out - 1)) * 8;
-      for (int c = 0; c < 8; ++c) b = fmaxf(b, fabsf(bp[c]));
-      b *= 2.8284272f;  // at least the norm of the eight
-    }
-#pragma unroll
-    for (int o = 4; o > 0; o >>= 1) {
-      a = fmaxf(a, __shfl_xor(a, o));
-      b = fmaxf(b, __shfl_xor(b, o));
-    }
-    if (t == 0) {
-      norms[(size_t)e * 2 * nb + jb] = a;
-      norms[(size_t)e * 2 * nb + nb + jb] = b;
-    }
-  }
-}
-
-// ---- fp32 blade rows -> split rows ------------------------------------------------------
-// One wave per row, a multivector per lane and pass.
-//
-// The exponent of a slot's hidden row comes from a bound, so that the up product's
-// epilogue can write it before the row's maximum is known.  In Frobenius norms of the
-// complex matrices |M(y_j)| <= |M(W_j)| |M(x)| + |M(b_j)|; the activations do not enlarge a
-// component (sigmoid's stay within 1), and an entry of M(h) is at most its norm.  The
-// bound is some 2^4 above the largest entry in practice, which leaves the parts their 22
-// bits down to 2^-12 of it.
-__global__ __launch_bounds__(256) void split_rows_kernel(const float* __restrict__ x, int N, int d,
-                                                         unsigned char* __restrict__ out,
-                                                         int32_t* __restrict__ row_exp, SplitHidden hid) {
-  const int lane = threadIdx.x & 63, t = blockIdx.x * 4 + (threadIdx.x >> 6);
-  if (t >= N) return;
-  const float* row = x + (size_t)t * d * 8;
-  uint32_t m = 0;
-  for (int i = lane; i < d; i += 64) {
-    float v[8];
-    load8(row + (size_t)i * 8, v);
-    m = max(m, pauli_mag(v));
-  }
-  const int s = split_exp(__builtin_bit_cast(float, wave_max_u32(m)));
-  const int d_pad = (d + 7) & ~7;
-  unsigned char* o = out + (size_t)t * pauli_split_row_bytes(d);
-  float n2 = 0.f;
-  for (int i = lane; i < d_pad; i += 64) {
-    float v[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f}, c0[4], c1[4];
-    if (i < d) load8(row + (size_t)i * 8, v);
-    blade_to_pauli(v, c0, c1);
 #pragma unroll
     for (int c = 0; c < 4; ++c) {
-      const float a = __builtin_ldexpf(c0[c], s), b = __builtin_ldexpf(c1[c], s);
-      n2 += a * a + b * b;
-    }
-    store_split_mv(o, d_pad, i, v, s);
-  }
-  if (hid.k == 0) {
-    if (lane == 0) row_exp[t] = s;
-    if (hid.one_offsets != nullptr && t == 0 && lane < 2) hid.one_offsets[lane] = lane * N;
-    return;
-  }
+      __builtin_amdgcn_sched_barrier(0);
+      uint4 B[2][3];  // (u, -v) for the real part, (v, u) for the imaginary one, of c0 and c1
 #pragma unroll
-  for (int q = 32; q > 0; q >>= 1) n2 += __shfl_xor(n2, q);
-  const float xn = __builtin_ldexpf(__builtin_sqrtf(n2), -s);
-  const int nb = (hid.d_ff + 7) / 8;
-  for (int q = 0; q < hid.k; ++q) {
-    const int e = hid.topk_idx[(size_t)t * hid.k + q];
-    float a = 0.f, b = 0.f;
-    for (int u = lane; u < nb; u += 64) {
-      a = fmaxf(a, hid.norms[(size_t)e * 2 * nb + u]);
-      b = fmaxf(b, hid.norms[(size_t)e * 2 * nb + nb + u]);
-    }
-#pragma unroll
-    for (int u = 32; u > 0; u >>= 1) {
-      a = fmaxf(a, __shfl_xor(a, u));
-      b = fmaxf(b, __shfl_xor(b, u));
-    }
-    if (lane == 0) {
-      // 1.5: |M(b)| = sqrt(2) |b|, and the rounding of the sums behind it
-      float bound = 1.01f * (a * xn) + 1.5f * b;
-      if (hid.act == kActSigmoid) bound = fmaxf(bound, 3.f);
-      const int r = hid.slot_pos[(size_t)t * hid.k + q];
-      row_exp[r] = s;
-      hid.h_exp[r] = bound == INFINITY ? 15 - 128 : split_exp(bound);
-    }
-  }
-}
-
-constexpr int kGmKBlock = 64;  // inputs whose maxima one workgroup of the first launch takes
-
-// geom_matmul, first launch: workgroups [0, wblocks) split the weight rows of a (four
-// channels each); the others take the largest Pauli entry of each column of b over a
-// block of 64 inputs.
-__global__ __launch_bounds__(256) void split_gm_first_kernel(const float* __restrict__ a, const float* __restrict__ b,
-                                                             int M, int K, int N, int wblocks,
-                                                             unsigned char* __restrict__ w, int w_stride,
-                                                             int32_t* __restrict__ col_exp,
-                                                             float* __restrict__ partial,
-                                                             int32_t* __restrict__ offsets) {
-  const int t = threadIdx.x;
-  if ((int)blockIdx.x < wblocks) {
-    const int j = blockIdx.x * 4 + (t >> 6);
-    if (j < M) split_w_channel(a + (size_t)j * K * 8, K, t & 63, w + (size_t)j * w_stride, col_exp + j);
-    return;
-  }
-  __shared__ uint32_t mx[8][32];
-  const int nb = (N + 31) / 32, q = blockIdx.x - wblocks, kb = q / nb, n = (q - kb * nb) * 32 + (t & 31);
-  if (q == 0 && t == 0) {
-    offsets[0] = 0;
-    offsets[1] = N;
-  }
-  uint32_t m = 0;
-  if (n < N) {
-#pragma unroll
-    for (int u = 0; u < kGmKBlock / 8; ++u) {
-      const int k = kb * kGmKBlock + u * 8 + (t >> 5);
-      if (k < K) {
-        float v[8];
-        load8(b + ((size_t)k * N + n) * 8, v);
-        m = max(m, pauli_mag(v));
+      for (int h = 0; h < 2; ++h) {
+        const uint32_t off = h * 2048 + (c >> 1) * 512 + (c & 1) * 8;
+        const float2 w0 = *reinterpret_cast<const float2*>(st + w_rd + off);         // (u, v), c0
+        const float2 w1 = *reinterpret_cast<const float2*>(st + (w_rd ^ 16) + off);  // c1
+        split_operands<0x80008000u, 0u>(B, h, split_flip(w0.x, neg), split_flip(w1.x, neg), split_flip(w0.y, neg),
+                                        split_flip(w1.y, neg));
       }
+      split_accumulate(acc, c, A, B, f & 1 ? -1.f : 1.f);
     }
-  }
-  mx[t >> 5][t & 31] = m;
-  __syncthreads();
-  if (t < 32 && n < N) {
+  };
+
+  const int n = (d_in + kSpK - 1) / kSpK;
+  issue(0);
+  auto steps = [&](auto pairs_tag) __attribute__((always_inline)) {
+    for (int f = 0; f < n; ++f) {
+      split_wait();  // step f may be read and the other stage, read by step f - 1, overwritten
+      if (f + 1 < n) issue(f + 1);
+      compute(f, pairs_tag);
+    }
+  };
+  if (row_end - row0 > 32) steps(std::integral_constant<int, 2>{});
+  else steps(std::integral_constant<int, 1>{});  // the tile's upper half holds no rows
+
 #pragma unroll
-    for (int r = 1; r < 8; ++r) m = max(m, mx[r][t]);
-    partial[(size_t)kb * N + n] = __builtin_bit_cast(float, m);
+  for (int cb = 0; cb < 2; ++cb) {
+    const int j = col0 + wj * 32 + cb * 16 + l16;
+    if (j >= d_out) continue;
+#pragma unroll
+    for (int rb = 0; rb < 4; ++rb)
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const int row = row0 + rb * 16 + wt * 8 + 2 * g + h;  // its halves b = 0, 1 are sums 2 h, 2 h + 1
+        if (row >= row_end) continue;
+        const auto &s0 = acc[rb][2 * cb], &s1 = acc[rb][2 * cb + 1];  // a = 0, 1
+        f32_store_mv<ACT, OUT>(s0[0][2 * h], s0[1][2 * h], s0[0][2 * h + 1], s0[1][2 * h + 1], s1[0][2 * h], s1[1][2 * h],
+                               s1[0][2 * h + 1], s1[1][2 * h + 1], bias, e, row, j, d_out, 0, P_max, Y, Ypre, nullptr);
+      }
   }
 }
 
-// geom_matmul, second launch: b (K, N) blade -> split rows of its transpose.  Tiles of 32
-// columns x 8 inputs through LDS, so the reads (32 consecutive columns of one input) and
-// the writes (one block of a half-row, 128 bytes) are contiguous.
-__global__ __launch_bounds__(256) void split_gm_rows_kernel(const float* __restrict__ b, int K, int N,
-                                                            const float* __restrict__ partial,
-                                                            unsigned char* __restrict__ x,
-                                                            int32_t* __restrict__ row_exp) {
-  __shared__ uint2 tile[32][2][2][8];  // [column][b][hi, lo][input]
-  __shared__ int se[32];
-  const int n0 = blockIdx.x * 32, k0 = blockIdx.y * 8, t = threadIdx.x;
-  if (t < 32) {
-    const int n = n0 + t;
-    uint32_t m = 0;
-    if (n < N)
-      for (int kb = 0; kb * kGmKBlock < K; ++kb)
-        m = max(m, __builtin_bit_cast(uint32_t, partial[(size_t)kb * N + n]));
-    se[t] = split_exp(__builtin_bit_cast(float, m));
-    if (k0 == 0 && n < N) row_exp[n] = se[t];
-  }
-  const int kk = t >> 5, nn = t & 31;
-  float v[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f}, c0[4], c1[4];
-  if (k0 + kk < K && n0 + nn < N) load8(b + ((size_t)(k0 + kk) * N + n0 + nn) * 8, v);
-  blade_to_pauli(v, c0, c1);
-  __syncthreads();
-  split4_f16(c0, se[nn], tile[nn][0][0][kk], tile[nn][0][1][kk]);
-  split4_f16(c1, se[nn], tile[nn][1][0][kk], tile[nn][1][1][kk]);
-  __syncthreads();
-  // thread: column t / 8, half-row b, hi or lo part, its half: 32 bytes
-  const int wn = t >> 3, wb = (t >> 2) & 1, part = (t >> 1) & 1, hf = t & 1;
-  if (n0 + wn < N) {  // (the block's padding inputs were read as zero)
-    const int dv = 2 * ((K + 7) / 8 * 8);
-    const uint2* s = &tile[wn][wb][part][hf * 4];
-    uint4* dst = reinterpret_cast<uint4*>(x + ((size_t)(n0 + wn) * 2 + wb) * dv * 8 + (size_t)(k0 / 8) * 128 +
-                                          part * 64 + hf * 32);
-    dst[0] = make_uint4(s[0].x, s[0].y, s[1].x, s[1].y);
-    dst[1] = make_uint4(s[2].x, s[2].y, s[3].x, s[3].y);
-  }
+template <int ACT, int OUT>
+int launch_split(const float* x, int x_rows, const int32_t* gather, int P_max, const float* w, const float* bias,
+                 const int32_t* offsets, int E, int d_in, int d_out, float* y, float* y_pre, hipStream_t st) {
+  const int n_xcd = 8;  // workgroups go to the XCDs round robin (8 on MI355X)
+  const long long tiles = ((long long)(P_max + kSpT - 1) / kSpT + E) * ((d_out + kSpN - 1) / kSpN);  // at most
+  pauli_split_kernel<ACT, OUT><<<(unsigned)((tiles + n_xcd - 1) / n_xcd * n_xcd), 256, 0, st>>>(
+      x, (uint64_t)x_rows * d_in * 32, gather, w, bias, offsets, E, d_in, d_out, P_max, n_xcd, y, y_pre);
+  return check_launch("pauli_split");
 }
 
 }  // namespace
+
+// One product: from 32 inputs and about 100 tiles of 64 x 64 on.  A tile's steps are a chain of
+// some 2.9 us per eight inputs whether one or two share a CU, and fewer tiles leave CUs idle that
+// the fp32 MFMA kernel's 16 x 32 tiles use (geom_matmul, us, split / fp32 MFMA: 64 tiles, K = 32 26 / 21, 64
+// 37 / 30, 128 61 / 49, 512 196 / 151; 128 tiles 28 / 29, 41 / 46, 67 / 76, 202 / 291; 512 tiles 51 / 72, 76 / 112, 118 / 218,
+// 378 / 1060; K = 16: 128 tiles 22 / 19, 512 41 / 47).
+bool pauli_split_pays(long long P, int d_in, int d_out) { return d_in >= 32 && P * d_out >= 100LL * 64 * 64; }
+
+// A layer's two products together, whose smaller one may fill less (layer calls, us, split / fp32 MFMA: d =
+// 128, F = 512, E = 32: 1024 rows 250 / 191, 2048 277 / 327, 8192 525 / 940; d = 64, F = 256, E = 8: 2048 rows
+// 143 / 99, 4096 155 / 169, 8192 187 / 274; d = 64, F = 256, E = 32: 2048 141 / 107, 4096 156 / 177; d = 100, F = 300,
+// E = 12: 1024 171 / 115, 2048 172 / 190, 4096 195 / 300; d = F = 128, E = 64: 1024 83 / 81, 2048 118 / 132; d =
+// 256, F = 1024, E = 64: 1024 453 / 701; d = 32, F = 64, E = 8: 8192 68 / 63).
+bool pauli_split_layer_pays(long long P, int E, int d, int F) {
+  const int m = std::min(d, F);
+  return m >= 64 && P * m >= 60LL * 64 * 64 && P >= 16LL * E;
+}
+
+bool pauli_split_fits(int E, long long x_rows, bool gathered, int d_in, int d_out) {
+  const uint64_t lim = (uint64_t)1 << 31;
+  return E >= 1 && E <= kSpMaxExperts && (uint64_t)(d_in + kSpK) * d_out * 64 < lim &&
+         (gathered ? (uint64_t)x_rows * d_in * 32 < lim : (uint64_t)kSpT * d_in * 32 < lim);
+}
+
+int pauli_split_linear(const float* x, int x_rows, const int32_t* gather, int P_max, const float* w, const float* bias,
+                       const int32_t* offsets, int E, int d_in, int d_out, int act, float* y, int y_layout, float* y_pre,
+                       hipStream_t stream) {
+  if (y_layout == kF32OutBlade)
+    return launch_split<kActNone, kF32OutBlade>(x, x_rows, gather, P_max, w, bias, offsets, E, d_in, d_out, y, nullptr, stream);
+  if (y_layout == kF32OutBladeT)
+    return launch_split<kActNone, kF32OutBladeT>(x, x_rows, gather, P_max, w, bias, offsets, E, d_in, d_out, y, nullptr, stream);
+#define YGG_SU(A) \
+  return launch_split<A, kF32OutPauliRows>(x, x_rows, gather, P_max, w, bias, offsets, E, d_in, d_out, y, y_pre, stream)
+  switch (act) {
+    case kActNone: YGG_SU(kActNone);
+    case kActGelu: YGG_SU(kActGelu);
+    case kActRelu: YGG_SU(kActRelu);
+    default: YGG_SU(kActSigmoid);
+  }
+#undef YGG_SU
+}
+
 }  // namespace ygg
-
-using namespace ygg;
-
-int ygg::pauli_split_weights(const float* w, int E, int d_out, int d_in, const float* bias, void* out, int32_t* col_exp,
-                             float* norms, hipStream_t stream) {
-  split_weights_kernel<<<(unsigned)(E * ((d_out + 7) / 8)), 256, 0, stream>>>(
-      w, d_out, d_in, bias, static_cast<unsigned char*>(out), col_exp, norms);
-  return check_launch("pauli_split_weights");
-}
-
-int ygg::pauli_split_rows(const float* x, int N, int d, void* out, int32_t* row_exp, const SplitHidden& hid,
-                          hipStream_t stream) {
-  if (N == 0) return 0;
-  split_rows_kernel<<<(unsigned)((N + 3) / 4), 256, 0, stream>>>(x, N, d, static_cast<unsigned char*>(out), row_exp,
-                                                                 hid);
-  return check_launch("pauli_split_rows");
-}
-
-size_t ygg::pauli_split_gm_partials(int K, int N) { return (size_t)((K + kGmKBlock - 1) / kGmKBlock) * N; }
-
-int ygg::pauli_split_gm_operands(const float* a, const float* b, int M, int K, int N, void* w, int32_t* col_exp,
-                                 void* x, int32_t* row_exp, float* partial, int32_t* offsets, hipStream_t stream) {
-  const int wblocks = (M + 3) / 4;
-  const unsigned bblocks = (unsigned)(((N + 31) / 32) * ((K + kGmKBlock - 1) / kGmKBlock));
-  split_gm_first_kernel<<<wblocks + bblocks, 256, 0, stream>>>(a, b, M, K, N, wblocks, static_cast<unsigned char*>(w),
-                                                               (int)pauli_split_row_bytes(K), col_exp, partial,
-                                                               offsets);
-  if (check_launch("pauli_split_gm_first")) return -1;
-  split_gm_rows_kernel<<<dim3((unsigned)((N + 31) / 32), (unsigned)((K + 7) / 8)), 256, 0, stream>>>(
-      b, K, N, partial, static_cast<unsigned char*>(x), row_exp);
-  return check_launch("pauli_split_gm_rows");
-}

@@ -8,9 +8,7 @@
 namespace ygg {
 
 enum PauliIn : int { kInBladeGather = 0, kInPauliRows = 1 };
-// split products (fp32 operands as two fp16 parts) write fp32 blade rows, blade columns
-// (d_out, P), or the split rows of the next product
-enum PauliOut : int { kOutPauliRows = 0, kOutBlade = 1, kOutBladeT = 2, kOutSplitRows = 3 };
+enum PauliOut : int { kOutPauliRows = 0, kOutBlade = 1 };
 
 struct PauliTileInfo {
   int e, row0, row_end, col0;

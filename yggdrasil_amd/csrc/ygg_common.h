@@ -187,57 +187,17 @@ int pauli_f32_up_routed(const float* x, const float* logits, int N, int E, int k
                         const float* w, const float* bias, int d_in, int d_out, int act, float* y_pauli,
                         float* y_pre, hipStream_t stream);
 
-// fp32 Pauli products on the fp16 MFMA units (pauli_gemm.hip, conversions in
-// pauli_split.hip): operands as two fp16 parts of values scaled by a power of two per
-// row and per output channel.  Split rows: two half-rows (b = 0, 1) per row, each
-// pauli_split_width(d) x 4 fp16: per block of eight multivectors (the last one padded
-// with zeros) the hi parts (c0 re, c0 im, c1 re, c1 im each), then the lo parts.  Split
-// weights: per (expert, output channel) the same blocks as format 3's 32-byte pair
-// records.  An exponent s says that the stored values are the true ones times 2^s.
-__host__ __device__ inline int pauli_split_width(int d) { return 2 * ((d + 7) / 8 * 8); }
-__host__ __device__ inline size_t pauli_split_row_bytes(int d) { return (size_t)pauli_split_width(d) * 16; }
-// whether the split product is the faster and no less exact one, and whether the sizes fit
-// the kernel's 32-bit offsets and its two chunks per tile
-bool pauli_split_pays(long long P, int E, int d_in, int d_out);
-bool pauli_split_fits(int E, int P_max, int x_rows, bool gathered, int d_in, int d_out, bool transposed);
-// one expert, no bias, output transposed: y_t (d_out, P_max, 8) blade order
-int pauli_split_linear_t(const void* x, const int32_t* row_exp, int P_max, const void* w, const int32_t* col_exp,
-                         const int32_t* offsets, int d_in, int d_out, float* y_t, hipStream_t stream);
-// grouped product of split rows in place: y (P_max, d_out, 8) fp32 blade order
-int pauli_split_linear(const void* x, const int32_t* row_exp, int P_max, const void* w, const int32_t* col_exp,
-                       const float* bias, const int32_t* offsets, int E, int d_in, int d_out, float* y,
+// fp32 Pauli products of enough rows on the bf16 MFMA units (pauli_split.hip), from the operands
+// of pauli_f32.hip: whether a product, or a layer's two, are faster there, whether the sizes fit the kernel's
+// 32-bit offsets, and the product itself (y_layout as pauli_f32.hip's kF32Out*: Pauli rows
+// with the activation, y_pre taking the blade rows before it when not NULL; blade rows;
+// blade columns (d_out, P_max)).
+bool pauli_split_pays(long long P, int d_in, int d_out);
+bool pauli_split_layer_pays(long long P, int E, int d, int F);
+bool pauli_split_fits(int E, long long x_rows, bool gathered, int d_in, int d_out);
+int pauli_split_linear(const float* x, int x_rows, const int32_t* gather, int P_max, const float* w, const float* bias,
+                       const int32_t* offsets, int E, int d_in, int d_out, int act, float* y, int y_layout, float* y_pre,
                        hipStream_t stream);
-// an expert's up product: rows gathered from x_rows split rows (row_exp per product row),
-// activation, h as split rows with the given exponents, and h_pre (when not NULL) the fp32
-// blade rows before the activation
-int pauli_split_up(const void* x, int x_rows, const int32_t* row_exp, const int32_t* gather, int P_max, const void* w,
-                   const int32_t* col_exp, const float* bias, const int32_t* offsets, int E, int d_in, int d_out,
-                   int act, void* h, const int32_t* h_exp, float* h_pre, hipStream_t stream);
-// prepared fp32 Pauli weights (format 4) -> split weights and col_exp (E d_out); norms (when
-// not NULL): per (expert, block of 8 channels) the largest norm of a channel's weights and
-// of its bias, 2 x pauli_split_norm_blocks(d_out) floats per expert
-inline int pauli_split_norm_blocks(int d_out) { return (d_out + 7) / 8; }
-int pauli_split_weights(const float* w, int E, int d_out, int d_in, const float* bias, void* out, int32_t* col_exp,
-                        float* norms, hipStream_t stream);
-// fp32 blade rows (N, d) -> split rows.  Exponents: row_exp[t] (k = 0), or for each of
-// the token's k slots at its product row, row_exp[slot_pos[t k + s]], and in h_exp there
-// an exponent for the hidden rows of act(W x + b), from a bound on their size
-struct SplitHidden {
-  int k = 0, d_ff = 0, act = 0;
-  const int32_t* slot_pos = nullptr;
-  const int32_t* topk_idx = nullptr;
-  const float* norms = nullptr;  // of pauli_split_weights
-  int32_t* h_exp = nullptr;
-  int32_t* one_offsets = nullptr;  // k = 0: when set, takes the one-expert offsets {0, N}
-};
-int pauli_split_rows(const float* x, int N, int d, void* out, int32_t* row_exp, const SplitHidden& hid,
-                     hipStream_t stream);
-// geom_matmul's operands: a (M, K) blade -> split weights and col_exp, b (K, N) blade ->
-// split rows of its transpose and row_exp, and the one-expert offsets {0, N};
-// `partial` holds pauli_split_gm_partials(K, N) floats
-size_t pauli_split_gm_partials(int K, int N);
-int pauli_split_gm_operands(const float* a, const float* b, int M, int K, int N, void* w, int32_t* col_exp, void* x,
-                            int32_t* row_exp, float* partial, int32_t* offsets, hipStream_t stream);
 
 // decode-shape int8 products (clifford_gemm.hip): whether (P_max rows, E
 // experts, format) takes the weight-streaming kernel, its number of K splits
@@ -308,25 +268,18 @@ size_t weight_grad_pauli_workspace_bytes(int P_max, int E, int d_in, int d_out);
 int weight_grad_pauli(const float* dy_pauli, const float* a_pauli, const int32_t* gather, const int32_t* offsets,
                       int P_max, int E, int d_in, int d_out, float* dW, float* db, void* workspace,
                       hipStream_t stream);
-// The same on the fp16 MFMA units from split rows (pauli_split.hip) of dy and a with
-// their exponents (a's per source row); same workspace.
-bool weight_grad_split_fits(int a_rows, bool gathered, int d_in, int d_out);
-int weight_grad_split(const void* dy, const int32_t* dy_exp, const void* a, int a_rows, const int32_t* a_exp,
-                      const int32_t* gather, const int32_t* offsets, int P_max, int E, int d_in, int d_out, float* dW,
-                      float* db, void* workspace, hipStream_t stream);
-// The activation's forward (g NULL) or backward (of g at h) over P blade rows of d
-// multivectors, as split rows.
-int activation_split_rows(const float* h, const float* g, size_t P, int d, int act, void* out, int32_t* row_exp,
-                          hipStream_t stream);
+// The same on the bf16 MFMA units, same operands and workspace (a_rows: rows of A), where that is faster
+bool weight_grad_split_pays(long long P, int E, long long a_rows, bool gathered, int d_in, int d_out);
+int weight_grad_split(const float* dy_pauli, const float* a_pauli, int a_rows, const int32_t* gather,
+                      const int32_t* offsets, int P_max, int E, int d_in, int d_out, float* dW, float* db, void* workspace,
+                      hipStream_t stream);
 // (out may alias g; out and out_pauli -- fp32 Pauli rows -- are each optional)
 int activation_backward(const float* h, const float* g, size_t n_mv, int act, float* out, float* out_pauli,
                         hipStream_t stream);
 int activation_forward(const float* h, size_t n_mv, int act, float* out, float* out_pauli, hipStream_t stream);
 int fill_zero_f32(float* p, size_t n, hipStream_t stream);  // n floats at p set to zero
-// dy goes out as blade rows, fp32 Pauli rows and / or split rows with their exponents
 int combine_backward(const float* dout, const float* y_sorted, int N, int k, int d, const float* topk_w,
-                     const int32_t* slot_pos, float* dy_sorted, float* dy_pauli, float* dtopk_w, hipStream_t stream,
-                     void* dy_split = nullptr, int32_t* dy_exp = nullptr);
+                     const int32_t* slot_pos, float* dy_sorted, float* dy_pauli, float* dtopk_w, hipStream_t stream);
 int dispatch_backward(const float* dxs, int N, int k, int d, const int32_t* slot_pos, const float* residual_grad,
                       float* dx, hipStream_t stream);
 

@@ -38,8 +38,9 @@ class MoEHLMConfig:
     top_k       k (<= 8)
     activation  'gelu' | 'relu' | 'sigmoid' (grade-wise)
     dtype       activation dtype: torch.float32 or torch.bfloat16
-    weight_format  fp32 layers: 'pauli_f32' (the default: complex 2x2 weights on the fp32 MFMA
-                units, 32 multiply-adds per multivector pair) or 'f32' (8x8 L(w) blocks on the
+    weight_format  fp32 layers: 'pauli_f32' (the default: complex 2x2 weights, 32
+                multiply-adds per multivector pair, on the fp32 MFMA units or, for enough rows, on the
+                bf16 ones with every value as three bf16 parts, which hold its 24 bits) or 'f32' (8x8 L(w) blocks on the
                 vector units, 64); bf16 layers: 'pauli' (the default when d_model and d_ff are
                 even), 'bf16' (8x8 L(w) blocks), 'int8' (per-output-channel int8, L(w) blocks) or
                 'int8_pauli' (per-output-channel int8 of the complex 2x2 weights: the one-launch

@@ -78,7 +78,8 @@ def geom_matmul(a: torch.Tensor, b: torch.Tensor, *, workspace: torch.Tensor | N
     """``out[m, n] = sum_k gp(a[m, k], b[k, n])`` (fp32, blade order).
 
     Drop-in for ``rune.ops.batched.geom_matmul`` (``rune/ops/batched.py:320-344``):
-    one fp32 Pauli MFMA product with ``a`` as the weight.  ``workspace`` (uint8,
+    one fp32 Pauli product with ``a`` as the weight, on the fp32 MFMA units or, from some 100
+    tiles of 64 x 64 on, the bf16 ones (three bf16 parts a value: its 24 bits).  ``workspace`` (uint8,
     at least :func:`geom_matmul_workspace_bytes`) and ``out`` may be given to reuse
     buffers across calls; otherwise they are allocated here.
     """

@@ -262,3 +262,19 @@ def test_layer_with_non_finite_rows(k):
         for e in range(E):
             assert torch.isfinite(b[e]).all() == (e not in hit)
             assert e in hit or torch.equal(a[e], b[e])
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("name,shape", [("router_weight", (3, 4)), ("router_weight", (4, 3)), ("router_bias", (3,)),
+                                        ("w_up", (4, 8, 10, 8)), ("w_down", (4, 16, 16, 8)), ("b_up", (3, 16, 8)),
+                                        ("b_down", (4, 14, 8))])
+def test_replaced_parameters_of_another_shape_are_refused(name, shape, dtype):
+    """A parameter replaced by one of another shape raises before its pointer reaches a kernel."""
+    import yggdrasil_amd
+
+    layer = yggdrasil_amd.CliffordMoELayer(
+        yggdrasil_amd.MoEHLMConfig(d_model=10, d_ff=16, n_experts=4, top_k=2, dtype=dtype), device="cuda")
+    setattr(layer, name, torch.nn.Parameter(torch.zeros(shape, device="cuda")))
+    say(f"{name} {shape}")
+    with torch.no_grad(), pytest.raises(ValueError, match=name):
+        layer.moe_forward(torch.randn(1, 5, 10, 8, device="cuda").to(dtype))

@@ -163,6 +163,10 @@ class CliffordMoELayer(nn.Module):
     def prepare(self):
         """Build the device weight layouts (done lazily; redone when parameters change)."""
         fmt = self.cfg.weight_format
+        E, d, F = self.cfg.n_experts, self.cfg.d_model, self.cfg.d_ff
+        for name, want in (("w_up", (E, F, d, 8)), ("b_up", (E, F, 8)), ("w_down", (E, d, F, 8)), ("b_down", (E, d, 8))):
+            if tuple(getattr(self, name).shape) != want:  # (replaced or parametrized: the kernels take the shapes of cfg)
+                raise ValueError(f"{name} must be {want}, got {tuple(getattr(self, name).shape)}")
         head = None
         if self.head_weight is not None:
             head = self.head_weight.detach().float().contiguous()
@@ -228,6 +232,10 @@ class CliffordMoELayer(nn.Module):
                 rw = rw.float().contiguous()
             if rb.dtype != torch.float32 or not rb.is_contiguous():
                 rb = rb.float().contiguous()
+            if tuple(rw.shape) != (E, 4):
+                raise ValueError(f"router_weight must be ({E}, 4), got {tuple(rw.shape)}")
+            if tuple(rb.shape) != (E,):
+                raise ValueError(f"router_bias must be ({E},), got {tuple(rb.shape)}")
         ops._dev(x, logits, residual, rw, rb, prep["b_up"], prep["b_down"])
         out, routing = ops.layer_forward(x, N, cfg.top_k, prep["w_up"], prep["w_down"], prep["b_up"], prep["b_down"],
                                          cfg.activation, logits, rw, rb, residual, ws, ws_bytes)

@@ -389,3 +389,19 @@ def test_bf16_layer_workspace_grows_with_the_batch():
     for d, F, E, k in ((128, 512, 32, 2), (256, 1024, 64, 2), (64, 128, 4, 1), (100, 302, 12, 3)):
         sizes = [L.ygg_moe_workspace_bytes(N, d, F, E, k, 1, 3) for N in range(1, 2100)]
         assert all(a <= b for a, b in zip(sizes, sizes[1:])), (d, F, E, k)
+
+
+def test_aux_loss_of_given_counts():
+    """The balance loss takes the counts that last_routing holds, whatever put them there: other types and
+    devices than a call's, and the attribute of a layer saved as a whole when it was a plain one."""
+    import yggdrasil_amd
+
+    layer = yggdrasil_amd.CliffordMoELayer(yggdrasil_amd.MoEHLMConfig(d_model=2, d_ff=2, n_experts=4, top_k=1))
+    assert layer.aux_loss().item() == 0.0
+    want = ((torch.tensor([0.1, 0.2, 0.3, 0.4]) - 0.25) ** 2).sum().item()
+    for counts in (torch.tensor([1, 2, 3, 4]), torch.tensor([1.0, 2.0, 3.0, 4.0]), torch.tensor([1, 2, 3, 4], dtype=torch.int32)):
+        layer.last_routing = dict(counts=counts)
+        assert layer.aux_loss().item() == pytest.approx(want, rel=1e-6)
+    del layer.__dict__["_last_routing"]
+    layer.__dict__["last_routing"] = dict(counts=torch.tensor([1, 2, 3, 4]))
+    assert layer.aux_loss().item() == pytest.approx(want, rel=1e-6)

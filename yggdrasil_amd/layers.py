@@ -144,7 +144,7 @@ class CliffordMoELayer(nn.Module):
     @property
     def last_routing(self):
         """The last call's ``topk_idx``, ``topk_w``, ``counts`` and ``offsets`` (None before the first)."""
-        r = self.__dict__.get("_last_routing")
+        r = self.__dict__.get("_last_routing", self.__dict__.get("last_routing"))  # (the second: layers saved before it)
         if isinstance(r, ops.LayerRouting):  # the tensors are made when they are asked for
             r = self.__dict__["_last_routing"] = r.arrays()
         return r
@@ -290,7 +290,12 @@ class CliffordMoELayer(nn.Module):
         """
         if self.last_routing is None:
             return torch.zeros((), device=self.w_up.device)
-        return ops.balance_loss(self.last_routing["counts"])
+        counts = self.last_routing["counts"]
+        if counts.is_cuda and counts.dtype == torch.int32 and counts.is_contiguous():
+            return ops.balance_loss(counts)
+        c = counts.float()  # counts that a caller has put there
+        f = c / (c.sum() + 1e-12)
+        return ((f - 1.0 / self.cfg.n_experts) ** 2).sum()
 
 
 class _MoEFunction(torch.autograd.Function):

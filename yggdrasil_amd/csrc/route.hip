@@ -390,15 +390,15 @@ using namespace ygg;
 namespace {
 // Whether a batch routes in one workgroup: its time grows with the tokens (16 at a time)
 // and the logits a lane holds, the two launches' does not (one / two, us: E = 8: 256 tokens
-// 6.9 / 8.0, 512 10.8 / 8.4, 1024 19.0 / 8.4; E = 32: 128 8.4 / 9.5, 256 13.0 / 9.6; E = 64:
-// 64 7.4 / 7.6, 128 9.2 / 8.1, 1024 43.3 / 8.7).
-bool route_in_one(int N, int E) { return N <= kSmallMaxN && N * ((E + 7) / 8 + 2) <= 900; }
+// 6.9 / 8.2, 384 8.8 / 8.3, 1024 19.0 / 8.4; E = 16: 256 8.3 / 8.4, 384 10.9 / 8.2; E = 32: 192 8.1 / 8.4, 256
+// 10.1 / 8.5; E = 64: 128 7.6 / 8.0, 192 11.0 / 8.0, 1024 43.5 / 8.7).
+bool route_in_one(int N, int E) { return N <= kSmallMaxN && N * ((E + 7) / 8 + 4) <= 1750; }
 
 // ... and the logits with it, while the workgroup's reading of x is short beside a launch of
-// its own (one / three launches, us, measured while both loaded a row in smaller batches and
-// the map after it: E = 8, d = 64: 128 tokens 6.0 / 6.5, 256 8.8 / 8.0; d = 256: 32 tokens
-// 5.9 / 7.0, 64 7.5 / 7.1, 256 19.1 / 9.3).
-bool energy_in_one(int N, int E, int d) { return route_in_one(N, E) && (long long)N * d <= 13000; }
+// its own (layer calls, one / separate, us: E = 8: d = 64: 128 tokens 15.0 / 15.9, 256 18.1 / 17.4; d = 128: 64
+// 16.0 / 17.0, 128 17.5 / 17.5; d = 256: 64 20.0 / 20.9, 128 22.5 / 21.4; d = 32: 256 17.3 / 17.0; E = 32: d = 128: 128
+// 18.5 / 18.7; d = 256: 64 20.7 / 21.5, 128 23.6 / 22.4; E = 64: d = 128: 128 20.3 / 21.3; d = 256: 64 21.5 / 22.6).
+bool energy_in_one(int N, int E, int d) { return route_in_one(N, E) && N <= 192 && (long long)N * d <= 17000; }
 
 // The grade-energy logits of energy_logits (the sums of the one-workgroup kernel, in its
 // order) for batches that do not route in one workgroup: eight lanes per token.

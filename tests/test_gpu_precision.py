@@ -278,3 +278,15 @@ def test_replaced_parameters_of_another_shape_are_refused(name, shape, dtype):
     say(f"{name} {shape}")
     with torch.no_grad(), pytest.raises(ValueError, match=name):
         layer.moe_forward(torch.randn(1, 5, 10, 8, device="cuda").to(dtype))
+
+
+def test_weight_preparation_of_any_aligned_floats():
+    """Weights that are a view into a flat buffer, four bytes off: both layouts as of an aligned copy."""
+    from yggdrasil_amd import ops
+
+    flat = torch.randn(3 * 37 * 50 * 8 + 1, device="cuda")
+    w = flat[1:].view(3, 37, 50, 8)
+    assert w.data_ptr() % 16 == 4
+    say("weights four bytes off")
+    assert torch.equal(ops.prepare_weights(w, "pauli_f32").data, ops.prepare_weights(w.clone(), "pauli_f32").data)
+    assert torch.equal(ops.prepare_adjoint_weights(w).data, ops.prepare_adjoint_weights(w.clone()).data)

@@ -466,7 +466,8 @@ __global__ __launch_bounds__(256) void pauli_f32_prep_adjoint_kernel(const float
   if (n >= (size_t)E * d_out * d_in) return;
   const int i = (int)(n % d_in);
   const size_t ej = n / d_in;
-  const float4 p0 = reinterpret_cast<const float4*>(W + n * 8)[0], p1 = reinterpret_cast<const float4*>(W + n * 8)[1];
+  typedef float f4_t __attribute__((ext_vector_type(4), aligned(4)));  // W: any aligned floats
+  const f4_t p0 = reinterpret_cast<const f4_t*>(W + n * 8)[0], p1 = reinterpret_cast<const f4_t*>(W + n * 8)[1];
   const float x[8] = {0.5f * p0.x, 0.5f * p0.y, 0.5f * p0.z, 0.5f * p0.w, 0.5f * p1.x, 0.5f * p1.y, 0.5f * p1.z, 0.5f * p1.w};
   float c0[4], c1[4];
   blade_to_pauli(x, c0, c1);  // c0 = (M00, M10), c1 = (M01, M11)

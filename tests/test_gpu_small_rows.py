@@ -1,5 +1,5 @@
-"""bf16 Pauli layers of few rows (products that stream the weights, K ranges of the down product) and the
-routing's paths by batch size."""
+"""bf16 Pauli layers of few rows (products that stream the weights), the routing's paths by batch size, weight
+gradients of few rows and int8 layers of more than decode size."""
 
 import numpy as np
 import pytest
@@ -14,16 +14,14 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("N,d,F,E,k,act", [
     (1, 2, 2, 1, 1, "gelu"),        # one input pair, one column
     (3, 30, 34, 3, 2, "relu"),      # chunks of 8 inputs with tails, columns off 32
-    (17, 66, 530, 7, 3, "gelu"),    # two and more row tiles, K ranges with a short last one
-    (40, 520, 72, 2, 1, "sigmoid"),  # up contraction past the activations' register range
+    (17, 66, 530, 7, 3, "gelu"),    # two and more row tiles, a contraction of many rounds of the ring
+    (40, 520, 72, 2, 1, "sigmoid"),  # a long up contraction
     (640, 36, 1030, 64, 2, "gelu"),  # the largest row count, empty and many experts
     (320, 64, 300, 5, 4, "none"),
 ])
 def test_layer(N, d, F, E, k, act):
     import yggdrasil_amd
 
-    if act == "none":
-        act = "relu"
     g = np.random.default_rng(N + F)
     x = bf16_round(g.standard_normal((N, d, 8)).astype(np.float32))
     lg = g.standard_normal((N, E)).astype(np.float32)
@@ -32,15 +30,23 @@ def test_layer(N, d, F, E, k, act):
     wd = bf16_round((g.standard_normal((E, d, F, 8)) / np.sqrt(8 * F)).astype(np.float32))
     bu, bd = ((0.1 * g.standard_normal(s)).astype(np.float32) for s in ((E, F, 8), (E, d, 8)))
     res = bf16_round(g.standard_normal((N, d, 8)).astype(np.float32))
-    cfg = yggdrasil_amd.MoEHLMConfig(d_model=d, d_ff=F, n_experts=E, top_k=k, activation=act, dtype=torch.bfloat16,
-                                     weight_format="pauli", router="logits")
-    layer = yggdrasil_amd.CliffordMoELayer(cfg, device="cuda")
-    layer.load_reference_weights(w_up=wu, b_up=bu, w_down=wd, b_down=bd)
     say(f"few rows N={N} d={d} F={F} E={E} k={k} {act}")
-    out = layer.moe_forward(torch.from_numpy(x).cuda().bfloat16()[None], logits=torch.from_numpy(lg).cuda(),
-                            residual=torch.from_numpy(res).cuda().bfloat16()[None])[0]
-    idx = layer.last_routing["topk_idx"].cpu().numpy()
-    w = layer.last_routing["topk_w"].cpu().numpy()
+    xt, lt, rt = torch.from_numpy(x).cuda().bfloat16(), torch.from_numpy(lg).cuda(), torch.from_numpy(res).cuda().bfloat16()
+    if act == "none":  # the operator takes it, a layer's configuration does not
+        from yggdrasil_amd import ops
+
+        wt = [ops.prepare_weights(torch.from_numpy(v).cuda(), "pauli") for v in (wu, wd)]
+        bt = [ops.prepare_bias(torch.from_numpy(v).cuda()) for v in (bu, bd)]
+        out, routing = ops.moe_forward(xt, k, wt[0], wt[1], bt[0], bt[1], act, logits=lt, residual=rt)
+    else:
+        cfg = yggdrasil_amd.MoEHLMConfig(d_model=d, d_ff=F, n_experts=E, top_k=k, activation=act, dtype=torch.bfloat16,
+                                         weight_format="pauli", router="logits")
+        layer = yggdrasil_amd.CliffordMoELayer(cfg, device="cuda")
+        layer.load_reference_weights(w_up=wu, b_up=bu, w_down=wd, b_down=bd)
+        out = layer.moe_forward(xt[None], logits=lt, residual=rt[None])[0]
+        routing = layer.last_routing
+    idx = routing["topk_idx"].cpu().numpy()
+    w = routing["topk_w"].cpu().numpy()
     ref = dense.moe_layer(x, idx, w, wu, bu, wd, bd, act, residual=res)
     assert normwise_err(out.float().cpu().numpy(), ref) < TOL_BF16
 
@@ -118,8 +124,8 @@ def test_adjoint_preparation_and_balance_loss():
     (160, 150, 70, 2, 2, "gelu"),
 ])
 def test_int8_layer_of_enough_rows(N, d, F, E, k, act):
-    """int8 weights in whole-number fp16 products: the layer on the dequantized weights (x, weights exact; h rounded
-    to 11 bits, y and the output to bf16), tokens over many binades, an expert without rows, a token of zeros."""
+    """int8 weights: the layer on the dequantized weights (x and weights exact; h, y and the output rounded to bf16),
+    tokens over many binades, an expert without rows, a token of zeros."""
     import yggdrasil_amd
 
     g = np.random.default_rng(N + F)

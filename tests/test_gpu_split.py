@@ -1,12 +1,10 @@
-"""fp32 products on the fp16 MFMA units (operands as two fp16 parts) against float64.
+"""fp32 products on the bf16 MFMA units (operands as three bf16 parts) against float64.
 
-The parts hold 22 bits of a value scaled by its row's (or output channel's) power of
-two, and the sums are fp32.  Error model of an output element: each of the two operands
-is off by at most 2^-23 of itself plus 2^-39 of its row's largest entry, lo * lo (at most
-2^-22 of the product) is left out, and the fp32 accumulators round 3 K / 8 times (K = 4 d_in
-real terms, in blocks of eight) by 2^-24 of partial sums of random terms.  In the 2-norm that
-stays below (2^-22 + 2^-24 sqrt(3 K / 16)) of the result: 6.6e-7 for d_in = 128, 1.1e-6 for
-512; the bound used is 2e-6.
+The parts hold the 24 bits of a value.  Error model of an output element: the products of parts that are
+left out are at most 2^-23 of a product, and the sums are fp32, one rounding of a full sum per eight inputs
+and those of the small sums, 2^-24 of partial sums of random terms.  In the 2-norm that stays below
+(2^-23 + 2^-24 sqrt(d_in / 8)) of the result: 3.6e-7 for d_in = 128, 6e-7 for 512; the bound used is 2e-6, which
+the fp32 MFMA units' sums (4 d_in terms in a chain of pairs) meet too.
 """
 
 import numpy as np
@@ -36,9 +34,17 @@ def _truth(a, b):
     return np.transpose(dense.linear(np.transpose(b, (1, 0, 2)), a), (1, 0, 2))
 
 
-@pytest.mark.parametrize("M,K,N", [(64, 128, 6400), (65, 129, 6333), (130, 136, 3300), (513, 143, 800), (66, 255, 6300)])
+def _split_product(rows, d_in, d_out):
+    from yggdrasil_amd._native import lib
+
+    return lib().ygg_f32_product_split(rows, d_in, d_out) == 1
+
+
+@pytest.mark.parametrize("M,K,N", [(64, 128, 6400), (65, 129, 6333), (130, 136, 3300), (513, 143, 800), (66, 255, 6300),
+                                   (100, 32, 4100), (13, 33, 31600), (8191, 41, 51)])
 def test_geom_matmul_sizes(M, K, N):
     """Sizes from which the split product runs, on and off its tiles (64 x 64, blocks of 8 inputs)."""
+    assert _split_product(N, K, M)
     g = np.random.default_rng(M + K + N)
     a = (g.standard_normal((M, K, 8)) / np.sqrt(8 * K)).astype(np.float32)
     b = g.standard_normal((K, N, 8)).astype(np.float32)
@@ -51,6 +57,7 @@ def test_geom_matmul_scales_and_non_finite():
     with an infinity or NaN: those give non-finite rows, and every other row is as without them."""
     g = np.random.default_rng(4)
     M, K, N = 70, 130, 6000
+    assert _split_product(N, K, M)
     a = (g.standard_normal((M, K, 8)) / np.sqrt(8 * K)).astype(np.float32)
     b = g.standard_normal((K, N, 8)).astype(np.float32)
     a *= np.ldexp(1.0, g.integers(-60, 40, (M, 1, 1))).astype(np.float32)
@@ -106,8 +113,8 @@ def test_layer(N, d, F, E, k, act, empty):
 
 
 @pytest.mark.parametrize("rows,d_in,d_out,bias,dtype", [
-    (6400, 128, 64, True, "f32"), (1637, 131, 257, False, "f32"),   # split product
-    (6399, 127, 65, True, "f32"), (1, 1, 1, True, "f32"), (33, 300, 5, False, "f32"),  # fp32 MFMA product
+    (6400, 128, 64, True, "f32"), (1637, 131, 257, False, "f32"), (6399, 127, 65, True, "f32"),  # split product
+    (6399, 128, 64, True, "f32"), (1, 1, 1, True, "f32"), (33, 300, 5, False, "f32"),  # fp32 MFMA product
     (200, 9, 40, True, "bf16"), (17, 128, 33, False, "bf16"), (0, 16, 8, True, "f32")])
 def test_clifford_linear_module(rows, d_in, d_out, bias, dtype):
     """The module on each of its paths, from a strided and from a misaligned input."""
@@ -124,6 +131,7 @@ def test_clifford_linear_module(rows, d_in, d_out, bias, dtype):
         if bias:
             lin.bias.copy_(torch.from_numpy(b))
     say(f"CliffordLinear {rows} x {d_in} -> {d_out} {dtype}")
+    assert _split_product(rows, d_in, d_out) == (rows * d_out >= 100 * 64 * 64 and d_in >= 32)
     shifted = torch.empty(rows * d_in * 8 + 1, dtype=dt, device="cuda")[1:].view(rows, d_in, 8)
     strided = torch.empty((rows, 2 * d_in, 8), dtype=dt, device="cuda")[:, ::2]
     shifted.copy_(x)

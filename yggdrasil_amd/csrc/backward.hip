@@ -403,10 +403,10 @@ __device__ __forceinline__ void store_db(float* __restrict__ dst, const float* t
 }
 
 // grid (chunks bound, ceil(d_out / T), ceil(d_in / T)), 256 threads: RS = 1, T = 64, a wave per
-// 32 x 32 quadrant; RS = 4, T = 32, the four waves take every fourth block of rows of one
-// 32 x 32 tile and add their sums in wave order through LDS.  RS = 4 serves the grids that
+// 32 x 32 quadrant; RS = 4, T = 32, the four waves take a quarter of the rows of one 32 x 32 tile
+// each and add their sums through LDS, (0 + 2) + (1 + 3).  RS = 4 serves the grids that
 // would leave CUs idle: a row is a chain of 16 MFMAs of 64 cycles, 0.5 us, so an expert's 64
-// rows took 31 us in one wave (512 rows over 8 experts, skewed, 64 x 256: 42 us each with
+// rows took 31 us in one wave (512 rows over 8 experts, skewed, 64 x 256: 36-42 us each with
 // the longest expert's chain, where the vector-ALU kernel on 32 x 32 tiles took 112).
 // part: (chunks, d_out, d_in, 8) Pauli sums [a][c][re, im]; dbpart: (chunks, d_out, 8)
 // Pauli-row sums [b][re, im][a] of D, or NULL.

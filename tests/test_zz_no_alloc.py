@@ -66,6 +66,10 @@ CASES = [
     ("fp32 Pauli, grade-energy router", torch.float32, "pauli_f32", 300, 33, 16, 32, 6, 2, "energy", False),
     ("fp32 Pauli, routed in the up product", torch.float32, "pauli_f32", 200, 37, 32, 64, 8, 2, "logits", True),
     ("bf16 L(w) blocks", torch.bfloat16, "bf16", 200, 40, 16, 32, 4, 3, "logits", False),
+    # sizes near the scratch's limit: the same products as with a workspace, whatever they need
+    ("int8, more than a decode batch", torch.bfloat16, "int8", 2000, 700, 128, 512, 32, 2, "logits", True),
+    ("fp32 Pauli, split products", torch.float32, "pauli_f32", 2000, 300, 128, 512, 16, 1, "logits", True),
+    ("bf16 Pauli, few rows", torch.bfloat16, "pauli", 640, 3, 128, 512, 32, 2, "energy", False),
 ]
 
 

@@ -233,7 +233,7 @@ def test_layer_with_non_finite_rows(k):
     """Tokens with a NaN or an infinity: their rows are not finite, every other row is as without them."""
     import yggdrasil_amd
 
-    N, d, F, E = 3000, 100, 130, 3
+    N, d, F, E = 3000, 129, 130, 3
     _split(N, d, F, E, k)
     torch.manual_seed(k)
     layer = yggdrasil_amd.CliffordMoELayer(

@@ -191,13 +191,14 @@ int launch_split(const float* x, int x_rows, const int32_t* gather, int P_max, c
 bool pauli_split_pays(long long P, int d_in, int d_out) { return d_in >= 32 && P * d_out >= 100LL * 64 * 64; }
 
 // A layer's two products together, whose smaller one may fill less (layer calls, us, split / fp32 MFMA: d =
-// 128, F = 512, E = 32: 1024 rows 250 / 191, 2048 277 / 327, 8192 525 / 940; d = 64, F = 256, E = 8: 2048 rows
-// 143 / 99, 4096 155 / 169, 8192 187 / 274; d = 64, F = 256, E = 32: 2048 141 / 107, 4096 156 / 177; d = 100, F = 300,
-// E = 12: 1024 171 / 115, 2048 172 / 190, 4096 195 / 300; d = F = 128, E = 64: 1024 83 / 81, 2048 118 / 132; d =
-// 256, F = 1024, E = 64: 1024 453 / 701; d = 32, F = 64, E = 8: 8192 68 / 63).
+// 128, F = 512, E = 32: 1024 rows 250 / 191, 2048 277 / 327, 8192 525 / 940; d = F = 128, E = 64: 1024 83 / 81,
+// 2048 118 / 132; d = 256, F = 1024, E = 64: 1024 453 / 701).  Layers narrower than 128 keep the fp32 units and
+// with them their outputs bit for bit, though 8192 rows of d = 64, F = 256, E = 8 take 274 us there and 187 here:
+// through the sigmoid's gate c / |c|, whose derivative has no bound, any other order of the
+// sums moves their gradients by up to 1.2e-5.
 bool pauli_split_layer_pays(long long P, int E, int d, int F) {
   const int m = std::min(d, F);
-  return m >= 64 && P * m >= 60LL * 64 * 64 && P >= 16LL * E;
+  return m >= 128 && P * m >= 60LL * 64 * 64 && P >= 16LL * E;
 }
 
 bool pauli_split_fits(int E, long long x_rows, bool gathered, int d_in, int d_out) {

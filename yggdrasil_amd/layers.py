@@ -163,21 +163,19 @@ class CliffordMoELayer(nn.Module):
     def prepare(self):
         """Build the device weight layouts (done lazily; redone when parameters change)."""
         fmt = self.cfg.weight_format
-        E, d, F = self.cfg.n_experts, self.cfg.d_model, self.cfg.d_ff
-        for name, want in (("w_up", (E, F, d, 8)), ("b_up", (E, F, 8)), ("w_down", (E, d, F, 8)), ("b_down", (E, d, 8))):
-            if tuple(getattr(self, name).shape) != want:  # (replaced or parametrized: the kernels take the shapes of cfg)
-                raise ValueError(f"{name} must be {want}, got {tuple(getattr(self, name).shape)}")
         head = None
         if self.head_weight is not None:
             head = self.head_weight.detach().float().contiguous()
-        self._prepared = dict(
-            key=self._param_versions(),
-            w_up=ops.prepare_weights(self.w_up.detach(), fmt),
-            w_down=ops.prepare_weights(self.w_down.detach(), fmt),
-            b_up=ops.prepare_bias(self.b_up.detach()),
-            b_down=ops.prepare_bias(self.b_down.detach()),
-            head=head,
-        )
+        w_up, w_down = ops.prepare_weights(self.w_up.detach(), fmt), ops.prepare_weights(self.w_down.detach(), fmt)
+        b_up, b_down = ops.prepare_bias(self.b_up.detach()), ops.prepare_bias(self.b_down.detach())
+        # replaced or parametrized: the layer's kernels take the shapes of cfg
+        E, d, F = self.cfg.n_experts, self.cfg.d_model, self.cfg.d_ff
+        for name, got, want in (("w_up", (w_up.E, w_up.d_out, w_up.d_in), (E, F, d)), ("b_up", b_up.shape, (E, F, 8)),
+                                ("w_down", (w_down.E, w_down.d_out, w_down.d_in), (E, d, F)),
+                                ("b_down", b_down.shape, (E, d, 8))):
+            if got != want:
+                raise ValueError(f"{name} must be of shape {want}, got {tuple(got)}")
+        self._prepared = dict(key=self._param_versions(), w_up=w_up, w_down=w_down, b_up=b_up, b_down=b_down, head=head)
         return self._prepared
 
     def _get_prepared(self):

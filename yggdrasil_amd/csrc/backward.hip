@@ -120,29 +120,22 @@ __global__ __launch_bounds__(256) void act_backward_kernel(const float* __restri
 // epilogues apply), for the backward's recompute of h from h before the activation.
 template <int ACT>
 __global__ __launch_bounds__(256) void act_forward_kernel(const float* __restrict__ h, size_t n_mv,
-                                                          float* __restrict__ out, float* __restrict__ out_pauli) {
+                                                          float* __restrict__ out_pauli) {
   const size_t n = (size_t)blockIdx.x * 256 + threadIdx.x;
   if (n >= n_mv) return;
   const float4* hp = reinterpret_cast<const float4*>(h + n * 8);
   const float4 h0 = hp[0], h1 = hp[1];
   float y[8] = {h0.x, h0.y, h0.z, h0.w, h1.x, h1.y, h1.z, h1.w};
   activate_blade<ACT>(y);
-  if (out != nullptr) {
-    float4* op = reinterpret_cast<float4*>(out + n * 8);
-    op[0] = make_float4(y[0], y[1], y[2], y[3]);
-    op[1] = make_float4(y[4], y[5], y[6], y[7]);
-  }
-  if (out_pauli != nullptr) store_pauli_f32(out_pauli + n * 8, y);
+  store_pauli_f32(out_pauli + n * 8, y);
 }
 
 // ---- combine backward: dy[slot] = w dout_t; dw[t, s] = <dout_t, y[slot]> ----------
-// One wave per token, a multivector per lane; dy goes out in blade order and/or as
-// fp32 Pauli rows (whichever is not NULL).
+// One wave per token, a multivector per lane; dy goes out as fp32 Pauli rows.
 __global__ __launch_bounds__(256) void combine_backward_kernel(const float* __restrict__ dout,
                                                                const float* __restrict__ y_sorted, int N, int k,
                                                                int d, const float* __restrict__ topk_w,
                                                                const int32_t* __restrict__ slot_pos,
-                                                               float* __restrict__ dy_sorted,
                                                                float* __restrict__ dy_pauli,
                                                                float* __restrict__ dtopk_w) {
   const int lane = threadIdx.x & 63;
@@ -161,12 +154,7 @@ __global__ __launch_bounds__(256) void combine_backward_kernel(const float* __re
 #pragma unroll
       for (int c = 0; c < 8; ++c) o[c] = w * gv[c];
       const size_t mv = row * d + i;
-      if (dy_sorted) {
-        float4* q = reinterpret_cast<float4*>(dy_sorted + mv * 8);
-        q[0] = make_float4(o[0], o[1], o[2], o[3]);
-        q[1] = make_float4(o[4], o[5], o[6], o[7]);
-      }
-      if (dy_pauli) store_pauli_f32(dy_pauli + mv * 8, o);
+      store_pauli_f32(dy_pauli + mv * 8, o);
       if (y_sorted) {
         const float4* yp = reinterpret_cast<const float4*>(y_sorted + mv * 8);
         const float4 y0 = yp[0], y1 = yp[1];
@@ -865,10 +853,10 @@ int activation_backward(const float* h, const float* g, size_t n_mv, int act, fl
   return check_launch("activation backward");
 }
 
-int activation_forward(const float* h, size_t n_mv, int act, float* out, float* out_pauli, hipStream_t stream) {
+int activation_forward(const float* h, size_t n_mv, int act, float* out_pauli, hipStream_t stream) {
   if (n_mv == 0) return 0;
   const dim3 grid((unsigned)((n_mv + 255) / 256));
-#define YGG_AF(A) hipLaunchKernelGGL(act_forward_kernel<A>, grid, dim3(256), 0, stream, h, n_mv, out, out_pauli)
+#define YGG_AF(A) hipLaunchKernelGGL(act_forward_kernel<A>, grid, dim3(256), 0, stream, h, n_mv, out_pauli)
   switch (act) {
     case kActNone: YGG_AF(kActNone); break;
     case kActGelu: YGG_AF(kActGelu); break;
@@ -892,10 +880,10 @@ int fill_zero_f32(float* p, size_t n, hipStream_t stream) {
 }
 
 int combine_backward(const float* dout, const float* y_sorted, int N, int k, int d, const float* topk_w,
-                     const int32_t* slot_pos, float* dy_sorted, float* dy_pauli, float* dtopk_w, hipStream_t stream) {
+                     const int32_t* slot_pos, float* dy_pauli, float* dtopk_w, hipStream_t stream) {
   if (N == 0) return 0;
   hipLaunchKernelGGL(combine_backward_kernel, dim3((N + 3) / 4), dim3(256), 0, stream, dout, y_sorted, N, k, d, topk_w,
-                     slot_pos, dy_sorted, dy_pauli, dtopk_w);
+                     slot_pos, dy_pauli, dtopk_w);
   return check_launch("combine backward");
 }
 

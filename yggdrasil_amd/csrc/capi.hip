@@ -519,11 +519,11 @@ YGG_API int ygg_moe_backward(const float* x, int N, int d, int F, int E, int k, 
   void* rws = take();
   float* xp = static_cast<float*>(take());
   float* h_pre = static_cast<float*>(take());
-  float* h = static_cast<float*>(take());
+  take();  // (h in blade order, which no kernel writes any more: the workspace's layout is kept)
   float* fp = static_cast<float*>(take());  // Pauli rows of h, then of dh_pre
   float* dh = static_cast<float*>(take());  // dh, then dh_pre in place
   float* y = static_cast<float*>(take());   // y, then dx rows
-  take();  // (a region of dy's size: the workspace's layout is kept)
+  take();  // (dy in blade order, likewise)
   float* dp = static_cast<float*>(take());  // Pauli rows of dy
   void* wg = take();                        // weight-gradient partial sums
 
@@ -564,10 +564,10 @@ YGG_API int ygg_moe_backward(const float* x, int N, int d, int F, int E, int k, 
     hp_in = h_pre;
   }
   // h as Pauli rows for the down product and its weight gradient
-  if (activation_forward(hp_in, P * F, act, nullptr, fp, stream)) return -1;
+  if (activation_forward(hp_in, P * F, act, fp, stream)) return -1;
   if (dtopk_w && product(fp, nullptr, w_down, b_down, F, d, y)) return -1;
   // combine backward -> dy; down backward -> dh, dW_down, db_down
-  if (combine_backward(dout, dtopk_w ? y : nullptr, N, k, d, tw, slot_pos, nullptr, dp, dtopk_w, stream)) return -1;
+  if (combine_backward(dout, dtopk_w ? y : nullptr, N, k, d, tw, slot_pos, dp, dtopk_w, stream)) return -1;
   if (product(dp, nullptr, w_down_adj, nullptr, d, F, dh)) return -1;
   if (weight_grad(dp, fp, nullptr, F, d, dw_down, db_down)) return -1;
   // activation backward -> Pauli rows of dh before the activation; up backward -> dx rows, dW_up, db_up

@@ -545,13 +545,20 @@ def run_train_config(torch, ops, name, c, steps, warmup):
                          router_bias=rb, workspace=ws_b, routing_grad=False, h_pre=h_pre)
 
     ms = time_fn(torch, step, steps, warmup)
+    P = N * k
+    flops_proj = 128.0 * d * F * P
+    res = dict(workload=name, N=N, d=d, E=E, k=k, F=F, dtype="f32", weights=c["fmt"], ms_per_step=ms,
+               tokens_per_s=N / (ms * 1e-3), step_tflops=6 * flops_proj / (ms * 1e-3) / 1e12)
+    if ops.lib().ygg_f32_layer_split(N, d, F, E, k):
+        # products (and weight gradients, from some 320 of their workgroups on) on the bf16 units, six part
+        # products for each of the Pauli form's multiply-adds; the latter have no entry of their own to time
+        return dict(res, products="three bf16 parts a value on the bf16 MFMA units",
+                    step_mfma_tflops=18 * flops_proj / (ms * 1e-3) / 1e12)
     # the weight gradients alone: up (rows of x through perm, F outputs) and down (h rows, d outputs)
     r = ops.route(logits if logits is not None else ops.router_energy_logits(x, rw, rb), k)
-    P = N * k
     dh = torch.randn(P, F, 8, generator=g, device="cuda")
     dy = torch.randn(P, d, 8, generator=g, device="cuda")
     h = torch.randn(P, F, 8, generator=g, device="cuda")
-    wg_kind = "mfma"  # the fp32 MFMA kernel on Pauli rows (large layers' backward uses its fp16-split form)
     dhp, xp = ops.pauli_rows_from_blade_f32(dh), ops.pauli_rows_from_blade_f32(x.reshape(N, d, 8))
     dyp, hp = ops.pauli_rows_from_blade_f32(dy), ops.pauli_rows_from_blade_f32(h)
     ws_w = torch.empty(ops.lib().ygg_grouped_weight_grad_pauli_f32_workspace_bytes(P, E, d, F), device="cuda",
@@ -560,11 +567,8 @@ def run_train_config(torch, ops, name, c, steps, warmup):
                                                                     workspace=ws_w), steps, warmup)
     ms_wg_down = time_fn(torch, lambda: ops.grouped_weight_grad_pauli(dyp, hp, r.offsets, E, workspace=ws_w),
                          steps, warmup)
-    flops_proj = 128.0 * d * F * P
-    return dict(workload=name, N=N, d=d, E=E, k=k, F=F, dtype="f32", weights=c["fmt"],
-                ms_per_step=ms, tokens_per_s=N / (ms * 1e-3), weight_grad_kernel=wg_kind,
+    return dict(res, products="fp32 MFMA units", weight_grad_kernel="mfma",
                 kernels_ms=dict(weight_grad_up=ms_wg_up, weight_grad_down=ms_wg_down),
-                step_tflops=6 * flops_proj / (ms * 1e-3) / 1e12,
                 # the reference's arithmetic (64 multiply-adds per multivector pair): an effective rate
                 weight_grad_dense_equiv_tflops=2 * flops_proj / ((ms_wg_up + ms_wg_down) * 1e-3) / 1e12,
                 # the MFMA work issued (the Pauli form's 32 multiply-adds per pair) against the fp32 peak
@@ -576,10 +580,10 @@ def run_gm(torch, ops, name, c, steps, warmup):
     g = torch.Generator(device="cuda")
     g.manual_seed(SEEDS[name])
     N, d, F = c["N"], c["d"], c["F"]
-    res = dict(workload=name, dtype="f32", kernels=["pauli_f32_prep_kernel", "pauli_f32_rows_t_kernel",
-                                                    "pauli_f32_kernel"],
-               frac_basis="MFMA work issued (the Pauli form's 32 multiply-adds per multivector pair) against "
-                          "the fp32 MFMA peak; dense_equiv_tflops counts the reference's 64 (an effective rate)")
+    res = dict(workload=name, dtype="f32",
+               frac_basis="MFMA work issued (the Pauli form's 32 multiply-adds per multivector pair, six part "
+                          "products each on the bf16 units) against the peak of the units it runs on; "
+                          "dense_equiv_tflops counts the reference's 64 (an effective rate)")
     for tag, M, K in (("up", F, d), ("down", d, F)):
         a = torch.randn(M, K, 8, generator=g, device="cuda") / (8.0 * K) ** 0.5
         b = torch.randn(K, N, 8, generator=g, device="cuda")
@@ -587,9 +591,12 @@ def run_gm(torch, ops, name, c, steps, warmup):
         out = torch.empty((M, N, 8), device="cuda")
         ms = time_fn(torch, lambda: ops.geom_matmul(a, b, workspace=ws, out=out), steps, warmup)
         flops = 128.0 * M * K * N  # the reference's arithmetic: 64 multiply-adds per multivector pair
+        split = bool(ops.lib().ygg_f32_product_split(N, K, M))
+        issued = flops / 2 * (6 if split else 1) / (ms * 1e-3)
         res[tag] = dict(M=M, K=K, N=N, ms=ms, tflops=flops / 2 / (ms * 1e-3) / 1e12,
-                        # against the fp32 units' peak: products on the fp16 units can pass 1
-                        mfma_frac_f32=flops / 2 / (ms * 1e-3) / PEAK_F32,
+                        kernels=["pauli_f32_prep_kernel", "pauli_f32_rows_t_kernel",
+                                 "pauli_split_kernel" if split else "pauli_f32_kernel"],
+                        mfma_frac=issued / (PEAK_BF16 if split else PEAK_F32), mfma_units="bf16" if split else "fp32",
                         dense_equiv_tflops=flops / (ms * 1e-3) / 1e12)
         del a, b, ws, out
     return res

@@ -1,5 +1,6 @@
-"""Cases where the size of one value must not cost another its bits: inputs that cancel, rows and channels
-of very different size, gradients of small rows beside large ones."""
+"""Cases where the size of one value must not cost another its bits (inputs that cancel, rows and channels of
+very different size, gradients of small rows beside large ones) or the batch a row its bits (few rows against
+the tiles); scratch, shapes and alignment that a path must take or refuse as every other path does."""
 
 import numpy as np
 import pytest
